@@ -123,6 +123,32 @@ enum MatType { MT_F64 = 0, MT_F32 = 1, MT_BF16 = 2 };
 /* most distinct column offsets of a stencil-pattern operator */
 constexpr int PAT_MAX = 8;
 
+/* row classes (kernels_class.hip): most distinct row forms, longest row */
+constexpr int CLS_MAX = 256;
+constexpr int CLS_ROW = 8;
+
+/* the distinct row forms of an operator, a form being a row's (column - row,
+   value) pairs in storage order: code[r] is row r's class, the tables hold
+   entry k of class c at [k n + c] */
+struct RowClasses {
+    int n = 0;                   /* classes (0: not kept) */
+    int row = 0;                 /* longest row */
+    bool analysed = false;
+    /* a constant stencil (forms that differ only in the entries left out):
+       its k offsets, ascending, and their values; code[r] is then the mask
+       of row r's entries */
+    int k = 0;
+    int off[CLS_ROW] = {};
+    double val[CLS_ROW] = {};
+    DBuf<unsigned char> code;    /* padded to whole 256-row blocks */
+    DBuf<int> idx;               /* n lengths, then row x n offsets */
+    /* row x n values, then n diagonals and n sums of magnitudes; in FP32 and
+       with bfloat16 values where the operator has such copies */
+    DBuf<double> v64;
+    DBuf<float> v32, v16;
+    void make_lowp(hipStream_t s, bool bf16);
+};
+
 /* CSR, 0-based, int32 indices, FP64 values; columns ascending with a diagonal
    entry in every row (the layout of src/matrix/CSR.h:13-28). */
 struct DevCsr {
@@ -150,9 +176,12 @@ struct DevCsr {
     int pk = 0;
     int poff[PAT_MAX] = {};
     bool cols_analysed = false; /* narrow copy and pattern considered */
-    /* the narrowest column form the row kernels may read: 2 the pattern,
-       1 the 16-bit offsets, 0 the int32 columns (bcmg_csr_set_columns) */
-    int col_mode = 2;
+    RowClasses cls;
+    /* the narrowest form the row kernels may read: 3 the row classes, 2 the
+       pattern, 1 the 16-bit offsets, 0 the int32 columns
+       (bcmg_csr_set_columns chooses among the last three) */
+    int col_mode = 3;
+    bool use_classes() const { return cls.n > 0 && col_mode >= 3; }
     bool use_pattern() const { return pk > 0 && col_mode >= 2; }
     bool use_narrow() const { return narrow && col_mode >= 1; }
     int group = 8;          /* lanes per row of the row-group kernels */
@@ -174,6 +203,10 @@ void resolve_tiles(Ctx &c, const std::vector<DevCsr *> &mats);
    pattern when those offsets take at most PAT_MAX values (one round trip
    for the lot) */
 void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats);
+/* find the row classes of every square operator in mats that has rows of at
+   most CLS_ROW entries (their tiles resolved) and at most CLS_MAX forms (one
+   round trip for the lot) */
+void make_classes(Ctx &c, const std::vector<DevCsr *> &mats);
 
 /* ------------------------------------------------------------- context */
 
@@ -183,8 +216,9 @@ struct Ctx {
     hipStream_t stream = nullptr;
     bool own_stream = true;     /* false: the caller's stream, not destroyed here */
     /* pinned host scalars used for the few device->host reads */
+    static constexpr size_t H_INTS = 16384;
     double *h_scalars = nullptr;
-    int *h_ints = nullptr;
+    int *h_ints = nullptr;      /* H_INTS of them */
     /* reduction scratch */
     DBuf<double> red;           /* partial sums (per block) + results */
     DBuf<int> iscratch;
@@ -334,13 +368,32 @@ inline const VT *pvals(const Level &lv)
    (the first sweep's iterate f / d is formed at each gather and for the row
    itself; x is not read) */
 enum RowOp { OP_SPMV = 0, OP_RESID = 1, OP_JACOBI = 2, OP_JACOBI_Z = 3 };
+/* where a sweep's divisor comes from: the array d, or d is the operator's
+   diagonal / its rows' sums of magnitudes, which an operator with row
+   classes holds per class (same values; d is then not read) */
+enum DivSource { DIV_ARRAY = 0, DIV_DIAG = 1, DIV_L1 = 2 };
+inline DivSource div_source(int relax_type) { return relax_type == 4 ? DIV_L1 : DIV_DIAG; }
 template <typename VT>
 void launch_rows(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const VT *x, const VT *f,
-                 const VT *d, VT *y);
+                 const VT *d, VT *y, DivSource div = DIV_ARRAY);
+/* kernels_class.hip: whether A's values of type mt are read as row classes
+   by VT kernels, and those kernels */
+template <typename VT>
+bool class_ok(const DevCsr &A, MatType mt);
+template <typename VT>
+void launch_rows_class(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const VT *x,
+                       const VT *f, const VT *d, VT *y, DivSource div);
+template <typename VT>
+void launch_jacobi_zero_class(hipStream_t s, const DevCsr &A, MatType mt, const VT *f, VT *y,
+                              DivSource div);
+void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const double *z, double *t,
+                            const double *r, const double *to, double *part);
 void launch_rows(hipStream_t s, const DevCsr &A, RowOp op, const double *x, const double *f,
                  const double *d, double *y);
+/* y = f / d: the first sweep on A from zero */
 template <typename VT>
-void launch_jacobi_zero(hipStream_t s, int n, const VT *f, const VT *d, VT *y);
+void launch_jacobi_zero(hipStream_t s, const DevCsr &A, MatType mt, const VT *f, const VT *d,
+                        VT *y, DivSource div);
 template <typename VT>
 void launch_prolong(hipStream_t s, int n, const int *agg, const VT *p, const VT *xc, VT *x);
 /* y = x + P x_c with y another buffer than x */
@@ -399,6 +452,9 @@ size_t red_size_for(int n);
    column j at j * cs + i * rs), skipped when act[j] == 0 */
 template <typename VT>
 bool relax_block_ok(const DevCsr &A);
+/* levels of at most this many rows fold neighbouring steps into one launch
+   (where a launch costs more than the work) */
+constexpr int SMALL_LEVEL_ROWS = 65536;
 /* whether the first two sweeps from zero run as one OP_JACOBI_Z pass on A */
 template <typename VT>
 bool fuse_zero_sweeps(const DevCsr &A, MatType mt);

@@ -246,7 +246,7 @@ int ctx_create(int device, hipStream_t ext, bcmg_ctx *out)
             BCMG_HIP(hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking));
         }
         BCMG_HIP(hipHostMalloc((void **)&ctx->c.h_scalars, 64 * sizeof(double), hipHostMallocDefault));
-        BCMG_HIP(hipHostMalloc((void **)&ctx->c.h_ints, 256 * sizeof(int), hipHostMallocDefault));
+        BCMG_HIP(hipHostMalloc((void **)&ctx->c.h_ints, Ctx::H_INTS * sizeof(int), hipHostMallocDefault));
         ctx->c.ensure_reductions(1);
         BCMG_HIP(hipStreamSynchronize(ctx->c.stream));
     } catch (...) {

@@ -293,6 +293,7 @@ void adaptive_coarsening(Ctx &c, const bcmg_params &p, BuildState &bs, DevCsr &A
     pending.clear();
     for (int i = 1; i < level; i++) pending.push_back(&H.L[i].Aown);
     make_narrow(c, pending);
+    make_classes(c, pending);
     double cx = 0, cw = 0;
     for (int i = 0; i < level; i++) {
         cx += H.L[i].mat().nnz;
@@ -364,7 +365,7 @@ void relax_level(Ctx &c, const Level &lv, MatType mt, int type, int sweeps, cons
                the first iterate f / d is formed where the second reads it) */
             k++;
             if (final_out && k == sweeps - 1 && s.x != final_out) out = final_out;
-            launch_rows<VT>(c.stream, A, mt, OP_JACOBI_Z, nullptr, f, d, out);
+            launch_rows<VT>(c.stream, A, mt, OP_JACOBI_Z, nullptr, f, d, out, div_source(type));
             s.x2 = s.x;
             s.x = out;
             s.zero = false;
@@ -372,14 +373,14 @@ void relax_level(Ctx &c, const Level &lv, MatType mt, int type, int sweeps, cons
         }
         if (final_out && k == sweeps - 1 && s.x != final_out) out = final_out;
         if (s.zero) {
-            launch_jacobi_zero<VT>(c.stream, A.n, f, d, out);
+            launch_jacobi_zero<VT>(c.stream, A, mt, f, d, out, div_source(type));
         } else {
             if (timing && !timed) {
                 hipEvent_t e0 = c.next_event();
                 e1 = c.next_event();
                 BCMG_HIP(hipEventRecord(e0, c.stream));
             }
-            launch_rows<VT>(c.stream, A, mt, OP_JACOBI, s.x, f, d, out);
+            launch_rows<VT>(c.stream, A, mt, OP_JACOBI, s.x, f, d, out, div_source(type));
             timed++;
         }
         s.x2 = s.x;
@@ -391,10 +392,6 @@ void relax_level(Ctx &c, const Level &lv, MatType mt, int type, int sweeps, cons
         c.ev_launches.push_back(timed);
     }
 }
-
-/* levels of at most this many rows restrict their residual in the launch
-   that forms it (where a launch costs more than the work) */
-constexpr int SMALL_LEVEL_ROWS = 65536;
 
 /* R's values in the cycle's type */
 template <typename VT>

@@ -1,0 +1,991 @@
+/*
+ * kernels_class.hip - row classes: operators whose rows take few distinct
+ * forms are read as one byte per row.
+ *
+ * A row's form is its list of (column - row, value) pairs in storage order.
+ * A constant-coefficient stencil has one form per combination of missing
+ * neighbours (27 for the 3D 7-point stencil, 9 for the 2D 5-point one), and
+ * where the aggregates repeat, so have its Galerkin coarse levels. An
+ * operator of at most CLS_MAX forms of at most CLS_ROW entries keeps, beside
+ * its CSR arrays, the class of each row (one byte) and the forms (a few KB);
+ * the row kernels stage the forms in LDS and stream the codes, so a sweep
+ * moves 25 bytes per row (x, f, the result and the code) instead of 89 (the
+ * 7-point stencil with one mask byte per row) or 132 (int32 columns). The
+ * products, their order and the divisors are those of the CSR row, so every
+ * result has the same bits.
+ *
+ * Where the forms differ only in which entries they have (constant
+ * coefficients, missing neighbours eliminated: one value per offset, at most
+ * CLS_ROW offsets) the byte is the mask of the entries present, and offsets
+ * and values are kernel arguments: no table, no barrier, and the gathers
+ * do not wait for the byte.
+ *
+ * Measured on level 0 of 3D Poisson 160^3 (4.1 M rows) and 2D 2048^2, FP64:
+ * product 56.7 and 57.7 us with the one-byte mask and streamed values, 24.0
+ * and 20.0 us from the table of forms, 13.5 and 12.1 us as a constant
+ * stencil; the L1 sweep 63.3 -> 18.1 us (5.7 TB/s of its 102 MB; FP32
+ * 30.9 -> 12.8 us). What bounds them now is the vectors' traffic through
+ * L2 and the last-level cache.
+ */
+#include "kernels_common.h"
+
+#include <algorithm>
+#include <cmath>
+#include <cstring>
+#include <utility>
+
+namespace bcmg {
+
+namespace {
+
+constexpr int CLS_SLOTS = 1024;   /* hash slots while the forms are collected */
+/* a block of 256 rows with more forms than this raises the overflow flag by
+   itself: an operator without repeated rows is told by its first blocks */
+constexpr int CLS_BLOCK_MAX = 128;
+constexpr unsigned long long HASH_EMPTY = 0ull;
+
+__device__ __forceinline__ unsigned long long mix64(unsigned long long z)
+{
+    z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+    z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+    return z ^ (z >> 31);
+}
+
+/* hash of row r's form (never HASH_EMPTY) */
+__device__ __forceinline__ unsigned long long row_hash(int r, const int *__restrict__ rp,
+                                                       const int *__restrict__ ci,
+                                                       const double *__restrict__ av)
+{
+    const int e0 = rp[r], e1 = rp[r + 1];
+    unsigned long long h = 0x9E3779B97F4A7C15ull * (unsigned)(e1 - e0 + 1);
+    for (int e = e0; e < e1; e++) {
+        h = mix64(h ^ (unsigned)(ci[e] - r));
+        h = mix64(h + (unsigned long long)__double_as_longlong(av[e]));
+    }
+    return h | 1ull;
+}
+
+/* work area of one operator's analysis (device) */
+struct ClassWork {
+    unsigned long long hash[CLS_SLOTS];
+    int rep[CLS_SLOTS];       /* smallest row with that hash */
+    int cls[CLS_SLOTS];       /* class of the slot, once numbered */
+    int count, over, ncls, pad;
+    /* the tables, entry k of class c at [k ncls + c]: lengths, then offsets;
+       values, then the diagonals and the sums of magnitudes (the smoother
+       divisors) */
+    int idx[(CLS_ROW + 1) * CLS_MAX];
+    double tv[(CLS_ROW + 2) * CLS_MAX];
+};
+
+__global__ __launch_bounds__(BS) void k_class_clear(ClassWork *w)
+{
+    for (int q = threadIdx.x; q < CLS_SLOTS; q += BS) {
+        w->hash[q] = HASH_EMPTY;
+        w->rep[q] = 0x7fffffff;
+        w->cls[q] = -1;
+    }
+    if (threadIdx.x == 0) w->count = w->over = w->ncls = 0;
+}
+
+/* step 1: the distinct row hashes of a 256-row block (an LDS table) go into
+   the operator's table with the smallest row that has them; more than
+   CLS_BLOCK_MAX in a block, or CLS_MAX in all, raises `over`, which later
+   blocks read first */
+__global__ __launch_bounds__(BS) void k_class_collect(int n, const int *__restrict__ rp,
+                                                      const int *__restrict__ ci,
+                                                      const double *__restrict__ av,
+                                                      ClassWork *w)
+{
+    constexpr int LS = 2 * BS;
+    __shared__ unsigned long long lh[LS];
+    __shared__ int lr[LS];
+    __shared__ int lcount, skip;
+    const int t = threadIdx.x;
+    for (int q = t; q < LS; q += BS) {
+        lh[q] = HASH_EMPTY;
+        lr[q] = 0x7fffffff;
+    }
+    if (t == 0) {
+        lcount = 0;
+        skip = __hip_atomic_load(&w->over, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (skip) return;
+    const int r = blockIdx.x * BS + t;
+    if (r < n) {
+        const unsigned long long h = row_hash(r, rp, ci, av);
+        /* LS >= 2 BS slots for at most BS hashes: the probe ends */
+        int s = (int)(h >> 40) & (LS - 1);
+        for (;;) {
+            const unsigned long long prev = atomicCAS(&lh[s], HASH_EMPTY, h);
+            if (prev == HASH_EMPTY) atomicAdd(&lcount, 1);
+            if (prev == HASH_EMPTY || prev == h) break;
+            s = (s + 1) & (LS - 1);
+        }
+        atomicMin(&lr[s], r);
+    }
+    __syncthreads();
+    if (lcount > CLS_BLOCK_MAX) {
+        if (t == 0) atomicOr(&w->over, 1);
+        return;
+    }
+    for (int q = t; q < LS; q += BS) {
+        const unsigned long long h = lh[q];
+        if (h == HASH_EMPTY) continue;
+        int s = (int)(h >> 20) & (CLS_SLOTS - 1);
+        for (int probe = 0;; probe++) {
+            if (probe == CLS_SLOTS) {
+                atomicOr(&w->over, 1);
+                break;
+            }
+            unsigned long long v =
+                __hip_atomic_load(&w->hash[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (v == HASH_EMPTY) {
+                v = atomicCAS(&w->hash[s], HASH_EMPTY, h);
+                if (v == HASH_EMPTY) {
+                    if (atomicAdd(&w->count, 1) >= CLS_MAX) atomicOr(&w->over, 1);
+                    v = h;
+                }
+            }
+            if (v == h) {
+                if (__hip_atomic_load(&w->rep[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >
+                    lr[q])
+                    atomicMin(&w->rep[s], lr[q]);
+                break;
+            }
+            s = (s + 1) & (CLS_SLOTS - 1);
+        }
+    }
+}
+
+/* step 2 (one block): number the forms by their smallest row and write the
+   tables (the divisors as k_diag and k_abs_rowsum form them) */
+__global__ __launch_bounds__(CLS_MAX) void k_class_tables(int crow, const int *__restrict__ rp,
+                                                          const int *__restrict__ ci,
+                                                          const double *__restrict__ av,
+                                                          ClassWork *w)
+{
+    __shared__ int slot[CLS_MAX], rep[CLS_MAX];
+    __shared__ int m;
+    const int t = threadIdx.x;
+    if (t == 0) m = 0;
+    __syncthreads();
+    if (w->over) return;
+    for (int q = t; q < CLS_SLOTS; q += CLS_MAX)
+        if (w->hash[q] != HASH_EMPTY) {
+            const int at = atomicAdd(&m, 1); /* at most CLS_MAX: over is clear */
+            slot[at] = q;
+            rep[at] = w->rep[q];
+        }
+    __syncthreads();
+    const int nc = m;
+    if (t == 0) w->ncls = nc;
+    if (t >= nc) return;
+    int c = 0;
+    for (int q = 0; q < nc; q++) c += rep[q] < rep[t] ? 1 : 0;
+    w->cls[slot[t]] = c;
+    const int r = rep[t], e0 = rp[r], len = rp[r + 1] - e0;
+    int *const idx = w->idx;
+    double *const tv = w->tv;
+    idx[c] = len;
+    double d = 0.0, s = 0.0;
+    for (int k = 0; k < crow; k++) {
+        const bool in = k < len;
+        const double v = in ? av[e0 + k] : 0.0;
+        const int o = in ? ci[e0 + k] - r : 0;
+        idx[(k + 1) * nc + c] = o;
+        tv[k * nc + c] = v;
+        if (in) {
+            if (o == 0) d = v;
+            s += fabs(v);
+        }
+    }
+    tv[crow * nc + c] = d;
+    tv[(crow + 1) * nc + c] = s;
+}
+
+/* step 3: each row's class, its form compared entry by entry with the
+   table's (a hash collision raises `over`); rows that pad the last block
+   get class 0 */
+__global__ __launch_bounds__(BS) void k_class_codes(int n, const int *__restrict__ rp,
+                                                    const int *__restrict__ ci,
+                                                    const double *__restrict__ av,
+                                                    ClassWork *w,
+                                                    unsigned char *__restrict__ code)
+{
+    const int *const idx = w->idx;
+    const double *const tv = w->tv;
+    const int r = blockIdx.x * BS + threadIdx.x;
+    if (r >= n) {
+        code[r] = 0;
+        return;
+    }
+    const int nc = w->ncls;
+    const unsigned long long h = row_hash(r, rp, ci, av);
+    int s = (int)(h >> 20) & (CLS_SLOTS - 1);
+    /* step 1 put h into the table and left empty slots: the probe ends */
+    while (w->hash[s] != h) s = (s + 1) & (CLS_SLOTS - 1);
+    const int c = w->cls[s];
+    const int e0 = rp[r], len = rp[r + 1] - e0;
+    bool same = idx[c] == len;
+    for (int k = 0; same && k < len; k++)
+        same = idx[(k + 1) * nc + c] == ci[e0 + k] - r &&
+               __double_as_longlong(tv[k * nc + c]) == __double_as_longlong(av[e0 + k]);
+    if (!same) atomicOr(&w->over, 1);
+    code[r] = (unsigned char)c;
+}
+
+/* the forms in FP32, or rounded to bfloat16 and widened; the divisors in FP32 */
+__global__ __launch_bounds__(BS) void k_class_lowp(int nv, int nall, const double *__restrict__ a,
+                                                   float *__restrict__ b, int bf16)
+{
+    const int i = blockIdx.x * BS + threadIdx.x;
+    if (i >= nall) return;
+    const float v = (float)a[i];
+    b[i] = (bf16 && i < nv) ? bf16_round(v) : v;
+}
+
+/* ---------------------------------------------------------- row kernels */
+
+/* the forms of an operator as the kernels take them */
+template <typename VT>
+struct ClassRef {
+    const unsigned char *code;
+    const int *idx;
+    const VT *tv;
+    int nc;      /* classes */
+    int crow;    /* longest row */
+};
+
+/* LDS: the values and one divisor row, then lengths and offsets */
+template <typename VT>
+inline size_t class_lds_bytes(int nc, int crow)
+{
+    return (size_t)nc * ((crow + 1) * sizeof(VT) + (crow + 1) * sizeof(int));
+}
+
+/* The forms into LDS: values [k nc + c] (k < crow), the divisor row at
+   k = crow (table row `drow`; not copied when negative), lengths and offsets
+   behind them. */
+template <typename VT>
+__device__ __forceinline__ void class_stage(const ClassRef<VT> &C, int drow, VT *&lv, int *&li)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_class[];
+    lv = reinterpret_cast<VT *>(smem_class);
+    li = reinterpret_cast<int *>(lv + (size_t)(C.crow + 1) * C.nc);
+    const int nv = C.crow * C.nc;
+#pragma unroll 1
+    for (int q = threadIdx.x; q < nv + C.nc; q += BS) {
+        li[q] = C.idx[q];
+        if (q < nv)
+            lv[q] = C.tv[q];
+        else if (drow >= 0)
+            lv[q] = C.tv[(size_t)drow * C.nc + (q - nv)];
+    }
+}
+
+/* Row r's sum from its form: all gathers go out at once (an absent entry
+   gathers the row's own element and adds nothing), the products are rounded
+   and added left to right from 0 in storage order (staged_row_sum's bits). */
+template <typename VT, int CR>
+__device__ __forceinline__ VT class_row_sum(int c, int nc, int crow, const VT *lv, const int *li,
+                                            const VT *__restrict__ x, int r)
+{
+    const int len = li[c];
+    VT g[CR], v[CR];
+    int j[CR];
+#pragma unroll
+    for (int k = 0; k < CR; k++) {
+        j[k] = r;
+        v[k] = 0;
+        if (k < crow) {
+            const int o = li[(k + 1) * nc + c];
+            v[k] = lv[k * nc + c];
+            j[k] = r + o;   /* the table holds offset 0 past the row's length */
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < CR; k++) g[k] = x[j[k]];
+    VT t = 0;
+#pragma unroll
+    for (int k = 0; k < CR; k++) t = k < len ? t + v[k] * g[k] : t;
+    return t;
+}
+
+template <typename VT, int OP, int CR, int RPT, bool DTAB>
+__global__ __launch_bounds__(BS) void k_rows_class(int n, ClassRef<VT> C, int drow,
+                                                   const VT *__restrict__ x,
+                                                   const VT *__restrict__ f,
+                                                   const VT *__restrict__ d, VT *__restrict__ y)
+{
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int r0 = b * (BS * RPT) + threadIdx.x;
+    int c[RPT];
+    VT fr[RPT], xr[RPT], dr[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int r = r0 + q * BS;
+        c[q] = 0;
+        fr[q] = xr[q] = 0;
+        dr[q] = 1;
+        if (r < n) {
+            c[q] = C.code[r];
+            if (OP != OP_SPMV) fr[q] = f[r];
+            if (OP == OP_JACOBI) xr[q] = x[r];
+            if (OP == OP_JACOBI && !DTAB) dr[q] = d[r];
+        }
+    }
+    VT *lv;
+    int *li;
+    class_stage<VT>(C, DTAB ? drow : -1, lv, li);
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int r = r0 + q * BS;
+        if (r >= n) return;
+        const VT t = class_row_sum<VT, CR>(c[q], C.nc, C.crow, lv, li, x, r);
+        if (DTAB) dr[q] = lv[C.crow * C.nc + c[q]];
+        if (OP == OP_SPMV)
+            y[r] = t;
+        else if (OP == OP_RESID)
+            y[r] = fr[q] - t;
+        else
+            y[r] = (fr[q] - t) / dr[q] + xr[q];
+    }
+}
+
+/* ------------------------------------------------------ constant stencils */
+
+/* offsets and values of the stencil, ascending (CSR order); the entries
+   past k are never in a mask */
+template <typename VT>
+struct StencilRef {
+    const unsigned char *mask;
+    int off[CLS_ROW];
+    VT v[CLS_ROW];
+    double a[CLS_ROW];   /* magnitudes in FP64: the L1 divisor */
+    VT diag;
+    int lo, hi;          /* smallest and largest offset */
+};
+
+/* Row r's entries g[k] summed under mask m (products rounded, added left to
+   right from 0), with DL1 also the row's sum of magnitudes as k_abs_rowsum
+   forms it. */
+template <typename VT, int K, bool DL1>
+__device__ __forceinline__ void stencil_sum(unsigned m, const StencilRef<VT> &S, const VT (&g)[K],
+                                            VT &t, VT &dl)
+{
+    t = 0;
+    double a = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        if ((m >> k) & 1u) {
+            t = t + S.v[k] * g[k];
+            if (DL1) a += S.a[k];
+        }
+    dl = (VT)a;
+}
+
+/* The gathers of W consecutive rows from r (W VT values are 16 bytes, or
+   W = 1). INNER: every r + off + W - 1 lies in [0, n), so the loads are
+   unconditional 16-byte ones (any alignment of VT); else each element is
+   loaded where its index is in range and its mask bit set. */
+template <typename VT, int K, int W, bool INNER>
+__device__ __forceinline__ void stencil_gather(const StencilRef<VT> &S, const VT *__restrict__ x,
+                                               int r, int n, const unsigned (&m)[W],
+                                               VT (&g)[W][K])
+{
+    if constexpr (INNER) {
+        typedef VT vec __attribute__((ext_vector_type(W == 1 ? 2 : W)));
+        typedef vec uvec __attribute__((aligned(sizeof(VT))));
+#pragma unroll
+        for (int k = 0; k < K; k++) {
+            if constexpr (W == 1) {
+                g[0][k] = x[r + S.off[k]];
+            } else {
+                const vec q = *reinterpret_cast<const uvec *>(x + r + S.off[k]);
+#pragma unroll
+                for (int w = 0; w < W; w++) g[w][k] = q[w];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int w = 0; w < W; w++)
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                g[w][k] = 0;
+                if (r + w < n && ((m[w] >> k) & 1u)) g[w][k] = x[r + w + S.off[k]];
+            }
+    }
+}
+
+/* Row operations on a constant stencil, W rows per thread. A block whose
+   gathers stay inside the vector whatever the masks issues every load at
+   once; the first and last blocks load under the masks. */
+template <typename VT, int OP, int K, int W, int DIV>
+__global__ __launch_bounds__(BS) void k_rows_stencil(int n, StencilRef<VT> S,
+                                                     const VT *__restrict__ x,
+                                                     const VT *__restrict__ f,
+                                                     const VT *__restrict__ d, VT *__restrict__ y)
+{
+    typedef VT vec __attribute__((ext_vector_type(W == 1 ? 2 : W)));
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int r0 = b * (BS * W);
+    const int r = r0 + threadIdx.x * W;
+    const bool inner = r0 + S.lo >= 0 && r0 + BS * W + S.hi <= n && r0 + BS * W <= n;
+    unsigned m[W];
+    VT g[W][K], fr[W], xr[W], dr[W];
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+        fr[w] = xr[w] = 0;
+        dr[w] = 1;
+    }
+    if (inner) {
+        if constexpr (W == 1) {
+            m[0] = S.mask[r];
+            stencil_gather<VT, K, W, true>(S, x, r, n, m, g);
+            if (OP != OP_SPMV) fr[0] = f[r];
+            if (OP == OP_JACOBI) xr[0] = x[r];
+            if (OP == OP_JACOBI && DIV == DIV_ARRAY) dr[0] = d[r];
+        } else {
+            const unsigned mm = W == 2 ? *reinterpret_cast<const unsigned short *>(S.mask + r)
+                                       : *reinterpret_cast<const unsigned *>(S.mask + r);
+            stencil_gather<VT, K, W, true>(S, x, r, n, m, g);
+            vec vf, vx, vd;
+            if (OP != OP_SPMV) vf = *reinterpret_cast<const vec *>(f + r);
+            if (OP == OP_JACOBI) vx = *reinterpret_cast<const vec *>(x + r);
+            if (OP == OP_JACOBI && DIV == DIV_ARRAY) vd = *reinterpret_cast<const vec *>(d + r);
+#pragma unroll
+            for (int w = 0; w < W; w++) {
+                m[w] = (mm >> (8 * w)) & 0xFFu;
+                if (OP != OP_SPMV) fr[w] = vf[w];
+                if (OP == OP_JACOBI) xr[w] = vx[w];
+                if (OP == OP_JACOBI && DIV == DIV_ARRAY) dr[w] = vd[w];
+            }
+        }
+    } else {
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            m[w] = 0;
+            if (r + w < n) {
+                m[w] = S.mask[r + w];
+                if (OP != OP_SPMV) fr[w] = f[r + w];
+                if (OP == OP_JACOBI) xr[w] = x[r + w];
+                if (OP == OP_JACOBI && DIV == DIV_ARRAY) dr[w] = d[r + w];
+            }
+        }
+        stencil_gather<VT, K, W, false>(S, x, r, n, m, g);
+    }
+    VT o[W];
+#pragma unroll
+    for (int w = 0; w < W; w++) {
+        VT t, dl;
+        stencil_sum<VT, K, OP == OP_JACOBI && DIV == DIV_L1>(m[w], S, g[w], t, dl);
+        if (OP == OP_SPMV)
+            o[w] = t;
+        else if (OP == OP_RESID)
+            o[w] = fr[w] - t;
+        else
+            o[w] = (fr[w] - t) / (DIV == DIV_L1 ? dl : DIV == DIV_DIAG ? S.diag : dr[w]) + xr[w];
+    }
+    if (W > 1 && inner) {
+        vec v;
+#pragma unroll
+        for (int w = 0; w < W; w++) v[w] = o[w];
+        *reinterpret_cast<vec *>(y + r) = v;
+    } else {
+#pragma unroll
+        for (int w = 0; w < W; w++)
+            if (r + w < n) y[r + w] = o[w];
+    }
+}
+
+/* k_spmv_dots on a constant stencil (the same 256-row blocks and trees) */
+template <int K, int KO>
+__global__ __launch_bounds__(BS) void k_spmv_dots_stencil(int n, StencilRef<double> S,
+                                                          const double *__restrict__ z,
+                                                          double *__restrict__ t,
+                                                          const double *__restrict__ rv,
+                                                          const double *__restrict__ to,
+                                                          double *__restrict__ part)
+{
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int r0 = b * BS;
+    const int r = r0 + threadIdx.x;
+    double sdot[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) sdot[k] = 0.0;
+    auto row = [&](auto inner) {
+        const unsigned m[1] = {S.mask[r]};
+        double g[1][KO];
+        const double zr = z[r], rr = rv[r];
+        const double tor = K > 2 ? to[r] : 0.0;
+        stencil_gather<double, KO, 1, decltype(inner)::value>(S, z, r, n, m, g);
+        double tr, unused;
+        stencil_sum<double, KO, false>(m[0], S, g[0], tr, unused);
+        t[r] = tr;
+        sdot[0] = rr * zr;
+        sdot[1] = tr * zr;
+        if (K > 2) sdot[K - 1] = tor * zr;
+    };
+    if (r0 + S.lo >= 0 && r0 + BS + S.hi <= n && r0 + BS <= n)
+        row(std::true_type{});
+    else if (r < n)
+        row(std::false_type{});
+    block_reduce_store<K>(sdot, part + (size_t)b * K);
+}
+
+/* one sweep from zero on a constant stencil */
+template <typename VT, int DIV>
+__global__ __launch_bounds__(BS) void k_jz_stencil(int n, StencilRef<VT> S,
+                                                   const VT *__restrict__ f, VT *__restrict__ y)
+{
+    const int i = blockIdx.x * BS + threadIdx.x;
+    if (i >= n) return;
+    VT t, dl, g[CLS_ROW];
+#pragma unroll
+    for (int k = 0; k < CLS_ROW; k++) g[k] = 0;
+    stencil_sum<VT, CLS_ROW, DIV == DIV_L1>(DIV == DIV_L1 ? S.mask[i] : 0u, S, g, t, dl);
+    y[i] = f[i] / (DIV == DIV_L1 ? dl : S.diag);
+}
+
+/* class codes -> entry masks */
+struct MaskTable {
+    unsigned char m[CLS_MAX];
+};
+__global__ __launch_bounds__(BS) void k_class_masks(int n, MaskTable T,
+                                                    unsigned char *__restrict__ code)
+{
+    const int r = blockIdx.x * BS + threadIdx.x;
+    if (r < n) code[r] = T.m[code[r]];
+}
+
+/* one sweep from zero, y = f / d with d from the row's class */
+template <typename VT>
+__global__ __launch_bounds__(BS) void k_jz_class(int n, ClassRef<VT> C, int drow,
+                                                 const VT *__restrict__ f, VT *__restrict__ y)
+{
+    const int i = blockIdx.x * BS + threadIdx.x;
+    if (i < n) y[i] = f[i] / C.tv[(size_t)drow * C.nc + C.code[i]];
+}
+
+/* k_spmv_dots on row classes: t = A z, per 256-row block the partial sums
+   of r.z, t.z and (K = 3) to.z over the same rows in the same tree */
+template <int K, int CR>
+__global__ __launch_bounds__(BS) void k_spmv_dots_class(int n, ClassRef<double> C,
+                                                        const double *__restrict__ z,
+                                                        double *__restrict__ t,
+                                                        const double *__restrict__ rv,
+                                                        const double *__restrict__ to,
+                                                        double *__restrict__ part)
+{
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int r = b * BS + threadIdx.x;
+    double sdot[K];
+#pragma unroll
+    for (int k = 0; k < K; k++) sdot[k] = 0.0;
+    double *lv;
+    int *li;
+    class_stage<double>(C, -1, lv, li);
+    __syncthreads();
+    if (r < n) {
+        const int c = C.code[r];
+        const double zr = z[r], rr = rv[r];
+        const double tor = K > 2 ? to[r] : 0.0;
+        const double tr = class_row_sum<double, CR>(c, C.nc, C.crow, lv, li, z, r);
+        t[r] = tr;
+        sdot[0] = rr * zr;
+        sdot[1] = tr * zr;
+        if (K > 2) sdot[K - 1] = tor * zr;
+    }
+    block_reduce_store<K>(sdot, part + (size_t)b * K);
+}
+
+template <typename VT>
+ClassRef<VT> class_ref(const DevCsr &A, MatType mt);
+template <>
+ClassRef<double> class_ref<double>(const DevCsr &A, MatType)
+{
+    return {A.cls.code.get(), A.cls.idx.get(), A.cls.v64.get(), A.cls.n, A.cls.row};
+}
+template <>
+ClassRef<float> class_ref<float>(const DevCsr &A, MatType mt)
+{
+    return {A.cls.code.get(), A.cls.idx.get(),
+            mt == MT_BF16 ? A.cls.v16.get() : A.cls.v32.get(), A.cls.n, A.cls.row};
+}
+
+template <typename VT>
+StencilRef<VT> stencil_ref(const DevCsr &A, MatType mt)
+{
+    StencilRef<VT> S;
+    const RowClasses &R = A.cls;
+    S.mask = R.code.get();
+    S.lo = R.off[0];
+    S.hi = R.off[R.k - 1];
+    S.diag = (VT)0;
+    for (int k = 0; k < CLS_ROW; k++) {
+        const bool in = k < R.k;
+        const double v = in ? R.val[k] : 0.0;
+        S.off[k] = in ? R.off[k] : 0;
+        S.a[k] = in ? std::fabs(v) : 0.0;
+        if (mt == MT_BF16)
+            S.v[k] = (VT)bf16_round((float)v);
+        else
+            S.v[k] = (VT)v;
+        if (in && R.off[k] == 0) S.diag = (VT)v;
+    }
+    return S;
+}
+
+/* rows per thread: the block stages the forms (nc (crow + 1) (4 + value)
+   bytes) for BS * RPT rows. Product with 1 / 2 / 4 rows: 27.2 / 24.0 / 23.3 us
+   at 4.1 M rows, 8.2 / 7.7 / 7.9 at 1 M, 3.4 / 3.9 / 5.2 at 262 144 (too few
+   blocks); sweeps 30.9 / 29.4 / 30.7 at 4.1 M */
+constexpr int CLS_RPT_BIG = 2;
+constexpr int CLS_BIG = 1 << 19;
+
+template <typename VT, int OP, int CR, int RPT>
+void rows_class_rpt(hipStream_t s, const DevCsr &A, const ClassRef<VT> &C, int drow, const VT *x,
+                    const VT *f, const VT *d, VT *y)
+{
+    const int nb = (A.n + BS * RPT - 1) / (BS * RPT);
+    const size_t lds = class_lds_bytes<VT>(C.nc, C.crow);
+    if (OP == OP_JACOBI && drow >= 0)
+        k_rows_class<VT, OP, CR, RPT, true><<<nb, BS, lds, s>>>(A.n, C, drow, x, f, d, y);
+    else
+        k_rows_class<VT, OP, CR, RPT, false><<<nb, BS, lds, s>>>(A.n, C, -1, x, f, d, y);
+}
+
+template <typename VT, int OP, int CR>
+void rows_class_cr(hipStream_t s, const DevCsr &A, const ClassRef<VT> &C, int drow, const VT *x,
+                   const VT *f, const VT *d, VT *y)
+{
+    if (A.n >= CLS_BIG)
+        rows_class_rpt<VT, OP, CR, CLS_RPT_BIG>(s, A, C, drow, x, f, d, y);
+    else
+        rows_class_rpt<VT, OP, CR, 1>(s, A, C, drow, x, f, d, y);
+}
+
+template <typename VT, int OP>
+void rows_class_op(hipStream_t s, const DevCsr &A, const ClassRef<VT> &C, int drow, const VT *x,
+                   const VT *f, const VT *d, VT *y)
+{
+    if (C.crow <= 5)
+        rows_class_cr<VT, OP, 5>(s, A, C, drow, x, f, d, y);
+    else if (C.crow <= 7)
+        rows_class_cr<VT, OP, 7>(s, A, C, drow, x, f, d, y);
+    else
+        rows_class_cr<VT, OP, CLS_ROW>(s, A, C, drow, x, f, d, y);
+}
+
+/* rows from which a thread takes two rows (FP64: 16-byte loads): product
+   with 1 / 2 rows 19.4 / 13.5 us at 4.1 M rows, 6.4 / 5.0 at 1 M; at 262 144
+   rows 2.88 / 2.99, where the launch is bound by latency and more threads
+   are better. FP32 with 4 rows was slower than with 2 (whole 160^3 FP32
+   solve 20.6 against 19.3 ms) */
+constexpr int STC_WIDE = 1 << 19;
+template <typename VT, int OP, int K, int W, int DIV>
+void rows_stencil_w(hipStream_t s, const DevCsr &A, const StencilRef<VT> &S, const VT *x,
+                    const VT *f, const VT *d, VT *y)
+{
+    const int nb = (A.n + BS * W - 1) / (BS * W);
+    k_rows_stencil<VT, OP, K, W, DIV><<<nb, BS, 0, s>>>(A.n, S, x, f, d, y);
+}
+
+template <typename VT, int OP, int K, int DIV>
+void rows_stencil_k(hipStream_t s, const DevCsr &A, const StencilRef<VT> &S, const VT *x,
+                    const VT *f, const VT *d, VT *y)
+{
+    /* the wide form's loads and stores of f, d and y are 16-byte aligned */
+    const uintptr_t al = reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(y) |
+                         (OP != OP_SPMV ? reinterpret_cast<uintptr_t>(f) : 0) |
+                         (OP == OP_JACOBI && DIV == DIV_ARRAY ? reinterpret_cast<uintptr_t>(d) : 0);
+    if (A.n >= STC_WIDE && (al & 15) == 0)
+        rows_stencil_w<VT, OP, K, 2, DIV>(s, A, S, x, f, d, y);
+    else
+        rows_stencil_w<VT, OP, K, 1, DIV>(s, A, S, x, f, d, y);
+}
+
+template <typename VT, int OP, int DIV>
+void rows_stencil_op(hipStream_t s, const DevCsr &A, const StencilRef<VT> &S, const VT *x,
+                     const VT *f, const VT *d, VT *y)
+{
+    const int k = A.cls.k;
+    if (k <= 5)
+        rows_stencil_k<VT, OP, 5, DIV>(s, A, S, x, f, d, y);
+    else if (k <= 7)
+        rows_stencil_k<VT, OP, 7, DIV>(s, A, S, x, f, d, y);
+    else
+        rows_stencil_k<VT, OP, CLS_ROW, DIV>(s, A, S, x, f, d, y);
+}
+
+/* the divisor's table row, or -1 for the caller's array */
+int div_row(const DevCsr &A, DivSource div)
+{
+    return div == DIV_DIAG ? A.cls.row : div == DIV_L1 ? A.cls.row + 1 : -1;
+}
+
+} // namespace
+
+namespace {
+
+/* Whether the forms (host copies of the tables) are one stencil with entries
+   left out: at most CLS_ROW offsets in all, each with one value (the same
+   bits). Then R.k, R.off and R.val hold it and T the mask of each class. */
+bool constant_stencil(RowClasses &R, const int *idx, const double *val, MaskTable &T)
+{
+    std::vector<std::pair<int, double>> ov;
+    for (int c = 0; c < R.n; c++)
+        for (int k = 0; k < idx[c]; k++) {
+            const int o = idx[(k + 1) * R.n + c];
+            const double v = val[k * R.n + c];
+            auto it = std::find_if(ov.begin(), ov.end(),
+                                   [&](const std::pair<int, double> &p) { return p.first == o; });
+            if (it == ov.end()) {
+                if (ov.size() == CLS_ROW) return false;
+                ov.emplace_back(o, v);
+            } else if (std::memcmp(&it->second, &v, sizeof(v)) != 0) {
+                return false;
+            }
+        }
+    std::sort(ov.begin(), ov.end(), [](const std::pair<int, double> &a,
+                                       const std::pair<int, double> &b) { return a.first < b.first; });
+    R.k = (int)ov.size();
+    for (int k = 0; k < R.k; k++) {
+        R.off[k] = ov[k].first;
+        R.val[k] = ov[k].second;
+    }
+    for (int c = 0; c < CLS_MAX; c++) {
+        unsigned m = 0;
+        for (int k = 0; c < R.n && k < idx[c]; k++)
+            for (int q = 0; q < R.k; q++)
+                if (R.off[q] == idx[(k + 1) * R.n + c]) m |= 1u << q;
+        T.m[c] = (unsigned char)m;
+    }
+    return true;
+}
+
+} // namespace
+
+/* operators of fewer rows relax in one workgroup (relax_block_ok) and are
+   not analysed */
+constexpr int CLS_MIN_ROWS = 4097;
+
+void make_classes(Ctx &c, const std::vector<DevCsr *> &mats)
+{
+    std::vector<DevCsr *> cand;
+    for (DevCsr *A : mats)
+        if (A->n == A->m && A->n >= CLS_MIN_ROWS && !A->cls.analysed && A->maxrow > 0 &&
+            A->maxrow <= CLS_ROW)
+            cand.push_back(A);
+    if (cand.empty()) return;
+    DBuf<ClassWork> work(cand.size());
+    /* first round trip: how many forms each operator has */
+    for (size_t k = 0; k < cand.size(); k++) {
+        DevCsr &A = *cand[k];
+        A.cls.analysed = true;
+        ClassWork *w = work.get() + k;
+        k_class_clear<<<1, BS, 0, c.stream>>>(w);
+        k_class_collect<<<(A.n + BS - 1) / BS, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(),
+                                                                 A.val.get(), w);
+        k_class_tables<<<1, CLS_MAX, 0, c.stream>>>(A.maxrow, A.row.get(), A.col.get(),
+                                                    A.val.get(), w);
+        BCMG_CHECK_LAUNCH();
+    }
+    struct Found {
+        DevCsr *A;
+        ClassWork *w;
+        int n;
+    };
+    std::vector<Found> found;
+    constexpr size_t HEADS = Ctx::H_INTS / 4;
+    for (size_t b = 0; b < cand.size(); b += HEADS) {
+        const size_t e = std::min(cand.size(), b + HEADS);
+        for (size_t k = b; k < e; k++)
+            BCMG_HIP(hipMemcpyAsync(c.h_ints + 4 * (k - b), &work.get()[k].count, 4 * sizeof(int),
+                                    hipMemcpyDeviceToHost, c.stream));
+        BCMG_HIP(hipStreamSynchronize(c.stream));
+        for (size_t k = b; k < e; k++) {
+            const int *h = c.h_ints + 4 * (k - b);
+            if (h[1] == 0) found.push_back({cand[k], work.get() + k, h[2]});
+        }
+    }
+    /* second: the codes' check and the tables, as many operators at a time
+       as the pinned staging holds */
+    for (size_t b = 0; b < found.size();) {
+        size_t e = b, at = 0;
+        std::vector<size_t> pos;
+        for (; e < found.size(); e++) {
+            const size_t row = found[e].A->maxrow, n = found[e].n;
+            const size_t need = 2 + (row + 1) * n + 2 * (row * n) + 1;
+            if (e > b && at + need > Ctx::H_INTS) break;
+            pos.push_back(at);
+            at += need;
+        }
+        for (size_t k = b; k < e; k++) {
+            DevCsr &A = *found[k].A;
+            ClassWork *w = found[k].w;
+            const size_t row = A.maxrow, n = found[k].n;
+            const int nblk = (A.n + BS - 1) / BS;
+            A.cls.code.alloc((size_t)nblk * BS);
+            k_class_codes<<<nblk, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(), A.val.get(),
+                                                     w, A.cls.code.get());
+            BCMG_CHECK_LAUNCH();
+            int *h = c.h_ints + pos[k - b];
+            BCMG_HIP(hipMemcpyAsync(h, &w->over, sizeof(int), hipMemcpyDeviceToHost, c.stream));
+            BCMG_HIP(hipMemcpyAsync(h + 1, w->idx, (row + 1) * n * sizeof(int),
+                                    hipMemcpyDeviceToHost, c.stream));
+            BCMG_HIP(hipMemcpyAsync(h + 1 + (row + 1) * n, w->tv, row * n * sizeof(double),
+                                    hipMemcpyDeviceToHost, c.stream));
+        }
+        BCMG_HIP(hipStreamSynchronize(c.stream));
+        for (size_t k = b; k < e; k++) {
+            DevCsr &A = *found[k].A;
+            RowClasses &R = A.cls;
+            const int *h = c.h_ints + pos[k - b];
+            if (h[0] != 0) {
+                R.code.release();
+                continue;
+            }
+            R.n = found[k].n;
+            R.row = A.maxrow;
+            const size_t ni = (size_t)(R.row + 1) * R.n, nv = (size_t)R.row * R.n;
+            std::vector<double> val(nv);
+            std::memcpy(val.data(), h + 1 + ni, nv * sizeof(double));
+            MaskTable T;
+            if (constant_stencil(R, h + 1, val.data(), T)) {
+                k_class_masks<<<(A.n + BS - 1) / BS, BS, 0, c.stream>>>(A.n, T, R.code.get());
+                BCMG_CHECK_LAUNCH();
+                continue;
+            }
+            R.idx.alloc(ni);
+            R.v64.alloc(nv + 2 * (size_t)R.n);
+            BCMG_HIP(hipMemcpyAsync(R.idx.get(), found[k].w->idx, ni * sizeof(int),
+                                    hipMemcpyDeviceToDevice, c.stream));
+            BCMG_HIP(hipMemcpyAsync(R.v64.get(), found[k].w->tv,
+                                    (nv + 2 * (size_t)R.n) * sizeof(double),
+                                    hipMemcpyDeviceToDevice, c.stream));
+        }
+        b = e;
+    }
+}
+
+void RowClasses::make_lowp(hipStream_t s, bool bf16)
+{
+    if (n == 0 || k > 0) return; /* a constant stencil's values are kernel arguments */
+    DBuf<float> &o = bf16 ? v16 : v32;
+    const int nv = row * n, nall = (row + 2) * n;
+    if (!o.get()) o.alloc(nall);
+    k_class_lowp<<<blocks_for(nall), BS, 0, s>>>(nv, nall, v64.get(), o.get(), bf16 ? 1 : 0);
+    BCMG_CHECK_LAUNCH();
+}
+
+template <typename VT>
+bool class_ok(const DevCsr &A, MatType mt)
+{
+    if (!A.use_classes()) return false;
+    if constexpr (std::is_same<VT, double>::value)
+        return mt == MT_F64;
+    else if (A.cls.k > 0)
+        return mt != MT_F64;
+    else
+        return mt == MT_F32 ? A.cls.v32.get() != nullptr
+                            : mt == MT_BF16 && A.cls.v16.get() != nullptr;
+}
+
+template <typename VT>
+void launch_rows_class(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const VT *x,
+                       const VT *f, const VT *d, VT *y, DivSource div)
+{
+    if (A.cls.k > 0) {
+        const StencilRef<VT> S = stencil_ref<VT>(A, mt);
+        if (op == OP_SPMV)
+            rows_stencil_op<VT, OP_SPMV, DIV_ARRAY>(s, A, S, x, f, d, y);
+        else if (op == OP_RESID)
+            rows_stencil_op<VT, OP_RESID, DIV_ARRAY>(s, A, S, x, f, d, y);
+        else if (div == DIV_ARRAY)
+            rows_stencil_op<VT, OP_JACOBI, DIV_ARRAY>(s, A, S, x, f, d, y);
+        else if (div == DIV_DIAG)
+            rows_stencil_op<VT, OP_JACOBI, DIV_DIAG>(s, A, S, x, f, d, y);
+        else
+            rows_stencil_op<VT, OP_JACOBI, DIV_L1>(s, A, S, x, f, d, y);
+        BCMG_CHECK_LAUNCH();
+        return;
+    }
+    const ClassRef<VT> C = class_ref<VT>(A, mt);
+    const int drow = div_row(A, div);
+    if (op == OP_SPMV)
+        rows_class_op<VT, OP_SPMV>(s, A, C, drow, x, f, d, y);
+    else if (op == OP_RESID)
+        rows_class_op<VT, OP_RESID>(s, A, C, drow, x, f, d, y);
+    else
+        rows_class_op<VT, OP_JACOBI>(s, A, C, drow, x, f, d, y);
+    BCMG_CHECK_LAUNCH();
+}
+
+template <typename VT>
+void launch_jacobi_zero_class(hipStream_t s, const DevCsr &A, MatType mt, const VT *f, VT *y,
+                              DivSource div)
+{
+    if (A.cls.k > 0) {
+        const StencilRef<VT> S = stencil_ref<VT>(A, mt);
+        if (div == DIV_L1)
+            k_jz_stencil<VT, DIV_L1><<<blocks_for(A.n), BS, 0, s>>>(A.n, S, f, y);
+        else
+            k_jz_stencil<VT, DIV_DIAG><<<blocks_for(A.n), BS, 0, s>>>(A.n, S, f, y);
+        BCMG_CHECK_LAUNCH();
+        return;
+    }
+    k_jz_class<VT><<<blocks_for(A.n), BS, 0, s>>>(A.n, class_ref<VT>(A, mt), div_row(A, div), f,
+                                                  y);
+    BCMG_CHECK_LAUNCH();
+}
+
+template <int K>
+static void spmv_dots_class_k(hipStream_t s, const DevCsr &A, const double *z, double *t,
+                              const double *r, const double *to, double *part)
+{
+    const int nb = (A.n + BS - 1) / BS;
+    if (A.cls.k > 0) {
+        const StencilRef<double> S = stencil_ref<double>(A, MT_F64);
+        if (A.cls.k <= 5)
+            k_spmv_dots_stencil<K, 5><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
+        else if (A.cls.k <= 7)
+            k_spmv_dots_stencil<K, 7><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
+        else
+            k_spmv_dots_stencil<K, CLS_ROW><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
+        return;
+    }
+    const ClassRef<double> C = class_ref<double>(A, MT_F64);
+    const size_t lds = class_lds_bytes<double>(C.nc, C.crow);
+    if (C.crow <= 5)
+        k_spmv_dots_class<K, 5><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
+    else if (C.crow <= 7)
+        k_spmv_dots_class<K, 7><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
+    else
+        k_spmv_dots_class<K, CLS_ROW><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
+}
+
+void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const double *z, double *t,
+                            const double *r, const double *to, double *part)
+{
+    if (k == 2)
+        spmv_dots_class_k<2>(s, A, z, t, r, to, part);
+    else
+        spmv_dots_class_k<3>(s, A, z, t, r, to, part);
+    BCMG_CHECK_LAUNCH();
+}
+
+#define BCMG_INSTANTIATE_CLASS(VT)                                                            \
+    template bool class_ok<VT>(const DevCsr &, MatType);                                      \
+    template void launch_rows_class<VT>(hipStream_t, const DevCsr &, MatType, RowOp,          \
+                                        const VT *, const VT *, const VT *, VT *, DivSource); \
+    template void launch_jacobi_zero_class<VT>(hipStream_t, const DevCsr &, MatType,          \
+                                               const VT *, VT *, DivSource);
+BCMG_INSTANTIATE_CLASS(double)
+BCMG_INSTANTIATE_CLASS(float)
+#undef BCMG_INSTANTIATE_CLASS
+
+} // namespace bcmg

@@ -31,6 +31,26 @@ __device__ __forceinline__ VT mval(float v) { return (VT)v; }
 template <typename VT>
 __device__ __forceinline__ VT mval(unsigned short h) { return (VT)__uint_as_float((unsigned)h << 16); }
 
+/* float -> bfloat16 bits (round to nearest even; NaN kept quiet) */
+__host__ __device__ __forceinline__ unsigned short to_bf16_bits(float f)
+{
+    unsigned u;
+    __builtin_memcpy(&u, &f, sizeof(u));
+    if ((u & 0x7F800000u) == 0x7F800000u && (u & 0x007FFFFFu))
+        return (unsigned short)((u >> 16) | 0x40u);
+    u += 0x7FFFu + ((u >> 16) & 1u);
+    return (unsigned short)(u >> 16);
+}
+
+/* f rounded to bfloat16, as a float */
+__host__ __device__ __forceinline__ float bf16_round(float f)
+{
+    const unsigned u = (unsigned)to_bf16_bits(f) << 16;
+    float r;
+    __builtin_memcpy(&r, &u, sizeof(r));
+    return r;
+}
+
 template <bool NT, typename T>
 __device__ __forceinline__ T ldm(const T *p)
 {

@@ -428,20 +428,12 @@ __global__ __launch_bounds__(BS) void k_convert(size_t n, const S *__restrict__ 
     if (i < n) b[i] = (D)a[i];
 }
 
-/* double -> bfloat16 (through float, round to nearest even; NaN kept quiet) */
+/* double -> bfloat16 (through float) */
 __global__ __launch_bounds__(BS) void k_to_bf16(size_t n, const double *__restrict__ a,
                                                 unsigned short *__restrict__ b)
 {
     const size_t i = (size_t)blockIdx.x * BS + threadIdx.x;
-    if (i >= n) return;
-    const float f = (float)a[i];
-    unsigned u = __float_as_uint(f);
-    if ((u & 0x7F800000u) == 0x7F800000u && (u & 0x007FFFFFu)) {
-        b[i] = (unsigned short)((u >> 16) | 0x40u);
-        return;
-    }
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    b[i] = (unsigned short)(u >> 16);
+    if (i < n) b[i] = to_bf16_bits((float)a[i]);
 }
 
 template <int K>
@@ -898,8 +890,8 @@ void analyze_rows(Ctx &c, DevCsr &A)
     launch_block_nnz(c, A);
     resolve_tiles(c, {&A});
     make_narrow(c, {&A});
+    make_classes(c, {&A});
 }
-
 
 /* square operators whose FP64 stream (12 B per entry) exceeds this are
    checked for a stencil pattern; the 16-bit copy is kept for streamed ones
@@ -977,13 +969,18 @@ void DevCsr::make_lowp(hipStream_t s, bool bf16)
         k_convert<double, float><<<nb, BS, 0, s>>>((size_t)nnz, val.get(), val32.get());
     }
     BCMG_CHECK_LAUNCH();
+    cls.make_lowp(s, bf16);
 }
 
 template <typename VT>
 void launch_rows(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const VT *x, const VT *f,
-                 const VT *d, VT *y)
+                 const VT *d, VT *y, DivSource div)
 {
     if (A.n <= 0) return;
+    if (op != OP_JACOBI_Z && class_ok<VT>(A, mt)) {
+        launch_rows_class<VT>(s, A, mt, op, x, f, d, y, div);
+        return;
+    }
     if constexpr (std::is_same<VT, double>::value) {
         if (mt != MT_F64) throw Error(BCMG_EINVAL, "FP64 vectors need FP64 matrix values");
         rows_op<double, double>(s, A, A.val.get(), op, x, f, d, y);
@@ -1007,6 +1004,11 @@ void launch_rows(hipStream_t s, const DevCsr &A, RowOp op, const double *x, cons
 template <typename VT>
 bool fuse_zero_sweeps(const DevCsr &A, MatType mt)
 {
+    /* row classes: a sweep from zero reads one byte and f per row, so two
+       light passes beat one with a division at every gather (160^3 FP32
+       47 us in one pass, 10.8 + 12.8 us in two), except where a launch costs
+       more than the work */
+    if (class_ok<VT>(A, mt)) return A.n <= SMALL_LEVEL_ROWS;
     /* a streamed FP64 operator: the division at every gather costs more
        than the pass it saves */
     const size_t vb = mt == MT_F64 ? 8 : mt == MT_F32 ? 4 : 2;
@@ -1111,10 +1113,15 @@ bool launch_resid_restrict(hipStream_t s, const DevCsr &A, MatType mt, const Dev
 }
 
 template <typename VT>
-void launch_jacobi_zero(hipStream_t s, int n, const VT *f, const VT *d, VT *y)
+void launch_jacobi_zero(hipStream_t s, const DevCsr &A, MatType mt, const VT *f, const VT *d,
+                        VT *y, DivSource div)
 {
-    if (n <= 0) return;
-    k_jacobi_zero<VT><<<blocks_for(n), BS, 0, s>>>(n, f, d, y);
+    if (A.n <= 0) return;
+    if (div != DIV_ARRAY && class_ok<VT>(A, mt)) {
+        launch_jacobi_zero_class<VT>(s, A, mt, f, y, div);
+        return;
+    }
+    k_jacobi_zero<VT><<<blocks_for(A.n), BS, 0, s>>>(A.n, f, d, y);
     BCMG_CHECK_LAUNCH();
 }
 
@@ -1184,7 +1191,7 @@ void launch_f2d(hipStream_t s, size_t n, const float *a, double *b)
 
 #define BCMG_INSTANTIATE(VT)                                                                 \
     template void launch_rows<VT>(hipStream_t, const DevCsr &, MatType, RowOp, const VT *,   \
-                                  const VT *, const VT *, VT *);                             \
+                                  const VT *, const VT *, VT *, DivSource);                  \
     template bool relax_block_ok<VT>(const DevCsr &);                                        \
     template void launch_relax_block<VT>(hipStream_t, const DevCsr &, MatType, const VT *,   \
                                          const VT *, const VT *, VT *, int, bool, int, long, \
@@ -1195,7 +1202,8 @@ void launch_f2d(hipStream_t s, size_t n, const float *a, double *b)
                                             const VT *, VT *);                               \
     template bool launch_resid_restrict<VT>(hipStream_t, const DevCsr &, MatType,            \
                                             const DevCsr &, const VT *, const VT *, VT *);   \
-    template void launch_jacobi_zero<VT>(hipStream_t, int, const VT *, const VT *, VT *);    \
+    template void launch_jacobi_zero<VT>(hipStream_t, const DevCsr &, MatType, const VT *,   \
+                                         const VT *, VT *, DivSource);                       \
     template void launch_prolong<VT>(hipStream_t, int, const int *, const VT *, const VT *,  \
                                      VT *);                                                  \
     template void launch_prolong_to<VT>(hipStream_t, int, const int *, const VT *,           \
@@ -1367,7 +1375,9 @@ void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const double *z, double *t
     double *part = c.red.get() + RED_SPMV;
     const int *rp = A.row.get();
     const double *av = A.val.get();
-    if (A.use_pattern()) {
+    if (class_ok<double>(A, MT_F64)) {
+        launch_spmv_dots_class(c.stream, A, k, z, t, r, to, part);
+    } else if (A.use_pattern()) {
         if (!stage_aligned(av, av))
             throw Error(BCMG_EINVAL, "SpMV: matrix values not 16-byte aligned");
         const size_t lds = pattern_lds_bytes(A.tile, sizeof(double));
