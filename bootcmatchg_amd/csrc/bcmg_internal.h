@@ -177,6 +177,7 @@ struct DevCsr {
     int poff[PAT_MAX] = {};
     bool cols_analysed = false; /* narrow copy and pattern considered */
     RowClasses cls;
+    int band = -1;              /* largest |column - row|; -1: not determined */
     /* the narrowest form the row kernels may read: 3 the row classes, 2 the
        pattern, 1 the 16-bit offsets, 0 the int32 columns
        (bcmg_csr_set_columns chooses among the last three) */
@@ -203,9 +204,9 @@ void resolve_tiles(Ctx &c, const std::vector<DevCsr *> &mats);
    pattern when those offsets take at most PAT_MAX values (one round trip
    for the lot) */
 void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats);
-/* find the row classes of every square operator in mats that has rows of at
-   most CLS_ROW entries (their tiles resolved) and at most CLS_MAX forms (one
-   round trip for the lot) */
+/* find the band and the row classes (at most CLS_MAX forms) of every square
+   operator in mats that has rows of at most CLS_ROW entries, their tiles
+   resolved (one round trip for the lot, a second for those with classes) */
 void make_classes(Ctx &c, const std::vector<DevCsr *> &mats);
 
 /* ------------------------------------------------------------- context */
@@ -472,6 +473,23 @@ struct BlockFuse {
     const VT *rv = nullptr;
     VT *fc = nullptr;
 };
+/* Several sweeps in one launch, on a constant stencil or an operator of short
+   rows, both of narrow band: how many of the next `sweeps` sweeps (zero: the
+   first of them is f / d) to make in one launch (0: no such launch pays) and
+   the rows *m that its workgroups own; whether one workgroup can take the
+   level; and the launch of `steps` neighbour-reading sweeps (after f / d with
+   zero): xout is another buffer than xin unless one workgroup does all
+   (m >= n); fu's restriction needs a constant stencil in one workgroup. A
+   constant stencil takes its divisor from div (DIV_DIAG or DIV_L1), other
+   rows from d. */
+template <typename VT>
+int slab_plan(const DevCsr &A, MatType mt, int sweeps, bool zero, int *m);
+template <typename VT>
+bool slab_one(const DevCsr &A, MatType mt);
+template <typename VT>
+void launch_slab(hipStream_t s, const DevCsr &A, MatType mt, int m, int steps, bool zero,
+                 DivSource div, const VT *d, const VT *f, const VT *xin, VT *xout,
+                 const BlockFuse<VT> &fu = BlockFuse<VT>());
 template <typename VT>
 void launch_relax_block(hipStream_t s, const DevCsr &A, MatType mt, const VT *d, const VT *f,
                         const VT *xin, VT *xout, int sweeps, bool zero, int ncols = 1,

@@ -343,6 +343,23 @@ void relax_level(Ctx &c, const Level &lv, MatType mt, int type, int sweeps, cons
     const VT *d = divisor<VT>(lv, type);
     if (sweeps == 0) return;
     const bool timing = level0 && c.time_smoother;
+    int m = 0;
+    for (int take; !timing && (take = slab_plan<VT>(A, mt, sweeps, s.zero, &m)) > 0;) {
+        /* several sweeps a launch; over several workgroups the result goes
+           to another buffer than x */
+        const bool to_final = final_out && take == sweeps;
+        VT *out = m >= A.n ? s.x : s.x2;
+        if (to_final && (s.zero || m >= A.n || s.x != final_out)) out = final_out;
+        launch_slab<VT>(c.stream, A, mt, m, take - (s.zero ? 1 : 0), s.zero, div_source(type), d,
+                        f, s.x, out);
+        if (out != s.x) {
+            s.x2 = s.x;
+            s.x = out;
+        }
+        s.zero = false;
+        sweeps -= take;
+        if (sweeps == 0) return;
+    }
     if (relax_block_ok<VT>(A) && !timing) {
         VT *out = (final_out && s.x != final_out) ? final_out : s.x;
         launch_relax_block<VT>(c.stream, A, mt, d, f, s.x, out, sweeps, s.zero);
@@ -410,6 +427,23 @@ bool post_lands_off(int sweeps, const VT *a, const VT *b, const VT *fo)
     if (!fo) return false;
     if (sweeps == 0) return a != fo;
     return ((sweeps - 1) % 2 == 0 ? a : b) == fo;
+}
+
+/* Where a launch that forms x + P x_c and sweeps puts its result: the other
+   iterate, or the preconditioner's output fo when no launch follows
+   (rest = 0). When the other iterate is that output and launches remain, a
+   third level-0 buffer (the multiplicative composites leave xb[0] free):
+   the remaining launches then alternate between two buffers that are not
+   the output, so the last one writes the output and no copy follows. */
+template <typename VT>
+VT *third_buffer(Boot &B, const LevelState<VT> &s, VT *fo, int rest)
+{
+    if (fo && fo != s.x) {
+        VT *third = bufs<VT>(B).xb[0].get();
+        if (rest == 0) return fo;
+        if (s.x2 == fo && third != s.x && third != fo) return third;
+    }
+    return s.x2;
 }
 
 /* inner-iteration tolerance of the K-cycle (src/SOLVER/GAMG_cycle.cu:5) */
@@ -487,7 +521,10 @@ void cycle(CycleRun<VT> &R, int l, const VT *fin)
     /* R holds the prolongator values: FP32 whenever the cycle runs in FP32 */
     const MatType rmt = std::is_same<VT, double>::value ? MT_F64 : MT_F32;
     VT *fc = W.f[l].get();
-    const bool blk = relax_block_ok<VT>(A) && !(top && c.time_smoother);
+    const bool timing = top && c.time_smoother;
+    /* one workgroup relaxes the level: as a constant stencil, or any rows */
+    const bool slab1 = !timing && slab_one<VT>(A, mt);
+    const bool blk = slab1 || (relax_block_ok<VT>(A) && !timing);
     bool restricted = false;
     if (blk && B.prm.prerelax_sweeps > 0 && rows_sequential<VT>(lv.R)) {
         /* a one-workgroup level: pre-smoothing, residual and restriction in
@@ -498,8 +535,12 @@ void cycle(CycleRun<VT> &R, int l, const VT *fin)
         fu.rci = lv.R.col.get();
         fu.rv = rvals<VT>(lv.R);
         fu.fc = fc;
-        launch_relax_block<VT>(c.stream, A, mt, divisor<VT>(lv, B.prm.relax_type), f, s.x, s.x,
-                               B.prm.prerelax_sweeps, s.zero, 1, 0, 1, nullptr, fu);
+        if (slab1)
+            launch_slab<VT>(c.stream, A, mt, A.n, B.prm.prerelax_sweeps - (s.zero ? 1 : 0),
+                            s.zero, div_source(B.prm.relax_type), nullptr, f, s.x, s.x, fu);
+        else
+            launch_relax_block<VT>(c.stream, A, mt, divisor<VT>(lv, B.prm.relax_type), f, s.x,
+                                   s.x, B.prm.prerelax_sweeps, s.zero, 1, 0, 1, nullptr, fu);
         s.zero = false;
         restricted = true;
     } else {
@@ -530,8 +571,11 @@ void cycle(CycleRun<VT> &R, int l, const VT *fin)
         }
     }
     bool prolong_in_block = false, prolong_in_sweep = false;
+    int slab_m = 0, slab_n = 0; /* sweeps that a slab launch makes from x + P x_c */
     if (!sc.zero) {
-        if (s.zero && !(blk && !lv.smoothed && B.prm.postrelax_sweeps > 0)) {
+        const bool fold = !lv.smoothed && B.prm.postrelax_sweeps > 0 && !timing;
+        if (fold) slab_n = slab_plan<VT>(A, mt, B.prm.postrelax_sweeps, false, &slab_m);
+        if (s.zero && !(fold && (blk || slab_n > 0))) {
             launch_fill<VT>(c.stream, A.n, VT(0), s.x);
             s.zero = false;
         }
@@ -540,6 +584,8 @@ void cycle(CycleRun<VT> &R, int l, const VT *fin)
             launch_rows<VT>(c.stream, lv.Pneg, std::is_same<VT, double>::value ? MT_F64 : MT_F32,
                             OP_RESID, sc.x, s.x, nullptr, s.x2);
             std::swap(s.x, s.x2);
+        } else if (slab_n > 0) {
+            /* the prolongation folded into the first slab launch (below) */
         } else if (blk && B.prm.postrelax_sweeps > 0) {
             /* a one-workgroup level: the prolongation folded into the
                post-smoothing launch (below) */
@@ -575,24 +621,26 @@ void cycle(CycleRun<VT> &R, int l, const VT *fin)
         s.zero = false;
         return;
     }
+    if (slab_n > 0) {
+        BlockFuse<VT> fu;
+        fu.agg = lv.agg.get();
+        fu.p = pvals<VT>(lv);
+        fu.xc = sc.x;
+        const int rest = B.prm.postrelax_sweeps - slab_n;
+        VT *fo = top ? R.final_out : nullptr;
+        VT *out = third_buffer<VT>(B, s, fo, rest);
+        launch_slab<VT>(c.stream, A, mt, slab_m, slab_n, s.zero, div_source(B.prm.relax_type),
+                        divisor<VT>(lv, B.prm.relax_type), f, s.x, out, fu);
+        s.x2 = s.x;
+        s.x = out;
+        s.zero = false;
+        relax_level<VT>(c, lv, mt, B.prm.relax_type, rest, f, s, fo, top);
+        return;
+    }
     if (prolong_in_sweep) {
-        /* the fused sweep writes the other iterate, or the preconditioner's
-           output when it is the last sweep. When the other iterate is that
-           output and sweeps remain, it writes a third level-0 buffer
-           instead (the multiplicative composites leave xb[0] free): the
-           remaining sweeps then alternate between two buffers that are not
-           the output, so the last one writes the output and no copy
-           follows. */
         const int rest = B.prm.postrelax_sweeps - 1;
         VT *fo = top ? R.final_out : nullptr;
-        VT *out = s.x2;
-        if (fo && fo != s.x) {
-            VT *third = bufs<VT>(B).xb[0].get();
-            if (rest == 0)
-                out = fo;
-            else if (s.x2 == fo && third != s.x && third != fo)
-                out = third;
-        }
+        VT *out = third_buffer<VT>(B, s, fo, rest);
         if (launch_jacobi_prolong<VT>(c.stream, A, mt, lv.agg.get(), pvals<VT>(lv), sc.x, s.x, f,
                                       divisor<VT>(lv, B.prm.relax_type), out)) {
             s.x2 = s.x;

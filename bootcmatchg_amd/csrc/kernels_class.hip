@@ -70,7 +70,7 @@ struct ClassWork {
     unsigned long long hash[CLS_SLOTS];
     int rep[CLS_SLOTS];       /* smallest row with that hash */
     int cls[CLS_SLOTS];       /* class of the slot, once numbered */
-    int count, over, ncls, pad;
+    int count, over, ncls, band;
     /* the tables, entry k of class c at [k ncls + c]: lengths, then offsets;
        values, then the diagonals and the sums of magnitudes (the smoother
        divisors) */
@@ -85,7 +85,24 @@ __global__ __launch_bounds__(BS) void k_class_clear(ClassWork *w)
         w->rep[q] = 0x7fffffff;
         w->cls[q] = -1;
     }
-    if (threadIdx.x == 0) w->count = w->over = w->ncls = 0;
+    if (threadIdx.x == 0) w->count = w->over = w->ncls = w->band = 0;
+}
+
+/* the largest |column - row| (columns ascend in a row) */
+__global__ __launch_bounds__(BS) void k_band(int n, const int *__restrict__ rp,
+                                             const int *__restrict__ ci, int *__restrict__ band)
+{
+    __shared__ int sm[BS / 64];
+    const int r = blockIdx.x * BS + threadIdx.x;
+    int o = 0;
+    if (r < n && rp[r + 1] > rp[r]) o = max(r - ci[rp[r]], ci[rp[r + 1] - 1] - r);
+#pragma unroll
+    for (int q = 32; q > 0; q >>= 1) o = max(o, __shfl_xor(o, q, 64));
+    if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = o;
+    __syncthreads();
+    if (threadIdx.x != 0) return;
+    for (int q = 1; q < BS / 64; q++) o = max(o, sm[q]);
+    if (o > __hip_atomic_load(band, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(band, o);
 }
 
 /* step 1: the distinct row hashes of a 256-row block (an LDS table) go into
@@ -550,6 +567,173 @@ __global__ __launch_bounds__(BS) void k_jz_stencil(int n, StencilRef<VT> S,
     y[i] = f[i] / (DIV == DIV_L1 ? dl : S.diag);
 }
 
+/* rows a slab workgroup of 1024 threads holds (four a thread: 64 KB of LDS in
+   FP64), and its own rows' least number where there are more workgroups than
+   CUs (the others are recomputed) */
+constexpr int SLAB_ROWS = 4096;
+/* the same with the rows in registers: one a thread (with four a thread, 128
+   VGPRs, four sweeps took 15-20 us, no less than four launches) */
+constexpr int SLAB_ROWS_REG = 1024;
+constexpr int SLAB_CUS = 256;
+constexpr int SLAB_MIN_SHARE = 1640;
+
+/* Several Jacobi/L1 sweeps of a constant stencil in one launch. A workgroup
+   owns rows [a, a + m) and keeps them and the rows within steps * B of them
+   (B the largest |offset|) in LDS: sweep t recomputes the rows within
+   (steps - t) B of its own, so no workgroup waits for another and x, f and
+   the masks are read and the result written once for all sweeps. Row sums,
+   divisors and the update are k_rows_stencil's, so the result has the bits
+   of separate sweeps. A level whose rows all fit one workgroup has no
+   redundant rows and takes any number of sweeps.
+   zero: x is known to be zero, the first sweep f / d is made while loading
+   (MODE 0 and 2; `steps` counts the sweeps after it). MODE 1: x starts as
+   x + P x_c (k_prolong's fma; x = 0 when zero). MODE 2 (one workgroup):
+   after the sweeps the residual rows are restricted into fu.fc as the
+   residual and SpMV kernels do. */
+template <typename VT, int K, int RPT, int MODE, int DIV>
+__global__ __launch_bounds__(1024) void k_stencil_slab(int n, StencilRef<VT> S, int m, int B,
+                                                       int steps, int zero,
+                                                       const VT *__restrict__ f,
+                                                       const VT *__restrict__ xin,
+                                                       VT *__restrict__ xout, BlockFuse<VT> fu)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_slab[];
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int a = b * m, e = min(a + m, n);
+    const int reach = steps * B;
+    const int lo = max(0, a - reach), hi = min(n, e + reach);
+    /* gathers of absent entries are not made, those of present ones stay in
+       [lo, hi): no pad is needed around the rows */
+    VT *cur = reinterpret_cast<VT *>(smem_slab);
+    VT *nxt = cur + (m + 2 * reach);
+    unsigned mk[RPT];
+    VT fr[RPT], dr[RPT];
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int i = lo + (int)threadIdx.x + 1024 * q;
+        mk[q] = 0;
+        fr[q] = 0;
+        dr[q] = 1;
+        if (i < hi) {
+            mk[q] = S.mask[i];
+            fr[q] = f[i];
+            VT x0 = 0;
+            if (MODE == 1)
+                x0 = fma(fu.p[i], fu.xc[fu.agg[i]], zero ? VT(0) : xin[i]);
+            else if (!zero)
+                x0 = xin[i];
+            VT t, dl, g[K];
+#pragma unroll
+            for (int k = 0; k < K; k++) g[k] = 0;
+            stencil_sum<VT, K, DIV == DIV_L1>(DIV == DIV_L1 ? mk[q] : 0u, S, g, t, dl);
+            dr[q] = DIV == DIV_L1 ? dl : S.diag;
+            cur[i - lo] = MODE != 1 && zero ? fr[q] / dr[q] : x0;
+        }
+    }
+    __syncthreads();
+    for (int t = 1; t <= steps; t++) {
+        const int wl = max(0, a - (steps - t) * B), wh = min(n, e + (steps - t) * B);
+#pragma unroll
+        for (int q = 0; q < RPT; q++) {
+            const int i = lo + (int)threadIdx.x + 1024 * q;
+            if (i >= wl && i < wh) {
+                VT sum = 0;
+                const VT *c = cur + (i - lo);
+#pragma unroll
+                for (int k = 0; k < K; k++)
+                    if ((mk[q] >> k) & 1u) sum = sum + S.v[k] * c[S.off[k]];
+                nxt[i - lo] = (fr[q] - sum) / dr[q] + c[0];
+            }
+        }
+        __syncthreads();
+        VT *const sw = cur;
+        cur = nxt;
+        nxt = sw;
+    }
+#pragma unroll
+    for (int q = 0; q < RPT; q++) {
+        const int i = lo + (int)threadIdx.x + 1024 * q;
+        if (i >= a && i < e) xout[i] = cur[i - lo];
+    }
+    if constexpr (MODE == 2) {
+#pragma unroll
+        for (int q = 0; q < RPT; q++) {
+            const int i = (int)threadIdx.x + 1024 * q;
+            if (i < n) {
+                VT sum = 0;
+#pragma unroll
+                for (int k = 0; k < K; k++)
+                    if ((mk[q] >> k) & 1u) sum = sum + S.v[k] * cur[i + S.off[k]];
+                nxt[i] = fr[q] - sum;
+            }
+        }
+        __syncthreads();
+        for (int I = threadIdx.x; I < fu.nc; I += 1024) {
+            VT t = 0;
+            const int e1 = fu.rrp[I + 1];
+            for (int j = fu.rrp[I]; j < e1; j++) t = t + fu.rv[j] * nxt[fu.rci[j]];
+            fu.fc[I] = t;
+        }
+    }
+}
+
+/* k_stencil_slab for any rows of at most CLS_ROW entries: the row of a thread
+   stays in registers (columns as LDS positions) and the divisor comes from
+   its array. Row sums in storage order from 0. */
+template <typename MT, typename VT, int MODE>
+__global__ __launch_bounds__(1024) void k_rows_slab(int n, const int *__restrict__ rp,
+                                                    const int *__restrict__ ci,
+                                                    const MT *__restrict__ av,
+                                                    const VT *__restrict__ d, int m, int B,
+                                                    int steps, int zero,
+                                                    const VT *__restrict__ f,
+                                                    const VT *__restrict__ xin,
+                                                    VT *__restrict__ xout, BlockFuse<VT> fu)
+{
+    __shared__ VT xs[2][SLAB_ROWS_REG];
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int a = b * m, e = min(a + m, n);
+    const int reach = steps * B;
+    const int lo = max(0, a - reach), hi = min(n, e + reach); /* at most SLAB_ROWS_REG rows */
+    const int t = threadIdx.x, i = lo + t;
+    VT *cur = xs[0], *nxt = xs[1];
+    VT v[CLS_ROW], fr = 0, dr = 1;
+    int c[CLS_ROW], len = 0;
+    if (i < hi) {
+        const int j0 = rp[i];
+        len = rp[i + 1] - j0;
+        fr = f[i];
+        dr = d[i];
+        VT x0 = 0;
+        if (MODE == 1)
+            x0 = fma(fu.p[i], fu.xc[fu.agg[i]], zero ? VT(0) : xin[i]);
+        else if (!zero)
+            x0 = xin[i];
+#pragma unroll
+        for (int k = 0; k < CLS_ROW; k++) {
+            v[k] = k < len ? mval<VT>(av[j0 + k]) : VT(0);
+            c[k] = k < len ? ci[j0 + k] - lo : 0;
+        }
+        cur[t] = MODE != 1 && zero ? fr / dr : x0;
+    }
+    __syncthreads();
+    for (int s = 1; s <= steps; s++) {
+        /* a row of the window has all its columns in [lo, hi) */
+        if (i >= a - (steps - s) * B && i < e + (steps - s) * B && i < hi) {
+            VT sum = 0;
+#pragma unroll
+            for (int k = 0; k < CLS_ROW; k++)
+                if (k < len) sum = sum + v[k] * cur[c[k]];
+            nxt[t] = (fr - sum) / dr + cur[t];
+        }
+        __syncthreads();
+        VT *const sw = cur;
+        cur = nxt;
+        nxt = sw;
+    }
+    if (i >= a && i < e) xout[i] = cur[t];
+}
+
 /* class codes -> entry masks */
 struct MaskTable {
     unsigned char m[CLS_MAX];
@@ -721,6 +905,70 @@ void rows_stencil_op(hipStream_t s, const DevCsr &A, const StencilRef<VT> &S, co
         rows_stencil_k<VT, OP, CLS_ROW, DIV>(s, A, S, x, f, d, y);
 }
 
+template <typename VT, int K, int RPT, int MODE>
+void slab_div(hipStream_t s, int n, const StencilRef<VT> &S, int m, int B, int steps, int zero,
+              DivSource div, const VT *f, const VT *xin, VT *xout, const BlockFuse<VT> &fu)
+{
+    const int nb = (n + m - 1) / m;
+    const size_t lds = 2 * (size_t)(m + 2 * steps * B) * sizeof(VT);
+    if (div == DIV_L1)
+        k_stencil_slab<VT, K, RPT, MODE, DIV_L1>
+            <<<nb, 1024, lds, s>>>(n, S, m, B, steps, zero, f, xin, xout, fu);
+    else
+        k_stencil_slab<VT, K, RPT, MODE, DIV_DIAG>
+            <<<nb, 1024, lds, s>>>(n, S, m, B, steps, zero, f, xin, xout, fu);
+    BCMG_CHECK_LAUNCH();
+}
+
+template <typename VT, int K, int MODE>
+void slab_rpt(hipStream_t s, int n, const StencilRef<VT> &S, int m, int B, int steps, int zero,
+              DivSource div, const VT *f, const VT *xin, VT *xout, const BlockFuse<VT> &fu)
+{
+    const int ext = std::min(n, m + 2 * steps * B);
+    if (ext <= 1024)
+        slab_div<VT, K, 1, MODE>(s, n, S, m, B, steps, zero, div, f, xin, xout, fu);
+    else if (ext <= 2048)
+        slab_div<VT, K, 2, MODE>(s, n, S, m, B, steps, zero, div, f, xin, xout, fu);
+    else if (ext <= 4096)
+        slab_div<VT, K, 4, MODE>(s, n, S, m, B, steps, zero, div, f, xin, xout, fu);
+    else
+        throw Error(BCMG_EINVAL, "stencil slab: too many rows");
+}
+
+template <typename MT, typename VT>
+void rows_slab(hipStream_t s, const DevCsr &A, const MT *av, int m, int B, int steps, int zero,
+               const VT *d, const VT *f, const VT *xin, VT *xout, const BlockFuse<VT> &fu)
+{
+    const int n = A.n, nb = (n + m - 1) / m;
+    const int ext = std::min(n, m + 2 * steps * B);
+    const size_t lds = 2 * (size_t)(m + 2 * steps * B) * sizeof(VT);
+    auto go = [&](auto kern) {
+        kern<<<nb, 1024, lds, s>>>(n, A.row.get(), A.col.get(), av, d, m, B, steps, zero, f, xin,
+                                   xout, fu);
+    };
+    const bool pro = fu.agg != nullptr;
+    if (ext > SLAB_ROWS_REG || fu.fc) throw Error(BCMG_EINVAL, "slab sweeps: too many rows");
+    if (pro)
+        go(k_rows_slab<MT, VT, 1>);
+    else
+        go(k_rows_slab<MT, VT, 0>);
+    BCMG_CHECK_LAUNCH();
+}
+
+template <typename VT, int MODE>
+void slab_k(hipStream_t s, const DevCsr &A, const StencilRef<VT> &S, int m, int B, int steps,
+            int zero, DivSource div, const VT *f, const VT *xin, VT *xout,
+            const BlockFuse<VT> &fu)
+{
+    const int k = A.cls.k;
+    if (k <= 5)
+        slab_rpt<VT, 5, MODE>(s, A.n, S, m, B, steps, zero, div, f, xin, xout, fu);
+    else if (k <= 7)
+        slab_rpt<VT, 7, MODE>(s, A.n, S, m, B, steps, zero, div, f, xin, xout, fu);
+    else
+        slab_rpt<VT, CLS_ROW, MODE>(s, A.n, S, m, B, steps, zero, div, f, xin, xout, fu);
+}
+
 /* the divisor's table row, or -1 for the caller's array */
 int div_row(const DevCsr &A, DivSource div)
 {
@@ -769,9 +1017,9 @@ bool constant_stencil(RowClasses &R, const int *idx, const double *val, MaskTabl
 
 } // namespace
 
-/* operators of fewer rows relax in one workgroup (relax_block_ok) and are
-   not analysed */
-constexpr int CLS_MIN_ROWS = 4097;
+/* smaller operators are not analysed: their sweeps take a few microseconds
+   in one workgroup (relax_block_ok) as they are */
+constexpr int CLS_MIN_ROWS = 512;
 
 void make_classes(Ctx &c, const std::vector<DevCsr *> &mats)
 {
@@ -787,9 +1035,10 @@ void make_classes(Ctx &c, const std::vector<DevCsr *> &mats)
         DevCsr &A = *cand[k];
         A.cls.analysed = true;
         ClassWork *w = work.get() + k;
+        const int nblk = (A.n + BS - 1) / BS;
         k_class_clear<<<1, BS, 0, c.stream>>>(w);
-        k_class_collect<<<(A.n + BS - 1) / BS, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(),
-                                                                 A.val.get(), w);
+        k_band<<<nblk, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(), &w->band);
+        k_class_collect<<<nblk, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(), A.val.get(), w);
         k_class_tables<<<1, CLS_MAX, 0, c.stream>>>(A.maxrow, A.row.get(), A.col.get(),
                                                     A.val.get(), w);
         BCMG_CHECK_LAUNCH();
@@ -809,6 +1058,7 @@ void make_classes(Ctx &c, const std::vector<DevCsr *> &mats)
         BCMG_HIP(hipStreamSynchronize(c.stream));
         for (size_t k = b; k < e; k++) {
             const int *h = c.h_ints + 4 * (k - b);
+            cand[k]->band = h[3];
             if (h[1] == 0) found.push_back({cand[k], work.get() + k, h[2]});
         }
     }
@@ -925,6 +1175,102 @@ void launch_rows_class(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, con
     BCMG_CHECK_LAUNCH();
 }
 
+/* whether the slab kernels take A: as a constant stencil, or its rows */
+template <typename VT>
+static bool slab_stencil(const DevCsr &A, MatType mt)
+{
+    return class_ok<VT>(A, mt) && A.cls.k > 0;
+}
+
+/* Rows of its own that a workgroup takes for `steps` neighbour-reading
+   sweeps (0: they do not fit; n: one workgroup), and the launch's time as
+   measured (us): 25 bytes a row at 6 TB/s and, for each 256 workgroups, which
+   run at a time, 3.0 + 0.4 per sweep and row of a thread on a constant
+   stencil, 4.0 + 0.6 per sweep with the rows in registers. */
+template <typename VT>
+static int slab_fit(const DevCsr &A, bool st, int steps, double *us)
+{
+    const int n = A.n;
+    const long long halo = 2ll * A.band * steps;
+    const int per_cu = ((n + SLAB_CUS - 1) / SLAB_CUS + 63) / 64 * 64;
+    int ext = 0;
+    for (int e = 1024; !ext && e <= (st ? SLAB_ROWS : SLAB_ROWS_REG); e *= 2)
+        if (per_cu + halo <= e || (st && n <= e)) ext = e;
+    if (!ext && st && SLAB_ROWS - halo >= SLAB_MIN_SHARE) ext = SLAB_ROWS;
+    if (!ext) return 0;
+    const int m = st && n <= ext ? n : (int)(ext - halo);
+    const int rounds = ((n + m - 1) / m + SLAB_CUS - 1) / SLAB_CUS;
+    const double per = st ? 0.4 * (ext / 1024) : 0.6;
+    *us = 2.0 + n * (25.0 / 6.0e6) + rounds * ((st ? 1.0 : 2.0) + steps * per);
+    return m < n ? m : n;
+}
+
+/* The next of `sweeps` sweeps that go into one slab launch: the split into
+   equal launches that takes least, if it takes less than a launch a sweep
+   (3 us and 25 bytes a row at 6 TB/s). */
+template <typename VT>
+int slab_plan(const DevCsr &A, MatType mt, int sweeps, bool zero, int *m)
+{
+    *m = 0;
+    const bool st = slab_stencil<VT>(A, mt);
+    if (sweeps < 1 || A.band < 0 || A.maxrow <= 0 || A.maxrow > CLS_ROW) return 0;
+    double best = sweeps * (3.0 + A.n * (25.0 / 6.0e6));
+    int take = 0;
+    for (int parts = 1; parts <= 8 && parts <= sweeps; parts++) {
+        const int t = (sweeps + parts - 1) / parts;
+        double us = 0.0;
+        const int mm = slab_fit<VT>(A, st, t - (zero ? 1 : 0), &us);
+        if (t < 2 && mm < A.n) continue;
+        if (mm > 0 && parts * us < best) {
+            best = parts * us;
+            take = t;
+            *m = mm;
+        }
+    }
+    return take;
+}
+
+template <typename VT>
+bool slab_one(const DevCsr &A, MatType mt)
+{
+    return slab_stencil<VT>(A, mt) && A.n <= SLAB_ROWS && A.band >= 0;
+}
+
+template <typename VT>
+void launch_slab(hipStream_t s, const DevCsr &A, MatType mt, int m, int steps, bool zero,
+                 DivSource div, const VT *d, const VT *f, const VT *xin, VT *xout,
+                 const BlockFuse<VT> &fu)
+{
+    const bool one = m >= A.n, st = slab_stencil<VT>(A, mt);
+    if (m <= 0 || A.band < 0 || (st && div == DIV_ARRAY) || (one && A.n > SLAB_ROWS))
+        throw Error(BCMG_EINVAL, "slab sweeps: not an operator of that kind");
+    const int B = one ? 0 : A.band;
+    if (!one && (fu.fc || ((!zero || fu.agg) && xin == xout)))
+        throw Error(BCMG_EINVAL, "slab sweeps: in place or restricting over several workgroups");
+    const int z = zero ? 1 : 0;
+    if (one) m = A.n;
+    if (!st) {
+        if constexpr (std::is_same<VT, double>::value) {
+            rows_slab(s, A, A.val.get(), m, B, steps, z, d, f, xin, xout, fu);
+        } else {
+            if (mt == MT_F32)
+                rows_slab(s, A, A.val32.get(), m, B, steps, z, d, f, xin, xout, fu);
+            else if (mt == MT_BF16)
+                rows_slab(s, A, A.val16.get(), m, B, steps, z, d, f, xin, xout, fu);
+            else
+                rows_slab(s, A, A.val.get(), m, B, steps, z, d, f, xin, xout, fu);
+        }
+        return;
+    }
+    const StencilRef<VT> S = stencil_ref<VT>(A, mt);
+    if (fu.agg)
+        slab_k<VT, 1>(s, A, S, m, B, steps, z, div, f, xin, xout, fu);
+    else if (fu.fc)
+        slab_k<VT, 2>(s, A, S, m, B, steps, z, div, f, xin, xout, fu);
+    else
+        slab_k<VT, 0>(s, A, S, m, B, steps, z, div, f, xin, xout, fu);
+}
+
 template <typename VT>
 void launch_jacobi_zero_class(hipStream_t s, const DevCsr &A, MatType mt, const VT *f, VT *y,
                               DivSource div)
@@ -982,6 +1328,11 @@ void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const double 
     template bool class_ok<VT>(const DevCsr &, MatType);                                      \
     template void launch_rows_class<VT>(hipStream_t, const DevCsr &, MatType, RowOp,          \
                                         const VT *, const VT *, const VT *, VT *, DivSource); \
+    template int slab_plan<VT>(const DevCsr &, MatType, int, bool, int *);                    \
+    template bool slab_one<VT>(const DevCsr &, MatType);                                      \
+    template void launch_slab<VT>(hipStream_t, const DevCsr &, MatType, int, int, bool,       \
+                                  DivSource, const VT *, const VT *, const VT *, VT *,        \
+                                  const BlockFuse<VT> &);                                     \
     template void launch_jacobi_zero_class<VT>(hipStream_t, const DevCsr &, MatType,          \
                                                const VT *, VT *, DivSource);
 BCMG_INSTANTIATE_CLASS(double)
