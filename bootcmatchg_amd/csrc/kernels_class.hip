@@ -374,18 +374,6 @@ __global__ __launch_bounds__(BS) void k_rows_class(int n, ClassRef<VT> C, int dr
 
 /* ------------------------------------------------------ constant stencils */
 
-/* offsets and values of the stencil, ascending (CSR order); the entries
-   past k are never in a mask */
-template <typename VT>
-struct StencilRef {
-    const unsigned char *mask;
-    int off[CLS_ROW];
-    VT v[CLS_ROW];
-    double a[CLS_ROW];   /* magnitudes in FP64: the L1 divisor */
-    VT diag;
-    int lo, hi;          /* smallest and largest offset */
-};
-
 /* Row r's entries g[k] summed under mask m (products rounded, added left to
    right from 0), with DL1 also the row's sum of magnitudes as k_abs_rowsum
    forms it. */
@@ -798,29 +786,6 @@ ClassRef<float> class_ref<float>(const DevCsr &A, MatType mt)
 {
     return {A.cls.code.get(), A.cls.idx.get(),
             mt == MT_BF16 ? A.cls.v16.get() : A.cls.v32.get(), A.cls.n, A.cls.row};
-}
-
-template <typename VT>
-StencilRef<VT> stencil_ref(const DevCsr &A, MatType mt)
-{
-    StencilRef<VT> S;
-    const RowClasses &R = A.cls;
-    S.mask = R.code.get();
-    S.lo = R.off[0];
-    S.hi = R.off[R.k - 1];
-    S.diag = (VT)0;
-    for (int k = 0; k < CLS_ROW; k++) {
-        const bool in = k < R.k;
-        const double v = in ? R.val[k] : 0.0;
-        S.off[k] = in ? R.off[k] : 0;
-        S.a[k] = in ? std::fabs(v) : 0.0;
-        if (mt == MT_BF16)
-            S.v[k] = (VT)bf16_round((float)v);
-        else
-            S.v[k] = (VT)v;
-        if (in && R.off[k] == 0) S.diag = (VT)v;
-    }
-    return S;
 }
 
 /* rows per thread: the block stages the forms (nc (crow + 1) (4 + value)

@@ -5,6 +5,8 @@
 #pragma once
 #include "bcmg_internal.h"
 
+#include <cmath>
+
 namespace bcmg {
 
 namespace {
@@ -330,6 +332,43 @@ __device__ __forceinline__ VT pattern_row_sum(unsigned m, const PatOffsets &po,
     for (int k = 0; k < PAT_MAX; k++)
         if ((m >> k) & 1u) t = t + v[k] * g[k];
     return t;
+}
+
+/* ------------------------------------------------------ constant stencils */
+
+/* offsets and values of the stencil, ascending (CSR order); the entries
+   past k are never in a mask */
+template <typename VT>
+struct StencilRef {
+    const unsigned char *mask;
+    int off[CLS_ROW];
+    VT v[CLS_ROW];
+    double a[CLS_ROW];   /* magnitudes in FP64: the L1 divisor */
+    VT diag;
+    int lo, hi;          /* smallest and largest offset */
+};
+
+template <typename VT>
+StencilRef<VT> stencil_ref(const DevCsr &A, MatType mt)
+{
+    StencilRef<VT> S;
+    const RowClasses &R = A.cls;
+    S.mask = R.code.get();
+    S.lo = R.off[0];
+    S.hi = R.off[R.k - 1];
+    S.diag = (VT)0;
+    for (int k = 0; k < CLS_ROW; k++) {
+        const bool in = k < R.k;
+        const double v = in ? R.val[k] : 0.0;
+        S.off[k] = in ? R.off[k] : 0;
+        S.a[k] = in ? std::fabs(v) : 0.0;
+        if (mt == MT_BF16)
+            S.v[k] = (VT)bf16_round((float)v);
+        else
+            S.v[k] = (VT)v;
+        if (in && R.off[k] == 0) S.diag = (VT)v;
+    }
+    return S;
 }
 
 /* LDS of the pattern kernels: the tile's values (room for the leading

@@ -331,6 +331,60 @@ __device__ __forceinline__ vec_t<VT, W> il_row(int r, int jg, const int *__restr
     return (fo - acc) / dr + xo;
 }
 
+/* il_row on a constant stencil (the same products in the same order): the
+   offsets and values are kernel arguments, so a lane loads the row's mask
+   byte in place of the row's bounds, columns and values, which 8 lanes of a
+   32-column FP32 row each loaded for themselves. An absent entry gathers the
+   row's own columns and adds nothing. 32 FP32 columns on 2048^2: level-0
+   sweep 351 -> 286 us (5.75 TB/s of its 1.64 GB), residual 327 -> 271 us,
+   last sweep 471 -> 402 us; the vector streams bound them. */
+template <typename VT, int OP, int W, int K, bool NT = false>
+__device__ __forceinline__ vec_t<VT, W> il_row_stencil(int r, int jg, const StencilRef<VT> &S,
+                                                       const VT *__restrict__ x,
+                                                       const VT *__restrict__ f,
+                                                       const VT *__restrict__ d, int lkp)
+{
+    using V = vec_t<VT, W>;
+    const unsigned m = S.mask[r];
+    const VT *xg = x + jg * W;
+    const size_t o = ((size_t)r << lkp) + jg * W;
+    V fo = V(0), xo = V(0), g[K];
+    VT dr = VT(1);
+    if (OP != OP_SPMV) fo = ldm<NT>(reinterpret_cast<const V *>(f + o));
+    if (OP == OP_JACOBI) {
+        xo = *reinterpret_cast<const V *>(x + o);
+        dr = d[r];
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++) {
+        const int c = ((m >> k) & 1u) ? r + S.off[k] : r;
+        g[k] = *reinterpret_cast<const V *>(xg + ((size_t)c << lkp));
+    }
+    V acc = V(0);
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        if ((m >> k) & 1u) acc = acc + S.v[k] * g[k];
+    if (OP == OP_SPMV) return acc;
+    if (OP == OP_RESID) return fo - acc;
+    return (fo - acc) / dr + xo;
+}
+
+/* a lane's W columns to y, the inactive ones left as they are */
+template <typename VT, int W, bool NT>
+__device__ __forceinline__ void il_store(vec_t<VT, W> res, VT *y, bool all, unsigned cw, int jg)
+{
+    using V = vec_t<VT, W>;
+    if (all) {
+        if (NT)
+            __builtin_nontemporal_store(res, reinterpret_cast<V *>(y));
+        else
+            *reinterpret_cast<V *>(y) = res;
+    } else {
+        for (int u = 0; u < W; u++)
+            if (word_on(cw, jg * W + u)) y[u] = vget<VT, W>(res, u);
+    }
+}
+
 /* PF entries of a row are gathered at once. 7 waves per SIMD (at most 72
    VGPRs) hold without spills for every instance launched: PF 8 only with
    FP32 values and vectors, PF 6 otherwise. NT: f and y, each touched once,
@@ -354,17 +408,63 @@ __global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(7))) void k_
     group_on(jg, W, cw, any, all);
     if (!any) return;
     const V res = il_row<MT, VT, OP, W, PF, NT>(r, jg, rp, ci, av, x, f, d, lkp);
-    const size_t o = ((size_t)r << lkp) + jg * W;
-    if (all) {
-        if (NT)
-            __builtin_nontemporal_store(res, reinterpret_cast<V *>(y + o));
-        else
-            *reinterpret_cast<V *>(y + o) = res;
-    } else {
-        for (int u = 0; u < W; u++)
-            if (word_on(cw, jg * W + u)) y[o + u] = vget<VT, W>(res, u);
-    }
+    il_store<VT, W, NT>(res, y + ((size_t)r << lkp) + jg * W, all, cw, jg);
 }
+
+/* k_rows_il on a constant stencil */
+template <typename VT, int OP, int W, int K, bool NT>
+__global__ __launch_bounds__(BS) void k_rows_il_stencil(int n, StencilRef<VT> S,
+                                                        const VT *__restrict__ x,
+                                                        const VT *__restrict__ f,
+                                                        const VT *__restrict__ d,
+                                                        VT *__restrict__ y, int lkp, int nc,
+                                                        const int *__restrict__ act)
+{
+    const unsigned cw = col_word(nc, act);
+    const int gpr = (nc + W - 1) / W;
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const long t = (long)b * BS + threadIdx.x;
+    const int r = (int)(t / gpr);
+    const int jg = (int)(t % gpr);
+    if (r >= n) return;
+    bool any, all;
+    group_on(jg, W, cw, any, all);
+    if (!any) return;
+    const vec_t<VT, W> res = il_row_stencil<VT, OP, W, K, NT>(r, jg, S, x, f, d, lkp);
+    il_store<VT, W, NT>(res, y + ((size_t)r << lkp) + jg * W, all, cw, jg);
+}
+
+/* The end of the sweeps into a column-major FP64 block (below): a lane's W
+   results to columns jg W ... of row r. Every thread of the block calls it. */
+template <typename VT, int W, bool TILE, bool NT>
+__device__ __forceinline__ void c64_store(int n, int b, int gpr, int r, int jg, bool any,
+                                          unsigned cw, vec_t<VT, W> res, double *__restrict__ z,
+                                          long ldz)
+{
+    if constexpr (!TILE) {
+        if (!any) return;
+#pragma unroll
+        for (int u = 0; u < W; u++) {
+            const int j = jg * W + u;
+            if (word_on(cw, j)) st_nt<NT>(z + (size_t)j * ldz + r, (double)vget<VT, W>(res, u));
+        }
+    } else {
+        /* rows [r0, r0 + rb) of the block; column j of local row q at
+           tile[j * (rb + 1) + q] (the pad spreads a row's columns over the
+           banks) */
+        __shared__ double tile[BS * W + MULTI_MAX_COLS];
+        const int rb = BS / gpr, pitch = rb + 1;
+        const int r0 = (int)((long)b * BS / gpr);
+        const int q = threadIdx.x / gpr;
+#pragma unroll
+        for (int u = 0; u < W; u++) tile[(jg * W + u) * pitch + q] = (double)vget<VT, W>(res, u);
+        __syncthreads();
+        for (int e = threadIdx.x; e < gpr * W * rb; e += BS) {
+            const int j = e / rb, qq = e - j * rb;
+            if (r0 + qq < n && word_on(cw, j))
+                st_nt<NT>(z + (size_t)j * ldz + r0 + qq, tile[j * pitch + qq]);
+        }
+    }}
 
 /* A Jacobi/L1 sweep of k_rows_il whose result goes straight to a
    column-major FP64 block (column j at z + j ldz), widened exactly: the
@@ -390,30 +490,27 @@ __global__ __launch_bounds__(BS) void k_jacobi_il_c64(
     if (r < n) group_on(jg, W, cw, any, all);
     vec_t<VT, W> res{};
     if (any) res = il_row<MT, VT, OP_JACOBI, W, PF, NT>(r, jg, rp, ci, av, x, f, d, lkp);
-    if constexpr (!TILE) {
-        if (!any) return;
-#pragma unroll
-        for (int u = 0; u < W; u++) {
-            const int j = jg * W + u;
-            if (word_on(cw, j)) st_nt<NT>(z + (size_t)j * ldz + r, (double)vget<VT, W>(res, u));
-        }
-    } else {
-        /* rows [r0, r0 + rb) of the block; column j of local row q at
-           tile[j * (rb + 1) + q] (the pad spreads a row's columns over the
-           banks) */
-        __shared__ double tile[BS * W + MULTI_MAX_COLS];
-        const int rb = BS / gpr, pitch = rb + 1;
-        const int r0 = (int)((long)b * BS / gpr);
-        const int q = threadIdx.x / gpr;
-#pragma unroll
-        for (int u = 0; u < W; u++) tile[(jg * W + u) * pitch + q] = (double)vget<VT, W>(res, u);
-        __syncthreads();
-        for (int e = threadIdx.x; e < gpr * W * rb; e += BS) {
-            const int j = e / rb, qq = e - j * rb;
-            if (r0 + qq < n && word_on(cw, j))
-                st_nt<NT>(z + (size_t)j * ldz + r0 + qq, tile[j * pitch + qq]);
-        }
-    }
+    c64_store<VT, W, TILE, NT>(n, b, gpr, r, jg, any, cw, res, z, ldz);
+}
+
+/* k_jacobi_il_c64 on a constant stencil */
+template <typename VT, int W, int K, bool TILE, bool NT>
+__global__ __launch_bounds__(BS) void k_jacobi_il_c64_stencil(
+    int n, StencilRef<VT> S, const VT *__restrict__ x, const VT *__restrict__ f,
+    const VT *__restrict__ d, double *__restrict__ z, long ldz, int lkp, int nc,
+    const int *__restrict__ act)
+{
+    const unsigned cw = col_word(nc, act);
+    const int gpr = (nc + W - 1) / W;
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const long t = (long)b * BS + threadIdx.x;
+    const int r = (int)(t / gpr);
+    const int jg = (int)(t % gpr);
+    bool any = false, all = false;
+    if (r < n) group_on(jg, W, cw, any, all);
+    vec_t<VT, W> res{};
+    if (any) res = il_row_stencil<VT, OP_JACOBI, W, K, NT>(r, jg, S, x, f, d, lkp);
+    c64_store<VT, W, TILE, NT>(n, b, gpr, r, jg, any, cw, res, z, ldz);
 }
 
 /* group-order row sums (k_rows<G>'s arithmetic) on interleaved blocks: G
@@ -828,10 +925,11 @@ __global__ void k_fcg_scalars_multi(double *scal, int nc, int first, const int *
    and written non-temporally (the columns' streams exceed the last-level
    cache). */
 constexpr int SD_PF = 8; /* entries whose indices are loaded at once */
-template <int K, bool NT>
+template <int K, bool NT, int KS = 0>
 __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__restrict__ rp,
                                                         const int *__restrict__ ci,
-                                                        const double *__restrict__ av, FcgCols F,
+                                                        const double *__restrict__ av,
+                                                        StencilRef<double> S, FcgCols F,
                                                         int nc, const int *__restrict__ mask,
                                                         double *__restrict__ part)
 {
@@ -854,7 +952,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const long ld = F.ld;
     int ra = 0, re = 0;
-    if (own) {
+    if (KS == 0 && own) {
         ra = rp[r];
         re = rp[r + 1];
     }
@@ -862,7 +960,24 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
 #pragma unroll
     for (int u = 0; u < CH; u++) t[u] = 0.0;
     const double *zj = F.Z + (size_t)j0 * ld;
-    if (all) {
+    if constexpr (KS > 0) {
+        /* a constant stencil: an absent entry gathers the row's own element
+           and adds nothing */
+        const unsigned m = own ? S.mask[r] : 0u;
+        const int ro = own ? r : 0;
+#pragma unroll
+        for (int q = 0; q < (KS > 0 ? KS : 1); q++) {
+            const bool in = (m >> q) & 1u;
+            const int c = in ? ro + S.off[q] : ro;
+            double g[CH];
+#pragma unroll
+            for (int u = 0; u < CH; u++)
+                if (all || on[u]) g[u] = zj[(size_t)u * ld + c];
+#pragma unroll
+            for (int u = 0; u < CH; u++)
+                if (in && (all || on[u])) t[u] = t[u] + S.v[q] * g[u];
+        }
+    } else if (all) {
         /* SD_PF entries' indices and values at once, then their gathers */
         for (int e0 = ra; e0 < re; e0 += SD_PF) {
             int cc[SD_PF];
@@ -1118,12 +1233,66 @@ inline FcgCols fcg_cols(const MultiFcg &M)
 
 } // namespace
 
+template <typename MT>
+constexpr MatType il_mt()
+{
+    return std::is_same<MT, double>::value ? MT_F64
+                                           : std::is_same<MT, float>::value ? MT_F32 : MT_BF16;
+}
+
+/* whether the interleaved kernels read A as a constant stencil: with a whole
+   vector of columns a lane */
+template <typename MT, typename VT>
+bool il_stencil_ok(const DevCsr &A, int nc)
+{
+    return nc >= (int)(16 / sizeof(VT)) && class_ok<VT>(A, il_mt<MT>()) && A.cls.k > 0;
+}
+
+template <typename VT, int OP, int K>
+void rows_il_stencil(hipStream_t s, int n, const StencilRef<VT> &S, const VT *x, const VT *f,
+                     const VT *d, VT *y, int lkp, int nc, const int *act)
+{
+    constexpr int W = 16 / sizeof(VT);
+    const unsigned g = (unsigned)blocks_for((long long)n * ((nc + W - 1) / W));
+    if (((size_t)n << lkp) * sizeof(VT) > NT_BYTES)
+        k_rows_il_stencil<VT, OP, W, K, true><<<g, BS, 0, s>>>(n, S, x, f, d, y, lkp, nc, act);
+    else
+        k_rows_il_stencil<VT, OP, W, K, false><<<g, BS, 0, s>>>(n, S, x, f, d, y, lkp, nc, act);
+}
+
+template <typename VT, int K>
+void c64_stencil(hipStream_t s, int n, const StencilRef<VT> &S, const VT *x, const VT *f,
+                 const VT *d, double *z, long ldz, int lkp, int nc, const int *act)
+{
+    constexpr int W = 16 / sizeof(VT);
+    const int gpr = (nc + W - 1) / W;
+    const unsigned g = (unsigned)blocks_for((long long)n * gpr);
+    const bool nt = ((size_t)n << lkp) * sizeof(VT) > NT_BYTES;
+    auto go = [&](auto kern) { kern<<<g, BS, 0, s>>>(n, S, x, f, d, z, ldz, lkp, nc, act); };
+    if (BS % gpr == 0)
+        nt ? go(k_jacobi_il_c64_stencil<VT, W, K, true, true>)
+           : go(k_jacobi_il_c64_stencil<VT, W, K, true, false>);
+    else
+        nt ? go(k_jacobi_il_c64_stencil<VT, W, K, false, true>)
+           : go(k_jacobi_il_c64_stencil<VT, W, K, false, false>);
+}
+
 template <typename MT, typename VT, int OP>
 void rows_il_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, const VT *f,
                    const VT *d, VT *y, int lkp, int nc, const int *act)
 {
     const int n = A.n;
     const int *rp = A.row.get(), *ci = A.col.get();
+    if (il_stencil_ok<MT, VT>(A, nc)) {
+        const StencilRef<VT> S = stencil_ref<VT>(A, il_mt<MT>());
+        if (A.cls.k <= 5)
+            rows_il_stencil<VT, OP, 5>(s, n, S, x, f, d, y, lkp, nc, act);
+        else if (A.cls.k <= 7)
+            rows_il_stencil<VT, OP, 7>(s, n, S, x, f, d, y, lkp, nc, act);
+        else
+            rows_il_stencil<VT, OP, CLS_ROW>(s, n, S, x, f, d, y, lkp, nc, act);
+        return;
+    }
     if (stream_ok<VT>(A)) {
         /* W columns per lane: a lane's columns stay inside the 2^lkp stride
            (W <= nc <= 2^lkp, both powers of two, or W = 1). Entries in
@@ -1170,6 +1339,16 @@ bool jacobi_il_c64_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT 
 {
     constexpr int WM = 16 / sizeof(VT);
     if (!stream_ok<VT>(A) || nc < WM) return false;
+    if (il_stencil_ok<MT, VT>(A, nc)) {
+        const StencilRef<VT> S = stencil_ref<VT>(A, il_mt<MT>());
+        if (A.cls.k <= 5)
+            c64_stencil<VT, 5>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
+        else if (A.cls.k <= 7)
+            c64_stencil<VT, 7>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
+        else
+            c64_stencil<VT, CLS_ROW>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
+        return true;
+    }
     constexpr bool all32 = std::is_same<MT, float>::value && std::is_same<VT, float>::value;
     const bool pf8 = all32 && A.maxrow > 6 && A.maxrow <= 8;
     const int n = A.n;
@@ -1588,25 +1767,32 @@ void launch_spmv_dots_multi(Ctx &c, const DevCsr &A, int k, MultiFcg &M, const i
     const unsigned grid = (unsigned)nb * (unsigned)nch;
     /* r, the previous direction and t of every column */
     const bool nt = (size_t)n * M.nc * 3 * sizeof(double) > NT_BYTES;
-    if (k == 2) {
-        if (nt)
-            k_spmv_dots_multi<2, true><<<grid, BS, 0, c.stream>>>(n, A.row.get(), A.col.get(),
-                                                                  A.val.get(), F, M.nc, mask,
-                                                                  part);
+    const bool st = class_ok<double>(A, MT_F64) && A.cls.k > 0;
+    const StencilRef<double> S = st ? stencil_ref<double>(A, MT_F64) : StencilRef<double>{};
+    auto go = [&](auto kern) {
+        kern<<<grid, BS, 0, c.stream>>>(n, A.row.get(), A.col.get(), A.val.get(), S, F, M.nc, mask,
+                                        part);
+    };
+    /* the stencil's entries as kernel arguments (KS of them), or CSR rows */
+    auto pick = [&](auto K, auto NT) {
+        constexpr int kk = decltype(K)::value;
+        constexpr bool nn = decltype(NT)::value;
+        if (!st)
+            go(k_spmv_dots_multi<kk, nn>);
+        else if (A.cls.k <= 5)
+            go(k_spmv_dots_multi<kk, nn, 5>);
+        else if (A.cls.k <= 7)
+            go(k_spmv_dots_multi<kk, nn, 7>);
         else
-            k_spmv_dots_multi<2, false><<<grid, BS, 0, c.stream>>>(n, A.row.get(), A.col.get(),
-                                                                   A.val.get(), F, M.nc, mask,
-                                                                   part);
+            go(k_spmv_dots_multi<kk, nn, CLS_ROW>);
+    };
+    using K2 = std::integral_constant<int, 2>;
+    using K3 = std::integral_constant<int, 3>;
+    if (k == 2) {
+        nt ? pick(K2{}, std::true_type{}) : pick(K2{}, std::false_type{});
         k_fcg_final_multi<2, false><<<M.nc, RED_FINAL_BS, 0, c.stream>>>(nb, part, F, mask);
     } else {
-        if (nt)
-            k_spmv_dots_multi<3, true><<<grid, BS, 0, c.stream>>>(n, A.row.get(), A.col.get(),
-                                                                  A.val.get(), F, M.nc, mask,
-                                                                  part);
-        else
-            k_spmv_dots_multi<3, false><<<grid, BS, 0, c.stream>>>(n, A.row.get(), A.col.get(),
-                                                                   A.val.get(), F, M.nc, mask,
-                                                                   part);
+        nt ? pick(K3{}, std::true_type{}) : pick(K3{}, std::false_type{});
         k_fcg_final_multi<3, false><<<M.nc, RED_FINAL_BS, 0, c.stream>>>(nb, part, F, mask);
     }
     BCMG_CHECK_LAUNCH();

@@ -161,3 +161,26 @@ def test_solves_same_bits(ctx, name, setting, prec):
     assert out[0][0] == out[1][0] and out[0][1] == out[1][1]
     assert np.array_equal(bits(out[0][2]), bits(out[1][2]))
     dA.free()
+
+
+@pytest.mark.parametrize("prec", [bc.PREC_FP64, bc.PREC_FP32])
+@pytest.mark.parametrize("name,k", [("poisson3d_41", 2), ("aniso2d_65", 5), ("poisson3d_17", 32),
+                                    ("eight_entries_91", 11), ("neumann2d_70", 4)])
+def test_columns_equal_single_solves(ctx, name, k, prec):
+    """Several right-hand sides: whole and partly filled vectors of columns
+    a lane, on constant stencils of 5, 7 and 8 entries and on classes."""
+    A = OPERATORS[name]()
+    n = len(A[0]) - 1
+    dA = bc.Csr(ctx, A)
+    B = bc.Boot(ctx, dA, bc.make_params(**dict(SETTINGS["V_L1_2sweeps"], itnlim=25)))
+    B.set_precision(prec)
+    bs = [bc.DeviceArray.from_numpy(ctx, ops.uniform_pm1(j, n)) for j in range(k)]
+    xs = [bc.DeviceArray(ctx, n) for _ in range(k)]
+    its, res, st = B.fcg_multi(bs, xs)
+    dx = bc.DeviceArray(ctx, n)
+    for j in range(k):
+        it, r = B.fcg(bs[j], dx)
+        assert st[j] == bc.OK and its[j] == it and res[j] == r
+        assert np.array_equal(bits(xs[j].numpy()), bits(dx.numpy())), j
+    B.free()
+    dA.free()
