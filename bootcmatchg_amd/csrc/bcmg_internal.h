@@ -387,7 +387,8 @@ void launch_rows_class(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, con
 template <typename VT>
 void launch_jacobi_zero_class(hipStream_t s, const DevCsr &A, MatType mt, const VT *f, VT *y,
                               DivSource div);
-void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const double *z, double *t,
+template <typename ZT>
+void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const ZT *z, double *t,
                             const double *r, const double *to, double *part);
 void launch_rows(hipStream_t s, const DevCsr &A, RowOp op, const double *x, const double *f,
                  const double *d, double *y);
@@ -417,9 +418,12 @@ void launch_dots(Ctx &c, int n, int k, const double *a0, const double *a1, const
                  const double *b, double *out);
 /* FCG v3 scalar recurrences on device; s = [alpha, beta, gamma, delta, theta, theta2, l2, ...] */
 void launch_fcg_scalars(hipStream_t s, double *scal);
-/* z = -theta zo + z; x += theta2 z; t = -theta to + t; r += -theta2 t; scal[6] = ||r|| */
-void launch_fcg_update(Ctx &c, int n, double *scal, const double *zo, double *z, double *x,
-                       const double *to, double *t, double *r);
+/* z = -theta zo + zc; x += theta2 z; t = -theta to + t; r += -theta2 t;
+   scal[6] = ||r||; zc is z itself or an FP32 cycle's result; r32 (or null)
+   receives r in FP32 */
+template <typename ZT>
+void launch_fcg_update(Ctx &c, int n, double *scal, const double *zo, const ZT *zc, double *z,
+                       double *x, const double *to, double *t, double *r, float *r32);
 /* first FCG step: x += theta v; r -= theta w; ||r|| (theta from scal[4]) */
 void launch_fcg_first(Ctx &c, int n, double *scal, const double *v, double *x,
                       const double *w, double *r);
@@ -427,8 +431,10 @@ void launch_fcg_first(Ctx &c, int n, double *scal, const double *v, double *x,
 void launch_true_residual(Ctx &c, const DevCsr &A, const double *b, const double *x, double *y,
                           double *r, double *scal);
 /* t = A z with the FCG products of z (k = 2: r.z, t.z; k = 3: also to.z) and
-   the scalar recurrence, all on the device */
-void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const double *z, double *t,
+   the scalar recurrence, all on the device; z in FP32 (an FP32 cycle's
+   result) where rows_sequential<double>(A) */
+template <typename ZT>
+void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const ZT *z, double *t,
                       const double *r, const double *to, double *scal);
 /* K-cycle inner iteration pieces: products of VT vectors in double into
    out[0..k); alpha and the breakdown flag; w -= alpha v; the coefficients;
@@ -545,13 +551,13 @@ void launch_scale_multi(hipStream_t s, int n, VT alpha, VT *x, long ld, int nc, 
 template <typename VT>
 void launch_rows_il(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const VT *x,
                     const VT *f, const VT *d, VT *y, int lkp, int nc, const int *act);
-/* the last Jacobi/L1 sweep of a cycle with its result widened into the
-   column-major FP64 block z (column j at z + j ldz); false when the operator
+/* the last Jacobi/L1 sweep of a cycle with its result written (in FP64
+   widened) into the column-major block z (column j at z + j ldz); false when the operator
    takes the group kernel or the block is narrower than one vector (the
    caller then sweeps and converts) */
-template <typename VT>
-bool launch_jacobi_il_c64(hipStream_t s, const DevCsr &A, MatType mt, const VT *x, const VT *f,
-                          const VT *d, double *z, long ldz, int lkp, int nc, const int *act);
+template <typename VT, typename ZT>
+bool launch_jacobi_il_cm(hipStream_t s, const DevCsr &A, MatType mt, const VT *x, const VT *f,
+                         const VT *d, ZT *z, long ldz, int lkp, int nc, const int *act);
 template <typename VT>
 void launch_jacobi_zero_il(hipStream_t s, int n, const VT *f, const VT *d, VT *y, int lkp,
                            int nc, const int *act);
@@ -583,6 +589,7 @@ void launch_from_il(hipStream_t s, int n, const S *a, D *b, long ldb, int lkp, i
 struct MultiFcg {
     double *V[2] = {nullptr, nullptr}, *W[2] = {nullptr, nullptr};
     double *Z = nullptr, *R = nullptr, *X = nullptr, *B = nullptr, *Y = nullptr;
+    bool z32 = false;          /* Z holds FP32 values (an FP32 cycle's result), stride ld */
     long ld = 0;
     int nc = 0;
     double *scal = nullptr;

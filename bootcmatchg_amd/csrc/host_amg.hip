@@ -968,8 +968,13 @@ int fcg_solve(Ctx &c, Boot &B, const double *b, double *x, int *iters, double *r
         throw Error(BCMG_EZERORHS, "initial residual is zero (the reference exits)");
     }
     precond_apply(c, B, r, v, true);
-    launch_spmv_dots(c, A, 2, v, w, r, nullptr, scal);
+    launch_spmv_dots<double>(c, A, 2, v, w, r, nullptr, scal);
     launch_fcg_first(c, n, scal, v, x, w, r);
+    /* A reduced-precision iteration keeps r and z in the cycle's FP32 where
+       the cycle meets FCG: the update writes r rounded beside r, the product
+       and the update widen z as they read it (no conversion passes). */
+    const bool z32 = B.prec != BCMG_PREC_FP64 && rows_sequential<double>(A);
+    if (z32) launch_d2f(c.stream, n, r, B.r32.get());
     /* d, q take the first direction; the next one goes to the other pair */
     std::swap(v, d);
     std::swap(w, q);
@@ -983,9 +988,15 @@ int fcg_solve(Ctx &c, Boot &B, const double *b, double *x, int *iters, double *r
         double *t = even ? w : q;
         const double *zo = even ? d : v;
         const double *to = even ? q : w;
-        precond_apply(c, B, r, z, true);
-        launch_spmv_dots(c, A, 3, z, t, r, to, scal);
-        launch_fcg_update(c, n, scal, zo, z, x, to, t, r);
+        if (z32) {
+            precond_apply_t<float>(c, B, B.r32.get(), B.z32.get(), true);
+            launch_spmv_dots<float>(c, A, 3, B.z32.get(), t, r, to, scal);
+            launch_fcg_update<float>(c, n, scal, zo, B.z32.get(), z, x, to, t, r, B.r32.get());
+        } else {
+            precond_apply(c, B, r, z, true);
+            launch_spmv_dots<double>(c, A, 3, z, t, r, to, scal);
+            launch_fcg_update<double>(c, n, scal, zo, z, z, x, to, t, r, nullptr);
+        }
         BCMG_HIP(hipMemcpyAsync(c.h_scalars + 8, scal + 6, sizeof(double), hipMemcpyDeviceToHost,
                                 c.stream));
         if (kcyc)
@@ -1055,8 +1066,9 @@ int fcg_solve(Ctx &c, Boot &B, const double *b, double *x, int *iters, double *r
         if (l2 <= rtol * delta0 || iter >= max_iter || !std::isfinite(l2)) break;
         B.restarts++;
         precond_apply(c, B, r, d, true);
-        launch_spmv_dots(c, A, 2, d, q, r, nullptr, scal);
+        launch_spmv_dots<double>(c, A, 2, d, q, r, nullptr, scal);
         launch_fcg_first(c, n, scal, d, x, q, r);
+        if (z32) launch_d2f(c.stream, n, r, B.r32.get());
         BCMG_HIP(hipMemcpyAsync(c.h_scalars + 8, scal + 6, sizeof(double), hipMemcpyDeviceToHost,
                                 c.stream));
         BCMG_HIP(hipStreamSynchronize(c.stream));

@@ -152,6 +152,7 @@ MultiWork &ensure_multi_into(Ctx &c, Boot &B, MultiWork &M, int kmax)
     } else {
         M.F.kflag = nullptr;
     }
+    M.F.z32 = B.prec != BCMG_PREC_FP64 && rows_sequential<double>(*B.A0);
     M.F.nc = M.kmax;
     M.F.maxit = B.prm.itnlim;
     if (B.prec != BCMG_PREC_FP64 && M.prec != B.prec) {
@@ -190,12 +191,28 @@ struct MRun {
     int nc;
     int lkp;    /* interleave stride 2^lkp of this application */
     const int *act;
-    /* when set, the sweep that writes final_out writes its result widened
-       into this column-major FP64 block instead (and sets *fused) */
-    double *z64 = nullptr;
+    /* when set, the sweep that writes final_out writes its result into this
+       column-major block instead (FP32 with z32, else FP64 widened) and sets
+       *fused */
+    void *zcm = nullptr;
+    bool z32 = false;
     long ldz = 0;
     bool *fused = nullptr;
 };
+
+template <typename VT>
+bool sweep_cm(MRun<VT> &R, const DevCsr &A, MatType mt, const VT *x, const VT *f, const VT *d)
+{
+    if constexpr (std::is_same<VT, float>::value) {
+        if (R.z32)
+            return launch_jacobi_il_cm<float, float>(R.c.stream, A, mt, x, f, d,
+                                                     static_cast<float *>(R.zcm), R.ldz, R.lkp,
+                                                     R.nc, R.act);
+    }
+    return launch_jacobi_il_cm<VT, double>(R.c.stream, A, mt, x, f, d,
+                                           static_cast<double *>(R.zcm), R.ldz, R.lkp, R.nc,
+                                           R.act);
+}
 
 /* relax_level of host_amg.hip on an interleaved block */
 template <typename VT>
@@ -224,10 +241,8 @@ void relax_level_m(MRun<VT> &R, const Level &lv, MatType mt, int type, int sweep
         if (last && s.x != final_out) out = final_out;
         if (s.zero) {
             launch_jacobi_zero_il<VT>(c.stream, A.n, f, d, out, lkp, R.nc, R.act);
-        } else if (last && R.z64 &&
-                   launch_jacobi_il_c64<VT>(c.stream, A, mt, s.x, f, d, R.z64, R.ldz, lkp, R.nc,
-                                            R.act)) {
-            /* the result is in z64 only; final_out is not written */
+        } else if (last && R.zcm && sweep_cm<VT>(R, A, mt, s.x, f, d)) {
+            /* the result is in zcm only; final_out is not written */
             out = final_out;
             *R.fused = true;
         } else {
@@ -362,17 +377,18 @@ void run_hierarchy_m(MRun<VT> &R, int k)
         R.st[l].x2 = W.xb[l].get();
         R.st[l].zero = true;
     }
-    MRun<VT> Rk{R.c, R.B, R.M, H, R.st, R.f0, R.final_out, R.nc, R.lkp, R.act, R.z64, R.ldz,
-                R.fused};
+    MRun<VT> Rk{R.c, R.B, R.M, H, R.st, R.f0, R.final_out, R.nc, R.lkp, R.act, R.zcm, R.z32,
+                R.ldz, R.fused};
     cycle_m<VT>(Rk, 1);
 }
 
 /* precond_apply_t of host_amg.hip from x = 0 on interleaved blocks. With
-   z64, a multiplicative or symmetrized composite may deliver its result
-   widened into that column-major FP64 block instead of x; *fused tells. */
+   zcm, a multiplicative or symmetrized composite may deliver its result in
+   that column-major block (FP32 with z32, else FP64) instead of x; *fused
+   tells. */
 template <typename VT>
 void precond_m(Ctx &c, Boot &B, MultiWork &M, const VT *r, VT *x, const int *act,
-               double *z64 = nullptr, long ldz = 0, bool *fused = nullptr)
+               void *zcm = nullptr, bool z32 = false, long ldz = 0, bool *fused = nullptr)
 {
     if (fused) *fused = false;
     CycleBufs<VT> &W = mbufs<VT>(M);
@@ -395,7 +411,7 @@ void precond_m(Ctx &c, Boot &B, MultiWork &M, const VT *r, VT *x, const int *act
         for (size_t t = 0; t < order.size(); t++) {
             const bool last = (t + 1 == order.size());
             MRun<VT> R{c,   B,   M,   *B.H[order[t]], st,   r, last ? x : nullptr,
-                       nc,  lkp, act, last ? z64 : nullptr, ldz, fused};
+                       nc,  lkp, act, last ? zcm : nullptr, z32, ldz, fused};
             run_hierarchy_m<VT>(R, order[t]);
         }
         if (fused && *fused) return;
@@ -421,8 +437,10 @@ void precond_m(Ctx &c, Boot &B, MultiWork &M, const VT *r, VT *x, const int *act
 
 /* Z = B(R) for the masked slots: R is turned into the cycle's interleaved
    layout (rounded to FP32 for a reduced-precision hierarchy), the cycles run,
-   and the result comes back column-major in FP64: written there by the
-   cycle's last sweep where that sweep can, converted after otherwise */
+   and the result comes back column-major: written there by the cycle's last
+   sweep where that sweep can, converted after otherwise. An FP32 cycle's
+   result stays in FP32 (FCG's kernels widen it as they read it: 12 bytes a
+   row and column less than writing and reading it in FP64, twice) */
 void precond_block(Ctx &c, Boot &B, MultiWork &M, const int *act)
 {
     const int n = B.A0->n;
@@ -431,14 +449,19 @@ void precond_block(Ctx &c, Boot &B, MultiWork &M, const int *act)
     bool fused = false;
     if (B.prec == BCMG_PREC_FP64) {
         launch_to_il<double, double>(c.stream, n, M.F.R, ld, M.r64.get(), lkp, nc, act);
-        precond_m<double>(c, B, M, M.r64.get(), M.z64.get(), act, M.F.Z, ld, &fused);
+        precond_m<double>(c, B, M, M.r64.get(), M.z64.get(), act, M.F.Z, false, ld, &fused);
         if (!fused)
             launch_from_il<double, double>(c.stream, n, M.z64.get(), M.F.Z, ld, lkp, nc, act);
         return;
     }
     launch_to_il<double, float>(c.stream, n, M.F.R, ld, M.r32.get(), lkp, nc, act);
-    precond_m<float>(c, B, M, M.r32.get(), M.z32.get(), act, M.F.Z, ld, &fused);
-    if (!fused) launch_from_il<float, double>(c.stream, n, M.z32.get(), M.F.Z, ld, lkp, nc, act);
+    precond_m<float>(c, B, M, M.r32.get(), M.z32.get(), act, M.F.Z, M.F.z32, ld, &fused);
+    if (fused) return;
+    if (M.F.z32)
+        launch_from_il<float, float>(c.stream, n, M.z32.get(), reinterpret_cast<float *>(M.F.Z),
+                                     ld, lkp, nc, act);
+    else
+        launch_from_il<float, double>(c.stream, n, M.z32.get(), M.F.Z, ld, lkp, nc, act);
 }
 
 void upload_flags(Ctx &c, MultiWork &M)

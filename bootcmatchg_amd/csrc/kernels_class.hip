@@ -305,9 +305,9 @@ __device__ __forceinline__ void class_stage(const ClassRef<VT> &C, int drow, VT 
 /* Row r's sum from its form: all gathers go out at once (an absent entry
    gathers the row's own element and adds nothing), the products are rounded
    and added left to right from 0 in storage order (staged_row_sum's bits). */
-template <typename VT, int CR>
+template <typename VT, int CR, typename XT = VT>
 __device__ __forceinline__ VT class_row_sum(int c, int nc, int crow, const VT *lv, const int *li,
-                                            const VT *__restrict__ x, int r)
+                                            const XT *__restrict__ x, int r)
 {
     const int len = li[c];
     VT g[CR], v[CR];
@@ -323,7 +323,7 @@ __device__ __forceinline__ VT class_row_sum(int c, int nc, int crow, const VT *l
         }
     }
 #pragma unroll
-    for (int k = 0; k < CR; k++) g[k] = x[j[k]];
+    for (int k = 0; k < CR; k++) g[k] = (VT)x[j[k]];
     VT t = 0;
 #pragma unroll
     for (int k = 0; k < CR; k++) t = k < len ? t + v[k] * g[k] : t;
@@ -396,8 +396,8 @@ __device__ __forceinline__ void stencil_sum(unsigned m, const StencilRef<VT> &S,
    W = 1). INNER: every r + off + W - 1 lies in [0, n), so the loads are
    unconditional 16-byte ones (any alignment of VT); else each element is
    loaded where its index is in range and its mask bit set. */
-template <typename VT, int K, int W, bool INNER>
-__device__ __forceinline__ void stencil_gather(const StencilRef<VT> &S, const VT *__restrict__ x,
+template <typename VT, int K, int W, bool INNER, typename XT = VT>
+__device__ __forceinline__ void stencil_gather(const StencilRef<VT> &S, const XT *__restrict__ x,
                                                int r, int n, const unsigned (&m)[W],
                                                VT (&g)[W][K])
 {
@@ -407,8 +407,9 @@ __device__ __forceinline__ void stencil_gather(const StencilRef<VT> &S, const VT
 #pragma unroll
         for (int k = 0; k < K; k++) {
             if constexpr (W == 1) {
-                g[0][k] = x[r + S.off[k]];
+                g[0][k] = (VT)x[r + S.off[k]];
             } else {
+                static_assert(std::is_same<XT, VT>::value, "wide gathers read x's own type");
                 const vec q = *reinterpret_cast<const uvec *>(x + r + S.off[k]);
 #pragma unroll
                 for (int w = 0; w < W; w++) g[w][k] = q[w];
@@ -420,7 +421,7 @@ __device__ __forceinline__ void stencil_gather(const StencilRef<VT> &S, const VT
 #pragma unroll
             for (int k = 0; k < K; k++) {
                 g[w][k] = 0;
-                if (r + w < n && ((m[w] >> k) & 1u)) g[w][k] = x[r + w + S.off[k]];
+                if (r + w < n && ((m[w] >> k) & 1u)) g[w][k] = (VT)x[r + w + S.off[k]];
             }
     }
 }
@@ -507,9 +508,9 @@ __global__ __launch_bounds__(BS) void k_rows_stencil(int n, StencilRef<VT> S,
 }
 
 /* k_spmv_dots on a constant stencil (the same 256-row blocks and trees) */
-template <int K, int KO>
+template <int K, int KO, typename ZT>
 __global__ __launch_bounds__(BS) void k_spmv_dots_stencil(int n, StencilRef<double> S,
-                                                          const double *__restrict__ z,
+                                                          const ZT *__restrict__ z,
                                                           double *__restrict__ t,
                                                           const double *__restrict__ rv,
                                                           const double *__restrict__ to,
@@ -524,9 +525,9 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_stencil(int n, StencilRef<doub
     auto row = [&](auto inner) {
         const unsigned m[1] = {S.mask[r]};
         double g[1][KO];
-        const double zr = z[r], rr = rv[r];
+        const double zr = (double)z[r], rr = rv[r];
         const double tor = K > 2 ? to[r] : 0.0;
-        stencil_gather<double, KO, 1, decltype(inner)::value>(S, z, r, n, m, g);
+        stencil_gather<double, KO, 1, decltype(inner)::value, ZT>(S, z, r, n, m, g);
         double tr, unused;
         stencil_sum<double, KO, false>(m[0], S, g[0], tr, unused);
         t[r] = tr;
@@ -744,9 +745,9 @@ __global__ __launch_bounds__(BS) void k_jz_class(int n, ClassRef<VT> C, int drow
 
 /* k_spmv_dots on row classes: t = A z, per 256-row block the partial sums
    of r.z, t.z and (K = 3) to.z over the same rows in the same tree */
-template <int K, int CR>
+template <int K, int CR, typename ZT>
 __global__ __launch_bounds__(BS) void k_spmv_dots_class(int n, ClassRef<double> C,
-                                                        const double *__restrict__ z,
+                                                        const ZT *__restrict__ z,
                                                         double *__restrict__ t,
                                                         const double *__restrict__ rv,
                                                         const double *__restrict__ to,
@@ -763,9 +764,9 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_class(int n, ClassRef<double> 
     __syncthreads();
     if (r < n) {
         const int c = C.code[r];
-        const double zr = z[r], rr = rv[r];
+        const double zr = (double)z[r], rr = rv[r];
         const double tor = K > 2 ? to[r] : 0.0;
-        const double tr = class_row_sum<double, CR>(c, C.nc, C.crow, lv, li, z, r);
+        const double tr = class_row_sum<double, CR, ZT>(c, C.nc, C.crow, lv, li, z, r);
         t[r] = tr;
         sdot[0] = rr * zr;
         sdot[1] = tr * zr;
@@ -1254,32 +1255,33 @@ void launch_jacobi_zero_class(hipStream_t s, const DevCsr &A, MatType mt, const 
     BCMG_CHECK_LAUNCH();
 }
 
-template <int K>
-static void spmv_dots_class_k(hipStream_t s, const DevCsr &A, const double *z, double *t,
+template <int K, typename ZT>
+static void spmv_dots_class_k(hipStream_t s, const DevCsr &A, const ZT *z, double *t,
                               const double *r, const double *to, double *part)
 {
     const int nb = (A.n + BS - 1) / BS;
     if (A.cls.k > 0) {
         const StencilRef<double> S = stencil_ref<double>(A, MT_F64);
         if (A.cls.k <= 5)
-            k_spmv_dots_stencil<K, 5><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
+            k_spmv_dots_stencil<K, 5, ZT><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
         else if (A.cls.k <= 7)
-            k_spmv_dots_stencil<K, 7><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
+            k_spmv_dots_stencil<K, 7, ZT><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
         else
-            k_spmv_dots_stencil<K, CLS_ROW><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
+            k_spmv_dots_stencil<K, CLS_ROW, ZT><<<nb, BS, 0, s>>>(A.n, S, z, t, r, to, part);
         return;
     }
     const ClassRef<double> C = class_ref<double>(A, MT_F64);
     const size_t lds = class_lds_bytes<double>(C.nc, C.crow);
     if (C.crow <= 5)
-        k_spmv_dots_class<K, 5><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
+        k_spmv_dots_class<K, 5, ZT><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
     else if (C.crow <= 7)
-        k_spmv_dots_class<K, 7><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
+        k_spmv_dots_class<K, 7, ZT><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
     else
-        k_spmv_dots_class<K, CLS_ROW><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
+        k_spmv_dots_class<K, CLS_ROW, ZT><<<nb, BS, lds, s>>>(A.n, C, z, t, r, to, part);
 }
 
-void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const double *z, double *t,
+template <typename ZT>
+void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const ZT *z, double *t,
                             const double *r, const double *to, double *part)
 {
     if (k == 2)
@@ -1288,6 +1290,10 @@ void launch_spmv_dots_class(hipStream_t s, const DevCsr &A, int k, const double 
         spmv_dots_class_k<3>(s, A, z, t, r, to, part);
     BCMG_CHECK_LAUNCH();
 }
+template void launch_spmv_dots_class<double>(hipStream_t, const DevCsr &, int, const double *,
+                                             double *, const double *, const double *, double *);
+template void launch_spmv_dots_class<float>(hipStream_t, const DevCsr &, int, const float *,
+                                            double *, const double *, const double *, double *);
 
 #define BCMG_INSTANTIATE_CLASS(VT)                                                            \
     template bool class_ok<VT>(const DevCsr &, MatType);                                      \

@@ -60,6 +60,15 @@ __device__ __forceinline__ T ldm(const T *p)
     return *p;
 }
 
+template <bool NT, typename T>
+__device__ __forceinline__ void st_nt(T *p, T v)
+{
+    if (NT)
+        __builtin_nontemporal_store(v, p);
+    else
+        *p = v;
+}
+
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 
 /* Staged LDS layout: element e of a block's source range [e0, e1) sits at
@@ -186,11 +195,12 @@ __device__ __forceinline__ void stage_entries(const IT *__restrict__ ci,
    entries in flight, and p = a_ij x_j (rounded) is added left to right from
    0 - the serial order. With short columns the stored value is the offset
    from the thread's row r. FZ gathers f_j / d_j in place of x_j (the
-   iterate of one sweep from zero, rounded as that sweep rounds it). */
-template <typename MT, typename VT, typename IT = int, bool FZ = false>
+   iterate of one sweep from zero, rounded as that sweep rounds it). x may be
+   stored in a narrower type than the sum's (widened exactly). */
+template <typename MT, typename VT, typename IT = int, bool FZ = false, typename XT = VT>
 __device__ __forceinline__ VT staged_row_sum(const IT *__restrict__ lcol,
                                              const MT *__restrict__ lval,
-                                             const VT *__restrict__ x, int kc, int kv, int len,
+                                             const XT *__restrict__ x, int kc, int kv, int len,
                                              int r = 0, const VT *__restrict__ zf = nullptr,
                                              const VT *__restrict__ zd = nullptr)
 {
@@ -224,7 +234,7 @@ __device__ __forceinline__ VT staged_row_sum(const IT *__restrict__ lcol,
         } else {
 #pragma unroll
             for (int u = 0; u < PF; u++)
-                if (u < kn) g[u] = x[c[u]];
+                if (u < kn) g[u] = (VT)x[c[u]];
         }
 #pragma unroll
         for (int u = 0; u < PF; u++)
@@ -299,10 +309,10 @@ __device__ __forceinline__ void pattern_block_rows(unsigned w, unsigned &m, int 
    set bit; all gathers go out at once and p = a_ij x_j (rounded) is added in
    that order - the CSR order, so the sum is staged_row_sum's bit for bit
    (FZ as there). */
-template <typename MT, typename VT, bool FZ = false>
+template <typename MT, typename VT, bool FZ = false, typename XT = VT>
 __device__ __forceinline__ VT pattern_row_sum(unsigned m, const PatOffsets &po,
                                               const MT *__restrict__ lv,
-                                              const VT *__restrict__ x, int r,
+                                              const XT *__restrict__ x, int r,
                                               const VT *__restrict__ zf = nullptr,
                                               const VT *__restrict__ zd = nullptr)
 {
@@ -315,7 +325,7 @@ __device__ __forceinline__ VT pattern_row_sum(unsigned m, const PatOffsets &po,
             if constexpr (FZ)
                 g[k] = zf[c];
             else
-                g[k] = x[c];
+                g[k] = (VT)x[c];
         }
     }
     if constexpr (FZ) {
@@ -440,21 +450,97 @@ __device__ __forceinline__ void kcycle_coef_apply(double *ks, double rtol)
     ks[9] = tau3 / tau4;
 }
 
+/* Sums of N values over the 64 lanes of a wave in the tree of
+   `for o = 32 .. 1: v += __shfl_down(v, o)` (lane 0's result: operands may
+   change places, a sum of two does not depend on it). The exchanges stay in
+   the vector registers: the halves of two values are exchanged in one swap
+   (lanes below 32 go on with the first, those above with the second; then
+   the same with rows of 16), and the steps inside a row are DPP moves, where
+   __shfl_down goes through the LDS unit (12 of its instructions a value;
+   with 24 values a wave, the 8-column FCG product spent a third of its time
+   there). N is padded to a multiple of 4: v[p] of row t (16 lanes each)
+   then holds the sum of value 4 p + 2 (t & 1) + (t >> 1). */
+__device__ __forceinline__ double dpair(unsigned hi, unsigned lo)
+{
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+template <bool ROWS>
+__device__ __forceinline__ double swap_add(double a, double b)
+{
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a);
+    const unsigned long long y = (unsigned long long)__double_as_longlong(b);
+    const unsigned xl = (unsigned)x, xh = (unsigned)(x >> 32);
+    const unsigned yl = (unsigned)y, yh = (unsigned)(y >> 32);
+    if constexpr (ROWS) {
+        const auto l = __builtin_amdgcn_permlane16_swap(xl, yl, false, false);
+        const auto h = __builtin_amdgcn_permlane16_swap(xh, yh, false, false);
+        return dpair(h[0], l[0]) + dpair(h[1], l[1]);
+    } else {
+        const auto l = __builtin_amdgcn_permlane32_swap(xl, yl, false, false);
+        const auto h = __builtin_amdgcn_permlane32_swap(xh, yh, false, false);
+        return dpair(h[0], l[0]) + dpair(h[1], l[1]);
+    }
+}
+
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double a)
+{
+    const unsigned long long x = (unsigned long long)__double_as_longlong(a);
+    const int l = __builtin_amdgcn_mov_dpp((int)(unsigned)x, CTRL, 0xf, 0xf, true);
+    const int h = __builtin_amdgcn_mov_dpp((int)(unsigned)(x >> 32), CTRL, 0xf, 0xf, true);
+    return dpair((unsigned)h, (unsigned)l);
+}
+
+/* sum over each row of 16 lanes: partners at distance 8 (rotation), 4 (mirror
+   of 8 lanes, then of 4), 2 and 1 */
+__device__ __forceinline__ double row_sum(double v)
+{
+    constexpr int ROR8 = 0x128, HALF_MIRROR = 0x141;
+    constexpr int QUAD_3210 = 0x1B, QUAD_2301 = 0x4E, QUAD_1032 = 0xB1;
+    v += dpp_move<ROR8>(v);
+    v += dpp_move<QUAD_3210>(dpp_move<HALF_MIRROR>(v));
+    v += dpp_move<QUAD_2301>(v);
+    v += dpp_move<QUAD_1032>(v);
+    return v;
+}
+
+template <int N>
+__device__ __forceinline__ void wave_sums(double (&v)[N])
+{
+    static_assert(N % 4 == 0, "values in fours");
+#pragma unroll
+    for (int p = 0; p < N / 2; p++) v[p] = swap_add<false>(v[2 * p], v[2 * p + 1]);
+#pragma unroll
+    for (int p = 0; p < N / 4; p++) v[p] = row_sum(swap_add<true>(v[2 * p], v[2 * p + 1]));
+}
+
+/* the wave's sums of K values into sh[k][wid] (from the first lane of a row) */
+template <int K, int NW>
+__device__ __forceinline__ void wave_sums_store(const double (&s)[K], double (&sh)[K][NW], int wid)
+{
+    constexpr int N = (K + 3) / 4 * 4;
+    double v[N];
+#pragma unroll
+    for (int k = 0; k < N; k++) v[k] = k < K ? s[k < K ? k : 0] : 0.0;
+    wave_sums(v);
+    const int lane = threadIdx.x & 63;
+    if ((lane & 15) == 0) {
+        const int row = lane >> 4;
+#pragma unroll
+        for (int p = 0; p < N / 4; p++) {
+            const int k = 4 * p + 2 * (row & 1) + (row >> 1);
+            if (k < K) sh[k][wid] = v[p];
+        }
+    }
+}
+
 /* fixed-order block reduction of K partial sums; thread 0 writes out[0..K) */
 template <int K>
 __device__ __forceinline__ void block_reduce_store(double (&s)[K], double *out)
 {
     __shared__ double sh[K][BS / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s[k] += __shfl_down(s[k], o, 64);
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < K; k++) sh[k][wid] = s[k];
-    }
+    wave_sums_store<K, BS / 64>(s, sh, threadIdx.x >> 6);
     __syncthreads();
     if (threadIdx.x == 0) {
 #pragma unroll
@@ -519,21 +605,25 @@ __device__ __forceinline__ bool fcg_final_sum(int nb, const double *__restrict__
     double s[K];
 #pragma unroll
     for (int k = 0; k < K; k++) s[k] = 0.0;
-    for (int b = threadIdx.x; b < nb; b += RED_FINAL_BS) {
+    /* U partials of a thread in flight, added in the same order */
+    constexpr int U = 8;
+    for (int b0 = threadIdx.x; b0 < nb; b0 += U * RED_FINAL_BS) {
+        double v[U][K];
 #pragma unroll
-        for (int k = 0; k < K; k++) s[k] += part[(size_t)b * K + k];
+        for (int u = 0; u < U; u++) {
+            const int b = b0 + u * RED_FINAL_BS;
+#pragma unroll
+            for (int k = 0; k < K; k++) v[u][k] = b < nb ? part[(size_t)b * K + k] : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (b0 + u * RED_FINAL_BS < nb) {
+#pragma unroll
+                for (int k = 0; k < K; k++) s[k] += v[u][k];
+            }
     }
     __shared__ double sh[K][RED_FINAL_BS / 64];
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int k = 0; k < K; k++) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s[k] += __shfl_down(s[k], o, 64);
-    }
-    if (lane == 0) {
-#pragma unroll
-        for (int k = 0; k < K; k++) sh[k][wid] = s[k];
-    }
+    wave_sums_store<K, RED_FINAL_BS / 64>(s, sh, threadIdx.x >> 6);
     __syncthreads();
     if (threadIdx.x != 0) return false;
 #pragma unroll

@@ -47,15 +47,6 @@ __device__ __forceinline__ bool word_on(unsigned w, int j)
     return j < 32 && ((w >> j) & 1u) != 0;
 }
 
-template <bool NT, typename T>
-__device__ __forceinline__ void st_nt(T *p, T v)
-{
-    if (NT)
-        __builtin_nontemporal_store(v, p);
-    else
-        *p = v;
-}
-
 /* Stream-order row kernel (the arithmetic of k_rows_staged): one row per
    thread and CH columns per block row (chunk blockIdx.y); p = a_ij * x_j
    rounded, then added left to right from 0.
@@ -436,28 +427,28 @@ __global__ __launch_bounds__(BS) void k_rows_il_stencil(int n, StencilRef<VT> S,
 
 /* The end of the sweeps into a column-major FP64 block (below): a lane's W
    results to columns jg W ... of row r. Every thread of the block calls it. */
-template <typename VT, int W, bool TILE, bool NT>
-__device__ __forceinline__ void c64_store(int n, int b, int gpr, int r, int jg, bool any,
-                                          unsigned cw, vec_t<VT, W> res, double *__restrict__ z,
-                                          long ldz)
+template <typename VT, typename ZT, int W, bool TILE, bool NT>
+__device__ __forceinline__ void cm_store(int n, int b, int gpr, int r, int jg, bool any,
+                                         unsigned cw, vec_t<VT, W> res, ZT *__restrict__ z,
+                                         long ldz)
 {
     if constexpr (!TILE) {
         if (!any) return;
 #pragma unroll
         for (int u = 0; u < W; u++) {
             const int j = jg * W + u;
-            if (word_on(cw, j)) st_nt<NT>(z + (size_t)j * ldz + r, (double)vget<VT, W>(res, u));
+            if (word_on(cw, j)) st_nt<NT>(z + (size_t)j * ldz + r, (ZT)vget<VT, W>(res, u));
         }
     } else {
         /* rows [r0, r0 + rb) of the block; column j of local row q at
            tile[j * (rb + 1) + q] (the pad spreads a row's columns over the
            banks) */
-        __shared__ double tile[BS * W + MULTI_MAX_COLS];
+        __shared__ ZT tile[BS * W + MULTI_MAX_COLS];
         const int rb = BS / gpr, pitch = rb + 1;
         const int r0 = (int)((long)b * BS / gpr);
         const int q = threadIdx.x / gpr;
 #pragma unroll
-        for (int u = 0; u < W; u++) tile[(jg * W + u) * pitch + q] = (double)vget<VT, W>(res, u);
+        for (int u = 0; u < W; u++) tile[(jg * W + u) * pitch + q] = (ZT)vget<VT, W>(res, u);
         __syncthreads();
         for (int e = threadIdx.x; e < gpr * W * rb; e += BS) {
             const int j = e / rb, qq = e - j * rb;
@@ -467,18 +458,18 @@ __device__ __forceinline__ void c64_store(int n, int b, int gpr, int r, int jg, 
     }}
 
 /* A Jacobi/L1 sweep of k_rows_il whose result goes straight to a
-   column-major FP64 block (column j at z + j ldz), widened exactly: the
+   column-major block (column j at z + j ldz; in FP64 widened exactly): the
    last sweep of a cycle hands its result to FCG this way instead of writing
    the interleaved block and converting it after. When the lanes per row
    divide the block (TILE), the block's rows are whole: the results pass
    through LDS so that each column's rows leave as one contiguous run;
    otherwise every lane stores its own columns. No thread leaves before the
    barrier. NT: f is read and z written non-temporally. */
-template <typename MT, typename VT, int W, int PF, bool TILE, bool NT>
-__global__ __launch_bounds__(BS) void k_jacobi_il_c64(
+template <typename MT, typename VT, typename ZT, int W, int PF, bool TILE, bool NT>
+__global__ __launch_bounds__(BS) void k_jacobi_il_cm(
     int n, const int *__restrict__ rp, const int *__restrict__ ci, const MT *__restrict__ av,
     const VT *__restrict__ x, const VT *__restrict__ f, const VT *__restrict__ d,
-    double *__restrict__ z, long ldz, int lkp, int nc, const int *__restrict__ act)
+    ZT *__restrict__ z, long ldz, int lkp, int nc, const int *__restrict__ act)
 {
     const unsigned cw = col_word(nc, act);
     const int gpr = (nc + W - 1) / W;
@@ -490,14 +481,14 @@ __global__ __launch_bounds__(BS) void k_jacobi_il_c64(
     if (r < n) group_on(jg, W, cw, any, all);
     vec_t<VT, W> res{};
     if (any) res = il_row<MT, VT, OP_JACOBI, W, PF, NT>(r, jg, rp, ci, av, x, f, d, lkp);
-    c64_store<VT, W, TILE, NT>(n, b, gpr, r, jg, any, cw, res, z, ldz);
+    cm_store<VT, ZT, W, TILE, NT>(n, b, gpr, r, jg, any, cw, res, z, ldz);
 }
 
-/* k_jacobi_il_c64 on a constant stencil */
-template <typename VT, int W, int K, bool TILE, bool NT>
-__global__ __launch_bounds__(BS) void k_jacobi_il_c64_stencil(
+/* k_jacobi_il_cm on a constant stencil */
+template <typename VT, typename ZT, int W, int K, bool TILE, bool NT>
+__global__ __launch_bounds__(BS) void k_jacobi_il_cm_stencil(
     int n, StencilRef<VT> S, const VT *__restrict__ x, const VT *__restrict__ f,
-    const VT *__restrict__ d, double *__restrict__ z, long ldz, int lkp, int nc,
+    const VT *__restrict__ d, ZT *__restrict__ z, long ldz, int lkp, int nc,
     const int *__restrict__ act)
 {
     const unsigned cw = col_word(nc, act);
@@ -510,7 +501,7 @@ __global__ __launch_bounds__(BS) void k_jacobi_il_c64_stencil(
     if (r < n) group_on(jg, W, cw, any, all);
     vec_t<VT, W> res{};
     if (any) res = il_row_stencil<VT, OP_JACOBI, W, K, NT>(r, jg, S, x, f, d, lkp);
-    c64_store<VT, W, TILE, NT>(n, b, gpr, r, jg, any, cw, res, z, ldz);
+    cm_store<VT, ZT, W, TILE, NT>(n, b, gpr, r, jg, any, cw, res, z, ldz);
 }
 
 /* group-order row sums (k_rows<G>'s arithmetic) on interleaved blocks: G
@@ -923,9 +914,11 @@ __global__ void k_fcg_scalars_multi(double *scal, int nc, int first, const int *
    rows that the first chunk brings into that XCD's L2 serve the others.
    NT: r, the previous direction and t, touched once per launch, are read
    and written non-temporally (the columns' streams exceed the last-level
-   cache). */
+   cache). 2048^2 x 32: 1.17 ms with z in FP64 and __shfl_down sums, 1.00 with
+   an FP32 cycle's z read as it is, 0.88 with the sums in registers
+   (4.0 GB at 4.5 TB/s). */
 constexpr int SD_PF = 8; /* entries whose indices are loaded at once */
-template <int K, bool NT, int KS = 0>
+template <int K, bool NT, typename ZT, int KS = 0>
 __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__restrict__ rp,
                                                         const int *__restrict__ ci,
                                                         const double *__restrict__ av,
@@ -933,7 +926,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
                                                         int nc, const int *__restrict__ mask,
                                                         double *__restrict__ part)
 {
-    __shared__ double sh[CH][K][BS / 64];
+    __shared__ double sh[CH * K][BS / 64];
     const int L = xcd_block(blockIdx.x, gridDim.x);
     const int nch = (nc + CH - 1) / CH, nb = (int)(gridDim.x / nch);
     const int b = L / nch;
@@ -949,7 +942,6 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
     if (!any) return;
     const int r = b * BS + threadIdx.x;
     const bool own = r < n;
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     const long ld = F.ld;
     int ra = 0, re = 0;
     if (KS == 0 && own) {
@@ -959,7 +951,8 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
     double t[CH];
 #pragma unroll
     for (int u = 0; u < CH; u++) t[u] = 0.0;
-    const double *zj = F.Z + (size_t)j0 * ld;
+    const ZT *const Z = reinterpret_cast<const ZT *>(F.Z);
+    const ZT *zj = Z + (size_t)j0 * ld;
     if constexpr (KS > 0) {
         /* a constant stencil: an absent entry gathers the row's own element
            and adds nothing */
@@ -969,13 +962,13 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
         for (int q = 0; q < (KS > 0 ? KS : 1); q++) {
             const bool in = (m >> q) & 1u;
             const int c = in ? ro + S.off[q] : ro;
-            double g[CH];
+            ZT g[CH];
 #pragma unroll
             for (int u = 0; u < CH; u++)
                 if (all || on[u]) g[u] = zj[(size_t)u * ld + c];
 #pragma unroll
             for (int u = 0; u < CH; u++)
-                if (in && (all || on[u])) t[u] = t[u] + S.v[q] * g[u];
+                if (in && (all || on[u])) t[u] = t[u] + S.v[q] * (double)g[u];
         }
     } else if (all) {
         /* SD_PF entries' indices and values at once, then their gathers */
@@ -992,11 +985,11 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
 #pragma unroll
             for (int q = 0; q < SD_PF; q++) {
                 if (e0 + q >= re) break;
-                double g[CH];
+                ZT g[CH];
 #pragma unroll
                 for (int u = 0; u < CH; u++) g[u] = zj[(size_t)u * ld + cc[q]];
 #pragma unroll
-                for (int u = 0; u < CH; u++) t[u] = t[u] + vv[q] * g[u];
+                for (int u = 0; u < CH; u++) t[u] = t[u] + vv[q] * (double)g[u];
             }
         }
     } else {
@@ -1005,41 +998,28 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
             const double v = av[e];
 #pragma unroll
             for (int u = 0; u < CH; u++)
-                if (on[u]) t[u] = t[u] + v * zj[(size_t)u * ld + c];
+                if (on[u]) t[u] = t[u] + v * (double)zj[(size_t)u * ld + c];
         }
     }
+    double sd[CH * K];
+#pragma unroll
+    for (int q = 0; q < CH * K; q++) sd[q] = 0.0;
 #pragma unroll
     for (int u = 0; u < CH; u++) {
-        if (!on[u]) continue;
+        if (!on[u] || !own) continue;
         const int j = j0 + u;
-        double sd[K];
-#pragma unroll
-        for (int k = 0; k < K; k++) sd[k] = 0.0;
-        if (own) {
-            const size_t o = (size_t)j * ld + r;
-            const int p = F.par[j];
-            const double zr = F.Z[o];
-            const double rr = ldm<NT>(F.R + o);
-            double *tv = slot(F.W0, F.W1, K == 2 ? 0 : (p ^ 1), j, ld);
-            if (NT)
-                __builtin_nontemporal_store(t[u], tv + r);
-            else
-                tv[r] = t[u];
-            sd[0] = rr * zr;
-            sd[1] = t[u] * zr;
-            if constexpr (K > 2) sd[K - 1] = ldm<NT>(slot(F.W0, F.W1, p, j, ld) + r) * zr;
-        }
-        /* the in-wave part of block_reduce_store<K> */
-#pragma unroll
-        for (int k = 0; k < K; k++) {
-#pragma unroll
-            for (int o = 32; o > 0; o >>= 1) sd[k] += __shfl_down(sd[k], o, 64);
-        }
-        if (lane == 0) {
-#pragma unroll
-            for (int k = 0; k < K; k++) sh[u][k][wid] = sd[k];
-        }
+        const size_t o = (size_t)j * ld + r;
+        const int p = F.par[j];
+        const double zr = (double)Z[o];
+        const double rr = ldm<NT>(F.R + o);
+        double *tv = slot(F.W0, F.W1, K == 2 ? 0 : (p ^ 1), j, ld);
+        st_nt<NT>(tv + r, t[u]);
+        sd[u * K] = rr * zr;
+        sd[u * K + 1] = t[u] * zr;
+        if constexpr (K > 2) sd[u * K + K - 1] = ldm<NT>(slot(F.W0, F.W1, p, j, ld) + r) * zr;
     }
+    /* the in-wave part of block_reduce_store<K>, all columns at once */
+    wave_sums_store<CH * K, BS / 64>(sd, sh, threadIdx.x >> 6);
     __syncthreads();
     /* the cross-wave part: thread u sums column j0 + u's wave results */
     const int u = threadIdx.x;
@@ -1048,7 +1028,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
 #pragma unroll
         for (int k = 0; k < K; k++) {
             double tt = 0.0;
-            for (int w = 0; w < BS / 64; w++) tt += sh[u][k][w];
+            for (int w = 0; w < BS / 64; w++) tt += sh[u * K + k][w];
             out[k] = tt;
         }
     }
@@ -1089,7 +1069,7 @@ __global__ __launch_bounds__(RED_FINAL_BS) void k_fcg_final_multi(int nb,
    new pair, x += theta2 z; t = -theta to + t; r += -theta2 t; ||r||^2.
    NT: the columns' ten streams exceed the last-level cache, so they are read
    and written non-temporally. */
-template <bool NT>
+template <bool NT, typename ZT>
 __global__ __launch_bounds__(BS) void k_fcg_update_multi(int n, FcgCols F,
                                                          double *__restrict__ part)
 {
@@ -1101,14 +1081,14 @@ __global__ __launch_bounds__(BS) void k_fcg_update_multi(int n, FcgCols F,
     const int p = F.par[j], q = p ^ 1;
     const double *zo = slot(F.V0, F.V1, p, j, ld);
     double *zn = slot(F.V0, F.V1, q, j, ld);
-    const double *zc = F.Z + (size_t)j * ld;
+    const ZT *zc = reinterpret_cast<const ZT *>(F.Z) + (size_t)j * ld;
     const double *to = slot(F.W0, F.W1, p, j, ld);
     double *t = slot(F.W0, F.W1, q, j, ld);
     double *x = F.X + (size_t)j * ld;
     double *r = F.R + (size_t)j * ld;
     double s[1] = {0.0};
     for (int i = blockIdx.x * BS + threadIdx.x; i < n; i += gridDim.x * BS) {
-        const double zi = fma(-theta, ldm<NT>(zo + i), ldm<NT>(zc + i));
+        const double zi = fma(-theta, ldm<NT>(zo + i), (double)ldm<NT>(zc + i));
         const double xi = fma(theta2, zi, ldm<NT>(x + i));
         const double ti = fma(-theta, ldm<NT>(to + i), ldm<NT>(t + i));
         const double ri = fma(-theta2, ti, ldm<NT>(r + i));
@@ -1130,6 +1110,7 @@ __global__ __launch_bounds__(BS) void k_fcg_update_multi(int n, FcgCols F,
 
 /* first FCG step (the arithmetic of k_fcg_first): the direction Z moves to
    pair 0, x += theta v, r -= theta w, ||r||^2 */
+template <typename ZT>
 __global__ __launch_bounds__(BS) void k_fcg_first_multi(int n, FcgCols F,
                                                         const int *__restrict__ mask,
                                                         double *__restrict__ part)
@@ -1138,14 +1119,14 @@ __global__ __launch_bounds__(BS) void k_fcg_first_multi(int n, FcgCols F,
     if (!mask[j]) return;
     const long ld = F.ld;
     const double theta = F.scal[(size_t)j * 8 + 4];
-    const double *v = F.Z + (size_t)j * ld;
+    const ZT *v = reinterpret_cast<const ZT *>(F.Z) + (size_t)j * ld;
     double *vs = F.V0 + (size_t)j * ld;
     const double *w = F.W0 + (size_t)j * ld;
     double *x = F.X + (size_t)j * ld;
     double *r = F.R + (size_t)j * ld;
     double s[1] = {0.0};
     for (int i = blockIdx.x * BS + threadIdx.x; i < n; i += gridDim.x * BS) {
-        const double vi = v[i];
+        const double vi = (double)v[i];
         vs[i] = vi;
         x[i] = fma(theta, vi, x[i]);
         const double ri = fma(-theta, w[i], r[i]);
@@ -1260,9 +1241,9 @@ void rows_il_stencil(hipStream_t s, int n, const StencilRef<VT> &S, const VT *x,
         k_rows_il_stencil<VT, OP, W, K, false><<<g, BS, 0, s>>>(n, S, x, f, d, y, lkp, nc, act);
 }
 
-template <typename VT, int K>
-void c64_stencil(hipStream_t s, int n, const StencilRef<VT> &S, const VT *x, const VT *f,
-                 const VT *d, double *z, long ldz, int lkp, int nc, const int *act)
+template <typename VT, typename ZT, int K>
+void cm_stencil(hipStream_t s, int n, const StencilRef<VT> &S, const VT *x, const VT *f,
+                const VT *d, ZT *z, long ldz, int lkp, int nc, const int *act)
 {
     constexpr int W = 16 / sizeof(VT);
     const int gpr = (nc + W - 1) / W;
@@ -1270,11 +1251,11 @@ void c64_stencil(hipStream_t s, int n, const StencilRef<VT> &S, const VT *x, con
     const bool nt = ((size_t)n << lkp) * sizeof(VT) > NT_BYTES;
     auto go = [&](auto kern) { kern<<<g, BS, 0, s>>>(n, S, x, f, d, z, ldz, lkp, nc, act); };
     if (BS % gpr == 0)
-        nt ? go(k_jacobi_il_c64_stencil<VT, W, K, true, true>)
-           : go(k_jacobi_il_c64_stencil<VT, W, K, true, false>);
+        nt ? go(k_jacobi_il_cm_stencil<VT, ZT, W, K, true, true>)
+           : go(k_jacobi_il_cm_stencil<VT, ZT, W, K, true, false>);
     else
-        nt ? go(k_jacobi_il_c64_stencil<VT, W, K, false, true>)
-           : go(k_jacobi_il_c64_stencil<VT, W, K, false, false>);
+        nt ? go(k_jacobi_il_cm_stencil<VT, ZT, W, K, false, true>)
+           : go(k_jacobi_il_cm_stencil<VT, ZT, W, K, false, false>);
 }
 
 template <typename MT, typename VT, int OP>
@@ -1331,22 +1312,22 @@ void rows_il_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, co
     }
 }
 
-/* the c64 sweep where k_rows_il's vector path runs (no group fallback);
+/* the column-major sweep where k_rows_il's vector path runs (no group fallback);
    false: not launched */
-template <typename MT, typename VT>
-bool jacobi_il_c64_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, const VT *f,
-                         const VT *d, double *z, long ldz, int lkp, int nc, const int *act)
+template <typename MT, typename VT, typename ZT>
+bool jacobi_il_cm_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, const VT *f,
+                        const VT *d, ZT *z, long ldz, int lkp, int nc, const int *act)
 {
     constexpr int WM = 16 / sizeof(VT);
     if (!stream_ok<VT>(A) || nc < WM) return false;
     if (il_stencil_ok<MT, VT>(A, nc)) {
         const StencilRef<VT> S = stencil_ref<VT>(A, il_mt<MT>());
         if (A.cls.k <= 5)
-            c64_stencil<VT, 5>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
+            cm_stencil<VT, ZT, 5>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
         else if (A.cls.k <= 7)
-            c64_stencil<VT, 7>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
+            cm_stencil<VT, ZT, 7>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
         else
-            c64_stencil<VT, CLS_ROW>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
+            cm_stencil<VT, ZT, CLS_ROW>(s, A.n, S, x, f, d, z, ldz, lkp, nc, act);
         return true;
     }
     constexpr bool all32 = std::is_same<MT, float>::value && std::is_same<VT, float>::value;
@@ -1356,24 +1337,24 @@ bool jacobi_il_c64_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT 
     const int gpr = (nc + WM - 1) / WM;
     const bool tile = (BS % gpr) == 0;
     const bool nt = ((size_t)n << lkp) * sizeof(VT) > NT_BYTES;
-#define C64(PF, TILE)                                                                        \
+#define CM(PF, TILE)                                                                        \
     do {                                                                                     \
         if (nt)                                                                              \
-            k_jacobi_il_c64<MT, VT, WM, PF, TILE, true><<<nb, BS, 0, s>>>(                   \
+            k_jacobi_il_cm<MT, VT, ZT, WM, PF, TILE, true><<<nb, BS, 0, s>>>(                   \
                 n, A.row.get(), A.col.get(), av, x, f, d, z, ldz, lkp, nc, act);             \
         else                                                                                 \
-            k_jacobi_il_c64<MT, VT, WM, PF, TILE, false><<<nb, BS, 0, s>>>(                  \
+            k_jacobi_il_cm<MT, VT, ZT, WM, PF, TILE, false><<<nb, BS, 0, s>>>(                  \
                 n, A.row.get(), A.col.get(), av, x, f, d, z, ldz, lkp, nc, act);             \
     } while (0)
     if (pf8 && tile)
-        C64((all32 ? 8 : 6), true);
+        CM((all32 ? 8 : 6), true);
     else if (pf8)
-        C64((all32 ? 8 : 6), false);
+        CM((all32 ? 8 : 6), false);
     else if (tile)
-        C64(6, true);
+        CM(6, true);
     else
-        C64(6, false);
-#undef C64
+        CM(6, false);
+#undef CM
     return true;
 }
 
@@ -1512,9 +1493,9 @@ void launch_rows_il(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const 
     BCMG_CHECK_LAUNCH();
 }
 
-template <typename VT>
-bool launch_jacobi_il_c64(hipStream_t s, const DevCsr &A, MatType mt, const VT *x, const VT *f,
-                          const VT *d, double *z, long ldz, int lkp, int nc, const int *act)
+template <typename VT, typename ZT>
+bool launch_jacobi_il_cm(hipStream_t s, const DevCsr &A, MatType mt, const VT *x, const VT *f,
+                         const VT *d, ZT *z, long ldz, int lkp, int nc, const int *act)
 {
     if (A.n <= 0 || nc <= 0) return true;
     if (nc > MULTI_MAX_COLS || nc > (1 << lkp))
@@ -1522,17 +1503,17 @@ bool launch_jacobi_il_c64(hipStream_t s, const DevCsr &A, MatType mt, const VT *
     bool done;
     if constexpr (std::is_same<VT, double>::value) {
         if (mt != MT_F64) throw Error(BCMG_EINVAL, "FP64 vectors need FP64 matrix values");
-        done = jacobi_il_c64_typed<double, double>(s, A, A.val.get(), x, f, d, z, ldz, lkp, nc,
+        done = jacobi_il_cm_typed<double, double>(s, A, A.val.get(), x, f, d, z, ldz, lkp, nc,
                                                    act);
     } else {
         if (mt == MT_F32)
-            done = jacobi_il_c64_typed<float, float>(s, A, A.val32.get(), x, f, d, z, ldz, lkp,
+            done = jacobi_il_cm_typed<float, float>(s, A, A.val32.get(), x, f, d, z, ldz, lkp,
                                                      nc, act);
         else if (mt == MT_BF16)
-            done = jacobi_il_c64_typed<unsigned short, float>(s, A, A.val16.get(), x, f, d, z,
+            done = jacobi_il_cm_typed<unsigned short, float>(s, A, A.val16.get(), x, f, d, z,
                                                               ldz, lkp, nc, act);
         else
-            done = jacobi_il_c64_typed<double, float>(s, A, A.val.get(), x, f, d, z, ldz, lkp,
+            done = jacobi_il_cm_typed<double, float>(s, A, A.val.get(), x, f, d, z, ldz, lkp,
                                                       nc, act);
     }
     BCMG_CHECK_LAUNCH();
@@ -1632,9 +1613,6 @@ void launch_from_il(hipStream_t s, int n, const S *a, D *b, long ldb, int lkp, i
 }
 
 #define BCMG_INSTANTIATE(VT)                                                                 \
-    template bool launch_jacobi_il_c64<VT>(hipStream_t, const DevCsr &, MatType, const VT *, \
-                                           const VT *, const VT *, double *, long, int, int,  \
-                                           const int *);                                      \
     template void launch_rows_il<VT>(hipStream_t, const DevCsr &, MatType, RowOp, const VT *, \
                                      const VT *, const VT *, VT *, int, int, const int *);    \
     template void launch_jacobi_zero_il<VT>(hipStream_t, int, const VT *, const VT *, VT *,  \
@@ -1650,6 +1628,17 @@ void launch_from_il(hipStream_t s, int n, const S *a, D *b, long ldb, int lkp, i
 BCMG_INSTANTIATE(double)
 BCMG_INSTANTIATE(float)
 #undef BCMG_INSTANTIATE
+template bool launch_jacobi_il_cm<double, double>(hipStream_t, const DevCsr &, MatType,
+                                                  const double *, const double *, const double *,
+                                                  double *, long, int, int, const int *);
+template bool launch_jacobi_il_cm<float, double>(hipStream_t, const DevCsr &, MatType,
+                                                 const float *, const float *, const float *,
+                                                 double *, long, int, int, const int *);
+template bool launch_jacobi_il_cm<float, float>(hipStream_t, const DevCsr &, MatType,
+                                                const float *, const float *, const float *,
+                                                float *, long, int, int, const int *);
+template void launch_from_il<float, float>(hipStream_t, int, const float *, float *, long, int,
+                                           int, const int *);
 template void launch_to_il<double, double>(hipStream_t, int, const double *, long, double *, int,
                                            int, const int *);
 template void launch_to_il<double, float>(hipStream_t, int, const double *, long, float *, int,
@@ -1746,6 +1735,7 @@ void launch_spmv_dots_multi(Ctx &c, const DevCsr &A, int k, MultiFcg &M, const i
     const int n = A.n;
     const FcgCols F = fcg_cols(M);
     if (!stream_ok<double>(A)) {
+        if (M.z32) throw Error(BCMG_EINVAL, "FCG product: FP32 z needs rows of the LDS tile");
         /* long rows: the single-column path's separate SpMV (k_rows<G>
            arithmetic into Y), products (k_dots) and recurrence */
         launch_rows_multi<double>(c.stream, A, MT_F64, OP_SPMV, M.Z, M.ld, nullptr, nullptr,
@@ -1774,17 +1764,21 @@ void launch_spmv_dots_multi(Ctx &c, const DevCsr &A, int k, MultiFcg &M, const i
                                         part);
     };
     /* the stencil's entries as kernel arguments (KS of them), or CSR rows */
-    auto pick = [&](auto K, auto NT) {
+    auto pick_z = [&](auto K, auto NT, auto zt) {
         constexpr int kk = decltype(K)::value;
         constexpr bool nn = decltype(NT)::value;
+        using ZT = decltype(zt);
         if (!st)
-            go(k_spmv_dots_multi<kk, nn>);
+            go(k_spmv_dots_multi<kk, nn, ZT>);
         else if (A.cls.k <= 5)
-            go(k_spmv_dots_multi<kk, nn, 5>);
+            go(k_spmv_dots_multi<kk, nn, ZT, 5>);
         else if (A.cls.k <= 7)
-            go(k_spmv_dots_multi<kk, nn, 7>);
+            go(k_spmv_dots_multi<kk, nn, ZT, 7>);
         else
-            go(k_spmv_dots_multi<kk, nn, CLS_ROW>);
+            go(k_spmv_dots_multi<kk, nn, ZT, CLS_ROW>);
+    };
+    auto pick = [&](auto K, auto NT) {
+        M.z32 ? pick_z(K, NT, float()) : pick_z(K, NT, double());
     };
     using K2 = std::integral_constant<int, 2>;
     using K3 = std::integral_constant<int, 3>;
@@ -1802,10 +1796,12 @@ void launch_fcg_update_multi(Ctx &c, int n, MultiFcg &M, double *part)
 {
     const int nb = red_blocks(n);
     const FcgCols F = fcg_cols(M);
-    if ((size_t)n * M.nc * 10 * sizeof(double) > NT_BYTES)
-        k_fcg_update_multi<true><<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, part);
+    const bool nt = (size_t)n * M.nc * 10 * sizeof(double) > NT_BYTES;
+    auto go = [&](auto kern) { kern<<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, part); };
+    if (M.z32)
+        nt ? go(k_fcg_update_multi<true, float>) : go(k_fcg_update_multi<false, float>);
     else
-        k_fcg_update_multi<false><<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, part);
+        nt ? go(k_fcg_update_multi<true, double>) : go(k_fcg_update_multi<false, double>);
     k_fcg_final_multi<1, true><<<M.nc, RED_FINAL_BS, 0, c.stream>>>(nb, part, F, M.act);
     BCMG_CHECK_LAUNCH();
 }
@@ -1814,7 +1810,10 @@ void launch_fcg_first_multi(Ctx &c, int n, MultiFcg &M, const int *mask, double 
 {
     const int nb = red_blocks(n);
     const FcgCols F = fcg_cols(M);
-    k_fcg_first_multi<<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, mask, part);
+    if (M.z32)
+        k_fcg_first_multi<float><<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, mask, part);
+    else
+        k_fcg_first_multi<double><<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, mask, part);
     k_fcg_final_multi<1, false><<<M.nc, RED_FINAL_BS, 0, c.stream>>>(nb, part, F, mask);
     BCMG_CHECK_LAUNCH();
 }

@@ -487,12 +487,14 @@ __global__ __launch_bounds__(RED_FINAL_BS) void k_fcg_final(int nb, const double
    triple inner product :6-83): t = A z, and per block the partial sums of
    alpha = r.z, beta = t.z (K = 2, first step) and gamma = to.z (K = 3),
    finished by k_fcg_final. The products use the z, r, to values the
-   epilogue loads anyway, so the separate triple-product pass is saved. */
-template <int K, bool NT, typename IT>
+   epilogue loads anyway, so the separate triple-product pass is saved. z is
+   read as the cycle left it: an FP32 cycle's result is widened here (exactly)
+   instead of in a pass of its own. */
+template <int K, bool NT, typename IT, typename ZT>
 __global__ __launch_bounds__(BS) void k_spmv_dots(int n, const int *__restrict__ rp,
                                                   const IT *__restrict__ ci,
                                                   const double *__restrict__ av,
-                                                  const double *__restrict__ z,
+                                                  const ZT *__restrict__ z,
                                                   double *__restrict__ t,
                                                   const double *__restrict__ rv,
                                                   const double *__restrict__ to,
@@ -511,7 +513,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots(int n, const int *__restrict__
     if (own) {
         ra = rp[r];
         re = rp[r + 1];
-        zr = z[r];
+        zr = (double)z[r];
         rr = rv[r];
         if (K > 2) tor = to[r];
     }
@@ -523,7 +525,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots(int n, const int *__restrict__
 #pragma unroll
     for (int k = 0; k < K; k++) sdot[k] = 0.0;
     if (own) {
-        const double tr = staged_row_sum<double, double, IT>(
+        const double tr = staged_row_sum<double, double, IT, false, ZT>(
             lcol, lval, z, ra - stage_base<IT>(e0), ra - stage_base<double>(e0), re - ra, r);
         t[r] = tr;
         sdot[0] = rr * zr;
@@ -535,12 +537,12 @@ __global__ __launch_bounds__(BS) void k_spmv_dots(int n, const int *__restrict__
 
 /* k_spmv_dots on a stencil-pattern operator (the reads of k_rows_pattern,
    the products and partials of k_spmv_dots) */
-template <int K, bool NT>
+template <int K, bool NT, typename ZT>
 __global__ __launch_bounds__(BS) void k_spmv_dots_pattern(int n, const int *__restrict__ rp,
                                                           const unsigned char *__restrict__ pm,
                                                           PatOffsets po,
                                                           const double *__restrict__ av,
-                                                          const double *__restrict__ z,
+                                                          const ZT *__restrict__ z,
                                                           double *__restrict__ t,
                                                           const double *__restrict__ rv,
                                                           const double *__restrict__ to,
@@ -556,7 +558,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_pattern(int n, const int *__re
     const unsigned w = ldm<NT>(reinterpret_cast<const unsigned *>(pm + r0) + (threadIdx.x & 63));
     double zr = 0.0, rr = 0.0, tor = 0.0;
     if (own) {
-        zr = z[r];
+        zr = (double)z[r];
         rr = rv[r];
         if (K > 2) tor = to[r];
     }
@@ -571,7 +573,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_pattern(int n, const int *__re
 #pragma unroll
     for (int k = 0; k < K; k++) sdot[k] = 0.0;
     if (own) {
-        const double tr = pattern_row_sum<double, double>(
+        const double tr = pattern_row_sum<double, double, false, ZT>(
             m, po, lval + (e0 - stage_base<double>(e0)) + pre, z, r);
         t[r] = tr;
         sdot[0] = rr * zr;
@@ -582,26 +584,34 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_pattern(int n, const int *__re
 }
 
 /* fused double_merged_axpy pair + ||r||^2 partials (src/SOLVER/FCG.cu:88-98,
-   536-558): z = -theta zo + z; x += theta2 z; t = -theta to + t; r += -theta2 t */
+   536-558): z = -theta zo + zc; x += theta2 z; t = -theta to + t;
+   r += -theta2 t. zc is the cycle's result (z itself, or an FP32 cycle's
+   block widened here); r32, when given, receives r rounded for the next FP32
+   cycle. NT, where the ten streams exceed the last-level cache: all but r,
+   which the next cycle reads, bypass it (160^3 solve 20.6 -> 20.3 ms FP64). */
+template <typename ZT, bool NT>
 __global__ __launch_bounds__(BS) void k_fcg_update(int n, const double *__restrict__ scal,
                                                    const double *__restrict__ zo,
-                                                   double *__restrict__ z,
+                                                   const ZT *zc, double *z,
                                                    double *__restrict__ x,
                                                    const double *__restrict__ to,
                                                    double *__restrict__ t,
                                                    double *__restrict__ r,
+                                                   float *__restrict__ r32,
                                                    double *__restrict__ part)
 {
     const double theta = scal[4], theta2 = scal[5];
     double s[1] = {0.0};
     for (int i = blockIdx.x * BS + threadIdx.x; i < n; i += gridDim.x * BS) {
-        const double zi = fma(-theta, zo[i], z[i]);
-        z[i] = zi;
-        x[i] = fma(theta2, zi, x[i]);
-        const double ti = fma(-theta, to[i], t[i]);
-        t[i] = ti;
+        const double zi = fma(-theta, ldm<NT>(zo + i), (double)zc[i]);
+        const double xi = fma(theta2, zi, ldm<NT>(x + i));
+        const double ti = fma(-theta, ldm<NT>(to + i), t[i]);
         const double ri = fma(-theta2, ti, r[i]);
+        st_nt<NT>(z + i, zi);
+        st_nt<NT>(x + i, xi);
+        st_nt<NT>(t + i, ti);
         r[i] = ri;
+        if (r32) r32[i] = (float)ri;
         s[0] = fma(ri, ri, s[0]);
     }
     block_reduce_store<1>(s, part + blockIdx.x);
@@ -1241,14 +1251,27 @@ void launch_fcg_scalars(hipStream_t s, double *scal)
     BCMG_CHECK_LAUNCH();
 }
 
-void launch_fcg_update(Ctx &c, int n, double *scal, const double *zo, double *z, double *x,
-                       const double *to, double *t, double *r)
+template <typename ZT>
+void launch_fcg_update(Ctx &c, int n, double *scal, const double *zo, const ZT *zc, double *z,
+                       double *x, const double *to, double *t, double *r, float *r32)
 {
     const int nb = red_blocks(n);
-    k_fcg_update<<<nb, BS, 0, c.stream>>>(n, scal, zo, z, x, to, t, r, c.red.get() + RED_UPD);
-    k_fcg_final<1><<<1, RED_FINAL_BS, 0, c.stream>>>(nb, c.red.get() + RED_UPD, scal);
+    double *part = c.red.get() + RED_UPD;
+    if ((size_t)n * 10 * sizeof(double) > NT_BYTES)
+        k_fcg_update<ZT, true><<<nb, BS, 0, c.stream>>>(n, scal, zo, zc, z, x, to, t, r, r32,
+                                                        part);
+    else
+        k_fcg_update<ZT, false><<<nb, BS, 0, c.stream>>>(n, scal, zo, zc, z, x, to, t, r, r32,
+                                                         part);
+    k_fcg_final<1><<<1, RED_FINAL_BS, 0, c.stream>>>(nb, part, scal);
     BCMG_CHECK_LAUNCH();
 }
+template void launch_fcg_update<double>(Ctx &, int, double *, const double *, const double *,
+                                        double *, double *, const double *, double *, double *,
+                                        float *);
+template void launch_fcg_update<float>(Ctx &, int, double *, const double *, const float *,
+                                       double *, double *, const double *, double *, double *,
+                                       float *);
 
 void launch_fcg_first(Ctx &c, int n, double *scal, const double *v, double *x, const double *w,
                       double *r)
@@ -1330,9 +1353,9 @@ BCMG_INSTANTIATE_K(float)
 #undef BCMG_INSTANTIATE_K
 
 /* the fused FCG SpMV + inner products over the stored column type IT */
-template <typename IT>
+template <typename IT, typename ZT>
 static void spmv_dots_typed(hipStream_t s, int nb, int n, int k, const int *rp, const IT *ci,
-                            const double *av, int nnz, int tile, const double *z, double *t,
+                            const double *av, int nnz, int tile, const ZT *z, double *t,
                             const double *r, const double *to, double *part)
 {
     const size_t lds = staged_lds_bytes(tile, sizeof(double), sizeof(IT));
@@ -1341,27 +1364,32 @@ static void spmv_dots_typed(hipStream_t s, int nb, int n, int k, const int *rp, 
     const bool nt = (size_t)nnz * (sizeof(IT) + sizeof(double)) > NT_BYTES;
     if (k == 2) {
         if (nt)
-            k_spmv_dots<2, true, IT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
+            k_spmv_dots<2, true, IT, ZT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
         else
-            k_spmv_dots<2, false, IT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
+            k_spmv_dots<2, false, IT, ZT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
     } else {
         if (nt)
-            k_spmv_dots<3, true, IT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
+            k_spmv_dots<3, true, IT, ZT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
         else
-            k_spmv_dots<3, false, IT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
+            k_spmv_dots<3, false, IT, ZT><<<nb, BS, lds, s>>>(n, rp, ci, av, z, t, r, to, part, tile);
     }
 }
 
 size_t red_size_for(int n) { return (size_t)RED_SPMV + 3 * (size_t)((n + BS - 1) / BS) + 64; }
 
-void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const double *z, double *t,
-                      const double *r, const double *to, double *scal)
+template <typename ZT>
+void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const ZT *z, double *t, const double *r,
+                      const double *to, double *scal)
 {
     const int n = A.n;
     if (!stream_ok<double>(A)) {
         /* long rows: separate SpMV, products and recurrence */
-        launch_rows(c.stream, A, OP_SPMV, z, nullptr, nullptr, t);
-        launch_dots(c, n, k, r, t, to, z, scal);
+        if constexpr (std::is_same<ZT, double>::value) {
+            launch_rows(c.stream, A, OP_SPMV, z, nullptr, nullptr, t);
+            launch_dots(c, n, k, r, t, to, z, scal);
+        } else {
+            throw Error(BCMG_EINVAL, "FCG product: FP32 z needs rows of the LDS tile");
+        }
         if (k == 2)
             k_fcg_first_scalars<<<1, 64, 0, c.stream>>>(scal);
         else
@@ -1376,7 +1404,7 @@ void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const double *z, double *t
     const int *rp = A.row.get();
     const double *av = A.val.get();
     if (class_ok<double>(A, MT_F64)) {
-        launch_spmv_dots_class(c.stream, A, k, z, t, r, to, part);
+        launch_spmv_dots_class<ZT>(c.stream, A, k, z, t, r, to, part);
     } else if (A.use_pattern()) {
         if (!stage_aligned(av, av))
             throw Error(BCMG_EINVAL, "SpMV: matrix values not 16-byte aligned");
@@ -1386,17 +1414,17 @@ void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const double *z, double *t
         const unsigned char *pm = A.pmask.get();
         if (k == 2) {
             if (nt)
-                k_spmv_dots_pattern<2, true><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
+                k_spmv_dots_pattern<2, true, ZT><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
                                                                         r, to, part);
             else
-                k_spmv_dots_pattern<2, false><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
+                k_spmv_dots_pattern<2, false, ZT><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
                                                                          r, to, part);
         } else {
             if (nt)
-                k_spmv_dots_pattern<3, true><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
+                k_spmv_dots_pattern<3, true, ZT><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
                                                                         r, to, part);
             else
-                k_spmv_dots_pattern<3, false><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
+                k_spmv_dots_pattern<3, false, ZT><<<nb, BS, lds, c.stream>>>(n, rp, pm, po, av, z, t,
                                                                          r, to, part);
         }
     } else if (A.use_narrow())
@@ -1411,5 +1439,9 @@ void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const double *z, double *t
         k_fcg_final<3><<<1, RED_FINAL_BS, 0, c.stream>>>(nb, part, scal);
     BCMG_CHECK_LAUNCH();
 }
+template void launch_spmv_dots<double>(Ctx &, const DevCsr &, int, const double *, double *,
+                                       const double *, const double *, double *);
+template void launch_spmv_dots<float>(Ctx &, const DevCsr &, int, const float *, double *,
+                                      const double *, const double *, double *);
 
 } // namespace bcmg
