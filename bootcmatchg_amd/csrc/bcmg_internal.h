@@ -149,6 +149,19 @@ struct RowClasses {
     void make_lowp(hipStream_t s, bool bf16);
 };
 
+/* a symmetric stencil with varying coefficients (kernels_sym.hip): k offsets
+   ascending, closed under negation; the diagonal and the upper diagonals as
+   arrays of ld rows, and the mask of each row's entries */
+struct SymStencil {
+    int k = 0;                   /* 0: not kept */
+    int off[PAT_MAX] = {};
+    long ld = 0;                 /* rows padded to whole 256-row blocks */
+    DBuf<unsigned char> mask;
+    DBuf<double> u;
+    DBuf<float> u32;
+    void make_lowp(hipStream_t s);
+};
+
 /* CSR, 0-based, int32 indices, FP64 values; columns ascending with a diagonal
    entry in every row (the layout of src/matrix/CSR.h:13-28). */
 struct DevCsr {
@@ -178,11 +191,14 @@ struct DevCsr {
     bool cols_analysed = false; /* narrow copy and pattern considered */
     RowClasses cls;
     int band = -1;              /* largest |column - row|; -1: not determined */
-    /* the narrowest form the row kernels may read: 3 the row classes, 2 the
+    SymStencil sym;
+    /* the narrowest form the row kernels may read: 3 the row classes or the
+       symmetric stencil, 2 the
        pattern, 1 the 16-bit offsets, 0 the int32 columns
        (bcmg_csr_set_columns chooses among the last three) */
     int col_mode = 3;
     bool use_classes() const { return cls.n > 0 && col_mode >= 3; }
+    bool use_sym() const { return sym.k > 0 && col_mode >= 3; }
     bool use_pattern() const { return pk > 0 && col_mode >= 2; }
     bool use_narrow() const { return narrow && col_mode >= 1; }
     int group = 8;          /* lanes per row of the row-group kernels */
@@ -208,6 +224,10 @@ void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats);
    operator in mats that has rows of at most CLS_ROW entries, their tiles
    resolved (one round trip for the lot, a second for those with classes) */
 void make_classes(Ctx &c, const std::vector<DevCsr *> &mats);
+/* the symmetric-stencil form of an uploaded operator without row classes */
+void make_sym(Ctx &c, DevCsr &A);
+/* A's distinct column offsets, ascending; false when more than PAT_MAX */
+bool find_offsets(Ctx &c, DevCsr &A, std::vector<int> &off);
 
 /* ------------------------------------------------------------- context */
 
@@ -377,6 +397,16 @@ inline DivSource div_source(int relax_type) { return relax_type == 4 ? DIV_L1 : 
 template <typename VT>
 void launch_rows(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const VT *x, const VT *f,
                  const VT *d, VT *y, DivSource div = DIV_ARRAY);
+/* kernels_sym.hip: whether A's values of type mt are read as a symmetric
+   stencil by VT kernels, and those kernels */
+template <typename VT>
+bool sym_ok(const DevCsr &A, MatType mt);
+template <typename VT>
+void launch_rows_sym(hipStream_t s, const DevCsr &A, RowOp op, const VT *x, const VT *f,
+                     const VT *d, VT *y, DivSource div);
+template <typename ZT>
+void launch_spmv_dots_sym(hipStream_t s, const DevCsr &A, int k, const ZT *z, double *t,
+                          const double *r, const double *to, double *part);
 /* kernels_class.hip: whether A's values of type mt are read as row classes
    by VT kernels, and those kernels */
 template <typename VT>

@@ -901,12 +901,37 @@ void analyze_rows(Ctx &c, DevCsr &A)
     resolve_tiles(c, {&A});
     make_narrow(c, {&A});
     make_classes(c, {&A});
+    make_sym(c, A);
 }
 
 /* square operators whose FP64 stream (12 B per entry) exceeds this are
    checked for a stencil pattern; the 16-bit copy is kept for streamed ones
    (above NT_BYTES) only */
 constexpr size_t PAT_MIN_BYTES = (size_t)128 << 20;
+
+bool find_offsets(Ctx &c, DevCsr &A, std::vector<int> &off)
+{
+    off.clear();
+    if (A.pk > 0) {
+        off.assign(A.poff, A.poff + A.pk);
+        return true;
+    }
+    DBuf<int> info(1 + PAT_SLOTS);
+    c.h_ints[0] = 0;
+    for (int q = 0; q < PAT_SLOTS; q++) c.h_ints[1 + q] = PAT_EMPTY;
+    BCMG_HIP(hipMemcpyAsync(info.get(), c.h_ints, (1 + PAT_SLOTS) * sizeof(int),
+                            hipMemcpyHostToDevice, c.stream));
+    k_pattern_offsets<<<(A.n + BS - 1) / BS, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(),
+                                                               info.get() + 1, info.get());
+    BCMG_CHECK_LAUNCH();
+    BCMG_HIP(hipMemcpyAsync(c.h_ints, info.get(), (1 + PAT_SLOTS) * sizeof(int),
+                            hipMemcpyDeviceToHost, c.stream));
+    BCMG_HIP(hipStreamSynchronize(c.stream));
+    for (int q = 0; q < PAT_SLOTS; q++)
+        if (c.h_ints[1 + q] != PAT_EMPTY) off.push_back(c.h_ints[1 + q]);
+    std::sort(off.begin(), off.end());
+    return c.h_ints[0] == 0 && !off.empty() && off.size() <= PAT_MAX;
+}
 
 void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats)
 {
@@ -980,6 +1005,7 @@ void DevCsr::make_lowp(hipStream_t s, bool bf16)
     }
     BCMG_CHECK_LAUNCH();
     cls.make_lowp(s, bf16);
+    if (!bf16) sym.make_lowp(s);
 }
 
 template <typename VT>
@@ -989,6 +1015,10 @@ void launch_rows(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const VT 
     if (A.n <= 0) return;
     if (op != OP_JACOBI_Z && class_ok<VT>(A, mt)) {
         launch_rows_class<VT>(s, A, mt, op, x, f, d, y, div);
+        return;
+    }
+    if (op != OP_JACOBI_Z && sym_ok<VT>(A, mt)) {
+        launch_rows_sym<VT>(s, A, op, x, f, d, y, div);
         return;
     }
     if constexpr (std::is_same<VT, double>::value) {
@@ -1018,7 +1048,7 @@ bool fuse_zero_sweeps(const DevCsr &A, MatType mt)
        light passes beat one with a division at every gather (160^3 FP32
        47 us in one pass, 10.8 + 12.8 us in two), except where a launch costs
        more than the work */
-    if (class_ok<VT>(A, mt)) return A.n <= SMALL_LEVEL_ROWS;
+    if (class_ok<VT>(A, mt) || sym_ok<VT>(A, mt)) return A.n <= SMALL_LEVEL_ROWS;
     /* a streamed FP64 operator: the division at every gather costs more
        than the pass it saves */
     const size_t vb = mt == MT_F64 ? 8 : mt == MT_F32 ? 4 : 2;
@@ -1405,6 +1435,8 @@ void launch_spmv_dots(Ctx &c, const DevCsr &A, int k, const ZT *z, double *t, co
     const double *av = A.val.get();
     if (class_ok<double>(A, MT_F64)) {
         launch_spmv_dots_class<ZT>(c.stream, A, k, z, t, r, to, part);
+    } else if (sym_ok<double>(A, MT_F64)) {
+        launch_spmv_dots_sym<ZT>(c.stream, A, k, z, t, r, to, part);
     } else if (A.use_pattern()) {
         if (!stage_aligned(av, av))
             throw Error(BCMG_EINVAL, "SpMV: matrix values not 16-byte aligned");

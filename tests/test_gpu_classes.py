@@ -1,10 +1,11 @@
 """Row classes (operators whose rows take few distinct forms, read as one byte
-per row): every row kernel gives the bits of the int32-column kernels, at the
-edges of the kernels' blocks and of the rules that choose them.
+per row) and symmetric stencils (half of the values, by diagonals): every row
+kernel gives the bits of the int32-column kernels, at the edges of the
+kernels' blocks and of the rules that choose them.
 
 bcmg_csr_set_columns(4) restricts a handle to its int32 columns; the default
 uses the classes where they are kept (no more than 256 forms of at most 8
-entries; more than 4096 rows)."""
+entries), else the symmetric stencil (at most 7 offsets, from 32 768 rows)."""
 import ctypes
 
 import numpy as np
@@ -59,9 +60,30 @@ def eight_entries(N):
     return csr(10.0 * sp.eye(N * N) - sp.kron(T, T) + sp.kron(U, U))
 
 
+def varying2d(N, asymmetric=False):
+    """5-point operator with varying symmetric coefficients; asymmetric
+    changes one lower entry by an ulp."""
+    n = N * N
+    rng = np.random.default_rng(N)
+    ex, ey = rng.uniform(1, 2, n - 1), rng.uniform(1, 2, n - N)
+    ex[np.arange(1, n) % N == 0] = 0.0
+    S = sp.csr_matrix(sp.diags([-ey, -ex, -ex, -ey], [-N, -1, 1, N], shape=(n, n)))
+    S.eliminate_zeros()
+    S = S + sp.diags(0.1 - np.asarray(S.sum(axis=1)).ravel())
+    row, col, val = csr(S)
+    if asymmetric:
+        val[row[n // 2]] = np.nextafter(val[row[n // 2]], 0.0)
+    return row, col, val
+
+
 OPERATORS = {
+    "lognormal3d_33": lambda: ops.lognormal3d(33, 4.0, seed=2),   # a symmetric stencil
+    "lognormal3d_53": lambda: ops.lognormal3d(53, 4.0, seed=2),   # two rows a thread, ragged
+    "varying2d_181": lambda: varying2d(181),                      # just analysed
+    "varying2d_401": lambda: varying2d(401),
+    "varying2d_401_asymmetric": lambda: varying2d(401, True),
     "poisson3d_17": lambda: ops.poisson3d(17),        # few blocks, all near an end
-    "aniso2d_65": lambda: ops.aniso2d(65, 0.01),      # 4225 rows: just analysed
+    "aniso2d_65": lambda: ops.aniso2d(65, 0.01),      # 4225 rows
     "poisson3d_41": lambda: ops.poisson3d(41),        # one row a thread, ragged
     "tridiagonal_4097": lambda: tridiagonal(4097),
     "tridiagonal_524289": lambda: tridiagonal((1 << 19) + 1),  # two rows a thread, one over
@@ -72,7 +94,7 @@ OPERATORS = {
     "diagonals_200": lambda: diagonals(20011, 200),
     "diagonals_257": lambda: diagonals(20011, 257),   # one form too many
     "eight_entries_91": lambda: eight_entries(91),
-    "lognormal3d_18": lambda: ops.lognormal3d(18, 4.0, seed=1),  # every row its own form
+    "lognormal3d_18": lambda: ops.lognormal3d(18, 4.0, seed=1),  # neither form
 }
 
 
@@ -117,7 +139,8 @@ def test_row_kernels_same_bits(ctx, name, offset):
     dA.free()
 
 
-@pytest.mark.parametrize("name", ["poisson3d_41", "aniso2d_725", "neumann2d_70"])
+@pytest.mark.parametrize("name", ["poisson3d_41", "aniso2d_725", "neumann2d_70",
+                                  "lognormal3d_53", "varying2d_181"])
 def test_special_values_stay_where_the_rows_read_them(ctx, name):
     """Infinities and NaN in x reach exactly the rows that have an entry
     there; a row without the entry is not touched."""
@@ -125,7 +148,7 @@ def test_special_values_stay_where_the_rows_read_them(ctx, name):
     n = len(A[0]) - 1
     rng = np.random.default_rng(6)
     x, f, d = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n), rng.uniform(7, 8, n)
-    N = 41 if name == "poisson3d_41" else 725 if name == "aniso2d_725" else 70
+    N = int(name.split("_")[1])
     x[[0, N - 1, N, 5 * N, n - N, n - 1]] = [np.inf, np.nan, -np.inf, np.nan, np.inf, -np.inf]
     dA = bc.Csr(ctx, A)
     got = row_ops(ctx, dA, n, x, f, d)
@@ -140,7 +163,8 @@ def test_special_values_stay_where_the_rows_read_them(ctx, name):
 
 @pytest.mark.parametrize("prec", [bc.PREC_FP64, bc.PREC_FP32, bc.PREC_BF16])
 @pytest.mark.parametrize("setting", ["V_L1_2sweeps", "H_jacobi_1sweep"])
-@pytest.mark.parametrize("name", ["poisson3d_41", "neumann2d_70", "aniso2d_725"])
+@pytest.mark.parametrize("name", ["poisson3d_41", "neumann2d_70", "aniso2d_725",
+                                  "lognormal3d_33", "varying2d_401"])
 def test_solves_same_bits(ctx, name, setting, prec):
     """Setup and FCG with level 0 read as classes and as int32 columns (the
     L1 and the diagonal divisor come from the forms in one, from their arrays
