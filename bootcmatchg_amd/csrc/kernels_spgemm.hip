@@ -20,12 +20,15 @@
  *     the touched columns are put in order at the end of the row; when the
  *     right rows are long (SG_SERIAL_MIN products per left entry or more) and
  *     hold distinct columns, no sort is needed: the left entries are taken
- *     one at a time, each adding its products column-parallel.
+ *     one at a time, each adding its products column-parallel;
+ *   - with SG_LDS_COLS columns or fewer the accumulators are in LDS and a
+ *     wavefront owns a column tile (k_sg_wave).
  * The pattern is symbolic (a cancelled entry stays), columns ascending. The
  * file is compiled with -ffp-contract=off: products and sums are rounded
  * separately, as in the serial restatement.
  */
 #include "bcmg_internal.h"
+#include "kernels_common.h"
 
 #include <algorithm>
 #include <climits>
@@ -36,7 +39,6 @@ namespace bcmg {
 
 namespace {
 
-constexpr int BS = 256;
 constexpr int SG_CAP = 1024;          /* products of a packed row, at most */
 constexpr int SG_KEYS = 2 * SG_CAP;   /* keys of a packed workgroup */
 constexpr int SG_CH = 2048;           /* products per chunk of a long row */
@@ -44,7 +46,11 @@ constexpr int SG_SORT = 2 * SG_CH;    /* touched columns sorted in LDS, at most 
 constexpr long long SG_DENSE_BYTES = 2ll << 30; /* dense accumulators, all workgroups */
 constexpr int SG_DENSE_BLOCKS = 1024;
 constexpr int SG_SERIAL_MIN = 64;     /* products per left entry for the serial mode */
-constexpr int SG_LDS_COLS = 4096;     /* columns of C for LDS accumulators */
+constexpr int SG_TILES = 16;          /* wavefronts (column tiles) of a row, at most */
+constexpr int SG_TILE = 1024;         /* columns of a tile, about */
+constexpr int SG_LDS_COLS = SG_TILES * SG_TILE; /* columns of C, at most, for LDS accumulators */
+constexpr int SG_AHEAD = 8;           /* loads of 64 right entries in flight */
+constexpr long long SG_UNTOUCHED = LLONG_MIN;   /* the bits of -0.0 */
 constexpr int SHORT_ROW = 64;         /* transpose rows ranked by one lane */
 constexpr int RANK_CHUNK = 4096;      /* columns per LDS load when ranking */
 constexpr unsigned long long SG_NONE = ~0ull;
@@ -52,7 +58,6 @@ constexpr int POS_BITS = 11;          /* position field: < 2048 */
 constexpr int ROW_SHIFT = 42;         /* row field above 31 column bits */
 constexpr long long SG_PER_PASS = 1ll << 28; /* slots + weights per batch of rows */
 
-inline int blocks_for(long long w) { return (int)((w + BS - 1) / BS); }
 
 /* first index t in [0, n) with a[t] >= x (n if none) */
 __device__ inline int lower_bound_i(const int *a, int n, int x)
@@ -121,8 +126,8 @@ __device__ inline int pow2_at_least(int v)
 
 /* per row: products u, output slots sl = min(products, columns of C) (a
    row has at most that many entries), packing weight ws, the long-row
-   list; the total of slots plus weights (what a batch of rows is bounded
-   by); *big = 1 if a row has 2^30 products or more */
+   list and how many of it have fewer than smin products per left entry; the
+   total of slots plus weights (what a batch of rows is bounded by); *big = 1 if a row has 2^30 products or more */
 __global__ __launch_bounds__(BS) void k_sg_count(int n, const int *__restrict__ Lrp,
                                                  const int *__restrict__ Lci,
                                                  const int *__restrict__ Rrp, long long m,
@@ -131,7 +136,7 @@ __global__ __launch_bounds__(BS) void k_sg_count(int n, const int *__restrict__ 
                                                  int *__restrict__ large,
                                                  int *__restrict__ nlarge,
                                                  unsigned long long *__restrict__ total,
-                                                 int *__restrict__ big)
+                                                 int *__restrict__ big, int smin)
 {
     const int i = blockIdx.x * BS + threadIdx.x;
     long long s = 0, slots = 0;
@@ -150,6 +155,7 @@ __global__ __launch_bounds__(BS) void k_sg_count(int n, const int *__restrict__ 
         } else {
             ws[i] = 0;
             large[atomicAdd(nlarge, 1)] = i;
+            if (s < (long long)smin * (Lrp[i + 1] - Lrp[i])) atomicAdd(nlarge + 2, 1);
         }
     }
     /* the batch cost of a row: its slots plus its packing weight */
@@ -330,7 +336,7 @@ __global__ __launch_bounds__(BS) void k_sg_dense(int nlarge, const int *__restri
         const int e_end = Lrp[r + 1];
         int ew0 = Lrp[r], pb0 = 0;   /* first window some later chunk needs */
         const bool serial = serial_min > 0 && (long long)U >= (long long)serial_min * (e_end - ew0);
-        if (serial && skip_serial) continue;   /* k_sg_serial_lds takes it */
+        if (serial && skip_serial) continue;   /* k_sg_wave takes it */
         int *const ocol = tcol + uoff[r];
         double *const oval = tval + uoff[r];
         if (threadIdx.x == 0) {
@@ -485,88 +491,137 @@ __global__ __launch_bounds__(BS) void k_sg_dense(int nlarge, const int *__restri
     }
 }
 
-/* The serial-mode long rows when C has at most SG_LDS_COLS columns: the
-   accumulator and the row marks live in LDS; the row's entries come out in
-   column order from a scan of the marks (no sort). Same order per column as
-   the serial mode of k_sg_dense. */
-__global__ __launch_bounds__(BS) void k_sg_serial_lds(int nlarge, const int *__restrict__ large,
-                                                      const int *__restrict__ Lrp,
-                                                      const int *__restrict__ Lci,
-                                                      const double *__restrict__ Lv,
-                                                      const int *__restrict__ Rrp,
-                                                      const int *__restrict__ Rci,
-                                                      const double *__restrict__ Rv,
-                                                      const int *__restrict__ u,
-                                                      const int *__restrict__ uoff,
-                                                      int *__restrict__ tcol,
-                                                      double *__restrict__ tval, int m,
-                                                      int serial_min, int *__restrict__ cnt)
+/* where R's rows cross the column tiles [t W, (t + 1) W): seg[row][t] is the
+   first entry of tile t, seg[row][nt] the row's end (a wavefront a row,
+   columns strictly ascending) */
+__global__ __launch_bounds__(BS) void k_sg_seg(int n, const int *__restrict__ rp,
+                                               const int *__restrict__ ci, int W, int nt,
+                                               int *__restrict__ seg)
 {
-    __shared__ double acc[SG_LDS_COLS];
-    __shared__ int mark[SG_LDS_COLS];
-    __shared__ int ws0[BS], wf0[BS];
-    __shared__ double wlv[BS];
-    __shared__ int sh[BS / 64];
-    for (int j = threadIdx.x; j < m; j += BS) mark[j] = -1;
-    __syncthreads();
-    for (int q = blockIdx.x; q < nlarge; q += gridDim.x) {
-        const int r = large[q];
-        const int U = u[r];
-        const int e_end = Lrp[r + 1];
-        const int eb = Lrp[r];
-        if (!((long long)U >= (long long)serial_min * (e_end - eb))) continue;
-        for (int e0 = eb; e0 < e_end; e0 += BS) {
-            const int e = e0 + threadIdx.x;
-            if (e < e_end) {
-                const int k = Lci[e];
-                wf0[threadIdx.x] = Rrp[k];
-                ws0[threadIdx.x] = Rrp[k + 1];
-                wlv[threadIdx.x] = Lv[e];
-            }
-            __syncthreads();
-            const int ne = min(BS, e_end - e0);
-            int pf = wf0[0] + threadIdx.x;
-            bool have = pf < ws0[0];
-            int pc = have ? Rci[pf] : 0;
-            double pv = have ? Rv[pf] : 0.0;
-            for (int t = 0; t < ne; t++) {
-                const int f1 = ws0[t];
-                const double lv = wlv[t];
-                const int nf = t + 1 < ne ? wf0[t + 1] + threadIdx.x : 0;
-                const bool nhave = t + 1 < ne && nf < ws0[t + 1];
-                const int nc = nhave ? Rci[nf] : 0;
-                const double nv = nhave ? Rv[nf] : 0.0;
-                for (int f = pf; have && f < f1; f += BS) {
-                    const int col = f == pf ? pc : Rci[f];
-                    const double prod = lv * (f == pf ? pv : Rv[f]);
-                    const bool first = mark[col] != q;
-                    acc[col] = (first ? 0.0 : acc[col]) + prod;
-                    if (first) mark[col] = q;
-                }
-                __syncthreads();
-                pf = nf;
-                have = nhave;
-                pc = nc;
-                pv = nv;
-            }
-        }
-        int *const ocol = tcol + uoff[r];
-        double *const oval = tval + uoff[r];
-        int base = 0;
-        for (int jb = 0; jb < m; jb += BS) {
-            const int j = jb + threadIdx.x;
-            const int fl = (j < m && mark[j] == q) ? 1 : 0;
-            int tot;
-            const int pos = base + block_scan_excl(fl, sh, &tot);
-            if (fl) {
-                ocol[pos] = j;
-                oval[pos] = acc[j];
-            }
-            base += tot;
-        }
-        if (threadIdx.x == 0) cnt[r] = base;
-        __syncthreads();
+    const int row = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    if (row >= n) return;
+    int *const o = seg + (long long)row * (nt + 1);
+    const int a = rp[row], b = rp[row + 1];
+    for (int f = a + lane; f < b; f += 64) {
+        const int t0 = f > a ? ci[f - 1] / W + 1 : 0, t1 = ci[f] / W;
+        for (int t = t0; t <= t1; t++) o[t] = f;
     }
+    const int last = b > a ? ci[b - 1] / W + 1 : 0;
+    for (int t = last + lane; t <= nt; t += 64) o[t] = b;
+}
+
+__device__ inline double lane_double(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)b, l);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+/* Long rows when C's columns fit LDS: a workgroup a row, a wavefront a column
+   tile of it with W accumulators in LDS. A wavefront walks the left entries
+   in order and adds the products of each one's segment of the right row, 64
+   lanes at a time: a right row's columns are distinct, so one LDS add
+   instruction never meets a column twice, and one wavefront's LDS
+   instructions execute in order - each column's sum is taken in the stated
+   order with no barrier between left entries. ds_add_f64 rounds as v_add_f64
+   does and returns nothing, so no step waits for the one before; the loads of
+   SG_AHEAD steps are issued ahead of their adds. An untouched column holds
+   -0.0: a product is added as prod + 0.0 (never -0.0), so a touched column is
+   never -0.0, and the row's columns come out in order by ballots. Rows next
+   to each other share right rows: an XCD takes consecutive ones.
+   The right rows bound it (12 bytes a product from L2 and the last-level
+   cache): T P with 2048 columns, 5.0e9 products, 4.6 ms (13 TB/s); R A with
+   4096 columns, 3.6e9 products, 5.6 ms (6.5 without the XCD order; A is
+   60 MB); both and T P of the level above 47.1 ms with a barrier per left
+   entry and a workgroup's lanes over one right row. Tiles of 512 / 2048
+   columns: the setup takes 2 % / 4 % longer. */
+__global__ __launch_bounds__(1024) void k_sg_wave(const int *__restrict__ large,
+                                                  const int *__restrict__ Lrp,
+                                                  const int *__restrict__ Lci,
+                                                  const double *__restrict__ Lv,
+                                                  const int *__restrict__ seg,
+                                                  const int *__restrict__ Rci,
+                                                  const double *__restrict__ Rv,
+                                                  const int *__restrict__ u,
+                                                  const int *__restrict__ uoff,
+                                                  int *__restrict__ tcol,
+                                                  double *__restrict__ tval, int W,
+                                                  int serial_min, int *__restrict__ cnt)
+{
+    extern __shared__ double sg_acc[];
+    __shared__ int wcnt[SG_TILES];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nt = blockDim.x >> 6;
+    const int r = large[xcd_block(blockIdx.x, gridDim.x)];
+    const int eb = Lrp[r], ee = Lrp[r + 1];
+    if (!((long long)u[r] >= (long long)serial_min * (ee - eb))) return;
+    double *const acc = sg_acc + wv * W;
+    for (int t = lane; t < W; t += 64) acc[t] = -0.0;
+    __syncthreads();
+    for (int e0 = eb; e0 < ee; e0 += 64) {
+        const int e = e0 + lane;
+        int s0 = 0, s1 = 0;
+        double lv = 0.0;
+        if (e < ee) {
+            const int *const o = seg + (long long)Lci[e] * (nt + 1) + wv;
+            s0 = o[0];
+            s1 = o[1];
+            lv = Lv[e];
+        }
+        unsigned long long todo = __ballot(s1 > s0);
+        int f = 0, f1 = 0;
+        double l = 0.0;
+        while (todo || f < f1) {
+            int cc[SG_AHEAD];
+            double vv[SG_AHEAD], ll[SG_AHEAD];
+#pragma unroll
+            for (int d = 0; d < SG_AHEAD; d++) {
+                if (f >= f1 && todo) {
+                    const int t = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    f = __builtin_amdgcn_readlane(s0, t);
+                    f1 = __builtin_amdgcn_readlane(s1, t);
+                    l = lane_double(lv, t);
+                }
+                const int p = f + lane;
+                const int pc = min(p, f1 - 1);
+                const int col = Rci[pc];
+                cc[d] = p < f1 ? col : -1;
+                vv[d] = Rv[pc];
+                ll[d] = l;
+                f += 64;
+            }
+#pragma unroll
+            for (int d = 0; d < SG_AHEAD; d++)
+                if (cc[d] >= 0)
+                    __hip_atomic_fetch_add(&sg_acc[cc[d]], ll[d] * vv[d] + 0.0, __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+        }
+    }
+    __syncthreads();
+    int mine = 0;
+    for (int t = lane; t < W; t += 64)
+        mine += __popcll(__ballot(__double_as_longlong(acc[t]) != SG_UNTOUCHED));
+    if (lane == 0) wcnt[wv] = mine;
+    __syncthreads();
+    int base = uoff[r], all = 0;
+    for (int w = 0; w < nt; w++) {
+        const int k = wcnt[w];
+        if (w < wv) base += k;
+        all += k;
+    }
+    for (int t = lane; t < W; t += 64) {
+        const double v = acc[t];
+        const bool have = __double_as_longlong(v) != SG_UNTOUCHED;
+        const unsigned long long b = __ballot(have);
+        if (have) {
+            const int o = base + __popcll(b & ((1ull << lane) - 1));
+            tcol[o] = wv * W + t;
+            tval[o] = v;
+        }
+        base += __popcll(b);
+    }
+    if (threadIdx.x == 0) cnt[r] = all;
 }
 
 /* compact the rows from their product-count slots into C (G lanes a row) */
@@ -796,20 +851,30 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
         return;
     }
     const long long mcols = R.m > 0 ? R.m : 1;
+    /* Long rows whose accumulators fit LDS go to k_sg_wave when their left
+       entries bring half a product per tile or more (below that most of its
+       steps add a lane or none; at 1.2 per tile, 16 384 columns, it takes
+       3.0 ms and the sorting form 4.9) and the tile pointers stay below R. */
+    const int tiles = (int)std::min<long long>((mcols + SG_TILE - 1) / SG_TILE, SG_TILES);
+    const int tile_w = (int)((mcols + 64ll * tiles - 1) / (64ll * tiles)) * 64;
+    const bool lds = right_unique && mcols <= SG_LDS_COLS &&
+                     (long long)R.n * (tiles + 1) <= 2ll * R.nnz;
+    const int smin = !right_unique ? 0 : lds ? std::max(1, tiles / 2) : SG_SERIAL_MIN;
     DBuf<int> u(n), sl(n), ws(n), cnt(n), large(n);
-    DBuf<int> flags(2);   /* long-row count, row with too many products */
+    /* long-row count, row with too many products, long rows below smin */
+    DBuf<int> flags(3);
     DBuf<unsigned long long> total(1);
-    BCMG_HIP(hipMemsetAsync(flags.get(), 0, 2 * sizeof(int), c.stream));
+    BCMG_HIP(hipMemsetAsync(flags.get(), 0, 3 * sizeof(int), c.stream));
     BCMG_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), c.stream));
     k_sg_count<<<blocks_for(n), BS, 0, c.stream>>>(n, L.rp, L.ci, R.rp, mcols, u.get(), sl.get(),
                                                    ws.get(), cnt.get(), large.get(), flags.get(),
-                                                   total.get(), flags.get() + 1);
+                                                   total.get(), flags.get() + 1, smin);
     BCMG_CHECK_LAUNCH();
     unsigned long long h_total = 0;
-    int h_flags[2] = {0, 0};
+    int h_flags[3] = {0, 0, 0};
     BCMG_HIP(hipMemcpyAsync(&h_total, total.get(), sizeof(h_total), hipMemcpyDeviceToHost,
                             c.stream));
-    BCMG_HIP(hipMemcpyAsync(h_flags, flags.get(), 2 * sizeof(int), hipMemcpyDeviceToHost,
+    BCMG_HIP(hipMemcpyAsync(h_flags, flags.get(), 3 * sizeof(int), hipMemcpyDeviceToHost,
                             c.stream));
     BCMG_HIP(hipStreamSynchronize(c.stream));
     const int h_nlarge = h_flags[0];
@@ -871,6 +936,7 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
     DBuf<double> acc;
     DBuf<int> stamp;
     int dblocks = 0;
+    DBuf<int> seg;
     for (size_t b = 0; b < nbatch; b++) {
         const int lo = blo[b], nr = bhi[b] - blo[b];
         const int *Lrp = L.rp + lo;
@@ -896,30 +962,36 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
             lrows = lbuf.get();
         }
         if (nl > 0) {
-            if (!acc.get()) {
-                /* dense accumulators: as many workgroups as the budget
-                   allows, stamps cleared once for every batch */
-                const long long per = 12 * mcols;
-                dblocks = (int)std::min<long long>(
-                    {(long long)h_nlarge, (long long)SG_DENSE_BLOCKS,
-                     std::max<long long>(1, SG_DENSE_BYTES / per)});
-                acc.alloc((size_t)dblocks * mcols);
-                stamp.alloc((size_t)dblocks * mcols);
-                BCMG_HIP(hipMemsetAsync(stamp.get(), 0xff, sizeof(int) * (size_t)dblocks * mcols,
-                                        c.stream));
+            if (lds) {
+                if (!seg.get()) {
+                    seg.alloc((size_t)R.n * (tiles + 1));
+                    k_sg_seg<<<blocks_for(64ll * R.n), BS, 0, c.stream>>>(R.n, R.rp, R.ci, tile_w,
+                                                                          tiles, seg.get());
+                }
+                k_sg_wave<<<nl, 64 * tiles, sizeof(double) * tiles * tile_w, c.stream>>>(
+                    lrows, Lrp, L.ci, L.v, seg.get(), R.ci, R.v, u.get() + lo, uoff.get(),
+                    tcol.get(), tval.get(), tile_w, smin, cnt.get() + lo);
+                BCMG_CHECK_LAUNCH();
             }
-            const int g = std::min(nl, dblocks);
-            const int smin = right_unique ? SG_SERIAL_MIN : 0;
-            const bool lds = smin > 0 && mcols <= SG_LDS_COLS;
-            if (lds)
-                k_sg_serial_lds<<<std::min(nl, SG_DENSE_BLOCKS), BS, 0, c.stream>>>(
+            if (!lds || h_flags[2] > 0) {
+                if (!acc.get()) {
+                    /* dense accumulators: as many workgroups as the budget
+                       allows, stamps cleared once for every batch */
+                    const long long per = 12 * mcols;
+                    dblocks = (int)std::min<long long>(
+                        {(long long)h_nlarge, (long long)SG_DENSE_BLOCKS,
+                         std::max<long long>(1, SG_DENSE_BYTES / per)});
+                    acc.alloc((size_t)dblocks * mcols);
+                    stamp.alloc((size_t)dblocks * mcols);
+                    BCMG_HIP(hipMemsetAsync(stamp.get(), 0xff,
+                                            sizeof(int) * (size_t)dblocks * mcols, c.stream));
+                }
+                k_sg_dense<<<std::min(nl, dblocks), BS, 0, c.stream>>>(
                     nl, lrows, Lrp, L.ci, L.v, R.rp, R.ci, R.v, u.get() + lo, uoff.get(),
-                    tcol.get(), tval.get(), (int)mcols, smin, cnt.get() + lo);
-            k_sg_dense<<<g, BS, 0, c.stream>>>(nl, lrows, Lrp, L.ci, L.v, R.rp, R.ci, R.v,
-                                               u.get() + lo, uoff.get(), tcol.get(), tval.get(),
-                                               acc.get(), stamp.get(), mcols, lo, smin,
-                                               lds ? 1 : 0, cnt.get() + lo);
-            BCMG_CHECK_LAUNCH();
+                    tcol.get(), tval.get(), acc.get(), stamp.get(), mcols, lo, smin, lds ? 1 : 0,
+                    cnt.get() + lo);
+                BCMG_CHECK_LAUNCH();
+            }
         }
         if (nbatch == 1) {
             const long long nnz = exclusive_scan(c, cnt.get(), C.row.get(), n, true);
