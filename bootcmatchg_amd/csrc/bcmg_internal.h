@@ -792,7 +792,7 @@ inline CsrRef ref_of(const DevCsr &A)
    right_unique: every row of R has distinct columns */
 void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_pass = 0,
             bool right_unique = true);
-/* T = A^T, each row in ascending column order */
+/* T = A^T, each row in ascending column order; A's rows have distinct columns */
 void transpose_csr(Ctx &c, const CsrRef &A, DevCsr &T);
 /* S = I - omega D^-1 A in A's pattern, omega = 4 / (3 ||D^-1 A||_inf) */
 double sa_smoother(Ctx &c, const DevCsr &A, const double *D, DBuf<double> &S);

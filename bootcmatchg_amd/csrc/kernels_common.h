@@ -25,6 +25,25 @@ __device__ __forceinline__ int xcd_block(int bid, int nb)
     return x * q + (x < rm ? x : rm) + l;
 }
 
+/* lane l's double, as a scalar */
+__device__ __forceinline__ double lane_double(double v, int l)
+{
+    const long long b = __double_as_longlong(v);
+    const unsigned lo = __builtin_amdgcn_readlane((int)b, l);
+    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+/* s + lane 0's v + lane 1's v + ..., added in this order, for the first n
+   lanes (v >= 0, and 0 in every lane from n on) */
+__device__ __forceinline__ double add_lanes_in_order(double s, double v, int n)
+{
+    for (int q = 0; q < 64 && q < n; q += 8)
+#pragma unroll
+        for (int t = 0; t < 8; t++) s += lane_double(v, q + t);
+    return s;
+}
+
 /* stored matrix value -> compute type (bfloat16: upper half of a float) */
 template <typename VT>
 __device__ __forceinline__ VT mval(double v) { return (VT)v; }
@@ -657,6 +676,10 @@ __device__ __forceinline__ void fcg_final_apply(const double (&res)[K], double *
         fcg_recurrence(scal);
     }
 }
+
+/* rows that a wavefront takes in the set-up's row kernels */
+constexpr int LANE_ROW = 16;
+inline bool long_rows(int n, long long nnz) { return n > 0 && nnz >= (long long)LANE_ROW * n; }
 
 inline int blocks_for(long long work) { return (int)((work + BS - 1) / BS); }
 

@@ -18,6 +18,7 @@
  * with compare-and-swap, so no lane ever waits on another lane of its wave.
  */
 #include "bcmg_internal.h"
+#include "kernels_common.h"
 #include "../../include/bcmg_log.h"
 
 #include <algorithm>
@@ -28,10 +29,8 @@ namespace bcmg {
 
 namespace {
 
-constexpr int BS = 256;
 constexpr int SCAN_CHUNK = BS * 4;
 
-inline int blocks_for(long long work) { return (int)((work + BS - 1) / BS); }
 
 /* ------------------------------------------------------------ scan */
 
@@ -111,29 +110,58 @@ __global__ __launch_bounds__(BS) void k_scan_apply(int n, const int *__restrict_
 
 /* --------------------------------------------------- diagonal, row sums */
 
+/* Rows of LANE_ROW entries or more on average take a wavefront each (G = 64),
+   shorter ones a lane: with 1218 entries a row (4096 rows) a lane's walk along
+   its row took 301 us (diagonal) and 302 us (sums), a wavefront's 16 and 79
+   (it adds lane by lane);
+   at 7 entries a lane's stays better (its 64 rows share the lines). */
+template <int G>
 __global__ __launch_bounds__(BS) void k_diag(int n, const int *__restrict__ rp,
                                              const int *__restrict__ ci,
                                              const double *__restrict__ av,
                                              double *__restrict__ D)
 {
-    const int i = blockIdx.x * BS + threadIdx.x;
+    const int i = (blockIdx.x * BS + threadIdx.x) / G;
     if (i >= n) return;
-    double d = 0.0;
-    for (int j = rp[i]; j < rp[i + 1]; j++)
-        if (ci[j] == i) d = av[j];
-    D[i] = d;
+    const int a = rp[i], b = rp[i + 1];
+    if (G == 1) {
+        double d = 0.0;
+        for (int j = a; j < b; j++)
+            if (ci[j] == i) d = av[j];
+        D[i] = d;
+        return;
+    }
+    const int lane = threadIdx.x & (G - 1);
+    int at = -1;
+    for (int j0 = a; j0 < b; j0 += G) {
+        const int j = j0 + lane;
+        const unsigned long long hit = __ballot(j < b && ci[j] == i);
+        if (hit) at = j0 + 63 - __clzll(hit);
+    }
+    if (lane == 0) D[i] = at >= 0 ? av[at] : 0.0;
 }
 
 /* sum_j |a_ij| in CSR order (src/matrix/CSR.cu:638-652) */
+template <int G>
 __global__ __launch_bounds__(BS) void k_abs_rowsum(int n, const int *__restrict__ rp,
                                                    const double *__restrict__ av,
                                                    double *__restrict__ M)
 {
-    const int i = blockIdx.x * BS + threadIdx.x;
+    const int i = (blockIdx.x * BS + threadIdx.x) / G;
     if (i >= n) return;
+    const int a = rp[i], b = rp[i + 1];
     double s = 0.0;
-    for (int j = rp[i]; j < rp[i + 1]; j++) s += fabs(av[j]);
-    M[i] = s;
+    if (G == 1) {
+        for (int j = a; j < b; j++) s += fabs(av[j]);
+        M[i] = s;
+        return;
+    }
+    const int lane = threadIdx.x & (G - 1);
+    for (int j0 = a; j0 < b; j0 += G) {
+        const int j = j0 + lane;
+        s = add_lanes_in_order(s, j < b ? fabs(av[j]) : 0.0, b - j0);
+    }
+    if (lane == 0) M[i] = s;
 }
 
 /* ------------------------------------------------------ matching weights */
@@ -968,13 +996,20 @@ long long exclusive_scan(Ctx &c, const int *in, int *out, int n, bool read_total
 
 void launch_diag(hipStream_t s, const DevCsr &A, double *D)
 {
-    k_diag<<<blocks_for(A.n), BS, 0, s>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D);
+    if (long_rows(A.n, A.nnz))
+        k_diag<64><<<blocks_for(64ll * A.n), BS, 0, s>>>(A.n, A.row.get(), A.col.get(),
+                                                         A.val.get(), D);
+    else
+        k_diag<1><<<blocks_for(A.n), BS, 0, s>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D);
     BCMG_CHECK_LAUNCH();
 }
 
 void launch_abs_rowsum(hipStream_t s, const DevCsr &A, double *M)
 {
-    k_abs_rowsum<<<blocks_for(A.n), BS, 0, s>>>(A.n, A.row.get(), A.val.get(), M);
+    if (long_rows(A.n, A.nnz))
+        k_abs_rowsum<64><<<blocks_for(64ll * A.n), BS, 0, s>>>(A.n, A.row.get(), A.val.get(), M);
+    else
+        k_abs_rowsum<1><<<blocks_for(A.n), BS, 0, s>>>(A.n, A.row.get(), A.val.get(), M);
     BCMG_CHECK_LAUNCH();
 }
 

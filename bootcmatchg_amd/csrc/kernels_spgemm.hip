@@ -51,8 +51,9 @@ constexpr int SG_TILE = 1024;         /* columns of a tile, about */
 constexpr int SG_LDS_COLS = SG_TILES * SG_TILE; /* columns of C, at most, for LDS accumulators */
 constexpr int SG_AHEAD = 8;           /* loads of 64 right entries in flight */
 constexpr long long SG_UNTOUCHED = LLONG_MIN;   /* the bits of -0.0 */
-constexpr int SHORT_ROW = 64;         /* transpose rows ranked by one lane */
+constexpr int WAVE_RANK = 256;        /* transpose rows ranked by one wavefront */
 constexpr int RANK_CHUNK = 4096;      /* columns per LDS load when ranking */
+constexpr int RANK_BITS = 32 * RANK_CHUNK; /* columns ranked by a bit each */
 constexpr unsigned long long SG_NONE = ~0ull;
 constexpr int POS_BITS = 11;          /* position field: < 2048 */
 constexpr int ROW_SHIFT = 42;         /* row field above 31 column bits */
@@ -127,8 +128,12 @@ __device__ inline int pow2_at_least(int v)
 /* per row: products u, output slots sl = min(products, columns of C) (a
    row has at most that many entries), packing weight ws, the long-row
    list and how many of it have fewer than smin products per left entry; the
-   total of slots plus weights (what a batch of rows is bounded by); *big = 1 if a row has 2^30 products or more */
-__global__ __launch_bounds__(BS) void k_sg_count(int n, const int *__restrict__ Lrp,
+   total of slots plus weights (what a batch of rows is bounded by); *big = 1
+   if a row has 2^30 products or more. G lanes a row, per_block (a multiple of
+   BS / G, at most 256) rows a workgroup with one atomic a counter: an atomic
+   per wavefront of one row each took 791 us at 65 536 rows. */
+template <int G>
+__global__ __launch_bounds__(BS) void k_sg_count(int n, int per_block, const int *__restrict__ Lrp,
                                                  const int *__restrict__ Lci,
                                                  const int *__restrict__ Rrp, long long m,
                                                  int *__restrict__ u, int *__restrict__ sl,
@@ -138,31 +143,50 @@ __global__ __launch_bounds__(BS) void k_sg_count(int n, const int *__restrict__ 
                                                  unsigned long long *__restrict__ total,
                                                  int *__restrict__ big, int smin)
 {
-    const int i = blockIdx.x * BS + threadIdx.x;
-    long long s = 0, slots = 0;
-    if (i < n) {
-        for (int e = Lrp[i]; e < Lrp[i + 1]; e++) {
+    __shared__ int list[256], nlist, nfew, at;
+    __shared__ unsigned long long part[BS / 64];
+    const int lane = threadIdx.x & (G - 1);
+    if (threadIdx.x == 0) nlist = nfew = 0;
+    __syncthreads();
+    unsigned long long t = 0;   /* the batch cost of the rows: slots plus packing weights */
+    const int i1 = min(n, (int)(blockIdx.x + 1) * per_block);
+    for (int i = blockIdx.x * per_block + threadIdx.x / G; i < i1; i += BS / G) {
+        const int b = Lrp[i + 1], a = Lrp[i];
+        long long s = 0;
+        for (int e = a + lane; e < b; e += G) {
             const int k = Lci[e];
             s += Rrp[k + 1] - Rrp[k];
         }
+#pragma unroll
+        for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+        if (lane != 0) continue;
         if (s >= (1ll << 30)) atomicOr(big, 1);
         u[i] = (int)(s < (1ll << 30) ? s : (1ll << 30));
-        slots = s < m ? s : m;
+        const long long slots = s < m ? s : m;
         sl[i] = (int)slots;
         cnt[i] = 0;
+        t += (unsigned long long)slots;
         if (s <= SG_CAP) {
             ws[i] = (int)s + 1;
+            t += s + 1;
         } else {
             ws[i] = 0;
-            large[atomicAdd(nlarge, 1)] = i;
-            if (s < (long long)smin * (Lrp[i + 1] - Lrp[i])) atomicAdd(nlarge + 2, 1);
+            list[atomicAdd(&nlist, 1)] = i;
+            if (s < (long long)smin * (b - a)) atomicAdd(&nfew, 1);
         }
     }
-    /* the batch cost of a row: its slots plus its packing weight */
-    unsigned long long t = (unsigned long long)slots + (i < n && s <= SG_CAP ? s + 1 : 0);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) t += __shfl_xor(t, o, 64);
-    if ((threadIdx.x & 63) == 0 && t) atomicAdd(total, t);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = t;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < BS / 64; w++) t += part[w];
+        if (t) atomicAdd(total, t);
+        if (nlist) at = atomicAdd(nlarge, nlist);
+        if (nfew) atomicAdd(nlarge + 2, nfew);
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < nlist) large[at + threadIdx.x] = list[threadIdx.x];
 }
 
 /* the packed rows of one workgroup (see the file comment) */
@@ -510,14 +534,6 @@ __global__ __launch_bounds__(BS) void k_sg_seg(int n, const int *__restrict__ rp
     for (int t = last + lane; t <= nt; t += 64) o[t] = b;
 }
 
-__device__ inline double lane_double(double v, int l)
-{
-    const long long b = __double_as_longlong(v);
-    const unsigned lo = __builtin_amdgcn_readlane((int)b, l);
-    const unsigned hi = __builtin_amdgcn_readlane((int)(b >> 32), l);
-    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-
 /* Long rows when C's columns fit LDS: a workgroup a row, a wavefront a column
    tile of it with W accumulators in LDS. A wavefront walks the left entries
    in order and adds the products of each one's segment of the right row, 64
@@ -552,9 +568,10 @@ __global__ __launch_bounds__(1024) void k_sg_wave(const int *__restrict__ large,
     extern __shared__ double sg_acc[];
     __shared__ int wcnt[SG_TILES];
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nt = blockDim.x >> 6;
-    const int r = large[xcd_block(blockIdx.x, gridDim.x)];
+    const int b0 = xcd_block(blockIdx.x, gridDim.x);
+    const int r = large ? large[b0] : b0;
     const int eb = Lrp[r], ee = Lrp[r + 1];
-    if (!((long long)u[r] >= (long long)serial_min * (ee - eb))) return;
+    if (u[r] <= SG_CAP || (long long)u[r] < (long long)serial_min * (ee - eb)) return;
     double *const acc = sg_acc + wv * W;
     for (int t = lane; t < W; t += 64) acc[t] = -0.0;
     __syncthreads();
@@ -646,80 +663,116 @@ __global__ __launch_bounds__(BS) void k_sg_gather(int n, const int *__restrict__
 
 /* ------------------------------------------------------------ transpose */
 
+/* A's rows by G lanes each */
+template <int G>
 __global__ __launch_bounds__(BS) void k_col_count(int n, const int *__restrict__ rp,
                                                   const int *__restrict__ ci,
                                                   int *__restrict__ cnt)
 {
-    const int i = blockIdx.x * BS + threadIdx.x;
+    const int i = (blockIdx.x * BS + threadIdx.x) / G;
     if (i >= n) return;
-    for (int e = rp[i]; e < rp[i + 1]; e++) atomicAdd(&cnt[ci[e]], 1);
+    const int b = rp[i + 1];
+    for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) atomicAdd(&cnt[ci[e]], 1);
 }
 
+template <int G>
 __global__ __launch_bounds__(BS) void k_col_fill(int n, const int *__restrict__ rp,
                                                  const int *__restrict__ ci,
                                                  const double *__restrict__ v,
                                                  int *__restrict__ cursor, int *__restrict__ tcol,
                                                  double *__restrict__ tval)
 {
-    const int i = blockIdx.x * BS + threadIdx.x;
+    const int i = (blockIdx.x * BS + threadIdx.x) / G;
     if (i >= n) return;
-    for (int e = rp[i]; e < rp[i + 1]; e++) {
+    const int b = rp[i + 1];
+    for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) {
         const int pos = atomicAdd(&cursor[ci[e]], 1);
         tcol[pos] = i;
         tval[pos] = v[e];
     }
 }
 
-/* Each row of the transpose in ascending column order: an entry's place is
-   its rank among the row's entries (column, then fill position for equal
-   columns). Rows up to SHORT_ROW entries: one lane each; longer rows are
-   listed for k_rank_long. */
-__global__ __launch_bounds__(BS) void k_rank_short(int nr, const int *__restrict__ rp,
-                                                   const int *__restrict__ cin,
-                                                   const double *__restrict__ vin,
-                                                   int *__restrict__ col, double *__restrict__ val,
-                                                   int *__restrict__ longl, int *__restrict__ nlong)
+/* Each row of the transpose in ascending column order (distinct columns): an
+   entry's place is its rank among the row's entries. A wavefront a row of up
+   to WAVE_RANK entries, compared lane against lane; longer rows are listed
+   for k_rank_long. 16 384 rows of 75 entries: 473 us with a lane a row (to
+   64 entries, the rest with the long ones), 31 so. */
+__global__ __launch_bounds__(BS) void k_rank(int nr, const int *__restrict__ rp,
+                                             const int *__restrict__ cin,
+                                             const double *__restrict__ vin,
+                                             int *__restrict__ col, double *__restrict__ val,
+                                             int *__restrict__ longl, int *__restrict__ nlong)
 {
-    const int I = blockIdx.x * BS + threadIdx.x;
+    const int I = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
     if (I >= nr) return;
-    const int a = rp[I], b = rp[I + 1];
-    if (b - a > SHORT_ROW) {
-        longl[atomicAdd(nlong, 1)] = I;
+    const int a = rp[I], len = rp[I + 1] - a;
+    if (len > WAVE_RANK) {
+        if (lane == 0) longl[atomicAdd(nlong, 1)] = I;
         return;
     }
-    for (int e = a; e < b; e++) {
-        const int c = cin[e];
-        int rank = 0;
-        for (int f = a; f < b; f++) {
-            const int d = cin[f];
-            rank += (d < c || (d == c && f < e)) ? 1 : 0;
-        }
-        col[a + rank] = c;
-        val[a + rank] = vin[e];
+    constexpr int Q = WAVE_RANK / 64;
+    int c[Q], rank[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        c[q] = q * 64 + lane < len ? cin[a + q * 64 + lane] : INT_MAX;
+        rank[q] = 0;
     }
+#pragma unroll
+    for (int f = 0; f < Q; f++) {
+        if (f * 64 >= len) break;
+        const int nf = min(64, len - f * 64);
+        for (int t = 0; t < nf; t++) {
+            const int d = __builtin_amdgcn_readlane(c[f], t);
+#pragma unroll
+            for (int q = 0; q < Q; q++) rank[q] += d < c[q] ? 1 : 0;
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+        if (q * 64 + lane < len) {
+            col[a + rank[q]] = c[q];
+            val[a + rank[q]] = vin[a + q * 64 + lane];
+        }
 }
 
-/* a long row per workgroup: ranks against the row's columns staged in LDS,
-   RANK_CHUNK at a time */
-__global__ __launch_bounds__(BS) void k_rank_long(const int *__restrict__ longl,
+/* A long row per workgroup, m columns. Up to RANK_BITS of them: the row's
+   columns set bits in LDS and an entry's rank is the number of bits below
+   its own (2048 rows of 1291 entries, 4096 columns: 979 us by comparing all
+   pairs, 24 so); more: ranks against the row's columns, RANK_CHUNK at a
+   time. */
+__global__ __launch_bounds__(BS) void k_rank_long(const int *__restrict__ longl, int m,
                                                   const int *__restrict__ rp,
                                                   const int *__restrict__ cin,
                                                   const double *__restrict__ vin,
                                                   int *__restrict__ col, double *__restrict__ val)
 {
     __shared__ int buf[RANK_CHUNK];
+    __shared__ int pre[RANK_CHUNK];
+    __shared__ int sh[BS / 64];
     const int I = longl[blockIdx.x];
     const int a = rp[I], len = rp[I + 1] - a;
-    if (len <= RANK_CHUNK) {
-        for (int t = threadIdx.x; t < len; t += BS) buf[t] = cin[a + t];
+    if (m <= RANK_BITS) {
+        unsigned *const bit = reinterpret_cast<unsigned *>(buf);
+        const int words = (m + 31) >> 5;
+        for (int t = threadIdx.x; t < words; t += BS) bit[t] = 0;
         __syncthreads();
         for (int e = threadIdx.x; e < len; e += BS) {
-            const int c = buf[e];
-            int rank = 0;
-            for (int f = 0; f < len; f++) {
-                const int d = buf[f];
-                rank += (d < c || (d == c && f < e)) ? 1 : 0;
-            }
+            const int c = cin[a + e];
+            atomicOr(&bit[c >> 5], 1u << (c & 31));
+        }
+        __syncthreads();
+        int base = 0;
+        for (int t0 = 0; t0 < words; t0 += BS) {
+            const int t = t0 + threadIdx.x;
+            int tot;
+            const int x = block_scan_excl(t < words ? __popc(bit[t]) : 0, sh, &tot);
+            if (t < words) pre[t] = base + x;
+            base += tot;
+        }
+        __syncthreads();
+        for (int e = threadIdx.x; e < len; e += BS) {
+            const int c = cin[a + e];
+            const int rank = pre[c >> 5] + __popc(bit[c >> 5] & ((1u << (c & 31)) - 1));
             col[a + rank] = c;
             val[a + rank] = vin[a + e];
         }
@@ -735,10 +788,7 @@ __global__ __launch_bounds__(BS) void k_rank_long(const int *__restrict__ longl,
             for (int t = threadIdx.x; t < nk; t += BS) buf[t] = cin[a + k0 + t];
             __syncthreads();
             if (e < len)
-                for (int t = 0; t < nk; t++) {
-                    const int d = buf[t];
-                    rank += (d < c || (d == c && k0 + t < e)) ? 1 : 0;
-                }
+                for (int t = 0; t < nk; t++) rank += buf[t] < c ? 1 : 0;
         }
         if (e < len) {
             col[a + rank] = c;
@@ -752,40 +802,64 @@ __global__ __launch_bounds__(BS) void k_rank_long(const int *__restrict__ longl,
 /* s_ij = a_ij / d_i (CSRm::matrixVectorScaling, src/matrix/CSR.cu:520-545)
    and the largest 0 + sum_j |s_ij| in storage order (CSR.cu:386-416): row
    sums are >= 0, so their bit patterns order as the values do */
-__global__ __launch_bounds__(BS) void k_sa_scale(int n, const int *__restrict__ rp,
+template <int G>
+__global__ __launch_bounds__(BS) void k_sa_scale(int n, int per_block, const int *__restrict__ rp,
                                                  const double *__restrict__ av,
                                                  const double *__restrict__ D,
                                                  double *__restrict__ sv,
                                                  unsigned long long *__restrict__ norm)
 {
-    const int i = blockIdx.x * BS + threadIdx.x;
-    double s = 0.0;
-    if (i < n) {
+    __shared__ unsigned long long part[BS / 64];
+    unsigned long long top = 0;
+    const int i1 = min(n, (int)(blockIdx.x + 1) * per_block);
+    for (int i = blockIdx.x * per_block + threadIdx.x / G; i < i1; i += BS / G) {
         const double d = D[i];
-        for (int e = rp[i]; e < rp[i + 1]; e++) {
-            const double t = av[e] / d;
-            sv[e] = t;
-            s += fabs(t);
+        const int a = rp[i], b = rp[i + 1];
+        double s = 0.0;
+        if (G == 1) {
+            for (int e = a; e < b; e++) {
+                const double t = av[e] / d;
+                sv[e] = t;
+                s += fabs(t);
+            }
+        } else {
+            for (int e0 = a; e0 < b; e0 += G) {
+                const int e = e0 + (int)(threadIdx.x & (G - 1));
+                double t = 0.0;
+                if (e < b) {
+                    t = av[e] / d;
+                    sv[e] = t;
+                }
+                s = add_lanes_in_order(s, fabs(t), b - e0);
+            }
         }
+        const unsigned long long y = s > 0.0 ? (unsigned long long)__double_as_longlong(s) : 0ull;
+        top = y > top ? y : top;
     }
-    unsigned long long b = (s > 0.0) ? (unsigned long long)__double_as_longlong(s) : 0ull;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-        const unsigned long long y = __shfl_xor(b, o, 64);
-        b = y > b ? y : b;
+        const unsigned long long y = __shfl_xor(top, o, 64);
+        top = y > top ? y : top;
     }
-    if ((threadIdx.x & 63) == 0 && b) atomicMax(norm, b);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = top;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < BS / 64; w++) top = part[w] > top ? part[w] : top;
+        if (top) atomicMax(norm, top);
+    }
 }
 
 /* s_ij = -omega s_ij, plus 1 on the diagonal (_applyOmega,
    src/AMG/matchingAggregation.cu:64-80) */
+template <int G>
 __global__ __launch_bounds__(BS) void k_sa_omega(int n, const int *__restrict__ rp,
                                                  const int *__restrict__ ci, double omega,
                                                  double *__restrict__ sv)
 {
-    const int i = blockIdx.x * BS + threadIdx.x;
+    const int i = (blockIdx.x * BS + threadIdx.x) / G;
     if (i >= n) return;
-    for (int e = rp[i]; e < rp[i + 1]; e++) {
+    const int b = rp[i + 1];
+    for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) {
         double t = -omega * sv[e];
         if (ci[e] == i) t += 1.;
         sv[e] = t;
@@ -809,6 +883,14 @@ __global__ __launch_bounds__(BS) void k_negate(long long n, double *__restrict__
 /* ================================================================ host */
 
 namespace {
+
+/* rows of a workgroup that takes several and ends with one atomic: about
+   1024 workgroups of BS / 64 rows (a lane each: BS) to 256 */
+int rows_per_block(int n, bool lng)
+{
+    const int step = lng ? BS / 64 : BS;
+    return std::min(256, std::max(1, (n / 1024 + step - 1) / step) * step);
+}
 
 /* gather rows [0, n) from their product slots into (col, val) by rp */
 void gather_rows(Ctx &c, int n, const int *uoff, const int *rp, const int *tcol,
@@ -866,9 +948,11 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
     DBuf<unsigned long long> total(1);
     BCMG_HIP(hipMemsetAsync(flags.get(), 0, 3 * sizeof(int), c.stream));
     BCMG_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), c.stream));
-    k_sg_count<<<blocks_for(n), BS, 0, c.stream>>>(n, L.rp, L.ci, R.rp, mcols, u.get(), sl.get(),
-                                                   ws.get(), cnt.get(), large.get(), flags.get(),
-                                                   total.get(), flags.get() + 1, smin);
+    const bool lng = long_rows(n, L.nnz);
+    const int per = rows_per_block(n, lng);
+    (lng ? k_sg_count<64> : k_sg_count<1>)<<<(n + per - 1) / per, BS, 0, c.stream>>>(
+        n, per, L.rp, L.ci, R.rp, mcols, u.get(), sl.get(), ws.get(), cnt.get(), large.get(),
+        flags.get(), total.get(), flags.get() + 1, smin);
     BCMG_CHECK_LAUNCH();
     unsigned long long h_total = 0;
     int h_flags[3] = {0, 0, 0};
@@ -968,9 +1052,13 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
                     k_sg_seg<<<blocks_for(64ll * R.n), BS, 0, c.stream>>>(R.n, R.rp, R.ci, tile_w,
                                                                           tiles, seg.get());
                 }
-                k_sg_wave<<<nl, 64 * tiles, sizeof(double) * tiles * tile_w, c.stream>>>(
-                    lrows, Lrp, L.ci, L.v, seg.get(), R.ci, R.v, u.get() + lo, uoff.get(),
-                    tcol.get(), tval.get(), tile_w, smin, cnt.get() + lo);
+                /* mostly long rows: by row, which keeps their order (the list
+                   is in order of arrival) */
+                const bool by_row = nl >= nr / 2;
+                k_sg_wave<<<by_row ? nr : nl, 64 * tiles, sizeof(double) * tiles * tile_w,
+                            c.stream>>>(by_row ? nullptr : lrows, Lrp, L.ci, L.v, seg.get(), R.ci,
+                                        R.v, u.get() + lo, uoff.get(), tcol.get(), tval.get(),
+                                        tile_w, smin, cnt.get() + lo);
                 BCMG_CHECK_LAUNCH();
             }
             if (!lds || h_flags[2] > 0) {
@@ -1048,25 +1136,29 @@ void transpose_csr(Ctx &c, const CsrRef &A, DevCsr &T)
     DBuf<int> nlong(1);
     BCMG_HIP(hipMemsetAsync(cnt.get(), 0, sizeof(int) * (nr > 0 ? nr : 1), c.stream));
     BCMG_HIP(hipMemsetAsync(nlong.get(), 0, sizeof(int), c.stream));
-    if (A.n > 0) k_col_count<<<blocks_for(A.n), BS, 0, c.stream>>>(A.n, A.rp, A.ci, cnt.get());
+    const bool lng = long_rows(A.n, A.nnz);
+    const int gb = blocks_for(lng ? 64ll * A.n : A.n);
+    if (A.n > 0)
+        (lng ? k_col_count<64> : k_col_count<1>)<<<gb, BS, 0, c.stream>>>(A.n, A.rp, A.ci,
+                                                                          cnt.get());
     BCMG_CHECK_LAUNCH();
     exclusive_scan(c, cnt.get(), T.row.get(), nr, false);
     BCMG_HIP(hipMemcpyAsync(cursor.get(), T.row.get(), sizeof(int) * ((size_t)nr + 1),
                             hipMemcpyDeviceToDevice, c.stream));
     if (A.n > 0)
-        k_col_fill<<<blocks_for(A.n), BS, 0, c.stream>>>(A.n, A.rp, A.ci, A.v, cursor.get(),
-                                                         fcol.get(), fval.get());
+        (lng ? k_col_fill<64> : k_col_fill<1>)<<<gb, BS, 0, c.stream>>>(
+            A.n, A.rp, A.ci, A.v, cursor.get(), fcol.get(), fval.get());
     if (nr > 0)
-        k_rank_short<<<blocks_for(nr), BS, 0, c.stream>>>(nr, T.row.get(), fcol.get(),
-                                                          fval.get(), T.col.get(), T.val.get(),
-                                                          longl.get(), nlong.get());
+        k_rank<<<blocks_for(64ll * nr), BS, 0, c.stream>>>(nr, T.row.get(), fcol.get(),
+                                                           fval.get(), T.col.get(), T.val.get(),
+                                                           longl.get(), nlong.get());
     BCMG_CHECK_LAUNCH();
     int h_long = 0;
     BCMG_HIP(hipMemcpyAsync(&h_long, nlong.get(), sizeof(int), hipMemcpyDeviceToHost, c.stream));
     BCMG_HIP(hipStreamSynchronize(c.stream));
     if (h_long > 0)
-        k_rank_long<<<h_long, BS, 0, c.stream>>>(longl.get(), T.row.get(), fcol.get(), fval.get(),
-                                                 T.col.get(), T.val.get());
+        k_rank_long<<<h_long, BS, 0, c.stream>>>(longl.get(), A.n, T.row.get(), fcol.get(),
+                                                 fval.get(), T.col.get(), T.val.get());
     BCMG_CHECK_LAUNCH();
     T.group = lanes_for(nr, A.nnz);
     launch_block_nnz(c, T);
@@ -1078,8 +1170,11 @@ double sa_smoother(Ctx &c, const DevCsr &A, const double *D, DBuf<double> &S)
     S.alloc(A.nnz > 0 ? (size_t)A.nnz : 1);
     DBuf<unsigned long long> nb(1);
     BCMG_HIP(hipMemsetAsync(nb.get(), 0, sizeof(unsigned long long), c.stream));
-    k_sa_scale<<<blocks_for(n), BS, 0, c.stream>>>(n, A.row.get(), A.val.get(), D, S.get(),
-                                                   nb.get());
+    const bool lng = long_rows(n, A.nnz);
+    const int gb = blocks_for(lng ? 64ll * n : n);
+    const int per = rows_per_block(n, lng);
+    (lng ? k_sa_scale<64> : k_sa_scale<1>)<<<(n + per - 1) / per, BS, 0, c.stream>>>(
+        n, per, A.row.get(), A.val.get(), D, S.get(), nb.get());
     BCMG_CHECK_LAUNCH();
     unsigned long long bits = 0;
     BCMG_HIP(hipMemcpyAsync(&bits, nb.get(), sizeof(bits), hipMemcpyDeviceToHost, c.stream));
@@ -1087,7 +1182,8 @@ double sa_smoother(Ctx &c, const DevCsr &A, const double *D, DBuf<double> &S)
     double norm;
     std::memcpy(&norm, &bits, sizeof(norm));
     const double omega = 4.0 / (3.0 * norm);
-    k_sa_omega<<<blocks_for(n), BS, 0, c.stream>>>(n, A.row.get(), A.col.get(), omega, S.get());
+    (lng ? k_sa_omega<64> : k_sa_omega<1>)<<<gb, BS, 0, c.stream>>>(n, A.row.get(), A.col.get(),
+                                                                    omega, S.get());
     BCMG_CHECK_LAUNCH();
     return omega;
 }
