@@ -20,6 +20,18 @@ namespace bcmg {
 
 namespace {
 
+/* The rows kernels by entries: operators up to ENTRY_SMALL rows (64 rows a
+   block), and above it rows of ENTRY_AVG entries or more on average (128).
+   Sweeps, rows form -> entry form, us: 5619 rows of up to 63 entries 9.1 -> 5.5,
+   10 172 7.3 -> 4.8, 69 004 x 11.3 6.2 -> 5.5, 214 477 x 13.6 15.1 -> 11.3,
+   637 953 x 11.5 23.5 -> 21.0 (5.1 TB/s from the caches); with 7 entries a row
+   and neighbours' columns next to each other the row form's gathers coalesce:
+   226 981 rows 5.8 against 8.1, 2.1 M 35.3 against 49. */
+constexpr int ENTRY_SMALL = SMALL_LEVEL_ROWS;
+constexpr int ENTRY_AVG = 9;
+/* k_rows_entry's sweep after a prolongation */
+constexpr int OP_JACOBI_P = 4;
+
 /* layout of the context's reduction scratch (doubles) */
 constexpr size_t RED_UPD = 3 * RED_MAX_BLOCKS + 16;   /* update/norm partials */
 constexpr size_t RED_SPMV = 4 * RED_MAX_BLOCKS + 32;  /* SpMV+dots partials */
@@ -82,6 +94,106 @@ __global__ __launch_bounds__(BS) void k_rows_staged(int n, const int *__restrict
         y[r] = (fr - t) / dr + xr;
 }
 
+/* Rows of irregular operators and small levels: a block of BS lanes owns R
+   rows; a lane takes an entry at a time (U of them in flight), gathers x for
+   it and leaves the product in LDS, and the row's lane adds its products in
+   CSR order - k_rows_staged's sum bit for bit. The row form gathers eight
+   entries of its row at a time and waits for each eight; here every gather of
+   the block is issued at once, which is what a small level with long rows
+   waits for, and no column goes through LDS. OP_JACOBI_P: the first sweep
+   after the prolongation, from x~ = x + P x_c formed where it is read
+   (k_prolong's fma at every gather and for the row itself), so y equals a
+   prolongation launch and a sweep launch; x~ is not stored (the sweep's result
+   replaces it). 6351 rows: 22.6 -> 7 us. */
+template <typename MT, typename VT, int OP, bool NT, int R, int U>
+__global__ __launch_bounds__(BS) void k_rows_entry(int n, const int *__restrict__ rp,
+                                                   const int *__restrict__ ci,
+                                                   const MT *__restrict__ av,
+                                                   const VT *__restrict__ x,
+                                                   const VT *__restrict__ f,
+                                                   const VT *__restrict__ d,
+                                                   VT *__restrict__ y,
+                                                   const int *__restrict__ agg,
+                                                   const VT *__restrict__ p,
+                                                   const VT *__restrict__ xc)
+{
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_ent[];
+    VT *const prod = reinterpret_cast<VT *>(smem_ent);
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int r0 = b * R;
+    const int r1 = min(r0 + R, n);
+    const int r = r0 + threadIdx.x;
+    const bool own = r < r1;
+    const int e0 = rp[r0];
+    const int cnt = rp[r1] - e0;
+    int ra = 0, re = 0;
+    VT fr = 0, dr = 1, xr = 0;
+    if (own) {
+        ra = rp[r] - e0;
+        re = rp[r + 1] - e0;
+        if (OP != OP_SPMV) fr = f[r];
+        if (OP == OP_JACOBI || OP == OP_JACOBI_P) {
+            dr = d[r];
+            xr = x[r];
+            if (OP == OP_JACOBI_P) xr = fma(p[r], xc[agg[r]], xr);
+        } else if (OP == OP_JACOBI_Z) {
+            dr = d[r];
+            xr = fr / dr;
+        }
+    }
+    const int *const cb = ci + e0;
+    const MT *const vb = av + e0;
+    for (int base = threadIdx.x; base < cnt; base += U * BS) {
+        int c[U];
+        VT v[U], g[U];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int e = min(base + u * BS, cnt - 1);
+            c[u] = ldm<NT>(cb + e);
+            v[u] = mval<VT>(ldm<NT>(vb + e));
+        }
+        if (OP == OP_JACOBI_Z) {
+            VT gd[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                g[u] = f[c[u]];
+                gd[u] = d[c[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) g[u] = g[u] / gd[u];
+        } else if (OP == OP_JACOBI_P) {
+            int a[U];
+            VT pc[U], gx[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                a[u] = agg[c[u]];
+                pc[u] = p[c[u]];
+                gx[u] = x[c[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < U; u++) g[u] = xc[a[u]];
+#pragma unroll
+            for (int u = 0; u < U; u++) g[u] = fma(pc[u], g[u], gx[u]);
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; u++) g[u] = x[c[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (base + u * BS < cnt) prod[base + u * BS] = v[u] * g[u];
+    }
+    __syncthreads();
+    if (!own) return;
+    VT t = 0;
+    for (int k = ra; k < re; k++) t = t + prod[k];
+    if (OP == OP_SPMV)
+        y[r] = t;
+    else if (OP == OP_RESID)
+        y[r] = fr - t;
+    else
+        y[r] = (fr - t) / dr + xr;
+}
+
 /* k_rows_staged on a stencil-pattern operator: the block reads its rows'
    one-byte masks, two row pointers (its first value and its end) and its
    values (into LDS); each row's value positions come from a block scan of
@@ -131,50 +243,6 @@ __global__ __launch_bounds__(BS) void k_rows_pattern(int n, const int *__restric
         y[r] = fr - t;
     else
         y[r] = (fr - t) / dr + xr;
-}
-
-/* The first Jacobi/L1 sweep after the prolongation, from x~ = x + P x_c
-   formed where it is read (k_prolong's fma at every gather and for the row
-   itself) and summed in column order from 0, so y equals a prolongation
-   launch followed by a sweep launch bit for bit; x~ is not stored (the
-   sweep's result replaces it). One thread per row: for small levels, where
-   the launch saved costs more than the dependent loads. */
-template <typename MT, typename VT>
-__global__ __launch_bounds__(BS) void k_jacobi_prolong(int n, const int *__restrict__ rp,
-                                                       const int *__restrict__ ci,
-                                                       const MT *__restrict__ av,
-                                                       const int *__restrict__ agg,
-                                                       const VT *__restrict__ p,
-                                                       const VT *__restrict__ xc,
-                                                       const VT *__restrict__ x,
-                                                       const VT *__restrict__ f,
-                                                       const VT *__restrict__ d,
-                                                       VT *__restrict__ y)
-{
-    const int r = blockIdx.x * BS + threadIdx.x;
-    if (r >= n) return;
-    const VT xr = fma(p[r], xc[agg[r]], x[r]);
-    const VT fr = f[r], dr = d[r];
-    const int j1 = rp[r + 1];
-    VT t = 0;
-    constexpr int PF = 8;
-    for (int j0 = rp[r]; j0 < j1; j0 += PF) {
-        int c[PF];
-        VT v[PF], g[PF];
-#pragma unroll
-        for (int u = 0; u < PF; u++)
-            if (j0 + u < j1) {
-                c[u] = ci[j0 + u];
-                v[u] = mval<VT>(av[j0 + u]);
-            }
-#pragma unroll
-        for (int u = 0; u < PF; u++)
-            if (j0 + u < j1) g[u] = fma(p[c[u]], xc[agg[c[u]]], x[c[u]]);
-#pragma unroll
-        for (int u = 0; u < PF; u++)
-            if (j0 + u < j1) t = t + v[u] * g[u];
-    }
-    y[r] = (fr - t) / dr + xr;
 }
 
 /* Setup of the pattern, step 1: the distinct column offsets of each 256-row
@@ -722,6 +790,33 @@ PatOffsets pattern_offsets(const DevCsr &A)
     return po;
 }
 
+template <typename MT, typename VT, int OP, bool NT, int R, int U>
+void launch_entry_as(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, const VT *f,
+                     const VT *d, VT *y, const int *agg, const VT *p, const VT *xc)
+{
+    const long long most = A.maxrow > 0 ? std::min<long long>(A.tile, (long long)R * A.maxrow)
+                                        : A.tile;
+    const size_t lds = (size_t)most * sizeof(VT);
+    k_rows_entry<MT, VT, OP, NT, R, U><<<(A.n + R - 1) / R, BS, lds, s>>>(
+        A.n, A.row.get(), A.col.get(), av, x, f, d, y, agg, p, xc);
+}
+
+template <typename MT, typename VT, int OP>
+bool launch_entry(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, const VT *f,
+                  const VT *d, VT *y, const int *agg = nullptr, const VT *p = nullptr,
+                  const VT *xc = nullptr)
+{
+    if (A.n <= ENTRY_SMALL)
+        launch_entry_as<MT, VT, OP, false, 64, 3>(s, A, av, x, f, d, y, agg, p, xc);
+    else if (A.nnz < (long long)ENTRY_AVG * A.n)
+        return false;
+    else if ((size_t)A.nnz * (4 + sizeof(MT)) > NT_BYTES)
+        launch_entry_as<MT, VT, OP, true, 128, 8>(s, A, av, x, f, d, y, agg, p, xc);
+    else
+        launch_entry_as<MT, VT, OP, false, 128, 8>(s, A, av, x, f, d, y, agg, p, xc);
+    return true;
+}
+
 template <typename MT, typename VT, int OP>
 void rows_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, const VT *f,
                 const VT *d, VT *y)
@@ -762,6 +857,7 @@ void rows_typed(hipStream_t s, const DevCsr &A, const MT *av, const VT *x, const
         }
         const size_t lds = staged_lds_bytes(A.tile, sizeof(MT));
         if (lds > 65536) throw Error(BCMG_EUNSUP, "row tile too large for this value type");
+        if (launch_entry<MT, VT, OP>(s, A, av, x, f, d, y)) return;
         if ((size_t)A.nnz * (4 + sizeof(MT)) > NT_BYTES)
             k_rows_staged<MT, VT, OP, true, int><<<nb, BS, lds, s>>>(n, rp, ci, av, x, f, d, y,
                                                                      A.tile);
@@ -1103,24 +1199,23 @@ bool launch_jacobi_prolong(hipStream_t s, const DevCsr &A, MatType mt, const int
 {
     if (!stream_ok<VT>(A)) return false;
     if (x == y) throw Error(BCMG_EINVAL, "prolongation sweep into its own input");
-    const int n = A.n;
-    const int *rp = A.row.get(), *ci = A.col.get();
-    if (n <= 0) return true;
+    if (A.n <= 0) return true;
+    bool done;
     if constexpr (std::is_same<VT, double>::value) {
         if (mt != MT_F64) throw Error(BCMG_EINVAL, "FP64 vectors need FP64 matrix values");
-        k_jacobi_prolong<double, double><<<blocks_for(n), BS, 0, s>>>(n, rp, ci, A.val.get(), agg,
-                                                                      p, xc, x, f, d, y);
+        done = launch_entry<double, double, OP_JACOBI_P>(s, A, A.val.get(), x, f, d, y, agg, p, xc);
     } else {
         if (mt == MT_F32)
-            k_jacobi_prolong<float, float><<<blocks_for(n), BS, 0, s>>>(
-                n, rp, ci, A.val32.get(), agg, p, xc, x, f, d, y);
+            done = launch_entry<float, float, OP_JACOBI_P>(s, A, A.val32.get(), x, f, d, y, agg,
+                                                           p, xc);
         else if (mt == MT_BF16)
-            k_jacobi_prolong<unsigned short, float><<<blocks_for(n), BS, 0, s>>>(
-                n, rp, ci, A.val16.get(), agg, p, xc, x, f, d, y);
+            done = launch_entry<unsigned short, float, OP_JACOBI_P>(s, A, A.val16.get(), x, f, d,
+                                                                    y, agg, p, xc);
         else
-            k_jacobi_prolong<double, float><<<blocks_for(n), BS, 0, s>>>(
-                n, rp, ci, A.val.get(), agg, p, xc, x, f, d, y);
+            done = launch_entry<double, float, OP_JACOBI_P>(s, A, A.val.get(), x, f, d, y, agg,
+                                                            p, xc);
     }
+    if (!done) return false;
     BCMG_CHECK_LAUNCH();
     return true;
 }
