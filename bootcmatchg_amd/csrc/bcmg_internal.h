@@ -11,6 +11,7 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <list>
 #include <map>
 #include <memory>
 #include <unordered_map>
@@ -53,19 +54,43 @@ void set_last_error(const std::string &msg);
    kernel still reads it is only reused by work queued after that kernel.
    hipMalloc/hipFree of large buffers cost milliseconds and hipFree
    synchronises the device; the setup allocates and drops hundreds of
-   temporaries, so it goes through the pool. */
+   temporaries, so it goes through the pool. Blocks of up to SUB_MAX bytes
+   are cut from chunks (CHUNK_MIN bytes, each twice the last up to CHUNK_MAX,
+   so at most about as much again as the blocks take), since a call each to
+   get and to give back some 250 of them cost a 226 981-row solve from host arrays 14 of 29 ms;
+   a chunk goes back to the device when all its blocks are free and trim or
+   free_released asks for it. */
 struct Pool {
-    std::multimap<size_t, void *> free_;
-    std::unordered_map<void *, size_t> cls_;
+    static constexpr size_t SUB_MAX = (size_t)16 << 20;
+    static constexpr size_t CHUNK_MIN = (size_t)8 << 20, CHUNK_MAX = (size_t)64 << 20;
+    struct Chunk {
+        char *base = nullptr;
+        size_t size = 0, used = 0;   /* used: bytes cut so far */
+        size_t out = 0;              /* blocks handed out */
+    };
+    struct Block {
+        size_t cls = 0;
+        Chunk *chunk = nullptr;      /* null: an allocation of its own */
+    };
+    std::multimap<size_t, std::pair<void *, Chunk *>> free_;
+    std::unordered_map<void *, Block> cls_;
+    std::list<Chunk> chunks_;
     size_t cached = 0, live = 0;
-    /* while set, released blocks are freed at once instead of cached (the
+    /* while set, released memory is freed at once instead of cached (the
        serving loop gives a closed lane's memory back to the device) */
     bool free_released = false;
+    /* while set, blocks are allocations of their own, which release can give
+       back one by one (a serving lane's) */
+    bool own_blocks = false;
     static size_t size_class(size_t bytes);
     void *alloc(size_t bytes);
     void release(void *p);
     void trim();
     ~Pool();
+
+  private:
+    void *cut(size_t cls, Chunk **from);
+    void free_chunks();
 };
 
 /* Allocations made on this thread while a PoolScope is active come from its
@@ -75,6 +100,16 @@ struct PoolScope {
     Pool *prev;
     explicit PoolScope(Pool *p);
     ~PoolScope();
+};
+
+/* allocations of this thread's pool are of their own while it is active */
+struct OwnBlocks {
+    Pool *pool = current_pool();
+    const bool prev = pool && pool->own_blocks;
+    OwnBlocks() { if (pool) pool->own_blocks = true; }
+    ~OwnBlocks() { if (pool) pool->own_blocks = prev; }
+    OwnBlocks(const OwnBlocks &) = delete;
+    OwnBlocks &operator=(const OwnBlocks &) = delete;
 };
 
 void *dev_alloc(Pool *pool, size_t bytes);

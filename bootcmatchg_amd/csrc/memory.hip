@@ -4,6 +4,8 @@
  */
 #include "bcmg_internal.h"
 
+#include <algorithm>
+
 namespace bcmg {
 
 namespace {
@@ -23,27 +25,71 @@ size_t Pool::size_class(size_t bytes)
     return (bytes + step - 1) & ~(step - 1);
 }
 
+namespace {
+void *device_block(size_t bytes)
+{
+    void *p = nullptr;
+    if (hipMalloc(&p, bytes) == hipSuccess) return p;
+    (void)hipGetLastError();
+    return nullptr;
+}
+} // namespace
+
+/* the next cls bytes of a chunk that has them, or of a new one (null: the
+   device has no room for a chunk) */
+void *Pool::cut(size_t cls, Chunk **from)
+{
+    Chunk *c = nullptr;
+    size_t last = 0;
+    for (Chunk &k : chunks_) {
+        last = std::max(last, k.size);
+        if (!c && k.size - k.used >= cls) c = &k;
+    }
+    if (!c) {
+        const size_t want = std::max(cls, std::min(CHUNK_MAX, std::max(CHUNK_MIN, 2 * last)));
+        char *base = static_cast<char *>(device_block(want));
+        if (!base) return nullptr;
+        try {
+            chunks_.emplace_back();
+        } catch (...) {
+            (void)hipFree(base);
+            throw;
+        }
+        c = &chunks_.back();
+        c->base = base;
+        c->size = want;
+    }
+    void *p = c->base + c->used;
+    c->used += cls;
+    *from = c;
+    return p;
+}
+
 void *Pool::alloc(size_t bytes)
 {
     const size_t cls = size_class(bytes);
     void *p = nullptr;
-    auto it = free_.find(cls);
-    if (it != free_.end()) {
-        p = it->second;
+    Chunk *from = nullptr;
+    auto it = free_.lower_bound(cls);
+    const auto end = free_.upper_bound(cls);
+    while (own_blocks && it != end && it->second.second) ++it;
+    if (it != end) {
+        p = it->second.first;
+        from = it->second.second;
         free_.erase(it);
         cached -= cls;
     } else {
-        if (hipMalloc(&p, cls) != hipSuccess) {
-            (void)hipGetLastError();
-            trim();
-            if (hipMalloc(&p, cls) != hipSuccess) {
-                (void)hipGetLastError();
-                throw Error(BCMG_ENOMEM, "device allocation of " + std::to_string(cls) +
-                                             " bytes failed");
-            }
+        for (int attempt = 0; !p && attempt < 2; attempt++) {
+            if (attempt) trim();
+            if (cls <= SUB_MAX && !own_blocks) p = cut(cls, &from);
+            if (!p) p = device_block(cls);
         }
+        if (!p)
+            throw Error(BCMG_ENOMEM, "device allocation of " + std::to_string(cls) +
+                                         " bytes failed");
     }
-    cls_[p] = cls;
+    cls_[p] = Block{cls, from};
+    if (from) from->out++;
     live += cls;
     return p;
 }
@@ -55,23 +101,53 @@ void Pool::release(void *p)
         (void)hipFree(p);
         return;
     }
-    const size_t cls = it->second;
+    const Block b = it->second;
     cls_.erase(it);
-    live -= cls;
-    if (free_released) {
+    live -= b.cls;
+    if (free_released && !b.chunk) {
         (void)hipFree(p);
         return;
     }
-    free_.emplace(cls, p);
-    cached += cls;
+    free_.emplace(b.cls, std::make_pair(p, b.chunk));
+    cached += b.cls;
+    if (b.chunk && --b.chunk->out == 0 && free_released) free_chunks();
+}
+
+/* give back the chunks none of whose blocks are out (hipFree waits for the
+   work that used them) */
+void Pool::free_chunks()
+{
+    for (auto it = free_.begin(); it != free_.end();) {
+        if (it->second.second && it->second.second->out == 0) {
+            cached -= it->first;
+            it = free_.erase(it);
+        } else {
+            ++it;
+        }
+    }
+    for (auto it = chunks_.begin(); it != chunks_.end();) {
+        if (it->out == 0) {
+            (void)hipFree(it->base);
+            it = chunks_.erase(it);
+        } else {
+            ++it;
+        }
+    }
 }
 
 void Pool::trim()
 {
-    if (!free_.empty()) (void)hipDeviceSynchronize();
-    for (auto &kv : free_) (void)hipFree(kv.second);
-    free_.clear();
-    cached = 0;
+    if (!free_.empty() || !chunks_.empty()) (void)hipDeviceSynchronize();
+    for (auto it = free_.begin(); it != free_.end();) {
+        if (!it->second.second) {
+            (void)hipFree(it->second.first);
+            cached -= it->first;
+            it = free_.erase(it);
+        } else {
+            ++it;
+        }
+    }
+    free_chunks();
 }
 
 Pool::~Pool() { trim(); }

@@ -207,6 +207,7 @@ struct Server {
         BCMG_HIP(hipStreamCreateWithFlags(&L->c.stream, hipStreamNonBlocking));
         L->B = &B;
         const size_t live0 = pool_live();
+        const OwnBlocks own;   /* evict_one gives them back */
         multi_work(L->c, B, L->M, k);
         L->E = std::make_unique<SlotEngine>(L->c, B, *L->M);
         L->slot_req.assign(k, Request());
@@ -316,6 +317,7 @@ struct Server {
             /* reduced-precision buffers are allocated now (see open_lane) */
             BCMG_HIP(hipStreamSynchronize(main.stream));
             const size_t live0 = pool_live();
+            const OwnBlocks own;
             ensure_multi_into(L.c, *L.B, *L.M, L.M->kmax);
             const size_t grown = pool_live() - live0;
             L.bytes += grown;
