@@ -626,6 +626,21 @@ bool launch_jacobi_il_cm(hipStream_t s, const DevCsr &A, MatType mt, const VT *x
 template <typename VT>
 void launch_jacobi_zero_il(hipStream_t s, int n, const VT *f, const VT *d, VT *y, int lkp,
                            int nc, const int *act);
+/* two steps of an interleaved block in one pass, on a constant stencil with
+   offsets -N, -1, 0, 1, N (il_pair_ok): y = a sweep of x's sweep, of f / d (x
+   is not read) or of x + P x_c */
+enum PairFirst { PAIR_SWEEP = 0, PAIR_ZERO = 1, PAIR_PROLONG = 2 };
+template <typename VT>
+struct PairProlong {
+    const int *agg = nullptr;
+    const VT *p = nullptr, *xc = nullptr;
+};
+template <typename VT>
+bool il_pair_ok(const DevCsr &A, MatType mt, int nc);
+template <typename VT>
+void launch_il_pair(hipStream_t s, const DevCsr &A, MatType mt, PairFirst first, const VT *x,
+                    const VT *f, const VT *d, VT *y, const PairProlong<VT> &P, int lkp, int nc,
+                    const int *act);
 template <typename VT>
 void launch_prolong_il(hipStream_t s, int n, const int *agg, const VT *p, const VT *xc, VT *x,
                        int lkp, int nc, const int *act);

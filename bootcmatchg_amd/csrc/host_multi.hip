@@ -217,7 +217,7 @@ bool sweep_cm(MRun<VT> &R, const DevCsr &A, MatType mt, const VT *x, const VT *f
 /* relax_level of host_amg.hip on an interleaved block */
 template <typename VT>
 void relax_level_m(MRun<VT> &R, const Level &lv, MatType mt, int type, int sweeps, const VT *f,
-                   MState<VT> &s, VT *final_out)
+                   MState<VT> &s, VT *final_out, const PairProlong<VT> &pro = PairProlong<VT>())
 {
     Ctx &c = R.c;
     const int lkp = R.lkp;
@@ -235,8 +235,28 @@ void relax_level_m(MRun<VT> &R, const Level &lv, MatType mt, int type, int sweep
         s.zero = false;
         return;
     }
+    const bool pairs = il_pair_ok<VT>(A, mt, R.nc);
+    bool prolong = pro.agg != nullptr;
     for (int k = 0; k < sweeps; k++) {
         VT *out = s.x2;
+        /* two steps in one launch; the sweep that hands its result to FCG
+           stays one of its own */
+        const int steps = prolong ? 1 : 2;
+        if (pairs && (prolong || (k + steps <= sweeps && !(R.zcm && final_out &&
+                                                           k + steps == sweeps)))) {
+            if (final_out && k + steps == sweeps && s.x != final_out) out = final_out;
+            launch_il_pair<VT>(c.stream, A, mt,
+                               prolong  ? PAIR_PROLONG
+                               : s.zero ? PAIR_ZERO
+                                        : PAIR_SWEEP,
+                               s.x, f, d, out, pro, lkp, R.nc, R.act);
+            k += steps - 1;
+            prolong = false;
+            s.x2 = s.x;
+            s.x = out;
+            s.zero = false;
+            continue;
+        }
         const bool last = final_out && k == sweeps - 1;
         if (last && s.x != final_out) out = final_out;
         if (s.zero) {
@@ -347,6 +367,7 @@ void cycle_m(MRun<VT> &R, int l, const VT *fin)
             if (l == L - 1) break;
         }
     }
+    PairProlong<VT> pro;
     if (!sc.zero) {
         if (s.zero) {
             launch_fill_il<VT>(c.stream, A.n, VT(0), s.x, lkp, R.nc, R.act);
@@ -358,13 +379,19 @@ void cycle_m(MRun<VT> &R, int l, const VT *fin)
                                std::is_same<VT, double>::value ? MT_F64 : MT_F32, OP_RESID,
                                sc.x, s.x, nullptr, s.x2, lkp, R.nc, R.act);
             std::swap(s.x, s.x2);
+        } else if (il_pair_ok<VT>(A, mt, R.nc) && !relax_block_ok<VT>(A) &&
+                   B.prm.postrelax_sweeps > (top && R.zcm ? 1 : 0)) {
+            /* folded into the first post-sweep */
+            pro.agg = lv.agg.get();
+            pro.p = pvals<VT>(lv);
+            pro.xc = sc.x;
         } else {
             launch_prolong_il<VT>(c.stream, A.n, lv.agg.get(), pvals<VT>(lv), sc.x, s.x, lkp,
                                   R.nc, R.act);
         }
     }
     relax_level_m<VT>(R, lv, mt, B.prm.relax_type, B.prm.postrelax_sweeps, f, s,
-                      top ? R.final_out : nullptr);
+                      top ? R.final_out : nullptr, pro);
 }
 
 template <typename VT>

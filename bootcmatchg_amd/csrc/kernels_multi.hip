@@ -504,6 +504,147 @@ __global__ __launch_bounds__(BS) void k_jacobi_il_cm_stencil(
     cm_store<VT, ZT, W, TILE, NT>(n, b, gpr, r, jg, any, cw, res, z, ldz);
 }
 
+constexpr int PAIR_BS = 512;
+
+template <typename VT, int W>
+__device__ __forceinline__ vec_t<VT, W> five_sum(unsigned m, const VT *v, vec_t<VT, W> a,
+                                                 vec_t<VT, W> b, vec_t<VT, W> c,
+                                                 vec_t<VT, W> d, vec_t<VT, W> e)
+{
+    vec_t<VT, W> acc = vec_t<VT, W>(0);
+    if (m & 1u) acc = acc + v[0] * a;
+    if (m & 2u) acc = acc + v[1] * b;
+    if (m & 4u) acc = acc + v[2] * c;
+    if (m & 8u) acc = acc + v[3] * d;
+    if (m & 16u) acc = acc + v[4] * e;
+    return acc;
+}
+
+/* Two steps of a five-entry stencil with offsets -N, -1, 0, 1, N in one pass
+   over the block: a first iterate (a sweep of x, f / d, or x + P x_c) and a
+   sweep of it, each element by the operations of its own kernel, so the
+   result equals two launches bit for bit. A workgroup owns tw of N positions
+   along the short offset (a lane W columns of one) and walks H positions
+   along the long one: the first step's neighbours along the walk stay in
+   registers, those beside it pass through LDS, one barrier a position, and
+   the loads of the next position are issued before it. The halo - HX
+   positions each side, one or two at each end - is computed again by its
+   neighbour; a position beside the tile is row i - 1 or i + 1 whatever N is,
+   and masks keep rows outside the operator out of the sums. 32 FP32 columns
+   on 2048^2, us: two sweeps 2 x 286 -> 331 (1.6 GB, 4.9 TB/s), f / d and a
+   sweep 174 + 286 -> 236, a prolongation and a sweep 186 + 286 -> 336; on
+   256 x 2048 two sweeps 2 x 33.6 -> 49. */
+template <typename VT, int W, int FIRST, bool NT>
+__global__ __launch_bounds__(PAIR_BS) void k_il_pair(
+    int n, int N, int tiles, int tw, int H, StencilRef<VT> S, const VT *__restrict__ x,
+    const VT *__restrict__ f, const VT *__restrict__ d, VT *__restrict__ y, PairProlong<VT> P,
+    int lkp, int nc, const int *__restrict__ act)
+{
+    using V = vec_t<VT, W>;
+    constexpr int HX = FIRST == PAIR_SWEEP ? 2 : 1;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_pair[];
+    const unsigned cw = col_word(nc, act);
+    const int gpr = (nc + W - 1) / W;
+    const int cells = (tw + 2 * HX) * gpr;
+    V *const ss = reinterpret_cast<V *>(smem_pair);      /* 2 positions of the first iterate */
+    V *const xs = ss + 2 * cells;                        /* and of x */
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int strip = b / tiles, tile = b - strip * tiles;
+    const int tid = threadIdx.x;
+    const int xl = tid / gpr, jg = tid - xl * gpr;
+    bool any, all;
+    group_on(jg, W, cw, any, all);
+    const bool work = tid < cells && any;
+    const int gx = tile * tw - HX + xl;
+    const int y0 = strip * H;
+    const int y1 = min(y0 + H, (n + N - 1) / N);
+    const bool outx = work && xl >= HX && xl < HX + tw && gx < N;
+    const int left = max(tid - gpr, 0), right = min(tid + gpr, cells - 1);
+    auto row = [&](int q) {
+        const long long i = (long long)q * N + gx;
+        return (int)(i < 0 ? 0 : i < n ? i : n - 1);
+    };
+    auto at = [&](int r) { return ((size_t)r << lkp) + jg * W; };
+    auto vec = [&](const VT *a, int r) { return *reinterpret_cast<const V *>(a + at(r)); };
+    V xm = V(0), x0 = V(0), xp = V(0), fq = V(0), cq = V(0);
+    VT dq = VT(1), pq = VT(0);
+    unsigned mq = 0;
+    int an = 0;
+    if (work) {
+        const int r = row(y0 - 1);
+        fq = vec(f, r);
+        dq = d[r];
+        mq = S.mask[r];
+        if (FIRST != PAIR_ZERO) x0 = vec(x, r);
+        if (FIRST == PAIR_SWEEP) {
+            xm = vec(x, row(y0 - 2));
+            xp = vec(x, row(y0));
+        }
+        if (FIRST == PAIR_PROLONG) {
+            pq = P.p[r];
+            cq = vec(P.xc, P.agg[r]);
+            an = P.agg[row(y0)];
+        }
+    }
+    V sm = V(0), s0 = V(0), fp = V(0);
+    VT dp = VT(1);
+    unsigned mp = 0;
+    for (int q = y0 - 1; q <= y1; q++) {
+        V xn = V(0), fn = V(0), cn = V(0);
+        VT dn = VT(1), pn = VT(0);
+        unsigned mn = 0;
+        if (work && q < y1) {
+            const int r = row(q + 1);
+            if (FIRST == PAIR_SWEEP) xn = vec(x, row(q + 2));
+            fn = ldm<NT>(reinterpret_cast<const V *>(f + at(r)));
+            dn = d[r];
+            mn = S.mask[r];
+            if (FIRST == PAIR_PROLONG) {
+                xn = vec(x, r);
+                pn = P.p[r];
+                cn = vec(P.xc, an);
+                an = P.agg[row(q + 2)];
+            }
+        }
+        const int cur = (q & 1) * cells, prev = cells - cur;
+        if (FIRST == PAIR_SWEEP && work) xs[cur + tid] = x0;
+        __syncthreads();
+        if (work) {
+            V s;
+            if (FIRST == PAIR_ZERO) {
+                s = fq / dq;
+            } else if (FIRST == PAIR_PROLONG) {
+                for (int u = 0; u < W; u++) s[u] = fma(pq, cq[u], x0[u]);
+            } else {
+                const V t = five_sum<VT, W>(mq, S.v, xm, xs[cur + left], x0, xs[cur + right], xp);
+                s = (fq - t) / dq + x0;
+            }
+            if (q > y0 && outx && (long long)(q - 1) * N + gx < n) {
+                const V t = five_sum<VT, W>(mp, S.v, sm, ss[prev + left], s0, ss[prev + right], s);
+                il_store<VT, W, NT>((fp - t) / dp + s0, y + at(row(q - 1)), all, cw, jg);
+            }
+            ss[cur + tid] = s;
+            sm = s0;
+            s0 = s;
+        }
+        fp = fq;
+        dp = dq;
+        mp = mq;
+        fq = fn;
+        dq = dn;
+        mq = mn;
+        if (FIRST == PAIR_SWEEP) {
+            xm = x0;
+            x0 = xp;
+            xp = xn;
+        } else {
+            x0 = xn;
+            pq = pn;
+            cq = cn;
+        }
+    }
+}
+
 /* group-order row sums (k_rows<G>'s arithmetic) on interleaved blocks: G
    lanes per row, one column at a time */
 template <typename MT, typename VT, int OP>
@@ -1493,6 +1634,64 @@ void launch_rows_il(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const 
     BCMG_CHECK_LAUNCH();
 }
 
+/* Below PAIR_MIN_N positions along the short offset the walk waits more than
+   it moves (65 536 rows, N = 32: 15.7 us against 2 x 6.9). PAIR_WGS: three
+   workgroups of 8 wavefronts fit a CU (76 VGPRs), so just under 768 make one
+   round; PAIR_H positions at most, as strips of 64 end in a half-empty round
+   (2048^2: 367 us; 32: 331; 16: 334; one round of 98: 343). */
+constexpr int PAIR_MIN_N = 128;
+constexpr int PAIR_WGS = 740;
+constexpr int PAIR_H = 32;
+
+template <typename VT>
+bool il_pair_ok(const DevCsr &A, MatType mt, int nc)
+{
+    const RowClasses &C = A.cls;
+    if (nc < (int)(16 / sizeof(VT)) || !class_ok<VT>(A, mt) || C.k != 5) return false;
+    const int N = C.off[4];
+    return N >= PAIR_MIN_N && C.off[0] == -N && C.off[1] == -1 && C.off[2] == 0 && C.off[3] == 1;
+}
+
+template <typename VT, int FIRST>
+void il_pair(hipStream_t s, const DevCsr &A, MatType mt, const VT *x, const VT *f, const VT *d,
+             VT *y, const PairProlong<VT> &P, int lkp, int nc, const int *act)
+{
+    constexpr int W = 16 / sizeof(VT), HX = FIRST == PAIR_SWEEP ? 2 : 1;
+    const int n = A.n, N = A.cls.off[4], gpr = (nc + W - 1) / W;
+    const int most = PAIR_BS / gpr - 2 * HX;
+    const int tiles = (N + most - 1) / most, tw = (N + tiles - 1) / tiles;
+    const int ny = (n + N - 1) / N;
+    const int H = (int)std::min<long long>(
+        PAIR_H, std::max<long long>(8, ((long long)ny * tiles + PAIR_WGS - 1) / PAIR_WGS));
+    const int cells = (tw + 2 * HX) * gpr, bs = (cells + 63) / 64 * 64;
+    const size_t lds = (size_t)(FIRST == PAIR_SWEEP ? 4 : 2) * cells * 16;
+    const unsigned g = (unsigned)((long long)tiles * ((ny + H - 1) / H));
+    const StencilRef<VT> S = stencil_ref<VT>(A, mt);
+    if (((size_t)n << lkp) * sizeof(VT) > NT_BYTES)
+        k_il_pair<VT, W, FIRST, true><<<g, bs, lds, s>>>(n, N, tiles, tw, H, S, x, f, d, y, P, lkp,
+                                                         nc, act);
+    else
+        k_il_pair<VT, W, FIRST, false><<<g, bs, lds, s>>>(n, N, tiles, tw, H, S, x, f, d, y, P,
+                                                          lkp, nc, act);
+}
+
+template <typename VT>
+void launch_il_pair(hipStream_t s, const DevCsr &A, MatType mt, PairFirst first, const VT *x,
+                    const VT *f, const VT *d, VT *y, const PairProlong<VT> &P, int lkp, int nc,
+                    const int *act)
+{
+    if (nc > MULTI_MAX_COLS || nc > (1 << lkp))
+        throw Error(BCMG_EINVAL, "interleaved block narrower than its columns");
+    if (x == y) throw Error(BCMG_EINVAL, "two steps into their own input");
+    if (first == PAIR_SWEEP)
+        il_pair<VT, PAIR_SWEEP>(s, A, mt, x, f, d, y, P, lkp, nc, act);
+    else if (first == PAIR_ZERO)
+        il_pair<VT, PAIR_ZERO>(s, A, mt, x, f, d, y, P, lkp, nc, act);
+    else
+        il_pair<VT, PAIR_PROLONG>(s, A, mt, x, f, d, y, P, lkp, nc, act);
+    BCMG_CHECK_LAUNCH();
+}
+
 template <typename VT, typename ZT>
 bool launch_jacobi_il_cm(hipStream_t s, const DevCsr &A, MatType mt, const VT *x, const VT *f,
                          const VT *d, ZT *z, long ldz, int lkp, int nc, const int *act)
@@ -1617,6 +1816,10 @@ void launch_from_il(hipStream_t s, int n, const S *a, D *b, long ldb, int lkp, i
                                      const VT *, const VT *, VT *, int, int, const int *);    \
     template void launch_jacobi_zero_il<VT>(hipStream_t, int, const VT *, const VT *, VT *,  \
                                             int, int, const int *);                          \
+    template bool il_pair_ok<VT>(const DevCsr &, MatType, int);                              \
+    template void launch_il_pair<VT>(hipStream_t, const DevCsr &, MatType, PairFirst,        \
+                                     const VT *, const VT *, const VT *, VT *,               \
+                                     const PairProlong<VT> &, int, int, const int *);        \
     template void launch_prolong_il<VT>(hipStream_t, int, const int *, const VT *, const VT *, \
                                         VT *, int, int, const int *);                        \
     template void launch_fill_il<VT>(hipStream_t, int, VT, VT *, int, int, const int *);     \
