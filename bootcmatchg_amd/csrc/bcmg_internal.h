@@ -626,6 +626,10 @@ bool launch_jacobi_il_cm(hipStream_t s, const DevCsr &A, MatType mt, const VT *x
 template <typename VT>
 void launch_jacobi_zero_il(hipStream_t s, int n, const VT *f, const VT *d, VT *y, int lkp,
                            int nc, const int *act);
+/* y = R (f - A x) on interleaved blocks in one launch; false: not launched */
+template <typename VT>
+bool launch_il_resid_restrict(hipStream_t s, const DevCsr &A, MatType mt, const DevCsr &R,
+                              const VT *x, const VT *f, VT *y, int lkp, int nc, const int *act);
 /* two steps of an interleaved block in one pass, on a constant stencil with
    offsets -N, -1, 0, 1, N (il_pair_ok): y = a sweep of x's sweep, of f / d (x
    is not read) or of x + P x_c */

@@ -350,13 +350,16 @@ void cycle_m(MRun<VT> &R, int l, const VT *fin)
     relax_level_m<VT>(R, lv, mt, B.prm.relax_type, B.prm.prerelax_sweeps, f, s, nullptr);
     const DevCsr &A = lv.mat();
     const VT *rsrc = f;
-    if (!s.zero) {
-        launch_rows_il<VT>(c.stream, A, mt, OP_RESID, s.x, f, nullptr, W.res.get(), lkp, R.nc,
-                           R.act);
-        rsrc = W.res.get();
+    if (s.zero || !launch_il_resid_restrict<VT>(c.stream, A, mt, lv.R, s.x, f, W.f[l].get(), lkp,
+                                                R.nc, R.act)) {
+        if (!s.zero) {
+            launch_rows_il<VT>(c.stream, A, mt, OP_RESID, s.x, f, nullptr, W.res.get(), lkp, R.nc,
+                               R.act);
+            rsrc = W.res.get();
+        }
+        launch_rows_il<VT>(c.stream, lv.R, std::is_same<VT, double>::value ? MT_F64 : MT_F32,
+                           OP_SPMV, rsrc, nullptr, nullptr, W.f[l].get(), lkp, R.nc, R.act);
     }
-    launch_rows_il<VT>(c.stream, lv.R, std::is_same<VT, double>::value ? MT_F64 : MT_F32,
-                       OP_SPMV, rsrc, nullptr, nullptr, W.f[l].get(), lkp, R.nc, R.act);
     MState<VT> &sc = R.st[l];
     sc.zero = true;
     if (B.prm.cycle_type == 3 && l != L - 1) {
