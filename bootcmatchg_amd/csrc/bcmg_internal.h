@@ -794,7 +794,7 @@ void launch_norm2_multi(Ctx &c, int n, MultiFcg &M, const int *mask, double *par
 void launch_spmv_dots_multi(Ctx &c, const DevCsr &A, int k, MultiFcg &M, const int *mask,
                             double *part);
 /* iteration update of the active columns, then their stopping test */
-void launch_fcg_update_multi(Ctx &c, int n, MultiFcg &M, double *part);
+void launch_fcg_update_multi(Ctx &c, const DevCsr &A, MultiFcg &M, double *part);
 /* first step of the masked columns (direction Z moves to pair 0) */
 void launch_fcg_first_multi(Ctx &c, int n, MultiFcg &M, const int *mask, double *part);
 /* R = B - A X and scal[8 j + 6] = ||R_j|| for masked columns (Y scratch) */

@@ -528,7 +528,7 @@ void enqueue_iteration_m(Ctx &c, Boot &B, MultiWork &M)
     const DevCsr &A = *B.A0;
     precond_block(c, B, M, M.F.act);
     launch_spmv_dots_multi(c, A, 3, M.F, M.F.act, M.part.get());
-    launch_fcg_update_multi(c, A.n, M.F, M.part.get());
+    launch_fcg_update_multi(c, A, M.F, M.part.get());
     BCMG_HIP(hipMemcpyAsync(M.h_flags, M.flags.get(), 3 * (size_t)M.kmax * sizeof(int),
                             hipMemcpyDeviceToHost, c.stream));
 }

@@ -1100,8 +1100,8 @@ __global__ void k_fcg_scalars_multi(double *scal, int nc, int first, const int *
    NT: r, the previous direction and t, touched once per launch, are read
    and written non-temporally (the columns' streams exceed the last-level
    cache). 2048^2 x 32: 1.17 ms with z in FP64 and __shfl_down sums, 1.00 with
-   an FP32 cycle's z read as it is, 0.88 with the sums in registers
-   (4.0 GB at 4.5 TB/s). */
+   an FP32 cycle's z read as it is, 0.88 with the sums in registers, 0.75
+   where a constant stencil leaves t to the update (2.7 GB). */
 constexpr int SD_PF = 8; /* entries whose indices are loaded at once */
 template <int K, bool NT, typename ZT, int KS = 0>
 __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__restrict__ rp,
@@ -1197,8 +1197,9 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_multi(int n, const int *__rest
         const int p = F.par[j];
         const double zr = (double)Z[o];
         const double rr = ldm<NT>(F.R + o);
-        double *tv = slot(F.W0, F.W1, K == 2 ? 0 : (p ^ 1), j, ld);
-        st_nt<NT>(tv + r, t[u]);
+        /* with a constant stencil the update forms t again from z */
+        if (K == 2 || KS == 0)
+            st_nt<NT>(slot(F.W0, F.W1, K == 2 ? 0 : (p ^ 1), j, ld) + r, t[u]);
         sd[u * K] = rr * zr;
         sd[u * K + 1] = t[u] * zr;
         if constexpr (K > 2) sd[u * K + K - 1] = ldm<NT>(slot(F.W0, F.W1, p, j, ld) + r) * zr;
@@ -1253,9 +1254,13 @@ __global__ __launch_bounds__(RED_FINAL_BS) void k_fcg_final_multi(int nb,
 /* FCG update (the arithmetic of k_fcg_update): z = -theta zo + Z into the
    new pair, x += theta2 z; t = -theta to + t; r += -theta2 t; ||r||^2.
    NT: the columns' ten streams exceed the last-level cache, so they are read
-   and written non-temporally. */
-template <bool NT, typename ZT>
-__global__ __launch_bounds__(BS) void k_fcg_update_multi(int n, FcgCols F,
+   and written non-temporally. KS > 0: t = A z is formed here from the
+   stencil's KS entries (k_spmv_dots_multi's operations), which saves storing
+   it there and reading it back: 2048^2 x 32, 1767 -> 1607 us (5.7 TB/s) and
+   the product launch 875 -> 749. (A single column gains nothing: its z is
+   fetched by several XCDs.) */
+template <bool NT, typename ZT, int KS = 0>
+__global__ __launch_bounds__(BS) void k_fcg_update_multi(int n, FcgCols F, StencilRef<double> S,
                                                          double *__restrict__ part)
 {
     const int j = blockIdx.y;
@@ -1273,9 +1278,22 @@ __global__ __launch_bounds__(BS) void k_fcg_update_multi(int n, FcgCols F,
     double *r = F.R + (size_t)j * ld;
     double s[1] = {0.0};
     for (int i = blockIdx.x * BS + threadIdx.x; i < n; i += gridDim.x * BS) {
-        const double zi = fma(-theta, ldm<NT>(zo + i), (double)ldm<NT>(zc + i));
+        double tz = 0.0;
+        if constexpr (KS > 0) {
+            const unsigned m = S.mask[i];
+            ZT g[KS];
+#pragma unroll
+            for (int k = 0; k < KS; k++) g[k] = zc[((m >> k) & 1u) ? i + S.off[k] : i];
+#pragma unroll
+            for (int k = 0; k < KS; k++)
+                if ((m >> k) & 1u) tz = tz + S.v[k] * (double)g[k];
+        } else {
+            tz = ldm<NT>(t + i);
+        }
+        const double zi = fma(-theta, ldm<NT>(zo + i),
+                              (double)(KS > 0 ? zc[i] : ldm<NT>(zc + i)));
         const double xi = fma(theta2, zi, ldm<NT>(x + i));
-        const double ti = fma(-theta, ldm<NT>(to + i), ldm<NT>(t + i));
+        const double ti = fma(-theta, ldm<NT>(to + i), tz);
         const double ri = fma(-theta2, ti, ldm<NT>(r + i));
         if (NT) {
             __builtin_nontemporal_store(zi, zn + i);
@@ -2073,16 +2091,32 @@ void launch_spmv_dots_multi(Ctx &c, const DevCsr &A, int k, MultiFcg &M, const i
     BCMG_CHECK_LAUNCH();
 }
 
-void launch_fcg_update_multi(Ctx &c, int n, MultiFcg &M, double *part)
+void launch_fcg_update_multi(Ctx &c, const DevCsr &A, MultiFcg &M, double *part)
 {
+    const int n = A.n;
     const int nb = red_blocks(n);
     const FcgCols F = fcg_cols(M);
     const bool nt = (size_t)n * M.nc * 10 * sizeof(double) > NT_BYTES;
-    auto go = [&](auto kern) { kern<<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, part); };
+    /* as launch_spmv_dots_multi decided */
+    const bool st = stream_ok<double>(A) && class_ok<double>(A, MT_F64) && A.cls.k > 0;
+    const StencilRef<double> S = st ? stencil_ref<double>(A, MT_F64) : StencilRef<double>{};
+    auto go = [&](auto kern) { kern<<<dim3(nb, M.nc), BS, 0, c.stream>>>(n, F, S, part); };
+    auto pick = [&](auto NT, auto zt) {
+        constexpr bool nn = decltype(NT)::value;
+        using ZT = decltype(zt);
+        if (!st)
+            go(k_fcg_update_multi<nn, ZT>);
+        else if (A.cls.k <= 5)
+            go(k_fcg_update_multi<nn, ZT, 5>);
+        else if (A.cls.k <= 7)
+            go(k_fcg_update_multi<nn, ZT, 7>);
+        else
+            go(k_fcg_update_multi<nn, ZT, CLS_ROW>);
+    };
     if (M.z32)
-        nt ? go(k_fcg_update_multi<true, float>) : go(k_fcg_update_multi<false, float>);
+        nt ? pick(std::true_type{}, float()) : pick(std::false_type{}, float());
     else
-        nt ? go(k_fcg_update_multi<true, double>) : go(k_fcg_update_multi<false, double>);
+        nt ? pick(std::true_type{}, double()) : pick(std::false_type{}, double());
     k_fcg_final_multi<1, true><<<M.nc, RED_FINAL_BS, 0, c.stream>>>(nb, part, F, M.act);
     BCMG_CHECK_LAUNCH();
 }
