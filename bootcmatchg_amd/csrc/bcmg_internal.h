@@ -639,6 +639,15 @@ struct PairProlong {
     const int *agg = nullptr;
     const VT *p = nullptr, *xc = nullptr;
 };
+/* several sweeps of a small level in one launch, after x, f / d (which the
+   caller counts as a sweep) or x + P x_c; il_slab_sweeps: how many at a time
+   of `sweeps` pay (0: none) */
+template <typename VT>
+int il_slab_sweeps(const DevCsr &A, MatType mt, int nc, int sweeps);
+template <typename VT>
+void launch_il_slab(hipStream_t s, const DevCsr &A, MatType mt, PairFirst first, int sweeps,
+                    const VT *x, const VT *f, const VT *d, VT *y, const PairProlong<VT> &P,
+                    int lkp, int nc, const int *act);
 template <typename VT>
 bool il_pair_ok(const DevCsr &A, MatType mt, int nc);
 template <typename VT>

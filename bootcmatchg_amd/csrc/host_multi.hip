@@ -214,6 +214,15 @@ bool sweep_cm(MRun<VT> &R, const DevCsr &A, MatType mt, const VT *x, const VT *f
                                            R.act);
 }
 
+/* the prolongation goes into the first launch of the post-smoothing */
+template <typename VT>
+bool fold_prolong_m(const MRun<VT> &R, const DevCsr &A, MatType mt, int sweeps, bool handed)
+{
+    const int own = sweeps - (handed ? 1 : 0);
+    if (own >= 2 && il_slab_sweeps<VT>(A, mt, R.nc, sweeps) > 0) return true;
+    return own >= 1 && il_pair_ok<VT>(A, mt, R.nc) && !relax_block_ok<VT>(A);
+}
+
 /* relax_level of host_amg.hip on an interleaved block */
 template <typename VT>
 void relax_level_m(MRun<VT> &R, const Level &lv, MatType mt, int type, int sweeps, const VT *f,
@@ -224,7 +233,9 @@ void relax_level_m(MRun<VT> &R, const Level &lv, MatType mt, int type, int sweep
     const DevCsr &A = lv.mat();
     const VT *d = divisor<VT>(lv, type);
     if (sweeps == 0) return;
-    if (relax_block_ok<VT>(A)) {
+    /* stencil sweeps in the level (the sweep from zero is pointwise) */
+    const int slab = il_slab_sweeps<VT>(A, mt, R.nc, sweeps - (s.zero ? 1 : 0));
+    if (slab == 0 && relax_block_ok<VT>(A)) {
         VT *out = (final_out && s.x != final_out) ? final_out : s.x;
         launch_relax_block<VT>(c.stream, A, mt, d, f, s.x, out, sweeps, s.zero, R.nc, 1,
                                1 << lkp, R.act);
@@ -241,6 +252,23 @@ void relax_level_m(MRun<VT> &R, const Level &lv, MatType mt, int type, int sweep
         VT *out = s.x2;
         /* two steps in one launch; the sweep that hands its result to FCG
            stays one of its own */
+        const int left = sweeps - k - (s.zero ? 1 : 0);
+        const int handed = R.zcm && final_out ? 1 : 0;
+        if (slab > 0 && left - handed >= 2) {
+            const int take = std::min(slab, left - handed);
+            k += take + (s.zero ? 1 : 0) - 1;
+            if (final_out && k == sweeps - 1 && s.x != final_out) out = final_out;
+            launch_il_slab<VT>(c.stream, A, mt,
+                               prolong  ? PAIR_PROLONG
+                               : s.zero ? PAIR_ZERO
+                                        : PAIR_SWEEP,
+                               take, s.x, f, d, out, pro, lkp, R.nc, R.act);
+            prolong = false;
+            s.x2 = s.x;
+            s.x = out;
+            s.zero = false;
+            continue;
+        }
         const int steps = prolong ? 1 : 2;
         if (pairs && (prolong || (k + steps <= sweeps && !(R.zcm && final_out &&
                                                            k + steps == sweeps)))) {
@@ -382,8 +410,7 @@ void cycle_m(MRun<VT> &R, int l, const VT *fin)
                                std::is_same<VT, double>::value ? MT_F64 : MT_F32, OP_RESID,
                                sc.x, s.x, nullptr, s.x2, lkp, R.nc, R.act);
             std::swap(s.x, s.x2);
-        } else if (il_pair_ok<VT>(A, mt, R.nc) && !relax_block_ok<VT>(A) &&
-                   B.prm.postrelax_sweeps > (top && R.zcm ? 1 : 0)) {
+        } else if (fold_prolong_m<VT>(R, A, mt, B.prm.postrelax_sweeps, top && R.zcm)) {
             /* folded into the first post-sweep */
             pro.agg = lv.agg.get();
             pro.p = pvals<VT>(lv);

@@ -427,6 +427,108 @@ __global__ __launch_bounds__(BS) void k_rows_il_stencil(int n, StencilRef<VT> S,
 
 constexpr int ILR_AHEAD = 2;
 
+constexpr int SLAB_BS = 1024;
+
+/* Several steps of a small narrow-band level in one launch: a workgroup keeps
+   its L rows and a halo of `halo` each side (the band per sweep, computed
+   again by the neighbours) in LDS, both iterates, and a barrier separates the
+   sweeps; f, the divisor and the mask of a lane's RPT cells stay in registers.
+   FIRST as in k_il_pair; each element by the operations of its own kernel, so
+   the bits are those of separate launches. What the halo's ends gather from
+   beyond the tile is wrong and moves inwards by a band a sweep: it stops
+   short of the L rows that are stored. 32 FP32 columns, us: 8192 rows, band 8,
+   four sweeps 17.2 -> 7.0, with the prolongation 22.0 -> 6.7; 65 536 rows,
+   band 32, four sweeps 26.4 -> 20.4; the 4096-row coarsest level 37.2 (a
+   workgroup a column) -> 25.9. */
+template <typename VT, int W, int K, int RPT, int FIRST>
+__global__ __launch_bounds__(SLAB_BS) void k_il_slab(
+    int n, int L, int halo, int sweeps, StencilRef<VT> S, const VT *__restrict__ x,
+    const VT *__restrict__ f, const VT *__restrict__ d, VT *__restrict__ y, PairProlong<VT> P,
+    int lkp, int nc, const int *__restrict__ act)
+{
+    using V = vec_t<VT, W>;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem_slab[];
+    const unsigned cw = col_word(nc, act);
+    const int gpr = (nc + W - 1) / W;
+    const int cells = (L + 2 * halo) * gpr;
+    V *cur = reinterpret_cast<V *>(smem_slab), *nxt = cur + cells;
+    const int r0 = blockIdx.x * L;
+    V fv[RPT];
+    VT dv[RPT];
+    unsigned m[RPT];
+    bool work[RPT];
+    auto cell = [&](int u, int &r, int &jg) {
+        const int c = threadIdx.x + u * SLAB_BS;
+        const int lr = c / gpr;
+        jg = c - lr * gpr;
+        r = r0 - halo + lr;
+        return c;
+    };
+#pragma unroll
+    for (int u = 0; u < RPT; u++) {
+        int r, jg;
+        const int c = cell(u, r, jg);
+        bool any, all;
+        group_on(jg, W, cw, any, all);
+        work[u] = c < cells && r >= 0 && r < n && any;
+        m[u] = 0;
+        dv[u] = VT(1);
+        fv[u] = V(0);
+        V v = V(0);
+        if (work[u]) {
+            const size_t o = ((size_t)r << lkp) + jg * W;
+            fv[u] = *reinterpret_cast<const V *>(f + o);
+            dv[u] = d[r];
+            m[u] = S.mask[r];
+            if (FIRST == PAIR_ZERO) {
+                v = fv[u] / dv[u];
+            } else {
+                v = *reinterpret_cast<const V *>(x + o);
+                if (FIRST == PAIR_PROLONG) {
+                    const VT p = P.p[r];
+                    const V xc = *reinterpret_cast<const V *>(
+                        P.xc + ((size_t)P.agg[r] << lkp) + jg * W);
+                    for (int w = 0; w < W; w++) v[w] = fma(p, xc[w], v[w]);
+                }
+            }
+        }
+        if (c < cells) cur[c] = v;
+    }
+    __syncthreads();
+    for (int s = 0; s < sweeps; s++) {
+#pragma unroll
+        for (int u = 0; u < RPT; u++) {
+            const int c = threadIdx.x + u * SLAB_BS;
+            if (!work[u]) continue;
+            V g[K];
+#pragma unroll
+            for (int k = 0; k < K; k++) {
+                const int q = ((m[u] >> k) & 1u) ? c + S.off[k] * gpr : c;
+                g[k] = cur[min(max(q, 0), cells - 1)];
+            }
+            const V own = cur[c];
+            V acc = V(0);
+#pragma unroll
+            for (int k = 0; k < K; k++)
+                if ((m[u] >> k) & 1u) acc = acc + S.v[k] * g[k];
+            nxt[c] = (fv[u] - acc) / dv[u] + own;
+        }
+        __syncthreads();
+        V *const t = cur;
+        cur = nxt;
+        nxt = t;
+    }
+#pragma unroll
+    for (int u = 0; u < RPT; u++) {
+        int r, jg;
+        const int c = cell(u, r, jg);
+        if (!work[u] || r < r0 || r >= r0 + L) continue;
+        bool any, all;
+        group_on(jg, W, cw, any, all);
+        il_store<VT, W, false>(cur[c], y + ((size_t)r << lkp) + jg * W, all, cw, jg);
+    }
+}
+
 /* y = R (f - A x) for a constant stencil A: a lane takes W columns of a row of
    R and forms the residuals it adds where it adds them, ILR_AHEAD at a time,
    each by k_rows_il_stencil's operations and the sum by k_rows_il's, so the
@@ -1696,6 +1798,107 @@ void launch_rows_il(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const 
     BCMG_CHECK_LAUNCH();
 }
 
+/* The slab of `sweeps` sweeps: the rows a workgroup stores and its cells per
+   lane (0: does not fit). */
+struct IlSlab {
+    int L = 0, rpt = 0;
+    double us = 0;
+};
+
+/* Predicted time: a launch, the loads and the store cost about 4.5 us, a sweep
+   of the cells 0.45 us per cell of a lane and round of workgroups (one a CU);
+   a sweep of its own 3 us and its bytes at 8 TB/s. */
+IlSlab il_slab_fit(int n, int band, int gpr, int sweeps)
+{
+    IlSlab best;
+    const int halo = band * sweeps;
+    for (int L = 16; L <= 512; L *= 2) {
+        const long long cells = (long long)(L + 2 * halo) * gpr;
+        const int rpt = (int)((cells + SLAB_BS - 1) / SLAB_BS);
+        if (rpt > 4) break;
+        const int rounds = (n + 256 * L - 1) / (256 * L);
+        const double us = 2.5 + rounds * (2.0 + sweeps * 0.45 * rpt);
+        if (best.rpt == 0 || us < best.us) best = IlSlab{L, rpt, us};
+    }
+    return best;
+}
+
+template <typename VT>
+int il_slab_sweeps(const DevCsr &A, MatType mt, int nc, int sweeps)
+{
+    constexpr int W = 16 / sizeof(VT);
+    if (nc < W || sweeps < 2 || !class_ok<VT>(A, mt) || A.cls.k <= 0) return 0;
+    const int band = std::max(-A.cls.off[0], A.cls.off[A.cls.k - 1]);
+    const int gpr = (nc + W - 1) / W;
+    /* the alternatives: a launch a sweep, half of one where sweeps pair, or
+       all of them in a workgroup a column */
+    const double one = (3.0 + (double)A.n * nc * (3 * sizeof(VT)) / 8e6) *
+                       (il_pair_ok<VT>(A, mt, nc) ? 0.6 : 1.0);
+    double best = relax_block_ok<VT>(A) ? 2.5 + sweeps * (0.1 + 0.45 * ((A.n + 1023) / 1024))
+                                        : sweeps * one;
+    int take = 0;
+    for (int s = 2; s <= sweeps; s++) {
+        const IlSlab p = il_slab_fit(A.n, band, gpr, s);
+        if (p.rpt == 0) break;
+        const int rest = sweeps % s;
+        const double us = (sweeps / s) * p.us + (rest ? std::min(p.us, rest * one) : 0.0);
+        if (us < best) {
+            best = us;
+            take = s;
+        }
+    }
+    return take;
+}
+
+template <typename VT, int K, int RPT>
+void il_slab_first(hipStream_t s, const DevCsr &A, MatType mt, PairFirst first, int L, int sweeps,
+                   int band, const VT *x, const VT *f, const VT *d, VT *y,
+                   const PairProlong<VT> &P, int lkp, int nc, const int *act)
+{
+    constexpr int W = 16 / sizeof(VT);
+    const int gpr = (nc + W - 1) / W;
+    const size_t lds = (size_t)2 * (L + 2 * band * sweeps) * gpr * 16;
+    const int g = (A.n + L - 1) / L;
+    const StencilRef<VT> S = stencil_ref<VT>(A, mt);
+    auto go = [&](auto kern) {
+        kern<<<g, SLAB_BS, lds, s>>>(A.n, L, band * sweeps, sweeps, S, x, f, d, y, P, lkp, nc, act);
+    };
+    if (first == PAIR_SWEEP)
+        go(k_il_slab<VT, W, K, RPT, PAIR_SWEEP>);
+    else if (first == PAIR_ZERO)
+        go(k_il_slab<VT, W, K, RPT, PAIR_ZERO>);
+    else
+        go(k_il_slab<VT, W, K, RPT, PAIR_PROLONG>);
+}
+
+template <typename VT>
+void launch_il_slab(hipStream_t s, const DevCsr &A, MatType mt, PairFirst first, int sweeps,
+                    const VT *x, const VT *f, const VT *d, VT *y, const PairProlong<VT> &P,
+                    int lkp, int nc, const int *act)
+{
+    constexpr int W = 16 / sizeof(VT);
+    if (nc > MULTI_MAX_COLS || nc > (1 << lkp))
+        throw Error(BCMG_EINVAL, "interleaved block narrower than its columns");
+    if (x == y) throw Error(BCMG_EINVAL, "several sweeps into their own input");
+    const int band = std::max(-A.cls.off[0], A.cls.off[A.cls.k - 1]);
+    const IlSlab p = il_slab_fit(A.n, band, (nc + W - 1) / W, sweeps);
+    if (p.rpt == 0) throw Error(BCMG_EINVAL, "several sweeps: the level's band is too wide");
+    auto pick = [&](auto k) {
+        constexpr int K = decltype(k)::value;
+        if (p.rpt == 1)
+            il_slab_first<VT, K, 1>(s, A, mt, first, p.L, sweeps, band, x, f, d, y, P, lkp, nc, act);
+        else if (p.rpt == 2)
+            il_slab_first<VT, K, 2>(s, A, mt, first, p.L, sweeps, band, x, f, d, y, P, lkp, nc, act);
+        else
+            il_slab_first<VT, K, 4>(s, A, mt, first, p.L, sweeps, band, x, f, d, y, P, lkp, nc, act);
+    };
+    if (A.cls.k <= 5)
+        pick(std::integral_constant<int, 5>{});
+    else
+        pick(std::integral_constant<int, CLS_ROW>{});
+    BCMG_CHECK_LAUNCH();
+}
+
 template <typename VT>
 bool launch_il_resid_restrict(hipStream_t s, const DevCsr &A, MatType mt, const DevCsr &R,
                               const VT *x, const VT *f, VT *y, int lkp, int nc, const int *act)
@@ -1909,6 +2112,10 @@ void launch_from_il(hipStream_t s, int n, const S *a, D *b, long ldb, int lkp, i
                                      const VT *, const VT *, VT *, int, int, const int *);    \
     template void launch_jacobi_zero_il<VT>(hipStream_t, int, const VT *, const VT *, VT *,  \
                                             int, int, const int *);                          \
+    template int il_slab_sweeps<VT>(const DevCsr &, MatType, int, int);                      \
+    template void launch_il_slab<VT>(hipStream_t, const DevCsr &, MatType, PairFirst, int,   \
+                                     const VT *, const VT *, const VT *, VT *,               \
+                                     const PairProlong<VT> &, int, int, const int *);        \
     template bool launch_il_resid_restrict<VT>(hipStream_t, const DevCsr &, MatType,         \
                                                const DevCsr &, const VT *, const VT *, VT *, \
                                                int, int, const int *);                       \

@@ -1,4 +1,5 @@
-"""Two steps of a five-point stencil in one pass over an interleaved block:
+"""Two steps of a five-point stencil in one pass over an interleaved block, and
+several sweeps of a small narrow-band one in one launch:
 solves of several columns equal single solves bit for bit, at the edges of the
 tiles, strips and column groups, for sweep counts that pair and that do not.
 """
@@ -28,6 +29,9 @@ def ctx():
     (lambda: ops.poisson2d(257), 32),         # several tiles and strips, ragged
     (lambda: ops.aniso2d(512, 0.01), 31),     # coarse levels of five entries too
     (lambda: neumann2d(150), 12),             # an L1 divisor that varies at the edges
+    (lambda: ops.poisson2d(33), 32),          # level 0 in slabs
+    (lambda: ops.aniso2d(64, 0.01), 9),
+    (lambda: ops.poisson3d(12), 32),          # seven entries
 ])
 @pytest.mark.parametrize("prec", [bc.PREC_FP64, bc.PREC_FP32])
 @pytest.mark.parametrize("pre,post", [(1, 1), (2, 2), (4, 4), (3, 5)])
