@@ -1936,6 +1936,10 @@ bool launch_il_resid_restrict(hipStream_t s, const DevCsr &A, MatType mt, const 
    round; PAIR_H positions at most, as strips of 64 end in a half-empty round
    (2048^2: 367 us; 32: 331; 16: 334; one round of 98: 343). */
 constexpr int PAIR_MIN_N = 128;
+/* and below PAIR_BYTES a vector of the block the walk of at least twelve
+   positions (13 to 15 us) costs more than two sweeps: 4 MB 15.1 us against
+   2 x 4.4, 17 MB 16.7 against 2 x 7.3, 67 MB 30 against 2 x 19.7 */
+constexpr size_t PAIR_BYTES = (size_t)32 << 20;
 constexpr int PAIR_WGS = 740;
 constexpr int PAIR_H = 32;
 
@@ -1944,6 +1948,7 @@ bool il_pair_ok(const DevCsr &A, MatType mt, int nc)
 {
     const RowClasses &C = A.cls;
     if (nc < (int)(16 / sizeof(VT)) || !class_ok<VT>(A, mt) || C.k != 5) return false;
+    if ((size_t)A.n * nc * sizeof(VT) < PAIR_BYTES) return false;
     const int N = C.off[4];
     return N >= PAIR_MIN_N && C.off[0] == -N && C.off[1] == -1 && C.off[2] == 0 && C.off[3] == 1;
 }
