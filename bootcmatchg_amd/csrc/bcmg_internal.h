@@ -852,9 +852,10 @@ inline CsrRef ref_of(const DevCsr &A)
    in the order of L's row then R's row (storage order); rows are taken in
    batches of at most per_pass output slots (min(products, columns of C) per
    row) plus packing weights (0: the library's default);
-   right_unique: every row of R has distinct columns */
+   right_unique: every row of R has strictly ascending columns; left_sorted:
+   every row of L */
 void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_pass = 0,
-            bool right_unique = true);
+            bool right_unique = true, bool left_sorted = true);
 /* T = A^T, each row in ascending column order; A's rows have distinct columns */
 void transpose_csr(Ctx &c, const CsrRef &A, DevCsr &T);
 /* S = I - omega D^-1 A in A's pattern, omega = 4 / (3 ||D^-1 A||_inf) */

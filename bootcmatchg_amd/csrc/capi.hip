@@ -913,19 +913,19 @@ int bcmg_spgemm(bcmg_ctx ctx, int nl, int ml, int mr, const int *lrow, const int
     d2h(ctx, cr.data(), rcol, sizeof(int) * rnnz);
     for (int c : cl) REQUIRE(c >= 0 && c < ml, "left operand: column index out of range");
     for (int c : cr) REQUIRE(c >= 0 && c < mr, "right operand: column index out of range");
-    bool right_unique = true;
-    for (int i = 0; i < ml && right_unique; i++)
-        for (int e = hr[i] + 1; e < hr[i + 1]; e++)
-            if (cr[e] <= cr[e - 1]) {
-                right_unique = false;
-                break;
-            }
+    auto ascending = [](const std::vector<int> &rp, const std::vector<int> &ci) {
+        for (size_t i = 0; i + 1 < rp.size(); i++)
+            for (int e = rp[i] + 1; e < rp[i + 1]; e++)
+                if (ci[e] <= ci[e - 1]) return false;
+        return true;
+    };
+    const bool right_unique = ascending(hr, cr), left_sorted = ascending(hl, cl);
     const CsrRef L{nl, ml, lnnz, lrow, lcol, lval};
     const CsrRef R{ml, mr, rnnz, rrow, rcol, rval};
     auto *h = new bcmg_csr_s();
     try {
         h->ctx = ctx;
-        spgemm(ctx->c, L, R, h->A, slots_per_pass, right_unique);
+        spgemm(ctx->c, L, R, h->A, slots_per_pass, right_unique, left_sorted);
         resolve_tiles(ctx->c, {&h->A});
         make_narrow(ctx->c, {&h->A});
     } catch (...) {

@@ -50,6 +50,10 @@ constexpr int SG_TILES = 16;          /* wavefronts (column tiles) of a row, at 
 constexpr int SG_TILE = 1024;         /* columns of a tile, about */
 constexpr int SG_LDS_COLS = SG_TILES * SG_TILE; /* columns of C, at most, for LDS accumulators */
 constexpr int SG_AHEAD = 8;           /* loads of 64 right entries in flight */
+constexpr int SGM_ROWS = 8;           /* rows of a dense tile */
+constexpr int SGM_AHEAD = 4;          /* right rows loaded at once */
+constexpr long long SGM_ELEMS = 1ll << 25; /* of a dense operand, at most (256 MiB) */
+constexpr double SGM_FILL = 12.0;
 constexpr long long SG_UNTOUCHED = LLONG_MIN;   /* the bits of -0.0 */
 constexpr int WAVE_RANK = 256;        /* transpose rows ranked by one wavefront */
 constexpr int RANK_CHUNK = 4096;      /* columns per LDS load when ranking */
@@ -641,6 +645,207 @@ __global__ __launch_bounds__(1024) void k_sg_wave(const int *__restrict__ large,
     if (threadIdx.x == 0) cnt[r] = all;
 }
 
+/* ------------------------------------------- dense operands
+
+   Where both operands are filled well the products outnumber what LDS adds
+   and gathered right rows can move, and the rows of C go through registers
+   instead: R as a dense array, L in tiles of SGM_ROWS rows whose used columns
+   are listed, a wavefront taking a tile's SGM_ROWS x 128 elements of C. An
+   absent entry is a zero: its product is a zero and adds nothing (the sums
+   start from +0 and are never -0), so each element is the stated sum in the
+   stated order; the operands must be finite (an infinity times an absent
+   zero is not zero), which is checked first. The pattern is the union of the
+   right rows' column bits, taken apart from the values. */
+
+/* flag[0] |= 1 if a value is not finite */
+__global__ __launch_bounds__(BS) void k_sgm_finite(long long n, const double *__restrict__ v,
+                                                   int *__restrict__ flag)
+{
+    bool bad = false;
+    for (long long i = (long long)blockIdx.x * BS + threadIdx.x; i < n;
+         i += (long long)gridDim.x * BS)
+        bad = bad || !isfinite(v[i]);
+    if (__ballot(bad) && (threadIdx.x & 63) == 0) atomicOr(flag, 1);
+}
+
+/* R's rows into Rd (pitch mp, zeroed) and their column bits (mw words of 64);
+   a wavefront a row, bits gathered in LDS (4 mw words) */
+__global__ __launch_bounds__(BS) void k_sgm_right(int n, const int *__restrict__ rp,
+                                                  const int *__restrict__ ci,
+                                                  const double *__restrict__ v, int mp, int mw,
+                                                  double *__restrict__ Rd,
+                                                  unsigned long long *__restrict__ bits)
+{
+    extern __shared__ unsigned sgm_bits[];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = blockIdx.x * (BS / 64) + wv;
+    unsigned *const b = sgm_bits + wv * 2 * mw;
+    for (int t = lane; t < 2 * mw; t += 64) b[t] = 0;
+    __syncthreads();
+    if (r < n)
+        for (int e = rp[r] + lane; e < rp[r + 1]; e += 64) {
+            const int c = ci[e];
+            Rd[(size_t)r * mp + c] = v[e];
+            atomicOr(&b[c >> 5], 1u << (c & 31));
+        }
+    __syncthreads();
+    if (r < n)
+        for (int t = lane; t < mw; t += 64)
+            bits[(size_t)r * mw + t] = b[2 * t] | (unsigned long long)b[2 * t + 1] << 32;
+}
+
+/* L's rows into tiles: Ld[(tile (K + 1) + k) SGM_ROWS + row in tile] (zeroed)
+   and the tile's used k (kw words of 32, zeroed); a wavefront a row */
+__global__ __launch_bounds__(BS) void k_sgm_left(int n, int K, int kw,
+                                                 const int *__restrict__ rp,
+                                                 const int *__restrict__ ci,
+                                                 const double *__restrict__ v,
+                                                 double *__restrict__ Ld,
+                                                 unsigned *__restrict__ used)
+{
+    const int r = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    if (r >= n) return;
+    const int tile = r / SGM_ROWS, q = r - tile * SGM_ROWS;
+    for (int e = rp[r] + lane; e < rp[r + 1]; e += 64) {
+        const int k = ci[e];
+        Ld[((size_t)tile * (K + 1) + k) * SGM_ROWS + q] = v[e];
+        atomicOr(&used[(size_t)tile * kw + (k >> 5)], 1u << (k & 31));
+    }
+}
+
+/* a tile's used k in ascending order, filled up to a multiple of SGM_AHEAD
+   with K (a row of zeros in Ld); a wavefront a tile */
+__global__ __launch_bounds__(64) void k_sgm_list(int K, int kw, const unsigned *__restrict__ used,
+                                                 int pitch, int *__restrict__ list,
+                                                 int *__restrict__ count)
+{
+    const int tile = blockIdx.x, lane = threadIdx.x;
+    int *const o = list + (size_t)tile * pitch;
+    int at = 0;
+    for (int k0 = 0; k0 < K; k0 += 64) {
+        const int k = k0 + lane;
+        const bool in = k < K && ((used[(size_t)tile * kw + (k >> 5)] >> (k & 31)) & 1u);
+        const unsigned long long b = __ballot(in);
+        if (in) o[at + __popcll(b & ((1ull << lane) - 1))] = k;
+        at += __popcll(b);
+    }
+    const int end = (at + SGM_AHEAD - 1) / SGM_AHEAD * SGM_AHEAD;
+    if (lane < end - at) o[at + lane] = K;
+    if (lane == 0) count[tile] = end;
+}
+
+/* C's rows: column bits (the union over the left entries), the number of
+   entries before each word, the columns and the count; a wavefront a row */
+__global__ __launch_bounds__(BS) void k_sgm_pattern(int n, const int *__restrict__ rp,
+                                                    const int *__restrict__ ci, int mw,
+                                                    const unsigned long long *__restrict__ rbits,
+                                                    const int *__restrict__ uoff,
+                                                    unsigned long long *__restrict__ cbits,
+                                                    int *__restrict__ before,
+                                                    int *__restrict__ tcol, int *__restrict__ cnt)
+{
+    const int r = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    if (r >= n) return;
+    const int a = rp[r], b = rp[r + 1];
+    int base = 0;
+    for (int w0 = 0; w0 < mw; w0 += 64) {
+        const int w = w0 + lane;
+        const int wc = min(w, mw - 1);
+        unsigned long long bits = 0;
+        for (int e = a; e < b; e += 8) {
+#pragma unroll
+            for (int u = 0; u < 8; u++)
+                bits |= rbits[(size_t)ci[min(e + u, b - 1)] * mw + wc];
+        }
+        if (w >= mw) bits = 0;
+        int x = __popcll(bits);
+        const int own = x;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(x, o, 64);
+            if (lane >= o) x += y;
+        }
+        const int first = base + x - own;
+        if (w < mw) {
+            cbits[(size_t)r * mw + w] = bits;
+            before[(size_t)r * mw + w] = first;
+        }
+        for (int t = 0; t < min(64, mw - w0); t++) {
+            const unsigned lo = __builtin_amdgcn_readlane((int)bits, t);
+            const unsigned hi = __builtin_amdgcn_readlane((int)(bits >> 32), t);
+            const unsigned long long word = lo | (unsigned long long)hi << 32;
+            const int at = __builtin_amdgcn_readlane(first, t);
+            if ((word >> lane) & 1ull)
+                tcol[uoff[r] + at + __popcll(word & ((1ull << lane) - 1))] = (w0 + t) * 64 + lane;
+        }
+        base += __builtin_amdgcn_readlane(x, 63);
+    }
+    if (lane == 0) cnt[r] = base;
+}
+
+/* The values: four wavefronts of a workgroup take four row tiles of the same
+   128 columns (their right loads meet in L1); a left value is a scalar. The
+   multiplier bounds it: 2048 x 4096 x 2048, 1.6 ms, 21 of 39 T operations/s
+   (multiply and add apart). */
+__global__ __launch_bounds__(BS) void k_sgm_values(int n, int K, int mp, int mw, int tiles,
+                                                   const int *__restrict__ list, int pitch,
+                                                   const int *__restrict__ count,
+                                                   const double *__restrict__ Ld,
+                                                   const double *__restrict__ Rd,
+                                                   const unsigned long long *__restrict__ cbits,
+                                                   const int *__restrict__ before,
+                                                   const int *__restrict__ uoff,
+                                                   double *__restrict__ tval)
+{
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int cols = mp / 128;
+    const int b = xcd_block(blockIdx.x, gridDim.x);
+    const int c = b % cols, tile = b / cols * (BS / 64) + wv;
+    if (tile >= tiles) return;
+    const int *const ks = list + (size_t)tile * pitch;
+    const double *const Lt = Ld + (size_t)tile * (K + 1) * SGM_ROWS;
+    const double *const Rt = Rd + c * 128 + lane;
+    double acc[SGM_ROWS][2];
+#pragma unroll
+    for (int q = 0; q < SGM_ROWS; q++) acc[q][0] = acc[q][1] = 0.0;
+    const int nk = count[tile];
+    for (int e = 0; e < nk; e += SGM_AHEAD) {
+        double rv[SGM_AHEAD][2];
+        int kk[SGM_AHEAD];
+#pragma unroll
+        for (int u = 0; u < SGM_AHEAD; u++) {
+            kk[u] = ks[e + u];
+            const double *const row = Rt + (size_t)(kk[u] < K ? kk[u] : 0) * mp;
+            rv[u][0] = row[0];
+            rv[u][1] = row[64];
+        }
+#pragma unroll
+        for (int u = 0; u < SGM_AHEAD; u++) {
+            const double *const l = Lt + (size_t)kk[u] * SGM_ROWS;
+#pragma unroll
+            for (int q = 0; q < SGM_ROWS; q++) {
+                acc[q][0] = acc[q][0] + l[q] * rv[u][0];
+                acc[q][1] = acc[q][1] + l[q] * rv[u][1];
+            }
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < SGM_ROWS; q++) {
+        const int r = tile * SGM_ROWS + q;
+        if (r >= n) break;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            const int w = 2 * c + h;
+            if (w >= mw) continue;
+            const unsigned long long bits = cbits[(size_t)r * mw + w];
+            if ((bits >> lane) & 1ull)
+                tval[uoff[r] + before[(size_t)r * mw + w] +
+                     __popcll(bits & ((1ull << lane) - 1))] = acc[q][h];
+        }
+    }
+}
+
 /* compact the rows from their product-count slots into C (G lanes a row) */
 template <int G>
 __global__ __launch_bounds__(BS) void k_sg_gather(int n, const int *__restrict__ uoff,
@@ -911,11 +1116,44 @@ void gather_rows(Ctx &c, int n, const int *uoff, const int *rp, const int *tcol,
 
 } // namespace
 
+namespace {
+
+/* all rows of C = L R with dense operands (every row long, one batch) */
+void dense_product(Ctx &c, const CsrRef &L, const CsrRef &R, const int *uoff, int *tcol,
+                   double *tval, int *cnt)
+{
+    const int n = L.n, K = L.m, mp = (R.m + 127) / 128 * 128, mw = (R.m + 63) / 64;
+    const int tiles = (n + SGM_ROWS - 1) / SGM_ROWS, kw = (K + 31) / 32;
+    const int pitch = (K + SGM_AHEAD - 1) / SGM_AHEAD * SGM_AHEAD;
+    DBuf<double> Rd((size_t)K * mp), Ld((size_t)tiles * (K + 1) * SGM_ROWS);
+    DBuf<unsigned long long> rbits((size_t)K * mw), cbits((size_t)n * mw);
+    DBuf<unsigned> used((size_t)tiles * kw);
+    DBuf<int> before((size_t)n * mw), list((size_t)tiles * pitch), count(tiles);
+    BCMG_HIP(hipMemsetAsync(Rd.get(), 0, sizeof(double) * (size_t)K * mp, c.stream));
+    BCMG_HIP(hipMemsetAsync(Ld.get(), 0, sizeof(double) * (size_t)tiles * (K + 1) * SGM_ROWS,
+                            c.stream));
+    BCMG_HIP(hipMemsetAsync(used.get(), 0, sizeof(unsigned) * (size_t)tiles * kw, c.stream));
+    k_sgm_right<<<(K + BS / 64 - 1) / (BS / 64), BS, (size_t)(BS / 64) * 2 * mw * sizeof(unsigned),
+                  c.stream>>>(K, R.rp, R.ci, R.v, mp, mw, Rd.get(), rbits.get());
+    k_sgm_left<<<blocks_for(64ll * n), BS, 0, c.stream>>>(n, K, kw, L.rp, L.ci, L.v, Ld.get(),
+                                                          used.get());
+    k_sgm_list<<<tiles, 64, 0, c.stream>>>(K, kw, used.get(), pitch, list.get(), count.get());
+    k_sgm_pattern<<<blocks_for(64ll * n), BS, 0, c.stream>>>(n, L.rp, L.ci, mw, rbits.get(), uoff,
+                                                             cbits.get(), before.get(), tcol, cnt);
+    const int grid = (tiles + BS / 64 - 1) / (BS / 64) * (mp / 128);
+    k_sgm_values<<<grid, BS, 0, c.stream>>>(n, K, mp, mw, tiles, list.get(), pitch, count.get(),
+                                            Ld.get(), Rd.get(), cbits.get(), before.get(), uoff,
+                                            tval);
+    BCMG_CHECK_LAUNCH();
+}
+
+} // namespace
+
 /* Rows are taken in batches of at most per_pass output slots plus packing
    weights (a row over it is a batch of its own), so that the temporaries
    stay bounded and their offsets fit 32 bits; one batch writes C directly. */
 void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_pass,
-            bool right_unique)
+            bool right_unique, bool left_sorted)
 {
     if (L.m != R.n) throw Error(BCMG_EINVAL, "spgemm: inner dimensions differ");
     if (per_pass <= 0) per_pass = SG_PER_PASS;
@@ -943,10 +1181,27 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
                      (long long)R.n * (tiles + 1) <= 2ll * R.nnz;
     const int smin = !right_unique ? 0 : lds ? std::max(1, tiles / 2) : SG_SERIAL_MIN;
     DBuf<int> u(n), sl(n), ws(n), cnt(n), large(n);
-    /* long-row count, row with too many products, long rows below smin */
-    DBuf<int> flags(3);
+    /* Dense operands when the filled parts of both multiply to 1 / SGM_FILL or
+       more and either fits SGM_ELEMS: 0.28 and 0.094 (2048 rows) win 4.5 ->
+       2.2 and 5.6 -> 3.0 ms with all their preparation, 0.053 (1125 rows)
+       breaks even, 0.011 loses (48^3's products 5.2 -> 6.3 ms). */
+    const bool fill = right_unique && left_sorted && n >= SGM_ROWS && mcols >= 128 &&
+                      mcols <= SG_LDS_COLS &&
+                      (long long)n * L.m <= SGM_ELEMS && (long long)L.m * mcols <= SGM_ELEMS &&
+                      (double)L.nnz * R.nnz * SGM_FILL >=
+                          (double)n * L.m * ((double)R.n * (double)mcols);
+    /* long-row count, row with too many products, long rows below smin, a
+       value that is not finite */
+    DBuf<int> flags(4);
     DBuf<unsigned long long> total(1);
-    BCMG_HIP(hipMemsetAsync(flags.get(), 0, 3 * sizeof(int), c.stream));
+    BCMG_HIP(hipMemsetAsync(flags.get(), 0, 4 * sizeof(int), c.stream));
+    if (fill) {
+        k_sgm_finite<<<std::min(1024, blocks_for(L.nnz)), BS, 0, c.stream>>>(L.nnz, L.v,
+                                                                             flags.get() + 3);
+        k_sgm_finite<<<std::min(1024, blocks_for(R.nnz)), BS, 0, c.stream>>>(R.nnz, R.v,
+                                                                             flags.get() + 3);
+        BCMG_CHECK_LAUNCH();
+    }
     BCMG_HIP(hipMemsetAsync(total.get(), 0, sizeof(unsigned long long), c.stream));
     const bool lng = long_rows(n, L.nnz);
     const int per = rows_per_block(n, lng);
@@ -955,10 +1210,10 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
         flags.get(), total.get(), flags.get() + 1, smin);
     BCMG_CHECK_LAUNCH();
     unsigned long long h_total = 0;
-    int h_flags[3] = {0, 0, 0};
+    int h_flags[4] = {0, 0, 0, 0};
     BCMG_HIP(hipMemcpyAsync(&h_total, total.get(), sizeof(h_total), hipMemcpyDeviceToHost,
                             c.stream));
-    BCMG_HIP(hipMemcpyAsync(h_flags, flags.get(), 3 * sizeof(int), hipMemcpyDeviceToHost,
+    BCMG_HIP(hipMemcpyAsync(h_flags, flags.get(), 4 * sizeof(int), hipMemcpyDeviceToHost,
                             c.stream));
     BCMG_HIP(hipStreamSynchronize(c.stream));
     const int h_nlarge = h_flags[0];
@@ -1045,7 +1300,9 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
             }
             lrows = lbuf.get();
         }
-        if (nl > 0) {
+        if (fill && nbatch == 1 && nl == n && h_flags[3] == 0) {
+            dense_product(c, L, R, uoff.get(), tcol.get(), tval.get(), cnt.get());
+        } else if (nl > 0) {
             if (lds) {
                 if (!seg.get()) {
                     seg.alloc((size_t)R.n * (tiles + 1));

@@ -63,3 +63,39 @@ def test_short_right_rows(ctx, per_entry):
     assert np.array_equal(row, orow)
     assert np.array_equal(col, ocol)
     assert np.array_equal(bits(val), bits(oval))
+
+
+def same(val, oval):
+    nan = np.isnan(oval)
+    return np.array_equal(np.isnan(val), nan) and np.array_equal(bits(val[~nan]), bits(oval[~nan]))
+
+
+@pytest.mark.parametrize("n,k,m,fl,fr,special", [
+    (8, 160, 128, 0.5, 0.5, True),        # one tile, one column block
+    (9, 161, 129, 0.6, 0.4, True),        # a row and a column beyond them
+    (67, 300, 1000, 0.9, 0.2, False),
+    (130, 1025, 640, 0.3, 0.35, True),
+    (40, 200, 300, 0.05, 0.9, False),     # below the fill that is taken
+])
+@pytest.mark.parametrize("change", ["", "infinite", "left order", "a short row"])
+def test_dense_operands(ctx, n, k, m, fl, fr, special, change):
+    """Well-filled operands, and what keeps the other form: a value that is
+    not finite, left rows out of order, a short row among long ones."""
+    rng = np.random.default_rng(n + k)
+    L = rows(rng, n, k, np.maximum(20, rng.binomial(k, fl, n)), special)
+    R = rows(rng, k, m, np.maximum(60, rng.binomial(m, fr, k)), special)
+    if change == "infinite":
+        L[2][len(L[2]) // 2] = np.inf
+    elif change == "left order":
+        for i in range(0, n, 3):
+            s = slice(L[0][i], L[0][i + 1])
+            p = rng.permutation(s.stop - s.start)
+            L[1][s], L[2][s] = L[1][s][p], L[2][s][p]
+    elif change == "a short row":
+        L = rows(rng, n, k, np.r_[1, np.maximum(20, rng.binomial(k, fl, n - 1))], special)
+    row, col, val = bc.spgemm(ctx, L, R, m).download()
+    with np.errstate(all="ignore"):
+        orow, ocol, oval = orc.spgemm(L, R, m)
+    assert np.array_equal(row, orow)
+    assert np.array_equal(col, ocol)
+    assert same(val, oval)
