@@ -91,13 +91,16 @@ int bcmg_csr_upload(bcmg_ctx ctx, int n, int nnz, const int *row, const int *col
                     const double *val, bcmg_csr *out);
 int bcmg_csr_download(bcmg_csr A, int *row, int *col, double *val);
 int bcmg_csr_info(bcmg_csr A, int *n, int *nnz);
-/* Bytes per column index that the FP64 row kernels read for A. A square
+/* Bytes per column index of the narrowest column copy kept for A. A square
    operator can get narrower copies of its columns at upload: 16-bit offsets
    (column minus row) when they all fit and it has more than 16.7 M entries
    (an FP64 stream above 192 MB), and a stencil pattern when it has more
    than 11.2 M entries (above 128 MB) and its offsets take at most 8
    distinct values (one byte per row: which offsets of a sorted table the
-   row has). The row kernels read the narrowest one that is kept: 0 the
+   row has). An operator whose rows take few distinct forms, or that is
+   symmetric with few offsets, is read from those instead (a byte per row;
+   see bcmg_csr_set_columns); otherwise the row kernels read the narrowest
+   copy that is kept: 0 the
    pattern (no per-entry column bytes, one byte per row, and only two row
    pointers per 256 rows), 2 the 16-bit offsets (FP32/BF16 value copies use
    them when their 32-bit-column stream also exceeds 192 MB), else 4.
@@ -105,7 +108,8 @@ int bcmg_csr_info(bcmg_csr A, int *n, int *nnz);
    (which always streams 32-bit columns); it lets a caller price a kernel's
    memory traffic. */
 int bcmg_csr_column_bytes(bcmg_csr A, int *bytes);
-/* Restricts the row kernels on A to a column form: bytes 0 (the pattern),
+/* Restricts the row kernels on A to a column form, in place of its row classes
+   or symmetric stencil too: bytes 0 (the pattern),
    2 (the 16-bit offsets) or 4 (the int32 columns); BCMG_EUNSUP when A has no
    such copy. Composites set up on A before the call keep the launches they
    captured. No counterpart in the reference: for A/B measurements and tests

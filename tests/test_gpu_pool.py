@@ -2,6 +2,8 @@
 leaves nothing behind, and what a context holds stays near what its blocks
 take.
 """
+import time
+
 import pytest
 
 import bootcmatchg_amd as bc
@@ -33,4 +35,8 @@ def test_closed_context_gives_its_memory_back(make):
         # the operator and its hierarchy (about 3 times its 12 bytes an entry),
         # set-up temporaries, chunks at most as large again: 8 MiB at least
         assert held - before <= (16 << 20) + 40 * 12 * len(A[1])
+        # the runtime may hand freed memory back a few milliseconds later
+        end = time.monotonic() + 1.0
+        while device_bytes_in_use() - before > 4 << 20 and time.monotonic() < end:
+            time.sleep(0.005)
         assert device_bytes_in_use() - before <= 4 << 20
