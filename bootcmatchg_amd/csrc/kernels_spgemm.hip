@@ -7,9 +7,12 @@
  * C(i,j) is 0 + the products L(i,e) R(e,j), taken over L's row i in storage
  * order and, within it, over R's row e in storage order (the reference's hash
  * SpGEMM adds with shared-memory atomics in arrival order, so it fixes no
- * order). A row's products are expanded into LDS under a 64-bit key
- * (row, column, position), bitonic-sorted, and each run of one (row, column)
- * is summed by one lane in position order:
+ * order). With right rows of distinct columns, four or more on average, a row
+ * of up to SG_CAP products is summed in an LDS hash table (k_sg_hash), and so
+ * is a longer one that no form below suits better and whose columns fit. Else a
+ * row's products are expanded into LDS under a 64-bit key (row, column,
+ * position), bitonic-sorted, and each run of one (row, column) is summed by
+ * one lane in position order:
  *   - rows with at most SG_CAP products are packed into workgroups by a
  *     prefix sum of (products + 1): a workgroup owns the rows whose prefix
  *     starts in its SG_CAP-slot range, and since such a row ends within the
@@ -346,7 +349,7 @@ __global__ __launch_bounds__(BS) void k_sg_dense(int nlarge, const int *__restri
                                                  int *__restrict__ tcol, double *__restrict__ tval,
                                                  double *acc_all, int *stamp_all, long long m,
                                                  int row_base, int serial_min, int skip_serial,
-                                                 int *__restrict__ cnt)
+                                                 int only_left, int *__restrict__ cnt)
 {
     __shared__ unsigned long long key[SG_CH];   /* also the sort buffer of SG_SORT ints */
     __shared__ double val[SG_CH];
@@ -365,6 +368,7 @@ __global__ __launch_bounds__(BS) void k_sg_dense(int nlarge, const int *__restri
         int ew0 = Lrp[r], pb0 = 0;   /* first window some later chunk needs */
         const bool serial = serial_min > 0 && (long long)U >= (long long)serial_min * (e_end - ew0);
         if (serial && skip_serial) continue;   /* k_sg_wave takes it */
+        if (only_left && cnt[r] != -1) continue;   /* k_sg_hash took it */
         int *const ocol = tcol + uoff[r];
         double *const oval = tval + uoff[r];
         if (threadIdx.x == 0) {
@@ -519,6 +523,153 @@ __global__ __launch_bounds__(BS) void k_sg_dense(int nlarge, const int *__restri
     }
 }
 
+/* Rows with lo < products <= hi when R's rows hold distinct columns: a
+   wavefront a row, its columns in an LDS hash table of H slots with their
+   sums. The left entries are taken in order, 64 lanes on a right row; its
+   columns are distinct, so an LDS add instruction meets no slot twice and each
+   sum is taken in the stated order (k_sg_wave's argument). The table's entries
+   then go to their ranks among the columns. A row with more than H columns
+   (lo >= H only) is left: its count becomes -1 and *left 1. smin > 0: only
+   rows below smin products per left entry. 64^3 smoothed, R A and T P of
+   level 0 (25 M products): 2.1 ms sorted, 0.6 so; R A of level 1 (51 M, 65 536
+   columns): 2.8 ms on dense accumulators, 0.7 so. LDS latency bounds it. */
+template <int H>
+__global__ __launch_bounds__(BS) void k_sg_hash(int n, int lo, int hi, int smin,
+                                                const int *__restrict__ Lrp,
+                                                const int *__restrict__ Lci,
+                                                const double *__restrict__ Lv,
+                                                const int *__restrict__ Rrp,
+                                                const int *__restrict__ Rci,
+                                                const double *__restrict__ Rv,
+                                                const int *__restrict__ u,
+                                                const int *__restrict__ uoff,
+                                                int *__restrict__ tcol, double *__restrict__ tval,
+                                                int *__restrict__ cnt, int *__restrict__ left)
+{
+    constexpr int Q = H / 64, SHIFT = 32 - __builtin_ctz(H);
+    __shared__ double vals[BS / 64][H];
+    __shared__ int keys[BS / 64][H];
+    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int r = xcd_block(blockIdx.x, gridDim.x) * (BS / 64) + wv;
+    if (r >= n) return;
+    const int U = u[r], eb = Lrp[r], ee = Lrp[r + 1];
+    if (U <= lo || U > hi) return;
+    if (smin > 0 && (long long)U >= (long long)smin * (ee - eb)) return;
+    int *const key = keys[wv];
+    double *const val = vals[wv];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        key[q * 64 + lane] = -1;
+        val[q * 64 + lane] = 0.0;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    bool full = false;
+    for (int e0 = eb; e0 < ee && !full; e0 += 64) {
+        const int e = e0 + lane;
+        int s0 = 0, s1 = 0;
+        double lv = 0.0;
+        if (e < ee) {
+            const int k = Lci[e];
+            s0 = Rrp[k];
+            s1 = Rrp[k + 1];
+            lv = Lv[e];
+        }
+        unsigned long long todo = __ballot(s1 > s0);
+        int f = 0, f1 = 0;
+        double l = 0.0;
+        while ((todo || f < f1) && !full) {
+            int cc[SG_AHEAD];
+            double vv[SG_AHEAD], ll[SG_AHEAD];
+#pragma unroll
+            for (int d = 0; d < SG_AHEAD; d++) {
+                if (f >= f1 && todo) {
+                    const int t = __builtin_ctzll(todo);
+                    todo &= todo - 1;
+                    f = __builtin_amdgcn_readlane(s0, t);
+                    f1 = __builtin_amdgcn_readlane(s1, t);
+                    l = lane_double(lv, t);
+                }
+                const int p = f + lane;
+                const int pc = min(p, f1 - 1);
+                const int col = Rci[pc];
+                cc[d] = p < f1 ? col : -1;
+                vv[d] = Rv[pc];
+                ll[d] = l;
+                f += 64;
+            }
+#pragma unroll
+            for (int d = 0; d < SG_AHEAD; d++) {
+                const int c = cc[d];
+                if (c < 0) continue;
+                int h = (int)(((unsigned)c * 2654435761u) >> SHIFT);
+                int tries = 0;
+                for (; tries < H; tries++) {
+                    int k = __hip_atomic_load(&key[h], __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (k == -1) k = atomicCAS(&key[h], -1, c);
+                    if (k == -1 || k == c) break;
+                    h = (h + 1) & (H - 1);
+                }
+                if (tries < H)
+                    __hip_atomic_fetch_add(&val[h], ll[d] * vv[d], __ATOMIC_RELAXED,
+                                           __HIP_MEMORY_SCOPE_WORKGROUP);
+                else
+                    full = true;
+            }
+            full = __ballot(full) != 0;
+        }
+    }
+    if (full) {
+        if (lane == 0) {
+            cnt[r] = -1;
+            *left = 1;
+        }
+        return;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    /* to the front of the table (a step writes at or before what it read) */
+    int k = 0;
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        const int c = key[q * 64 + lane];
+        const double v = val[q * 64 + lane];
+        const unsigned long long b = __ballot(c >= 0);
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        if (c >= 0) {
+            const int at = k + __popcll(b & ((1ull << lane) - 1));
+            key[at] = c;
+            val[at] = v;
+        }
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+        k += __popcll(b);
+    }
+    int mine[Q], rank[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) {
+        mine[q] = q * 64 + lane < k ? key[q * 64 + lane] : INT_MAX;
+        rank[q] = 0;
+    }
+#pragma unroll
+    for (int g = 0; g < Q; g++) {
+        if (g * 64 >= k) break;
+        const int ng = min(64, k - g * 64);
+        for (int t = 0; t < ng; t++) {
+            const int d = __builtin_amdgcn_readlane(mine[g], t);
+#pragma unroll
+            for (int q = 0; q < Q; q++)
+                if (q * 64 < k) rank[q] += d < mine[q] ? 1 : 0;
+        }
+    }
+    const int o = uoff[r];
+#pragma unroll
+    for (int q = 0; q < Q; q++)
+        if (q * 64 + lane < k) {
+            tcol[o + rank[q]] = mine[q];
+            tval[o + rank[q]] = val[q * 64 + lane];
+        }
+    if (lane == 0) cnt[r] = k;
+}
+
 /* where R's rows cross the column tiles [t W, (t + 1) W): seg[row][t] is the
    first entry of tile t, seg[row][nt] the row's end (a wavefront a row,
    columns strictly ascending) */
@@ -567,7 +718,8 @@ __global__ __launch_bounds__(1024) void k_sg_wave(const int *__restrict__ large,
                                                   const int *__restrict__ uoff,
                                                   int *__restrict__ tcol,
                                                   double *__restrict__ tval, int W,
-                                                  int serial_min, int *__restrict__ cnt)
+                                                  int serial_min, int only_left,
+                                                  int *__restrict__ cnt)
 {
     extern __shared__ double sg_acc[];
     __shared__ int wcnt[SG_TILES];
@@ -576,6 +728,7 @@ __global__ __launch_bounds__(1024) void k_sg_wave(const int *__restrict__ large,
     const int r = large ? large[b0] : b0;
     const int eb = Lrp[r], ee = Lrp[r + 1];
     if (u[r] <= SG_CAP || (long long)u[r] < (long long)serial_min * (ee - eb)) return;
+    if (only_left && cnt[r] != -1) return;   /* k_sg_hash took it */
     double *const acc = sg_acc + wv * W;
     for (int t = lane; t < W; t += 64) acc[t] = -0.0;
     __syncthreads();
@@ -1179,7 +1332,16 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
     const int tile_w = (int)((mcols + 64ll * tiles - 1) / (64ll * tiles)) * 64;
     const bool lds = right_unique && mcols <= SG_LDS_COLS &&
                      (long long)R.n * (tiles + 1) <= 2ll * R.nnz;
-    const int smin = !right_unique ? 0 : lds ? std::max(1, tiles / 2) : SG_SERIAL_MIN;
+    /* rows by hash where the right rows have four entries or more on average:
+       a left entry is a step of a wavefront, and with one product each (the
+       tentative prolongator) 2048 of them took 5.2 ms against 0.9 sorted; below
+       four products per left entry and tile it also goes before k_sg_wave,
+       which takes what has too many columns (T P with 16 384 columns and 19
+       products per left entry: 3.0 ms
+       against 1.1) */
+    const bool hashed = right_unique && R.nnz >= 4ll * R.n;
+    const int wmin = std::max(1, tiles / 2);
+    const int smin = !right_unique ? 0 : !lds ? SG_SERIAL_MIN : hashed ? 4 * tiles : wmin;
     DBuf<int> u(n), sl(n), ws(n), cnt(n), large(n);
     /* Dense operands when the filled parts of both multiply to 1 / SGM_FILL or
        more and either fits SGM_ELEMS: 0.28 and 0.094 (2048 rows) win 4.5 ->
@@ -1280,7 +1442,17 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
         const int lo = blo[b], nr = bhi[b] - blo[b];
         const int *Lrp = L.rp + lo;
         exclusive_scan(c, sl.get() + lo, uoff.get(), nr, false);
-        const long long S = exclusive_scan(c, ws.get() + lo, soff.get(), nr, true);
+        auto hash = [&](auto kern, int above, int upto, int below) {
+            kern<<<(nr + BS / 64 - 1) / (BS / 64), BS, 0, c.stream>>>(
+                nr, above, upto, below, Lrp, L.ci, L.v, R.rp, R.ci, R.v, u.get() + lo, uoff.get(),
+                tcol.get(), tval.get(), cnt.get() + lo, flags.get() + 1);
+        };
+        if (hashed) {
+            hash(k_sg_hash<512>, 0, 512, 0);
+            hash(k_sg_hash<1024>, 512, SG_CAP, 0);
+        }
+        const long long S =
+            hashed ? 0 : exclusive_scan(c, ws.get() + lo, soff.get(), nr, true);
         const int nb = (int)((S + SG_CAP - 1) / SG_CAP);
         if (nb > 0)
             k_sg_small<<<nb, BS, 0, c.stream>>>(nr, Lrp, L.ci, L.v, R.rp, R.ci, R.v,
@@ -1303,7 +1475,7 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
         if (fill && nbatch == 1 && nl == n && h_flags[3] == 0) {
             dense_product(c, L, R, uoff.get(), tcol.get(), tval.get(), cnt.get());
         } else if (nl > 0) {
-            if (lds) {
+            auto wave = [&](int least, int only_left) {
                 if (!seg.get()) {
                     seg.alloc((size_t)R.n * (tiles + 1));
                     k_sg_seg<<<blocks_for(64ll * R.n), BS, 0, c.stream>>>(R.n, R.rp, R.ci, tile_w,
@@ -1315,10 +1487,23 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
                 k_sg_wave<<<by_row ? nr : nl, 64 * tiles, sizeof(double) * tiles * tile_w,
                             c.stream>>>(by_row ? nullptr : lrows, Lrp, L.ci, L.v, seg.get(), R.ci,
                                         R.v, u.get() + lo, uoff.get(), tcol.get(), tval.get(),
-                                        tile_w, smin, cnt.get() + lo);
+                                        tile_w, least, only_left, cnt.get() + lo);
                 BCMG_CHECK_LAUNCH();
+            };
+            if (lds && h_flags[2] < h_nlarge) wave(smin, 0);
+            /* the others: by hash where their columns fit, the rest on dense
+               accumulators */
+            int rest = !lds || h_flags[2] > 0;
+            if (rest && hashed) {
+                BCMG_HIP(hipMemsetAsync(flags.get() + 1, 0, sizeof(int), c.stream));
+                hash(k_sg_hash<1024>, SG_CAP, INT_MAX, lds ? smin : 0);
+                BCMG_CHECK_LAUNCH();
+                BCMG_HIP(hipMemcpyAsync(&rest, flags.get() + 1, sizeof(int),
+                                        hipMemcpyDeviceToHost, c.stream));
+                BCMG_HIP(hipStreamSynchronize(c.stream));
             }
-            if (!lds || h_flags[2] > 0) {
+            if (rest && lds && hashed) wave(wmin, 1);
+            if (rest) {
                 if (!acc.get()) {
                     /* dense accumulators: as many workgroups as the budget
                        allows, stamps cleared once for every batch */
@@ -1333,8 +1518,8 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
                 }
                 k_sg_dense<<<std::min(nl, dblocks), BS, 0, c.stream>>>(
                     nl, lrows, Lrp, L.ci, L.v, R.rp, R.ci, R.v, u.get() + lo, uoff.get(),
-                    tcol.get(), tval.get(), acc.get(), stamp.get(), mcols, lo, smin, lds ? 1 : 0,
-                    cnt.get() + lo);
+                    tcol.get(), tval.get(), acc.get(), stamp.get(), mcols, lo, lds ? wmin : smin, lds ? 1 : 0,
+                    hashed ? 1 : 0, cnt.get() + lo);
                 BCMG_CHECK_LAUNCH();
             }
         }

@@ -99,3 +99,26 @@ def test_dense_operands(ctx, n, k, m, fl, fr, special, change):
     assert np.array_equal(row, orow)
     assert np.array_equal(col, ocol)
     assert same(val, oval)
+
+
+@pytest.mark.parametrize("m", [1500, 60000])
+@pytest.mark.parametrize("stride", [8, 4, 1])
+def test_hashed_rows(ctx, m, stride):
+    """Right row k holds the eight columns from stride k on, so a left row of t
+    entries has 8 t products and 8 + stride (t - 1) columns: tables just full
+    and one entry too small, rows on both sides of each product bound."""
+    rng = np.random.default_rng(stride)
+    k = (m - 8) // stride + 1
+    col = (np.arange(k)[:, None] * stride + np.arange(8)).ravel()
+    R = (np.arange(0, 8 * k + 1, 8).astype(np.int32), col.astype(np.int32),
+         rng.uniform(-1, 1, 8 * k))
+    counts = [t for t in (0, 1, 63, 64, 65, 127, 128, 129, 255, 256, 300, 1017, 1018) if t <= k]
+    row = np.concatenate(([0], np.cumsum(counts))).astype(np.int32)
+    start = [int(rng.integers(0, k - t + 1)) for t in counts]
+    L = (row, np.concatenate([np.arange(s, s + t) for s, t in zip(start, counts)])
+         .astype(np.int32), rng.uniform(-1, 1, row[-1]))
+    crow, ccol, cval = bc.spgemm(ctx, L, R, m).download()
+    orow, ocol, oval = orc.spgemm(L, R, m)
+    assert np.array_equal(crow, orow)
+    assert np.array_equal(ccol, ocol)
+    assert np.array_equal(bits(cval), bits(oval))
