@@ -53,8 +53,8 @@ constexpr int SG_TILES = 16;          /* wavefronts (column tiles) of a row, at 
 constexpr int SG_TILE = 1024;         /* columns of a tile, about */
 constexpr int SG_LDS_COLS = SG_TILES * SG_TILE; /* columns of C, at most, for LDS accumulators */
 constexpr int SG_AHEAD = 8;           /* loads of 64 right entries in flight */
-constexpr int SGM_ROWS = 8;           /* rows of a dense tile */
-constexpr int SGM_AHEAD = 4;          /* right rows loaded at once */
+constexpr int SGM_ROWS = 16;          /* rows of a dense tile */
+constexpr int SGM_AHEAD = 2;          /* right rows loaded at once */
 constexpr long long SGM_ELEMS = 1ll << 25; /* of a dense operand, at most (256 MiB) */
 constexpr double SGM_FILL = 12.0;
 constexpr long long SG_UNTOUCHED = LLONG_MIN;   /* the bits of -0.0 */
@@ -847,44 +847,46 @@ __global__ __launch_bounds__(BS) void k_sgm_right(int n, const int *__restrict__
             bits[(size_t)r * mw + t] = b[2 * t] | (unsigned long long)b[2 * t + 1] << 32;
 }
 
-/* L's rows into tiles: Ld[(tile (K + 1) + k) SGM_ROWS + row in tile] (zeroed)
-   and the tile's used k (kw words of 32, zeroed); a wavefront a row */
+/* L's rows into tiles, a workgroup a tile: Ld[(tile (K + 1) + k) SGM_ROWS +
+   row in tile] (zeroed), and the tile's used k in ascending order (gathered as
+   bits in LDS, kw words), filled up to a multiple of SGM_AHEAD with K, a row of
+   zeros in Ld */
 __global__ __launch_bounds__(BS) void k_sgm_left(int n, int K, int kw,
                                                  const int *__restrict__ rp,
                                                  const int *__restrict__ ci,
                                                  const double *__restrict__ v,
-                                                 double *__restrict__ Ld,
-                                                 unsigned *__restrict__ used)
+                                                 double *__restrict__ Ld, int pitch,
+                                                 int *__restrict__ list, int *__restrict__ count)
 {
-    const int r = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (r >= n) return;
-    const int tile = r / SGM_ROWS, q = r - tile * SGM_ROWS;
-    for (int e = rp[r] + lane; e < rp[r + 1]; e += 64) {
-        const int k = ci[e];
-        Ld[((size_t)tile * (K + 1) + k) * SGM_ROWS + q] = v[e];
-        atomicOr(&used[(size_t)tile * kw + (k >> 5)], 1u << (k & 31));
+    extern __shared__ unsigned sgm_used[];
+    __shared__ int sh[BS / 64];
+    const int tile = blockIdx.x, wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    for (int t = threadIdx.x; t < kw; t += BS) sgm_used[t] = 0;
+    __syncthreads();
+    for (int q = wv; q < SGM_ROWS; q += BS / 64) {
+        const int r = tile * SGM_ROWS + q;
+        if (r >= n) break;
+        const int b = rp[r + 1];
+        for (int e = rp[r] + lane; e < b; e += 64) {
+            const int k = ci[e];
+            Ld[((size_t)tile * (K + 1) + k) * SGM_ROWS + q] = v[e];
+            atomicOr(&sgm_used[k >> 5], 1u << (k & 31));
+        }
     }
-}
-
-/* a tile's used k in ascending order, filled up to a multiple of SGM_AHEAD
-   with K (a row of zeros in Ld); a wavefront a tile */
-__global__ __launch_bounds__(64) void k_sgm_list(int K, int kw, const unsigned *__restrict__ used,
-                                                 int pitch, int *__restrict__ list,
-                                                 int *__restrict__ count)
-{
-    const int tile = blockIdx.x, lane = threadIdx.x;
+    __syncthreads();
     int *const o = list + (size_t)tile * pitch;
-    int at = 0;
-    for (int k0 = 0; k0 < K; k0 += 64) {
-        const int k = k0 + lane;
-        const bool in = k < K && ((used[(size_t)tile * kw + (k >> 5)] >> (k & 31)) & 1u);
-        const unsigned long long b = __ballot(in);
-        if (in) o[at + __popcll(b & ((1ull << lane) - 1))] = k;
-        at += __popcll(b);
+    int base = 0;
+    for (int t0 = 0; t0 < kw; t0 += BS) {
+        const int t = t0 + threadIdx.x;
+        unsigned w = t < kw ? sgm_used[t] : 0u;
+        int tot;
+        int at = base + block_scan_excl(__popc(w), sh, &tot);
+        for (; w; w &= w - 1) o[at++] = t * 32 + __builtin_ctz(w);
+        base += tot;
     }
-    const int end = (at + SGM_AHEAD - 1) / SGM_AHEAD * SGM_AHEAD;
-    if (lane < end - at) o[at + lane] = K;
-    if (lane == 0) count[tile] = end;
+    const int end = (base + SGM_AHEAD - 1) / SGM_AHEAD * SGM_AHEAD;
+    if ((int)threadIdx.x < end - base) o[base + threadIdx.x] = K;
+    if (threadIdx.x == 0) count[tile] = end;
 }
 
 /* C's rows: column bits (the union over the left entries), the number of
@@ -938,8 +940,9 @@ __global__ __launch_bounds__(BS) void k_sgm_pattern(int n, const int *__restrict
 
 /* The values: four wavefronts of a workgroup take four row tiles of the same
    128 columns (their right loads meet in L1); a left value is a scalar. The
-   multiplier bounds it: 2048 x 4096 x 2048, 1.6 ms, 21 of 39 T operations/s
-   (multiply and add apart). */
+   multiplier bounds it: 2048 x 4096 x 2048, 1.5 ms, 23 of 39 T operations/s
+   (multiply and add apart); eight rows a tile and four right rows ahead 1.6,
+   and 2.4 against 1.9 ms at 4096 columns. */
 __global__ __launch_bounds__(BS) void k_sgm_values(int n, int K, int mp, int mw, int tiles,
                                                    const int *__restrict__ list, int pitch,
                                                    const int *__restrict__ count,
@@ -1280,17 +1283,14 @@ void dense_product(Ctx &c, const CsrRef &L, const CsrRef &R, const int *uoff, in
     const int pitch = (K + SGM_AHEAD - 1) / SGM_AHEAD * SGM_AHEAD;
     DBuf<double> Rd((size_t)K * mp), Ld((size_t)tiles * (K + 1) * SGM_ROWS);
     DBuf<unsigned long long> rbits((size_t)K * mw), cbits((size_t)n * mw);
-    DBuf<unsigned> used((size_t)tiles * kw);
     DBuf<int> before((size_t)n * mw), list((size_t)tiles * pitch), count(tiles);
     BCMG_HIP(hipMemsetAsync(Rd.get(), 0, sizeof(double) * (size_t)K * mp, c.stream));
     BCMG_HIP(hipMemsetAsync(Ld.get(), 0, sizeof(double) * (size_t)tiles * (K + 1) * SGM_ROWS,
                             c.stream));
-    BCMG_HIP(hipMemsetAsync(used.get(), 0, sizeof(unsigned) * (size_t)tiles * kw, c.stream));
     k_sgm_right<<<(K + BS / 64 - 1) / (BS / 64), BS, (size_t)(BS / 64) * 2 * mw * sizeof(unsigned),
                   c.stream>>>(K, R.rp, R.ci, R.v, mp, mw, Rd.get(), rbits.get());
-    k_sgm_left<<<blocks_for(64ll * n), BS, 0, c.stream>>>(n, K, kw, L.rp, L.ci, L.v, Ld.get(),
-                                                          used.get());
-    k_sgm_list<<<tiles, 64, 0, c.stream>>>(K, kw, used.get(), pitch, list.get(), count.get());
+    k_sgm_left<<<tiles, BS, sizeof(unsigned) * kw, c.stream>>>(n, K, kw, L.rp, L.ci, L.v, Ld.get(),
+                                                               pitch, list.get(), count.get());
     k_sgm_pattern<<<blocks_for(64ll * n), BS, 0, c.stream>>>(n, L.rp, L.ci, mw, rbits.get(), uoff,
                                                              cbits.get(), before.get(), tcol, cnt);
     const int grid = (tiles + BS / 64 - 1) / (BS / 64) * (mp / 128);
@@ -1345,7 +1345,7 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
     DBuf<int> u(n), sl(n), ws(n), cnt(n), large(n);
     /* Dense operands when the filled parts of both multiply to 1 / SGM_FILL or
        more and either fits SGM_ELEMS: 0.28 and 0.094 (2048 rows) win 4.5 ->
-       2.2 and 5.6 -> 3.0 ms with all their preparation, 0.053 (1125 rows)
+       2.0 and 5.6 -> 2.4 ms with all their preparation, 0.053 (1125 rows)
        breaks even, 0.011 loses (48^3's products 5.2 -> 6.3 ms). */
     const bool fill = right_unique && left_sorted && n >= SGM_ROWS && mcols >= 128 &&
                       mcols <= SG_LDS_COLS &&

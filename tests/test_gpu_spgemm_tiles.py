@@ -71,8 +71,10 @@ def same(val, oval):
 
 
 @pytest.mark.parametrize("n,k,m,fl,fr,special", [
-    (8, 160, 128, 0.5, 0.5, True),        # one tile, one column block
-    (9, 161, 129, 0.6, 0.4, True),        # a row and a column beyond them
+    (16, 160, 128, 0.5, 0.5, True),       # one tile, one column block
+    (17, 161, 129, 0.6, 0.4, True),       # a row and a column beyond them
+    (8, 160, 128, 0.5, 0.5, True),        # fewer rows than a tile
+    (9, 161, 129, 0.6, 0.4, True),
     (67, 300, 1000, 0.9, 0.2, False),
     (130, 1025, 640, 0.3, 0.35, True),
     (40, 200, 300, 0.05, 0.9, False),     # below the fill that is taken
