@@ -100,6 +100,8 @@ def lib():
 
 
 PREC_FP64, PREC_FP32, PREC_BF16 = 0, 1, 2
+# bcmg_level_multi: steps of a multi-column cycle that share a launch
+MULTI_RESTRICT, MULTI_PAIRS, MULTI_SLAB = 1, 2, 4
 
 
 class SetupTimes(ctypes.Structure):
@@ -339,6 +341,12 @@ class Boot:
         nnz = ctypes.c_int()
         _check(lib().bcmg_level_size(self.h, k, l, ctypes.byref(n), ctypes.byref(nnz)))
         return n.value, nnz.value
+
+    def level_multi(self, k, l, columns):
+        """MULTI_* of level l's launches on blocks of `columns` right-hand sides."""
+        v = ctypes.c_int()
+        _check(lib().bcmg_level_multi(self.h, k, l, columns, ctypes.byref(v)))
+        return v.value
 
     def level_A(self, k, l):
         n, nnz = self.level_size(k, l)

@@ -626,7 +626,10 @@ bool launch_jacobi_il_cm(hipStream_t s, const DevCsr &A, MatType mt, const VT *x
 template <typename VT>
 void launch_jacobi_zero_il(hipStream_t s, int n, const VT *f, const VT *d, VT *y, int lkp,
                            int nc, const int *act);
-/* y = R (f - A x) on interleaved blocks in one launch; false: not launched */
+/* y = R (f - A x) on interleaved blocks in one launch; false: not launched
+   (il_resid_restrict_ok) */
+template <typename VT>
+bool il_resid_restrict_ok(const DevCsr &A, MatType mt, const DevCsr &R, int nc);
 template <typename VT>
 bool launch_il_resid_restrict(hipStream_t s, const DevCsr &A, MatType mt, const DevCsr &R,
                               const VT *x, const VT *f, VT *y, int lkp, int nc, const int *act);
@@ -873,6 +876,8 @@ int fcg_solve(Ctx &c, Boot &B, const double *b, double *x, int *iters, double *r
 /* k right-hand sides at once (device pointers b[j], x[j]); per column the
    iterations, final residual and status (BCMG_OK, BCMG_EZERORHS,
    BCMG_EBREAKDOWN) of fcg_solve on that column alone, bit for bit */
+/* BCMG_MULTI_* of level l of hierarchy k on blocks of nc columns */
+int level_launches_multi(const Boot &B, int k, int l, int nc);
 void fcg_multi(Ctx &c, Boot &B, int k, const double *const *b, double *const *x, int *iters,
                double *resid, int *status);
 double a_norm(Ctx &c, const DevCsr &A, const double *x, double *tmp);

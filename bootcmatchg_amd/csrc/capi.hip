@@ -760,6 +760,16 @@ int bcmg_level_Pcsr(bcmg_boot B, int k, int l, int *row, int *col, double *val)
     API_END
 }
 
+int bcmg_level_multi(bcmg_boot B, int k, int l, int columns, int *launches)
+{
+    if (!launches) return BCMG_EINVAL;
+    API_BEGIN
+    (void)get_level(B, k, l);
+    REQUIRE(columns >= 1 && columns <= MULTI_MAX_COLS, "columns: 1 to 32");
+    *launches = level_launches_multi(B->B, k, l, columns);
+    API_END
+}
+
 int bcmg_level_DM(bcmg_boot B, int k, int l, double *D, double *M, int *hasD, int *hasM)
 {
     API_BEGIN

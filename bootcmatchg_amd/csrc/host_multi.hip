@@ -424,6 +424,25 @@ void cycle_m(MRun<VT> &R, int l, const VT *fin)
                       top ? R.final_out : nullptr, pro);
 }
 
+/* BCMG_MULTI_* of a level's launches (the first visit of it) */
+template <typename VT>
+int level_launches_m(const Boot &B, const Hierarchy &H, int l, int nc)
+{
+    const Level &lv = H.L[l];
+    const DevCsr &A = lv.mat();
+    const MatType mt = level_mt(B, l);
+    const bool last = l + 1 == H.num_levels();
+    const int sweeps = last ? B.prm.relaxnumber_coarse : B.prm.prerelax_sweeps;
+    int out = 0;
+    if (il_slab_sweeps<VT>(A, mt, nc, sweeps - 1) > 0)
+        out |= BCMG_MULTI_SLAB;
+    else if (sweeps >= 2 && il_pair_ok<VT>(A, mt, nc) && !relax_block_ok<VT>(A))
+        out |= BCMG_MULTI_PAIRS;
+    if (!last && sweeps > 0 && il_resid_restrict_ok<VT>(A, mt, lv.R, nc))
+        out |= BCMG_MULTI_RESTRICT;
+    return out;
+}
+
 template <typename VT>
 void run_hierarchy_m(MRun<VT> &R, int k)
 {
@@ -841,6 +860,12 @@ void fcg_block(Ctx &c, Boot &B, int k, const double *const *b, double *const *x,
 }
 
 } // namespace
+
+int level_launches_multi(const Boot &B, int k, int l, int nc)
+{
+    return B.prec == BCMG_PREC_FP64 ? level_launches_m<double>(B, *B.H[k], l, nc)
+                                    : level_launches_m<float>(B, *B.H[k], l, nc);
+}
 
 void fcg_multi(Ctx &c, Boot &B, int k, const double *const *b, double *const *x, int *iters,
                double *resid, int *status)

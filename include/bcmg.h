@@ -206,6 +206,16 @@ int bcmg_boot_info(bcmg_boot B, int *n_hrc, double *estimated_ratio);
 /* number of levels of hierarchy k (AMG hierarchy->num_levels, AMG.cu:51) */
 int bcmg_hier_levels(bcmg_boot B, int k);
 int bcmg_level_size(bcmg_boot B, int k, int l, int *n, int *nnz);
+/* Which steps of level l of hierarchy k share a launch in the cycles of
+   bcmg_fcg_multi and of the serving loop on blocks of `columns` right-hand
+   sides (1 to 32): the sweeps before the coarse correction (on the coarsest
+   level: its sweeps) two in a pass over the block or several in a small level,
+   and the residual with its restriction. Results are the same bits in every
+   form. No counterpart in the reference: for measurements and tests. */
+#define BCMG_MULTI_RESTRICT 1
+#define BCMG_MULTI_PAIRS 2
+#define BCMG_MULTI_SLAB 4
+int bcmg_level_multi(bcmg_boot B, int k, int l, int columns, int *launches);
 /* hierarchy k's summary (AMG::Hierarchy::finalize_cmplx / finalize_wcmplx
    and the average coarsening ratio, src/AMG/AMG.cu:218-237,
    src/AMG/matchingAggregation.cu:330-333,406; printed by

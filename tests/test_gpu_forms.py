@@ -1,0 +1,40 @@
+"""The rules that choose a kernel form, seen through the library's queries."""
+import pytest
+
+import bootcmatchg_amd as bc
+from bootcmatchg_amd import operators as ops
+
+from common import SETTINGS
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    c = bc.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("make", [lambda: ops.poisson3d(20), lambda: ops.aniso2d(90, 0.05)])
+@pytest.mark.parametrize("prec,k", [(bc.PREC_FP64, 2), (bc.PREC_FP32, 4), (bc.PREC_FP32, 32)])
+def test_a_residual_is_formed_once(ctx, make, prec, k):
+    """The residual and its restriction share a launch, which forms a residual
+    for every entry of R, where R holds a fine row once at most: not with a
+    smoothed prolongator."""
+    dA = bc.Csr(ctx, make())
+    for aggrtype in (0, 1):
+        B = bc.Boot(ctx, dA, bc.make_params(**dict(SETTINGS["V_L1_2sweeps"], aggrtype=aggrtype)))
+        B.set_precision(prec)
+        entries = len(B.level_Pcsr(0, 0)[1])
+        assert (entries > dA.n) == (aggrtype == 1)
+        assert bool(B.level_multi(0, 0, k) & bc.MULTI_RESTRICT) == (aggrtype == 0)
+        B.free()
+    dA.free()
+
+
+def test_query_refuses_what_is_not_there(ctx):
+    B = bc.Boot(ctx, bc.Csr(ctx, ops.poisson2d(40)), bc.make_params())
+    for k, l, columns in [(1, 0, 4), (-1, 0, 4), (0, 99, 4), (0, 0, 0), (0, 0, 33)]:
+        with pytest.raises(bc.BcmgError):
+            B.level_multi(k, l, columns)
