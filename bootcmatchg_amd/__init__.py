@@ -100,6 +100,7 @@ def lib():
 
 
 PREC_FP64, PREC_FP32, PREC_BF16 = 0, 1, 2
+COLUMNS_ANY = -1
 # bcmg_level_multi: steps of a multi-column cycle that share a launch
 MULTI_RESTRICT, MULTI_PAIRS, MULTI_SLAB = 1, 2, 4
 
@@ -251,7 +252,8 @@ class Csr:
 
     def set_columns(self, nbytes):
         """Restrict the row kernels to a column form: 0 the stencil pattern,
-        2 the 16-bit offsets, 4 the int32 columns (same results)."""
+        2 the 16-bit offsets, 4 the int32 columns (same results);
+        COLUMNS_ANY lifts the restriction."""
         _check(lib().bcmg_csr_set_columns(self.h, nbytes))
 
     def download(self):

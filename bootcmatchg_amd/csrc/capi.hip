@@ -419,6 +419,8 @@ int bcmg_csr_set_columns(bcmg_csr A, int bytes)
             return BCMG_EUNSUP;
         }
         A->A.col_mode = 2;
+    } else if (bytes == BCMG_COLUMNS_ANY) {
+        A->A.col_mode = 3;
     } else {
         return BCMG_EINVAL;
     }

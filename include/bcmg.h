@@ -111,9 +111,10 @@ int bcmg_csr_column_bytes(bcmg_csr A, int *bytes);
 /* Restricts the row kernels on A to a column form, in place of its row classes
    or symmetric stencil too: bytes 0 (the pattern),
    2 (the 16-bit offsets) or 4 (the int32 columns); BCMG_EUNSUP when A has no
-   such copy. Composites set up on A before the call keep the launches they
+   such copy; BCMG_COLUMNS_ANY lifts the restriction. Composites set up on A before the call keep the launches they
    captured. No counterpart in the reference: for A/B measurements and tests
    of the column forms. */
+#define BCMG_COLUMNS_ANY (-1)
 int bcmg_csr_set_columns(bcmg_csr A, int bytes);
 /* Replaces CSRm::free (src/matrix/CSR.cu:160-181). */
 int bcmg_csr_free(bcmg_csr A);

@@ -38,3 +38,15 @@ def test_query_refuses_what_is_not_there(ctx):
     for k, l, columns in [(1, 0, 4), (-1, 0, 4), (0, 99, 4), (0, 0, 0), (0, 0, 33)]:
         with pytest.raises(bc.BcmgError):
             B.level_multi(k, l, columns)
+
+
+def test_a_restriction_to_a_column_form_is_lifted(ctx):
+    """bcmg_csr_set_columns(4) hides the narrower forms, BCMG_COLUMNS_ANY gives
+    them back."""
+    dA = bc.Csr(ctx, ops.poisson3d(120))
+    assert dA.column_bytes == 0
+    dA.set_columns(4)
+    assert dA.column_bytes == 4
+    dA.set_columns(bc.COLUMNS_ANY)
+    assert dA.column_bytes == 0
+    dA.free()
