@@ -101,6 +101,7 @@ def lib():
 
 PREC_FP64, PREC_FP32, PREC_BF16 = 0, 1, 2
 COLUMNS_ANY = -1
+FORM_COLUMNS, FORM_CLASSES, FORM_STENCIL, FORM_SYMMETRIC = 0, 1, 2, 3
 # bcmg_level_multi: steps of a multi-column cycle that share a launch
 MULTI_RESTRICT, MULTI_PAIRS, MULTI_SLAB = 1, 2, 4
 
@@ -244,11 +245,20 @@ class Csr:
 
     @property
     def column_bytes(self):
-        """Bytes per column index the streamed row kernels read (0 with the
-        stencil pattern, 2 with the 16-bit column-minus-row copy, else 4)."""
+        """Bytes per column index of the narrowest column copy (0 with the
+        stencil pattern, 2 with the 16-bit column-minus-row copy, else 4);
+        the row kernels read it when `form` is FORM_COLUMNS."""
         b = ctypes.c_int()
         _check(lib().bcmg_csr_column_bytes(self.h, ctypes.byref(b)))
         return b.value
+
+    @property
+    def form(self):
+        """What the FP64 row kernels read: FORM_COLUMNS (values and columns),
+        FORM_CLASSES, FORM_STENCIL or FORM_SYMMETRIC."""
+        f = ctypes.c_int()
+        _check(lib().bcmg_csr_form(self.h, ctypes.byref(f)))
+        return f.value
 
     def set_columns(self, nbytes):
         """Restrict the row kernels to a column form: 0 the stencil pattern,

@@ -402,6 +402,16 @@ int bcmg_csr_column_bytes(bcmg_csr A, int *bytes)
     return BCMG_OK;
 }
 
+int bcmg_csr_form(bcmg_csr A, int *form)
+{
+    if (!A || !form) return BCMG_EINVAL;
+    const DevCsr &M = A->A;
+    *form = class_ok<double>(M, MT_F64) ? (M.cls.k > 0 ? BCMG_FORM_STENCIL : BCMG_FORM_CLASSES)
+            : sym_ok<double>(M, MT_F64) ? BCMG_FORM_SYMMETRIC
+                                        : BCMG_FORM_COLUMNS;
+    return BCMG_OK;
+}
+
 int bcmg_csr_set_columns(bcmg_csr A, int bytes)
 {
     if (!A) return BCMG_EINVAL;

@@ -97,17 +97,28 @@ int bcmg_csr_info(bcmg_csr A, int *n, int *nnz);
    (an FP64 stream above 192 MB), and a stencil pattern when it has more
    than 11.2 M entries (above 128 MB) and its offsets take at most 8
    distinct values (one byte per row: which offsets of a sorted table the
-   row has). An operator whose rows take few distinct forms, or that is
-   symmetric with few offsets, is read from those instead (a byte per row;
-   see bcmg_csr_set_columns); otherwise the row kernels read the narrowest
-   copy that is kept: 0 the
-   pattern (no per-entry column bytes, one byte per row, and only two row
-   pointers per 256 rows), 2 the 16-bit offsets (FP32/BF16 value copies use
-   them when their 32-bit-column stream also exceeds 192 MB), else 4.
+   row has): 0 the pattern (no per-entry column bytes, one byte per row, and
+   only two row pointers per 256 rows), 2 the 16-bit offsets (FP32/BF16 value
+   copies use them when their 32-bit-column stream also exceeds 192 MB), else
+   4. The row kernels read the narrowest copy that is kept unless
+   bcmg_csr_form tells another form, which goes before them.
    Results are the same bits in every form. No counterpart in the reference
-   (which always streams 32-bit columns); it lets a caller price a kernel's
-   memory traffic. */
+   (which always streams 32-bit columns). */
 int bcmg_csr_column_bytes(bcmg_csr A, int *bytes);
+/* What the FP64 row kernels read for A; with bcmg_csr_column_bytes it lets a
+   caller price their memory traffic. BCMG_FORM_COLUMNS: values, columns of
+   bcmg_csr_column_bytes each and row pointers. BCMG_FORM_CLASSES: a byte per
+   row, the class of its form, and a table of the forms (a few KB).
+   BCMG_FORM_STENCIL: a byte per row, the mask of its entries in a constant
+   stencil. BCMG_FORM_SYMMETRIC: a byte per row and the values of the diagonal
+   and of the upper diagonals. In the last three a sweep of a hierarchy's L1 or
+   diagonal divisor reads no divisor array (with BCMG_FORM_SYMMETRIC: the L1
+   one). No counterpart in the reference. */
+#define BCMG_FORM_COLUMNS 0
+#define BCMG_FORM_CLASSES 1
+#define BCMG_FORM_STENCIL 2
+#define BCMG_FORM_SYMMETRIC 3
+int bcmg_csr_form(bcmg_csr A, int *form);
 /* Restricts the row kernels on A to a column form, in place of its row classes
    or symmetric stencil too: bytes 0 (the pattern),
    2 (the 16-bit offsets) or 4 (the int32 columns); BCMG_EUNSUP when A has no

@@ -5,6 +5,7 @@ import bootcmatchg_amd as bc
 from bootcmatchg_amd import operators as ops
 
 from common import SETTINGS
+from test_gpu_classes import neumann2d
 
 pytestmark = pytest.mark.gpu
 
@@ -50,3 +51,19 @@ def test_a_restriction_to_a_column_form_is_lifted(ctx):
     dA.set_columns(bc.COLUMNS_ANY)
     assert dA.column_bytes == 0
     dA.free()
+
+
+def test_the_form_that_the_row_kernels_read(ctx):
+    """bcmg_csr_form names the form, restricted and not, also where no narrow
+    column copy is kept (below 11.2 M entries bcmg_csr_column_bytes says 4)."""
+    for make, form in [(lambda: ops.poisson3d(24), bc.FORM_STENCIL),
+                       (lambda: neumann2d(70), bc.FORM_CLASSES),
+                       (lambda: ops.lognormal3d(33, 4.0, seed=2), bc.FORM_SYMMETRIC),
+                       (lambda: ops.lognormal3d(18, 4.0, seed=1), bc.FORM_COLUMNS)]:
+        dA = bc.Csr(ctx, make())
+        assert dA.form == form and dA.column_bytes == 4
+        dA.set_columns(4)
+        assert dA.form == bc.FORM_COLUMNS
+        dA.set_columns(bc.COLUMNS_ANY)
+        assert dA.form == form
+        dA.free()
