@@ -364,14 +364,29 @@ def spmv_bytes(n, nnz, cb=4):
     return (8 + cb) * nnz + 4 * (n + 1) + 2 * 8 * n
 
 
-def streamed_bytes(n, nnz, cb, vectors):
-    """Bytes a level-0 row kernel streams on this constant-coefficient operator:
-    (cb = 0) the mask byte of each row, offsets and values being kernel
-    arguments, else 8-byte values, cb-byte columns and the row pointers; plus
-    `vectors` 8-byte vectors of n."""
+# bcmg_csr_form's values
+FORM_COLUMNS, FORM_CLASSES, FORM_STENCIL, FORM_SYMMETRIC = range(4)
+
+
+def streamed_bytes(n, nnz, form, cb, vectors):
+    """Bytes a level-0 row kernel streams: `vectors` 8-byte vectors of n and, by
+    the operator's form, one byte per row (row classes, constant stencil), that
+    and the values of the diagonal and the upper diagonals (symmetric stencil),
+    or 8-byte values with one byte per row and two row pointers per 256 rows
+    (cb = 0) or cb-byte columns and a row pointer per row."""
+    v = vectors * 8 * n
+    if form in (FORM_CLASSES, FORM_STENCIL):
+        return n + v
+    if form == FORM_SYMMETRIC:
+        return n + 8 * (n + (nnz - n) // 2) + v
     if cb == 0:
-        return n + vectors * 8 * n
-    return (8 + cb) * nnz + 4 * (n + 1) + vectors * 8 * n
+        return 8 * nnz + n + 8 * ((n + 255) // 256) + v
+    return (8 + cb) * nnz + 4 * (n + 1) + v
+
+
+def sweep_vectors(form):
+    """The vectors of an L1 sweep: u, f, u' and, from the columns, the divisor."""
+    return 4 if form == FORM_COLUMNS else 3
 
 
 # Measured HBM bytes per level-0 SpMV launch at 160^3 (same PMC runs and
@@ -573,7 +588,7 @@ def main():
     # fine-level SpMV bandwidth (algorithmic bytes / event-timed launch)
     dy = bc.DeviceArray(ctx, n)
     spmv_ms = bc.time_spmv(ctx, dA, db, dy, 50)
-    cb = dA.column_bytes
+    form, cb = dA.form, dA.column_bytes
     # algorithmic bytes count 32-bit columns (the operator's own format); the
     # library reads a constant stencil here and moves far fewer, so rates
     # against the HBM peak are of the streamed bytes
@@ -594,8 +609,7 @@ def main():
 
     sweep_avg_ms = sm_ms / max(sm_launches, 1)
     sweep_b = sweep_bytes(n, nnz)
-    # the sweep's vectors: u, f, u' (the divisor is the mask's)
-    sweep_s = streamed_bytes(n, nnz, cb, 3 if cb == 0 else 4)
+    sweep_s = streamed_bytes(n, nnz, form, cb, sweep_vectors(form))
     achieved = sweep_s / (sweep_avg_ms * 1e-3) / 1e9
 
     cpu = None
@@ -666,27 +680,28 @@ def main():
         "true_rel_residual": true_rel,
         "cached_hierarchy_solves_per_s": args.steps / (tc1 - tc0),
         "spmv_gbs": spmv_gbs,
-        "spmv_frac_of_hbm": streamed_bytes(n, nnz, cb, 2) / (spmv_ms * 1e-3) / 1e9
+        "spmv_frac_of_hbm": streamed_bytes(n, nnz, form, cb, 2) / (spmv_ms * 1e-3) / 1e9
                             / HBM_PEAK_GBS,
         "spmv": {"kernel": "level-0 y = A x (k_rows_stencil<OP_SPMV> on a constant stencil, "
                            "else k_rows_staged<OP_SPMV>)",
                  "bytes_per_launch": spmv_bytes(n, nnz), "avg_launch_ms": spmv_ms,
-                 "achieved_gbs": spmv_gbs, "column_bytes": cb,
-                 "streamed_bytes_per_launch": streamed_bytes(n, nnz, cb, 2),
-                 "traffic_bytes": SPMV_TRAFFIC_BYTES_160 if (N == GRID and cb == 0) else None,
-                 "working_set_bytes": streamed_bytes(n, nnz, cb, 2), "mall_bytes": MALL_BYTES},
+                 "achieved_gbs": spmv_gbs, "column_bytes": cb, "form": form,
+                 "streamed_bytes_per_launch": streamed_bytes(n, nnz, form, cb, 2),
+                 "traffic_bytes": SPMV_TRAFFIC_BYTES_160 if (N == GRID and form == FORM_STENCIL) else None,
+                 "working_set_bytes": streamed_bytes(n, nnz, form, cb, 2), "mall_bytes": MALL_BYTES},
         "solve_roofline": solve_rl,
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": SWEEP_TRAFFIC_BYTES_160 if (N == GRID and cb == 0) else None,
+                     "traffic": SWEEP_TRAFFIC_BYTES_160 if (N == GRID and form == FORM_STENCIL) else None,
                      "kernel": "level-0 Jacobi/L1 sweep (k_rows_stencil<OP_JACOBI> on a constant "
                                "stencil, else k_rows_staged<OP_JACOBI>)",
                      "bytes_per_launch": sweep_b, "avg_launch_ms": sweep_avg_ms,
-                     "launches": sm_launches, "column_bytes": cb,
+                     "launches": sm_launches, "column_bytes": cb, "form": form,
                      "streamed_bytes_per_launch": sweep_s,
                      "algorithmic_gbs": sweep_b / (sweep_avg_ms * 1e-3) / 1e9,
-                     "note": "achieved = streamed_bytes_per_launch (one mask byte per row, u "
-                             "gathered once, f, u') / event-timed launch; bytes_per_launch "
+                     "note": "achieved = streamed_bytes_per_launch (the form that is read, 2: one "
+                             "mask byte per row; u gathered once, f, u') / event-timed "
+                             "launch; bytes_per_launch "
                              "is the reference algorithm's count (8-byte values, 32-bit "
                              "columns, row pointers, four vectors), algorithmic_gbs its "
                              "rate; traffic is the measured HBM bytes"},
