@@ -4,6 +4,7 @@
  */
 #pragma once
 #include "bcmg_internal.h"
+#include "rows.h"
 
 #include <cmath>
 

@@ -130,8 +130,7 @@ __global__ __launch_bounds__(BS) void k_rows_multi_g(int n, int G, const int *__
                                                      const int *__restrict__ act)
 {
     const int b = xcd_block(blockIdx.x, gridDim.x);
-    const int tid = b * BS + threadIdx.x;
-    const int row = tid / G;
+    const int row = group_row(b, threadIdx.x, G);
     const int lane = threadIdx.x & (G - 1);
     if (row >= n) return;
     const int j0 = rp[row], j1 = rp[row + 1];
@@ -803,8 +802,7 @@ __global__ __launch_bounds__(BS) void k_rows_il_g(int n, int G, const int *__res
                                                   int lkp, int nc, const int *__restrict__ act)
 {
     const int b = xcd_block(blockIdx.x, gridDim.x);
-    const int tid = b * BS + threadIdx.x;
-    const int row = tid / G;
+    const int row = group_row(b, threadIdx.x, G);
     const int lane = threadIdx.x & (G - 1);
     if (row >= n) return;
     const int j0 = rp[row], j1 = rp[row + 1];

@@ -736,8 +736,7 @@ __global__ __launch_bounds__(BS) void k_stage(int n, const int *__restrict__ rp,
                                               const int *__restrict__ stoff,
                                               int *__restrict__ Jst, double *__restrict__ tst)
 {
-    const int tid = blockIdx.x * BS + threadIdx.x;
-    const int i = tid / G;
+    const int i = group_row(blockIdx.x, threadIdx.x, G);
     const int lane = threadIdx.x & (G - 1);
     if (i >= n) return;
     const int I = agg[i];
@@ -761,8 +760,7 @@ __global__ __launch_bounds__(BS) void k_rap_count(int nc, const int *__restrict_
                                                   unsigned char *__restrict__ first,
                                                   int *__restrict__ cnt)
 {
-    const int tid = blockIdx.x * BS + threadIdx.x;
-    const int I = tid / G;
+    const int I = group_row(blockIdx.x, threadIdx.x, G);
     const int lane = threadIdx.x & (G - 1);
     if (I >= nc) return; /* the whole group: its lanes share I */
     const int s0 = stoff[I], s1 = stoff[I + 1];
@@ -812,8 +810,7 @@ __global__ __launch_bounds__(BS) void k_rap_fill(int nc, const int *__restrict__
                                                  const int *__restrict__ rpc,
                                                  int *__restrict__ colc, double *__restrict__ valc)
 {
-    const int tid = blockIdx.x * BS + threadIdx.x;
-    const int I = tid / G;
+    const int I = group_row(blockIdx.x, threadIdx.x, G);
     const int lane = threadIdx.x & (G - 1);
     if (I >= nc) return; /* the whole group: its lanes share I */
     const int s0 = stoff[I], s1 = stoff[I + 1];

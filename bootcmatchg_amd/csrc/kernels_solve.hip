@@ -405,8 +405,7 @@ __global__ __launch_bounds__(BS) void k_rows(int n, const int *__restrict__ rp,
                                              VT *__restrict__ y)
 {
     const int b = xcd_block(blockIdx.x, gridDim.x);
-    const int tid = b * BS + threadIdx.x;
-    const int row = tid / G;
+    const int row = group_row(b, threadIdx.x, G);
     const int lane = threadIdx.x & (G - 1);
     if (row >= n) return;
     const int j0 = rp[row], j1 = rp[row + 1];

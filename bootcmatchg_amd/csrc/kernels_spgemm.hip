@@ -1011,8 +1011,7 @@ __global__ __launch_bounds__(BS) void k_sg_gather(int n, const int *__restrict__
                                                   int *__restrict__ ccol,
                                                   double *__restrict__ cval)
 {
-    const int tid = blockIdx.x * BS + threadIdx.x;
-    const int row = tid / G;
+    const int row = group_row(blockIdx.x, threadIdx.x, G);
     const int lane = threadIdx.x & (G - 1);
     if (row >= n) return;
     const int s = uoff[row], d = Crp[row], len = Crp[row + 1] - d;
