@@ -121,24 +121,24 @@ __global__ __launch_bounds__(BS) void k_diag(int n, const int *__restrict__ rp,
                                              const double *__restrict__ av,
                                              double *__restrict__ D)
 {
-    const int i = (blockIdx.x * BS + threadIdx.x) / G;
-    if (i >= n) return;
-    const int a = rp[i], b = rp[i + 1];
-    if (G == 1) {
-        double d = 0.0;
-        for (int j = a; j < b; j++)
-            if (ci[j] == i) d = av[j];
-        D[i] = d;
-        return;
-    }
     const int lane = threadIdx.x & (G - 1);
-    int at = -1;
-    for (int j0 = a; j0 < b; j0 += G) {
-        const int j = j0 + lane;
-        const unsigned long long hit = __ballot(j < b && ci[j] == i);
-        if (hit) at = j0 + 63 - __clzll(hit);
+    for (long long i = group_row(blockIdx.x, threadIdx.x, G); i < n; i += row_step(gridDim.x, G)) {
+        const int a = rp[i], b = rp[i + 1];
+        if (G == 1) {
+            double d = 0.0;
+            for (int j = a; j < b; j++)
+                if (ci[j] == i) d = av[j];
+            D[i] = d;
+            continue;
+        }
+        int at = -1;
+        for (int j0 = a; j0 < b; j0 += G) {
+            const int j = j0 + lane;
+            const unsigned long long hit = __ballot(j < b && ci[j] == i);
+            if (hit) at = j0 + 63 - __clzll(hit);
+        }
+        if (lane == 0) D[i] = at >= 0 ? av[at] : 0.0;
     }
-    if (lane == 0) D[i] = at >= 0 ? av[at] : 0.0;
 }
 
 /* sum_j |a_ij| in CSR order (src/matrix/CSR.cu:638-652) */
@@ -147,21 +147,21 @@ __global__ __launch_bounds__(BS) void k_abs_rowsum(int n, const int *__restrict_
                                                    const double *__restrict__ av,
                                                    double *__restrict__ M)
 {
-    const int i = (blockIdx.x * BS + threadIdx.x) / G;
-    if (i >= n) return;
-    const int a = rp[i], b = rp[i + 1];
-    double s = 0.0;
-    if (G == 1) {
-        for (int j = a; j < b; j++) s += fabs(av[j]);
-        M[i] = s;
-        return;
-    }
     const int lane = threadIdx.x & (G - 1);
-    for (int j0 = a; j0 < b; j0 += G) {
-        const int j = j0 + lane;
-        s = add_lanes_in_order(s, j < b ? fabs(av[j]) : 0.0, b - j0);
+    for (long long i = group_row(blockIdx.x, threadIdx.x, G); i < n; i += row_step(gridDim.x, G)) {
+        const int a = rp[i], b = rp[i + 1];
+        double s = 0.0;
+        if (G == 1) {
+            for (int j = a; j < b; j++) s += fabs(av[j]);
+            M[i] = s;
+            continue;
+        }
+        for (int j0 = a; j0 < b; j0 += G) {
+            const int j = j0 + lane;
+            s = add_lanes_in_order(s, j < b ? fabs(av[j]) : 0.0, b - j0);
+        }
+        if (lane == 0) M[i] = s;
     }
-    if (lane == 0) M[i] = s;
 }
 
 /* ------------------------------------------------------ matching weights */
@@ -994,8 +994,8 @@ long long exclusive_scan(Ctx &c, const int *in, int *out, int n, bool read_total
 void launch_diag(hipStream_t s, const DevCsr &A, double *D)
 {
     if (long_rows(A.n, A.nnz))
-        k_diag<64><<<blocks_for(64ll * A.n), BS, 0, s>>>(A.n, A.row.get(), A.col.get(),
-                                                         A.val.get(), D);
+        k_diag<64><<<group_blocks(A.n, 64), BS, 0, s>>>(A.n, A.row.get(), A.col.get(),
+                                                        A.val.get(), D);
     else
         k_diag<1><<<blocks_for(A.n), BS, 0, s>>>(A.n, A.row.get(), A.col.get(), A.val.get(), D);
     BCMG_CHECK_LAUNCH();
@@ -1004,7 +1004,7 @@ void launch_diag(hipStream_t s, const DevCsr &A, double *D)
 void launch_abs_rowsum(hipStream_t s, const DevCsr &A, double *M)
 {
     if (long_rows(A.n, A.nnz))
-        k_abs_rowsum<64><<<blocks_for(64ll * A.n), BS, 0, s>>>(A.n, A.row.get(), A.val.get(), M);
+        k_abs_rowsum<64><<<group_blocks(A.n, 64), BS, 0, s>>>(A.n, A.row.get(), A.val.get(), M);
     else
         k_abs_rowsum<1><<<blocks_for(A.n), BS, 0, s>>>(A.n, A.row.get(), A.val.get(), M);
     BCMG_CHECK_LAUNCH();

@@ -677,16 +677,18 @@ __global__ __launch_bounds__(BS) void k_sg_seg(int n, const int *__restrict__ rp
                                                const int *__restrict__ ci, int W, int nt,
                                                int *__restrict__ seg)
 {
-    const int row = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (row >= n) return;
-    int *const o = seg + (long long)row * (nt + 1);
-    const int a = rp[row], b = rp[row + 1];
-    for (int f = a + lane; f < b; f += 64) {
-        const int t0 = f > a ? ci[f - 1] / W + 1 : 0, t1 = ci[f] / W;
-        for (int t = t0; t <= t1; t++) o[t] = f;
+    const int lane = threadIdx.x & 63;
+    for (long long row = group_row(blockIdx.x, threadIdx.x, 64); row < n;
+         row += row_step(gridDim.x, 64)) {
+        int *const o = seg + row * (nt + 1);
+        const int a = rp[row], b = rp[row + 1];
+        for (int f = a + lane; f < b; f += 64) {
+            const int t0 = f > a ? ci[f - 1] / W + 1 : 0, t1 = ci[f] / W;
+            for (int t = t0; t <= t1; t++) o[t] = f;
+        }
+        const int last = b > a ? ci[b - 1] / W + 1 : 0;
+        for (int t = last + lane; t <= nt; t += 64) o[t] = b;
     }
-    const int last = b > a ? ci[b - 1] / W + 1 : 0;
-    for (int t = last + lane; t <= nt; t += 64) o[t] = b;
 }
 
 /* Long rows when C's columns fit LDS: a workgroup a row, a wavefront a column
@@ -899,7 +901,7 @@ __global__ __launch_bounds__(BS) void k_sgm_pattern(int n, const int *__restrict
                                                     int *__restrict__ before,
                                                     int *__restrict__ tcol, int *__restrict__ cnt)
 {
-    const int r = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
+    const int r = group_row(blockIdx.x, threadIdx.x, 64), lane = threadIdx.x & 63;
     if (r >= n) return;
     const int a = rp[r], b = rp[r + 1];
     int base = 0;
@@ -1029,10 +1031,11 @@ __global__ __launch_bounds__(BS) void k_col_count(int n, const int *__restrict__
                                                   const int *__restrict__ ci,
                                                   int *__restrict__ cnt)
 {
-    const int i = (blockIdx.x * BS + threadIdx.x) / G;
-    if (i >= n) return;
-    const int b = rp[i + 1];
-    for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) atomicAdd(&cnt[ci[e]], 1);
+    for (long long i = group_row(blockIdx.x, threadIdx.x, G); i < n; i += row_step(gridDim.x, G)) {
+        const int b = rp[i + 1];
+        for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G)
+            atomicAdd(&cnt[ci[e]], 1);
+    }
 }
 
 template <int G>
@@ -1042,13 +1045,13 @@ __global__ __launch_bounds__(BS) void k_col_fill(int n, const int *__restrict__ 
                                                  int *__restrict__ cursor, int *__restrict__ tcol,
                                                  double *__restrict__ tval)
 {
-    const int i = (blockIdx.x * BS + threadIdx.x) / G;
-    if (i >= n) return;
-    const int b = rp[i + 1];
-    for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) {
-        const int pos = atomicAdd(&cursor[ci[e]], 1);
-        tcol[pos] = i;
-        tval[pos] = v[e];
+    for (long long i = group_row(blockIdx.x, threadIdx.x, G); i < n; i += row_step(gridDim.x, G)) {
+        const int b = rp[i + 1];
+        for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) {
+            const int pos = atomicAdd(&cursor[ci[e]], 1);
+            tcol[pos] = (int)i;
+            tval[pos] = v[e];
+        }
     }
 }
 
@@ -1063,36 +1066,38 @@ __global__ __launch_bounds__(BS) void k_rank(int nr, const int *__restrict__ rp,
                                              int *__restrict__ col, double *__restrict__ val,
                                              int *__restrict__ longl, int *__restrict__ nlong)
 {
-    const int I = (blockIdx.x * BS + threadIdx.x) >> 6, lane = threadIdx.x & 63;
-    if (I >= nr) return;
-    const int a = rp[I], len = rp[I + 1] - a;
-    if (len > WAVE_RANK) {
-        if (lane == 0) longl[atomicAdd(nlong, 1)] = I;
-        return;
-    }
     constexpr int Q = WAVE_RANK / 64;
-    int c[Q], rank[Q];
-#pragma unroll
-    for (int q = 0; q < Q; q++) {
-        c[q] = q * 64 + lane < len ? cin[a + q * 64 + lane] : INT_MAX;
-        rank[q] = 0;
-    }
-#pragma unroll
-    for (int f = 0; f < Q; f++) {
-        if (f * 64 >= len) break;
-        const int nf = min(64, len - f * 64);
-        for (int t = 0; t < nf; t++) {
-            const int d = __builtin_amdgcn_readlane(c[f], t);
-#pragma unroll
-            for (int q = 0; q < Q; q++) rank[q] += d < c[q] ? 1 : 0;
+    const int lane = threadIdx.x & 63;
+    for (long long I = group_row(blockIdx.x, threadIdx.x, 64); I < nr;
+         I += row_step(gridDim.x, 64)) {
+        const int a = rp[I], len = rp[I + 1] - a;
+        if (len > WAVE_RANK) {
+            if (lane == 0) longl[atomicAdd(nlong, 1)] = (int)I;
+            continue;
         }
-    }
+        int c[Q], rank[Q];
 #pragma unroll
-    for (int q = 0; q < Q; q++)
-        if (q * 64 + lane < len) {
-            col[a + rank[q]] = c[q];
-            val[a + rank[q]] = vin[a + q * 64 + lane];
+        for (int q = 0; q < Q; q++) {
+            c[q] = q * 64 + lane < len ? cin[a + q * 64 + lane] : INT_MAX;
+            rank[q] = 0;
         }
+#pragma unroll
+        for (int f = 0; f < Q; f++) {
+            if (f * 64 >= len) break;
+            const int nf = min(64, len - f * 64);
+            for (int t = 0; t < nf; t++) {
+                const int d = __builtin_amdgcn_readlane(c[f], t);
+#pragma unroll
+                for (int q = 0; q < Q; q++) rank[q] += d < c[q] ? 1 : 0;
+            }
+        }
+#pragma unroll
+        for (int q = 0; q < Q; q++)
+            if (q * 64 + lane < len) {
+                col[a + rank[q]] = c[q];
+                val[a + rank[q]] = vin[a + q * 64 + lane];
+            }
+    }
 }
 
 /* A long row per workgroup, m columns. Up to RANK_BITS of them: the row's
@@ -1216,13 +1221,13 @@ __global__ __launch_bounds__(BS) void k_sa_omega(int n, const int *__restrict__ 
                                                  const int *__restrict__ ci, double omega,
                                                  double *__restrict__ sv)
 {
-    const int i = (blockIdx.x * BS + threadIdx.x) / G;
-    if (i >= n) return;
-    const int b = rp[i + 1];
-    for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) {
-        double t = -omega * sv[e];
-        if (ci[e] == i) t += 1.;
-        sv[e] = t;
+    for (long long i = group_row(blockIdx.x, threadIdx.x, G); i < n; i += row_step(gridDim.x, G)) {
+        const int b = rp[i + 1];
+        for (int e = rp[i] + (int)(threadIdx.x & (G - 1)); e < b; e += G) {
+            double t = -omega * sv[e];
+            if (ci[e] == i) t += 1.;
+            sv[e] = t;
+        }
     }
 }
 
@@ -1290,7 +1295,7 @@ void dense_product(Ctx &c, const CsrRef &L, const CsrRef &R, const int *uoff, in
                   c.stream>>>(K, R.rp, R.ci, R.v, mp, mw, Rd.get(), rbits.get());
     k_sgm_left<<<tiles, BS, sizeof(unsigned) * kw, c.stream>>>(n, K, kw, L.rp, L.ci, L.v, Ld.get(),
                                                                pitch, list.get(), count.get());
-    k_sgm_pattern<<<blocks_for(64ll * n), BS, 0, c.stream>>>(n, L.rp, L.ci, mw, rbits.get(), uoff,
+    k_sgm_pattern<<<(n + BS / 64 - 1) / (BS / 64), BS, 0, c.stream>>>(n, L.rp, L.ci, mw, rbits.get(), uoff,
                                                              cbits.get(), before.get(), tcol, cnt);
     const int grid = (tiles + BS / 64 - 1) / (BS / 64) * (mp / 128);
     k_sgm_values<<<grid, BS, 0, c.stream>>>(n, K, mp, mw, tiles, list.get(), pitch, count.get(),
@@ -1477,7 +1482,7 @@ void spgemm(Ctx &c, const CsrRef &L, const CsrRef &R, DevCsr &C, long long per_p
             auto wave = [&](int least, int only_left) {
                 if (!seg.get()) {
                     seg.alloc((size_t)R.n * (tiles + 1));
-                    k_sg_seg<<<blocks_for(64ll * R.n), BS, 0, c.stream>>>(R.n, R.rp, R.ci, tile_w,
+                    k_sg_seg<<<group_blocks(R.n, 64), BS, 0, c.stream>>>(R.n, R.rp, R.ci, tile_w,
                                                                           tiles, seg.get());
                 }
                 /* mostly long rows: by row, which keeps their order (the list
@@ -1578,7 +1583,7 @@ void transpose_csr(Ctx &c, const CsrRef &A, DevCsr &T)
     BCMG_HIP(hipMemsetAsync(cnt.get(), 0, sizeof(int) * (nr > 0 ? nr : 1), c.stream));
     BCMG_HIP(hipMemsetAsync(nlong.get(), 0, sizeof(int), c.stream));
     const bool lng = long_rows(A.n, A.nnz);
-    const int gb = blocks_for(lng ? 64ll * A.n : A.n);
+    const int gb = group_blocks(A.n, lng ? 64 : 1);
     if (A.n > 0)
         (lng ? k_col_count<64> : k_col_count<1>)<<<gb, BS, 0, c.stream>>>(A.n, A.rp, A.ci,
                                                                           cnt.get());
@@ -1590,7 +1595,7 @@ void transpose_csr(Ctx &c, const CsrRef &A, DevCsr &T)
         (lng ? k_col_fill<64> : k_col_fill<1>)<<<gb, BS, 0, c.stream>>>(
             A.n, A.rp, A.ci, A.v, cursor.get(), fcol.get(), fval.get());
     if (nr > 0)
-        k_rank<<<blocks_for(64ll * nr), BS, 0, c.stream>>>(nr, T.row.get(), fcol.get(),
+        k_rank<<<group_blocks(nr, 64), BS, 0, c.stream>>>(nr, T.row.get(), fcol.get(),
                                                            fval.get(), T.col.get(), T.val.get(),
                                                            longl.get(), nlong.get());
     BCMG_CHECK_LAUNCH();
@@ -1612,7 +1617,7 @@ double sa_smoother(Ctx &c, const DevCsr &A, const double *D, DBuf<double> &S)
     DBuf<unsigned long long> nb(1);
     BCMG_HIP(hipMemsetAsync(nb.get(), 0, sizeof(unsigned long long), c.stream));
     const bool lng = long_rows(n, A.nnz);
-    const int gb = blocks_for(lng ? 64ll * n : n);
+    const int gb = group_blocks(n, lng ? 64 : 1);
     const int per = rows_per_block(n, lng);
     (lng ? k_sa_scale<64> : k_sa_scale<1>)<<<(n + per - 1) / per, BS, 0, c.stream>>>(
         n, per, A.row.get(), A.val.get(), D, S.get(), nb.get());

@@ -17,4 +17,19 @@ constexpr int group_row(unsigned block, unsigned thread, int G)
     return (int)(block * (unsigned)(ROW_BS / G) + thread / (unsigned)G);
 }
 
+/* Workgroups for n rows of G lanes. A launch takes less than 2^32 lanes, which
+   a wavefront a row reaches at 2^26 rows: the grid is capped at 2^31 lanes and
+   the kernels step by it (row_step). */
+constexpr int group_blocks(int n, int G)
+{
+    const long long rows = ROW_BS / G, b = (n + rows - 1) / rows;
+    return (int)(b < (1 << 23) ? b : (1 << 23));
+}
+
+/* rows that a whole grid takes at once */
+constexpr long long row_step(unsigned blocks, int G)
+{
+    return (long long)blocks * (ROW_BS / G);
+}
+
 } // namespace bcmg

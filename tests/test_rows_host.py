@@ -33,3 +33,20 @@ def test_rows_of_lane_groups(tmp_path):
             }
     """)
     assert out == ""
+
+
+def test_grids_of_lane_groups(tmp_path):
+    """A launch stays below 2^32 lanes and its steps reach every row once: a
+    wavefront a row at 2^26 rows and more, a lane a row at 2^31 - 1."""
+    out = run_cpp(tmp_path, """
+    for (int G = 1; G <= 64; G *= 2)
+        for (int n : {1, 3, 4, 255, 256, 257, 1 << 25, (1 << 25) + 1, 1 << 26, (1 << 26) + 5,
+                      (1 << 30) + 7, 0x7fffffff}) {
+            const unsigned long long blocks = group_blocks(n, G);
+            const long long step = row_step((unsigned)blocks, G);
+            if (blocks == 0 || blocks * ROW_BS >= 1ull << 32) std::printf("grid %d %d\\n", G, n);
+            if (step < n && blocks != 1u << 23) std::printf("short %d %d\\n", G, n);
+            if (step - n >= ROW_BS / G) std::printf("empty blocks %d %d\\n", G, n);
+        }
+    """)
+    assert out == ""
