@@ -439,7 +439,7 @@ __global__ __launch_bounds__(BS) void k_rows_stencil(int n, StencilRef<VT> S,
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int r0 = b * (BS * W);
     const int r = r0 + threadIdx.x * W;
-    const bool inner = r0 + S.lo >= 0 && r0 + BS * W + S.hi <= n && r0 + BS * W <= n;
+    const bool inner = rows_inside(r0, BS * W, S.lo, S.hi, n);
     unsigned m[W];
     VT g[W][K], fr[W], xr[W], dr[W];
 #pragma unroll
@@ -535,7 +535,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_stencil(int n, StencilRef<doub
         sdot[1] = tr * zr;
         if (K > 2) sdot[K - 1] = tor * zr;
     };
-    if (r0 + S.lo >= 0 && r0 + BS + S.hi <= n && r0 + BS <= n)
+    if (rows_inside(r0, BS, S.lo, S.hi, n))
         row(std::true_type{});
     else if (r < n)
         row(std::false_type{});

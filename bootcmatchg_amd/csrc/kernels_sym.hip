@@ -177,7 +177,7 @@ __global__ __launch_bounds__(BS) void k_rows_sym(int n, SymRef<MT> S, const VT *
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int r0 = b * (BS * W);
     const int r = r0 + threadIdx.x * W;
-    const bool inner = r0 + S.lo >= 0 && r0 + BS * W + S.hi <= n;
+    const bool inner = rows_inside(r0, BS * W, S.lo, S.hi, n);
     constexpr bool SD = OP == OP_JACOBI && DIV == DIV_L1;
     VT fr[W], xr[W], dr[W], t[W], sd[W];
 #pragma unroll
@@ -240,8 +240,8 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_sym(int n, SymRef<double> S,
         const double zr = (double)z[r], rr = rv[r];
         const double tor = K > 2 ? to[r] : 0.0;
         double tr[1], unused[1];
-        sym_rows<double, double, ZT, KO, 1, false>(n, r, r0 + S.lo >= 0 && r0 + BS + S.hi <= n, S,
-                                                   z, tr, unused);
+        sym_rows<double, double, ZT, KO, 1, false>(n, r, rows_inside(r0, BS, S.lo, S.hi, n), S, z,
+                                                   tr, unused);
         t[r] = tr[0];
         sdot[0] = rr * zr;
         sdot[1] = tr[0] * zr;

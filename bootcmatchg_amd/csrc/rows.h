@@ -17,6 +17,13 @@ constexpr int group_row(unsigned block, unsigned thread, int G)
     return (int)(block * (unsigned)(ROW_BS / G) + thread / (unsigned)G);
 }
 
+/* Whether rows [r0, r0 + rows) lie in [0, n) with every neighbour at offsets lo
+   to hi (r0 + hi passes 2^31 from 2^30 rows on). */
+constexpr bool rows_inside(int r0, int rows, int lo, int hi, int n)
+{
+    return r0 + lo >= 0 && (long long)r0 + rows + (hi > 0 ? hi : 0) <= n;
+}
+
 /* Workgroups for n rows of G lanes. A launch takes less than 2^32 lanes, which
    a wavefront a row reaches at 2^26 rows: the grid is capped at 2^31 lanes and
    the kernels step by it (row_step). */

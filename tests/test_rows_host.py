@@ -50,3 +50,20 @@ def test_grids_of_lane_groups(tmp_path):
         }
     """)
     assert out == ""
+
+
+def test_blocks_inside_the_operator(tmp_path):
+    """A block is inside where every row's neighbours are: against 64 bits, with
+    offsets and rows up to 2^31."""
+    out = run_cpp(tmp_path, """
+    for (long long n : {512ll, 4097ll, (1ll << 30) + 9, (3ll << 29) + 11, 0x7fffffffll})
+        for (long long lo : {-n + 1, -5ll, 0ll, 3ll})
+            for (long long hi : {-2ll, 0ll, 7ll, n / 2, n - 1})
+                for (long long r0 : {0ll, 256ll, n / 512 * 256, n / 256 * 256 - 256}) {
+                    if (hi < lo || r0 < 0 || r0 >= n) continue;
+                    const bool want = r0 + lo >= 0 && r0 + 256 + hi <= n && r0 + 256 <= n;
+                    if (rows_inside((int)r0, 256, (int)lo, (int)hi, (int)n) != want)
+                        std::printf("n %lld lo %lld hi %lld r0 %lld\\n", n, lo, hi, r0);
+                }
+    """)
+    assert out == ""
