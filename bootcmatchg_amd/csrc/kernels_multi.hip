@@ -12,6 +12,7 @@
  * Columns whose flag in `act` is 0 are skipped (act == nullptr: all nc).
  */
 #include "kernels_common.h"
+#include "slab_plan.h"
 
 namespace bcmg {
 
@@ -425,8 +426,6 @@ __global__ __launch_bounds__(BS) void k_rows_il_stencil(int n, StencilRef<VT> S,
 }
 
 constexpr int ILR_AHEAD = 2;
-
-constexpr int SLAB_BS = 1024;
 
 /* Several steps of a small narrow-band level in one launch: a workgroup keeps
    its L rows and a halo of `halo` each side (the band per sweep, computed
@@ -1794,31 +1793,6 @@ void launch_rows_il(hipStream_t s, const DevCsr &A, MatType mt, RowOp op, const 
             rows_il_op<double, float>(s, A, A.val.get(), op, x, f, d, y, lkp, nc, act);
     }
     BCMG_CHECK_LAUNCH();
-}
-
-/* The slab of `sweeps` sweeps: the rows a workgroup stores and its cells per
-   lane (0: does not fit). */
-struct IlSlab {
-    int L = 0, rpt = 0;
-    double us = 0;
-};
-
-/* Predicted time: a launch, the loads and the store cost about 4.5 us, a sweep
-   of the cells 0.45 us per cell of a lane and round of workgroups (one a CU);
-   a sweep of its own 3 us and its bytes at 8 TB/s. */
-IlSlab il_slab_fit(int n, int band, int gpr, int sweeps)
-{
-    IlSlab best;
-    const int halo = band * sweeps;
-    for (int L = 16; L <= 512; L *= 2) {
-        const long long cells = (long long)(L + 2 * halo) * gpr;
-        const int rpt = (int)((cells + SLAB_BS - 1) / SLAB_BS);
-        if (rpt > 4) break;
-        const int rounds = (n + 256 * L - 1) / (256 * L);
-        const double us = 2.5 + rounds * (2.0 + sweeps * 0.45 * rpt);
-        if (best.rpt == 0 || us < best.us) best = IlSlab{L, rpt, us};
-    }
-    return best;
 }
 
 template <typename VT>

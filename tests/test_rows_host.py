@@ -8,7 +8,7 @@ CSRC = os.path.join(ROOT, "bootcmatchg_amd", "csrc")
 
 def run_cpp(tmp_path, body):
     src = tmp_path / "t.cpp"
-    src.write_text('#include "rows.h"\n#include <algorithm>\n#include <cstdio>\n#include <initializer_list>\nusing namespace bcmg;\n'
+    src.write_text('#include "rows.h"\n#include "slab_plan.h"\n#include <algorithm>\n#include <cstdio>\n#include <initializer_list>\nusing namespace bcmg;\n'
                    "int main() {\n%s\nreturn 0;\n}\n" % body)
     exe = str(tmp_path / "t")
     subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-I", CSRC, str(src), "-o",
@@ -64,6 +64,27 @@ def test_blocks_inside_the_operator(tmp_path):
                     const bool want = r0 + lo >= 0 && r0 + 256 + hi <= n && r0 + 256 <= n;
                     if (rows_inside((int)r0, 256, (int)lo, (int)hi, (int)n) != want)
                         std::printf("n %lld lo %lld hi %lld r0 %lld\\n", n, lo, hi, r0);
+                }
+    """)
+    assert out == ""
+
+
+def test_slabs_fit_their_workgroup(tmp_path):
+    """The rows of a slab with its halo, for bands up to 2^31 and many sweeps:
+    what is taken has the cells that four a lane hold, the rest is refused."""
+    out = run_cpp(tmp_path, """
+    for (int band : {0, 1, 8, 63, 64, 2048, 1 << 20, 1 << 28, (1 << 29) + 1, 1 << 30, 0x7ffffffe})
+        for (int sweeps : {2, 3, 4, 16, 1000, 100000})
+            for (int gpr : {1, 2, 3, 16})
+                for (int n : {1, 4096, 1 << 20, 0x7fffffff}) {
+                    const IlSlab p = il_slab_fit(n, band, gpr, sweeps);
+                    const double least = (16.0 + 2.0 * band * sweeps) * gpr;
+                    const double cells = (p.L + 2.0 * band * sweeps) * gpr;
+                    const bool fits = p.rpt >= 1 && p.rpt <= 4 && cells <= p.rpt * SLAB_BS &&
+                                      cells > (p.rpt - 1) * SLAB_BS && p.us > 0;
+                    if (least <= 4 * SLAB_BS ? !fits : p.rpt != 0)
+                        std::printf("band %d sweeps %d gpr %d n %d: L %d rpt %d\\n", band, sweeps,
+                                    gpr, n, p.L, p.rpt);
                 }
     """)
     assert out == ""
