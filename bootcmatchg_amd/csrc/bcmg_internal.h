@@ -11,7 +11,6 @@
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
-#include <list>
 #include <map>
 #include <memory>
 #include <unordered_map>
@@ -21,6 +20,7 @@
 #include <vector>
 
 #include "../../include/bcmg.h"
+#include "chunks.h"
 
 namespace bcmg {
 
@@ -54,28 +54,21 @@ void set_last_error(const std::string &msg);
    kernel still reads it is only reused by work queued after that kernel.
    hipMalloc/hipFree of large buffers cost milliseconds and hipFree
    synchronises the device; the setup allocates and drops hundreds of
-   temporaries, so it goes through the pool. Blocks of up to SUB_MAX bytes
-   are cut from chunks (CHUNK_MIN bytes, each twice the last up to CHUNK_MAX,
-   so at most about as much again as the blocks take), since a call each to
-   get and to give back some 250 of them cost a 226 981-row solve from host arrays 14 of 29 ms;
-   a chunk goes back to the device when all its blocks are free and trim or
-   free_released asks for it. */
+   temporaries, so it goes through the pool. Blocks of up to Chunks::SUB_MAX
+   bytes are cut from chunks (8 to 32 MB), since a call each to get and to give
+   back some 250 of them cost a 226 981-row solve from host arrays 14 of 29 ms.
+   trim and free_released give back the cached blocks and the chunks that have
+   no block out: of a chunk with one, up to CHUNK_MAX, the rest stays and
+   serves the context's other blocks. */
 struct Pool {
-    static constexpr size_t SUB_MAX = (size_t)16 << 20;
-    static constexpr size_t CHUNK_MIN = (size_t)8 << 20, CHUNK_MAX = (size_t)64 << 20;
-    struct Chunk {
-        char *base = nullptr;
-        size_t size = 0, used = 0;   /* used: bytes cut so far */
-        size_t out = 0;              /* blocks handed out */
-    };
     struct Block {
         size_t cls = 0;
-        Chunk *chunk = nullptr;      /* null: an allocation of its own */
+        bool cut = false;            /* from a chunk, else an allocation of its own */
     };
-    std::multimap<size_t, std::pair<void *, Chunk *>> free_;
+    std::multimap<size_t, void *> free_;   /* cached allocations of their own */
     std::unordered_map<void *, Block> cls_;
-    std::list<Chunk> chunks_;
-    size_t cached = 0, live = 0;
+    Chunks chunks_;
+    size_t live = 0;
     /* while set, released memory is freed at once instead of cached (the
        serving loop gives a closed lane's memory back to the device) */
     bool free_released = false;
@@ -89,7 +82,8 @@ struct Pool {
     ~Pool();
 
   private:
-    void *cut(size_t cls, Chunk **from);
+    void *cached(size_t cls);
+    void *cut(size_t cls);
     void free_chunks();
 };
 

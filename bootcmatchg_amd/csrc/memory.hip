@@ -4,8 +4,6 @@
  */
 #include "bcmg_internal.h"
 
-#include <algorithm>
-
 namespace bcmg {
 
 namespace {
@@ -35,61 +33,47 @@ void *device_block(size_t bytes)
 }
 } // namespace
 
-/* the next cls bytes of a chunk that has them, or of a new one (null: the
-   device has no room for a chunk) */
-void *Pool::cut(size_t cls, Chunk **from)
+/* a cached allocation of its own of that class, or null */
+void *Pool::cached(size_t cls)
 {
-    Chunk *c = nullptr;
-    size_t last = 0;
-    for (Chunk &k : chunks_) {
-        last = std::max(last, k.size);
-        if (!c && k.size - k.used >= cls) c = &k;
-    }
-    if (!c) {
-        const size_t want = std::max(cls, std::min(CHUNK_MAX, std::max(CHUNK_MIN, 2 * last)));
-        char *base = static_cast<char *>(device_block(want));
-        if (!base) return nullptr;
-        try {
-            chunks_.emplace_back();
-        } catch (...) {
-            (void)hipFree(base);
-            throw;
-        }
-        c = &chunks_.back();
-        c->base = base;
-        c->size = want;
-    }
-    void *p = c->base + c->used;
-    c->used += cls;
-    *from = c;
+    const auto it = free_.find(cls);
+    if (it == free_.end()) return nullptr;
+    void *const p = it->second;
+    free_.erase(it);
     return p;
+}
+
+/* cls bytes of a new chunk (null: the device has no room for one) */
+void *Pool::cut(size_t cls)
+{
+    const size_t size = chunks_.next_size(cls);
+    char *const base = static_cast<char *>(device_block(size));
+    if (!base) return nullptr;
+    try {
+        chunks_.add(base, size);
+    } catch (...) {
+        (void)hipFree(base);
+        throw;
+    }
+    return chunks_.take(cls);
 }
 
 void *Pool::alloc(size_t bytes)
 {
     const size_t cls = size_class(bytes);
-    void *p = nullptr;
-    Chunk *from = nullptr;
-    auto it = free_.lower_bound(cls);
-    const auto end = free_.upper_bound(cls);
-    while (own_blocks && it != end && it->second.second) ++it;
-    if (it != end) {
-        p = it->second.first;
-        from = it->second.second;
-        free_.erase(it);
-        cached -= cls;
-    } else {
-        for (int attempt = 0; !p && attempt < 2; attempt++) {
-            if (attempt) trim();
-            if (cls <= SUB_MAX && !own_blocks) p = cut(cls, &from);
-            if (!p) p = device_block(cls);
-        }
-        if (!p)
-            throw Error(BCMG_ENOMEM, "device allocation of " + std::to_string(cls) +
-                                         " bytes failed");
+    const bool small = cls <= Chunks::SUB_MAX && !own_blocks;
+    Block b{cls, true};
+    void *p = small ? chunks_.take(cls) : nullptr;
+    if (!p && (p = cached(cls))) b.cut = false;
+    for (int attempt = 0; !p && attempt < 2; attempt++) {
+        if (attempt) trim();
+        if (small) p = cut(cls);
+        if (!p && (p = device_block(cls))) b.cut = false;
     }
-    cls_[p] = Block{cls, from};
-    if (from) from->out++;
+    if (!p)
+        throw Error(BCMG_ENOMEM,
+                    "device allocation of " + std::to_string(cls) + " bytes failed");
+    cls_[p] = b;
     live += cls;
     return p;
 }
@@ -104,49 +88,27 @@ void Pool::release(void *p)
     const Block b = it->second;
     cls_.erase(it);
     live -= b.cls;
-    if (free_released && !b.chunk) {
+    if (b.cut) {
+        if (chunks_.give(static_cast<char *>(p), b.cls) && free_released) free_chunks();
+    } else if (free_released) {
         (void)hipFree(p);
-        return;
+    } else {
+        free_.emplace(b.cls, p);
     }
-    free_.emplace(b.cls, std::make_pair(p, b.chunk));
-    cached += b.cls;
-    if (b.chunk && --b.chunk->out == 0 && free_released) free_chunks();
 }
 
 /* give back the chunks none of whose blocks are out (hipFree waits for the
    work that used them) */
 void Pool::free_chunks()
 {
-    for (auto it = free_.begin(); it != free_.end();) {
-        if (it->second.second && it->second.second->out == 0) {
-            cached -= it->first;
-            it = free_.erase(it);
-        } else {
-            ++it;
-        }
-    }
-    for (auto it = chunks_.begin(); it != chunks_.end();) {
-        if (it->out == 0) {
-            (void)hipFree(it->base);
-            it = chunks_.erase(it);
-        } else {
-            ++it;
-        }
-    }
+    for (char *base : chunks_.take_whole()) (void)hipFree(base);
 }
 
 void Pool::trim()
 {
     if (!free_.empty() || !chunks_.empty()) (void)hipDeviceSynchronize();
-    for (auto it = free_.begin(); it != free_.end();) {
-        if (!it->second.second) {
-            (void)hipFree(it->second.first);
-            cached -= it->first;
-            it = free_.erase(it);
-        } else {
-            ++it;
-        }
-    }
+    for (auto &kv : free_) (void)hipFree(kv.second);
+    free_.clear();
     free_chunks();
 }
 
