@@ -247,8 +247,10 @@ void resolve_tiles(Ctx &c, const std::vector<DevCsr *> &mats);
 /* build the narrow column copy of every square operator in mats above the
    non-temporal size whose column offsets all fit 16 bits, and its stencil
    pattern when those offsets take at most PAT_MAX values (one round trip
-   for the lot) */
-void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats);
+   for the lot). Operators with row classes or a symmetric stencil, whose
+   columns the row kernels do not read, get them only when asked for
+   (bcmg_csr_set_columns): at 160^3 they are 61 MB. */
+void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats, bool asked = false);
 /* find the band and the row classes (at most CLS_MAX forms) of every square
    operator in mats that has rows of at most CLS_ROW entries, their tiles
    resolved (one round trip for the lot, a second for those with classes) */

@@ -145,6 +145,14 @@ void d2h(bcmg_ctx ctx, void *dst, const void *src, size_t bytes)
     BCMG_HIP(hipStreamSynchronize(ctx->c.stream));
 }
 
+/* the narrow column copies of an operator that is read in another form */
+void narrow_copies(bcmg_csr A)
+{
+    if (A->A.cls.n == 0 && A->A.sym.k == 0) return;
+    CtxScope scope_(A->ctx);
+    make_narrow(A->ctx->c, {&A->A}, true);
+}
+
 } // namespace
 
 extern "C" {
@@ -398,8 +406,10 @@ int bcmg_csr_info(bcmg_csr A, int *n, int *nnz)
 int bcmg_csr_column_bytes(bcmg_csr A, int *bytes)
 {
     if (!A || !bytes) return BCMG_EINVAL;
+    API_BEGIN
+    narrow_copies(A);
     *bytes = A->A.use_pattern() ? 0 : A->A.use_narrow() ? 2 : 4;
-    return BCMG_OK;
+    API_END
 }
 
 int bcmg_csr_form(bcmg_csr A, int *form)
@@ -415,6 +425,8 @@ int bcmg_csr_form(bcmg_csr A, int *form)
 int bcmg_csr_set_columns(bcmg_csr A, int bytes)
 {
     if (!A) return BCMG_EINVAL;
+    API_BEGIN
+    narrow_copies(A);
     if (bytes == 4) {
         A->A.col_mode = 0;
     } else if (bytes == 2) {
@@ -434,7 +446,7 @@ int bcmg_csr_set_columns(bcmg_csr A, int bytes)
     } else {
         return BCMG_EINVAL;
     }
-    return BCMG_OK;
+    API_END
 }
 
 int bcmg_csr_free(bcmg_csr A)

@@ -292,8 +292,8 @@ void adaptive_coarsening(Ctx &c, const bcmg_params &p, BuildState &bs, DevCsr &A
     resolve_tiles(c, pending);
     pending.clear();
     for (int i = 1; i < level; i++) pending.push_back(&H.L[i].Aown);
-    make_narrow(c, pending);
     make_classes(c, pending);
+    make_narrow(c, pending);
     double cx = 0, cw = 0;
     for (int i = 0; i < level; i++) {
         cx += H.L[i].mat().nnz;

@@ -1024,9 +1024,9 @@ void analyze_rows(Ctx &c, DevCsr &A)
 {
     launch_block_nnz(c, A);
     resolve_tiles(c, {&A});
-    make_narrow(c, {&A});
     make_classes(c, {&A});
     make_sym(c, A);
+    make_narrow(c, {&A});
 }
 
 /* square operators whose FP64 stream (12 B per entry) exceeds this are
@@ -1058,11 +1058,12 @@ bool find_offsets(Ctx &c, DevCsr &A, std::vector<int> &off)
     return c.h_ints[0] == 0 && !off.empty() && off.size() <= PAT_MAX;
 }
 
-void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats)
+void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats, bool asked)
 {
     std::vector<DevCsr *> cand;
     for (DevCsr *A : mats)
-        if (A->n == A->m && (size_t)A->nnz * 12 > PAT_MIN_BYTES && !A->cols_analysed)
+        if (A->n == A->m && (size_t)A->nnz * 12 > PAT_MIN_BYTES && !A->cols_analysed &&
+            (asked || (A->cls.n == 0 && A->sym.k == 0)))
             cand.push_back(A);
     if (cand.empty()) return;
     const int nc = (int)cand.size();

@@ -67,3 +67,28 @@ def test_the_form_that_the_row_kernels_read(ctx):
         dA.set_columns(bc.COLUMNS_ANY)
         assert dA.form == form
         dA.free()
+
+
+def test_a_stencil_keeps_no_column_copies(ctx):
+    """An upload holds the CSR arrays, a byte a row and a chunk of small blocks;
+    the 16-bit columns and the pattern of a constant stencil (57 + 4 MB at
+    160^3) come when they are asked for."""
+    from test_gpu_serving import device_bytes_in_use
+
+    def rounded(b):                              # the pool's size classes
+        step = 1 << (b.bit_length() - 3)
+        return (b + step - 1) // step * step
+
+    A = ops.poisson3d(160)
+    n, nnz = len(A[0]) - 1, len(A[1])
+    c = bc.Context(0)
+    c.sync()
+    before = device_bytes_in_use()
+    dA = bc.Csr(c, A)
+    held = device_bytes_in_use() - before
+    assert dA.form == bc.FORM_STENCIL
+    assert held <= rounded(8 * nnz) + rounded(4 * nnz) + rounded(4 * (n + 1)) + (34 << 20)
+    assert dA.column_bytes == 0
+    assert device_bytes_in_use() - before >= held + 2 * nnz
+    dA.free()
+    c.close()
