@@ -151,6 +151,10 @@ enum MatType { MT_F64 = 0, MT_F32 = 1, MT_BF16 = 2 };
 
 /* most distinct column offsets of a stencil-pattern operator */
 constexpr int PAT_MAX = 8;
+/* the table they are found in: a flag (too many) and the slots */
+constexpr int PAT_SLOTS = 2 * PAT_MAX;
+constexpr int PAT_EMPTY = (int)0x80000000; /* no offset col - row equals it */
+constexpr int OFFSET_INTS = 1 + PAT_SLOTS;
 
 /* row classes (kernels_class.hip): most distinct row forms, longest row */
 constexpr int CLS_MAX = 256;
@@ -253,12 +257,17 @@ void resolve_tiles(Ctx &c, const std::vector<DevCsr *> &mats);
 void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats, bool asked = false);
 /* find the band and the row classes (at most CLS_MAX forms) of every square
    operator in mats that has rows of at most CLS_ROW entries, their tiles
-   resolved (one round trip for the lot, a second for those with classes) */
+   resolved (one round trip for the lot) */
 void make_classes(Ctx &c, const std::vector<DevCsr *> &mats);
-/* the symmetric-stencil form of an uploaded operator without row classes */
-void make_sym(Ctx &c, DevCsr &A);
-/* A's distinct column offsets, ascending; false when more than PAT_MAX */
-bool find_offsets(Ctx &c, DevCsr &A, std::vector<int> &off);
+/* the symmetric-stencil form of an uploaded operator without row classes, its
+   distinct column offsets being off; whether its size allows one */
+void make_sym(Ctx &c, DevCsr &A, const std::vector<int> &off);
+bool sym_candidate(const DevCsr &A);
+/* A's distinct column offsets into info (OFFSET_INTS ints, set to 0 and then to
+   PAT_EMPTY), queued; with run, only where *run is not 0 by then. From the host
+   copy: the offsets, ascending; false when more than PAT_MAX. */
+void launch_offsets(hipStream_t s, const DevCsr &A, int *info, const int *run);
+bool offsets_found(const int *info, std::vector<int> &off);
 
 /* ------------------------------------------------------------- context */
 

@@ -249,16 +249,17 @@ __global__ __launch_bounds__(BS) void k_rows_pattern(int n, const int *__restric
    block (an LDS table of 2 PAT_MAX slots) are inserted into the operator's
    table gtab of as many slots (PAT_EMPTY where unused: a slot, once set,
    keeps its value, so no value is inserted twice); more distinct offsets
-   than slots, in a block or in all, raise flag[0]. */
-constexpr int PAT_SLOTS = 2 * PAT_MAX;
-constexpr int PAT_EMPTY = (int)0x80000000; /* no offset col - row equals it */
+   than slots, in a block or in all, raise flag[0]. With `run`, only where
+   *run is not 0. */
 __global__ __launch_bounds__(BS) void k_pattern_offsets(int n, const int *__restrict__ rp,
                                                         const int *__restrict__ ci,
                                                         int *__restrict__ gtab,
-                                                        int *__restrict__ flag)
+                                                        int *__restrict__ flag,
+                                                        const int *__restrict__ run)
 {
     __shared__ int tab[PAT_SLOTS];
     __shared__ int over;
+    if (run && *run == 0) return;
     if (threadIdx.x < PAT_SLOTS) tab[threadIdx.x] = PAT_EMPTY;
     if (threadIdx.x == 0) over = 0;
     __syncthreads();
@@ -1020,42 +1021,25 @@ void resolve_tiles(Ctx &c, const std::vector<DevCsr *> &mats)
     }
 }
 
-void analyze_rows(Ctx &c, DevCsr &A)
-{
-    launch_block_nnz(c, A);
-    resolve_tiles(c, {&A});
-    make_classes(c, {&A});
-    make_sym(c, A);
-    make_narrow(c, {&A});
-}
-
 /* square operators whose FP64 stream (12 B per entry) exceeds this are
    checked for a stencil pattern; the 16-bit copy is kept for streamed ones
    (above NT_BYTES) only */
 constexpr size_t PAT_MIN_BYTES = (size_t)128 << 20;
 
-bool find_offsets(Ctx &c, DevCsr &A, std::vector<int> &off)
+void launch_offsets(hipStream_t s, const DevCsr &A, int *info, const int *run)
+{
+    k_pattern_offsets<<<(A.n + BS - 1) / BS, BS, 0, s>>>(A.n, A.row.get(), A.col.get(), info + 1,
+                                                        info, run);
+    BCMG_CHECK_LAUNCH();
+}
+
+bool offsets_found(const int *info, std::vector<int> &off)
 {
     off.clear();
-    if (A.pk > 0) {
-        off.assign(A.poff, A.poff + A.pk);
-        return true;
-    }
-    DBuf<int> info(1 + PAT_SLOTS);
-    c.h_ints[0] = 0;
-    for (int q = 0; q < PAT_SLOTS; q++) c.h_ints[1 + q] = PAT_EMPTY;
-    BCMG_HIP(hipMemcpyAsync(info.get(), c.h_ints, (1 + PAT_SLOTS) * sizeof(int),
-                            hipMemcpyHostToDevice, c.stream));
-    k_pattern_offsets<<<(A.n + BS - 1) / BS, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(),
-                                                               info.get() + 1, info.get());
-    BCMG_CHECK_LAUNCH();
-    BCMG_HIP(hipMemcpyAsync(c.h_ints, info.get(), (1 + PAT_SLOTS) * sizeof(int),
-                            hipMemcpyDeviceToHost, c.stream));
-    BCMG_HIP(hipStreamSynchronize(c.stream));
     for (int q = 0; q < PAT_SLOTS; q++)
-        if (c.h_ints[1 + q] != PAT_EMPTY) off.push_back(c.h_ints[1 + q]);
+        if (info[1 + q] != PAT_EMPTY) off.push_back(info[1 + q]);
     std::sort(off.begin(), off.end());
-    return c.h_ints[0] == 0 && !off.empty() && off.size() <= PAT_MAX;
+    return info[0] == 0 && !off.empty() && off.size() <= PAT_MAX;
 }
 
 void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats, bool asked)
@@ -1085,7 +1069,7 @@ void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats, bool asked)
                                                      A.col16.get(), in);
         }
         k_pattern_offsets<<<nblk, BS, 0, c.stream>>>(A.n, A.row.get(), A.col.get(), in + 2,
-                                                     in + 1);
+                                                     in + 1, nullptr);
     }
     BCMG_CHECK_LAUNCH();
     std::vector<int> h((size_t)nc * W);

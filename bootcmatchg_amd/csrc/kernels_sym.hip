@@ -307,12 +307,14 @@ void rows_sym_k(hipStream_t s, const DevCsr &A, const VT *x, const VT *f, const 
    latency and gain little */
 constexpr int SYM_MIN_ROWS = 32768;
 
-void make_sym(Ctx &c, DevCsr &A)
+bool sym_candidate(const DevCsr &A)
 {
-    if (A.n != A.m || A.n < SYM_MIN_ROWS || A.cls.n > 0 || A.maxrow <= 0 || A.maxrow > PAT_MAX - 1)
-        return;
-    std::vector<int> off;
-    if (!find_offsets(c, A, off)) return;
+    return A.n == A.m && A.n >= SYM_MIN_ROWS && A.nnz <= (long long)(PAT_MAX - 1) * A.n;
+}
+
+void make_sym(Ctx &c, DevCsr &A, const std::vector<int> &off)
+{
+    if (!sym_candidate(A) || A.cls.n > 0 || A.maxrow <= 0 || A.maxrow > PAT_MAX - 1) return;
     /* odd in number and closed under negation: the middle one is 0 */
     const int k = (int)off.size();
     if (k < 3 || k % 2 == 0) return;

@@ -1,11 +1,13 @@
 """The rules that choose a kernel form, seen through the library's queries."""
+import numpy as np
 import pytest
+import scipy.sparse as sp
 
 import bootcmatchg_amd as bc
 from bootcmatchg_amd import operators as ops
 
-from common import SETTINGS
-from test_gpu_classes import neumann2d
+from common import SETTINGS, bits
+from test_gpu_classes import csr, neumann2d, row_ops
 
 pytestmark = pytest.mark.gpu
 
@@ -92,3 +94,21 @@ def test_a_stencil_keeps_no_column_copies(ctx):
     assert device_bytes_in_use() - before >= held + 2 * nnz
     dA.free()
     c.close()
+
+
+@pytest.mark.parametrize("kinds", [1, 63, 64, 65, 255, 256, 257])
+def test_tables_of_any_length(ctx, kinds):
+    """Row classes as many as the head of the analysis holds (64), as there may
+    be (256) and one more: the kernels' bits are those of the columns. (A form
+    fills a hundred rows at a time: a block of 256 rows may hold 128 at most.)"""
+    n = 26011
+    dA = bc.Csr(ctx, csr(sp.diags(1.0 + (np.arange(n) // 100 % kinds) / 1024.0)))
+    assert dA.form == (bc.FORM_STENCIL if kinds == 1 else
+                       bc.FORM_CLASSES if kinds <= 256 else bc.FORM_COLUMNS)
+    rng = np.random.default_rng(8)
+    x, f, d = rng.uniform(-1, 1, n), rng.uniform(-1, 1, n), rng.uniform(7, 8, n)
+    got = row_ops(ctx, dA, n, x, f, d)
+    dA.set_columns(4)
+    for g, w in zip(got, row_ops(ctx, dA, n, x, f, d)):
+        assert np.array_equal(bits(g), bits(w))
+    dA.free()
