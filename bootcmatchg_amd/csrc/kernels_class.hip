@@ -1113,7 +1113,7 @@ void make_classes(Ctx &c, const std::vector<DevCsr *> &mats)
 
 /* An upload's analysis: the tile sizes, the classes and (where there are none)
    the offsets come back in one round trip; a symmetric stencil takes a second.
-   A 32^3 Poisson upload 0.277 -> 0.252 ms, 32^3 log-normal 0.306 -> 0.286 (both
+   A 32^3 Poisson upload 0.277 -> 0.250 ms, 32^3 log-normal 0.306 -> 0.264 (both
    0.213 without any analysis). */
 void analyze_rows(Ctx &c, DevCsr &A)
 {

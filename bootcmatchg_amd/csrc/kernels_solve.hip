@@ -245,12 +245,31 @@ __global__ __launch_bounds__(BS) void k_rows_pattern(int n, const int *__restric
         y[r] = (fr - t) / dr + xr;
 }
 
+/* a value into a table of PAT_SLOTS slots (PAT_EMPTY where unused: a slot, once
+   set, keeps its value, so no value is inserted twice); false: full. The search
+   starts at the value's own slot: from the first on, every block's offsets met
+   at the same words (32 768 rows of 7 entries: 22.8 -> 4.4 us). */
+template <int SCOPE>
+__device__ __forceinline__ bool insert_offset(int *tab, int o)
+{
+    static_assert(PAT_SLOTS == 16, "four bits of the hash");
+    const unsigned s0 = (unsigned)o * 2654435761u >> 28;
+    for (int k = 0; k < PAT_SLOTS; k++) {
+        int *const p = tab + ((s0 + k) & (PAT_SLOTS - 1));
+        const int v = __hip_atomic_load(p, __ATOMIC_RELAXED, SCOPE);
+        if (v == o) return true;
+        if (v == PAT_EMPTY) {
+            const int prev = atomicCAS(p, PAT_EMPTY, o);
+            if (prev == PAT_EMPTY || prev == o) return true;
+        }
+    }
+    return false;
+}
+
 /* Setup of the pattern, step 1: the distinct column offsets of each 256-row
-   block (an LDS table of 2 PAT_MAX slots) are inserted into the operator's
-   table gtab of as many slots (PAT_EMPTY where unused: a slot, once set,
-   keeps its value, so no value is inserted twice); more distinct offsets
-   than slots, in a block or in all, raise flag[0]. With `run`, only where
-   *run is not 0. */
+   block (an LDS table) are inserted into the operator's table gtab; more
+   distinct offsets than slots, in a block or in all, raise flag[0]. With
+   `run`, only where *run is not 0. */
 __global__ __launch_bounds__(BS) void k_pattern_offsets(int n, const int *__restrict__ rp,
                                                         const int *__restrict__ ci,
                                                         int *__restrict__ gtab,
@@ -266,36 +285,13 @@ __global__ __launch_bounds__(BS) void k_pattern_offsets(int n, const int *__rest
     const int r = blockIdx.x * BS + threadIdx.x;
     if (r < n) {
         const int k1 = rp[r + 1];
-        for (int k = rp[r]; k < k1; k++) {
-            const int o = ci[k] - r;
-            int s = 0;
-            for (; s < PAT_SLOTS; s++) {
-                const int v = __hip_atomic_load(&tab[s], __ATOMIC_RELAXED,
-                                                __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (v == o) break;
-                if (v == PAT_EMPTY) {
-                    const int prev = atomicCAS(&tab[s], PAT_EMPTY, o);
-                    if (prev == PAT_EMPTY || prev == o) break;
-                }
-            }
-            if (s == PAT_SLOTS) over = 1;
-        }
+        for (int k = rp[r]; k < k1; k++)
+            if (!insert_offset<__HIP_MEMORY_SCOPE_WORKGROUP>(tab, ci[k] - r)) over = 1;
     }
     __syncthreads();
     if (threadIdx.x == 0 && over) atomicOr(flag, 1);
-    if (threadIdx.x >= PAT_SLOTS) return;
-    const int o = tab[threadIdx.x];
-    if (o == PAT_EMPTY) return;
-    int s = 0;
-    for (; s < PAT_SLOTS; s++) {
-        const int v = __hip_atomic_load(&gtab[s], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (v == o) break;
-        if (v == PAT_EMPTY) {
-            const int prev = atomicCAS(&gtab[s], PAT_EMPTY, o);
-            if (prev == PAT_EMPTY || prev == o) break;
-        }
-    }
-    if (s == PAT_SLOTS) atomicOr(flag, 1);
+    if (threadIdx.x >= PAT_SLOTS || tab[threadIdx.x] == PAT_EMPTY) return;
+    if (!insert_offset<__HIP_MEMORY_SCOPE_AGENT>(gtab, tab[threadIdx.x])) atomicOr(flag, 1);
 }
 
 /* step 3: the row masks over the sorted offset table (every offset of the

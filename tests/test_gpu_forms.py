@@ -112,3 +112,24 @@ def test_tables_of_any_length(ctx, kinds):
     for g, w in zip(got, row_ops(ctx, dA, n, x, f, d)):
         assert np.array_equal(bits(g), bits(w))
     dA.free()
+
+
+@pytest.mark.parametrize("count", [1, 2, 8, 9, 16, 17])
+def test_offsets_of_any_number(ctx, count):
+    """The table of a large operator's distinct column offsets (16 slots): up to
+    8 make a pattern, which is read with the bits of the columns."""
+    n = 12_000_000 // count + 4099
+    off = [0] + [37 * k * k + 11 * k for k in range(1, count)]
+    vals = [1.0 + 0.25 * k for k in range(count)]
+    S = sp.diags([np.full(n - o, v) for o, v in zip(off, vals)], off, format="csr")
+    S.data *= 1.0 + (np.arange(S.nnz) % 1009) / 2048.0   # no classes
+    dA = bc.Csr(ctx, (S.indptr.astype(np.int32), S.indices.astype(np.int32), S.data))
+    assert dA.form == bc.FORM_COLUMNS and dA.column_bytes == (0 if count <= 8 else 4)
+    x = bc.DeviceArray.from_numpy(ctx, ops.uniform_pm1(2, n))
+    y = bc.DeviceArray(ctx, n)
+    bc.spmv(ctx, dA, x, y)
+    got = y.numpy()
+    dA.set_columns(4)
+    bc.spmv(ctx, dA, x, y)
+    assert np.array_equal(bits(got), bits(y.numpy()))
+    dA.free()
