@@ -466,7 +466,7 @@ __global__ __launch_bounds__(BS) void k_rows_stencil(int n, StencilRef<VT> S,
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int r0 = b * (BS * W);
     const int r = r0 + threadIdx.x * W;
-    const bool inner = rows_inside(r0, BS * W, S.lo, S.hi, n);
+    const bool inner = S.inner.holds(r0, BS * W);
     unsigned m[W];
     VT g[W][K], fr[W], xr[W], dr[W];
 #pragma unroll
@@ -562,7 +562,7 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_stencil(int n, StencilRef<doub
         sdot[1] = tr * zr;
         if (K > 2) sdot[K - 1] = tor * zr;
     };
-    if (rows_inside(r0, BS, S.lo, S.hi, n))
+    if (S.inner.holds(r0, BS))
         row(std::true_type{});
     else if (r < n)
         row(std::false_type{});

@@ -375,7 +375,7 @@ struct StencilRef {
     VT v[CLS_ROW];
     double a[CLS_ROW];   /* magnitudes in FP64: the L1 divisor */
     VT diag;
-    int lo, hi;          /* smallest and largest offset */
+    InnerRows inner;
 };
 
 template <typename VT>
@@ -384,8 +384,7 @@ StencilRef<VT> stencil_ref(const DevCsr &A, MatType mt)
     StencilRef<VT> S;
     const RowClasses &R = A.cls;
     S.mask = R.code.get();
-    S.lo = R.off[0];
-    S.hi = R.off[R.k - 1];
+    S.inner = inner_rows(A.n, R.off[0], R.off[R.k - 1]);
     S.diag = (VT)0;
     for (int k = 0; k < CLS_ROW; k++) {
         const bool in = k < R.k;

@@ -36,7 +36,7 @@ struct SymRef {
     long ld;
     int off[PAT_MAX];
     int up[PAT_MAX]; /* diagonal that holds entry k */
-    int lo, hi;
+    InnerRows inner;
 };
 
 /* step 1: the diagonals and masks (rows that pad the last block get none) */
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(BS) void k_rows_sym(int n, SymRef<MT> S, const VT *
     const int b = xcd_block(blockIdx.x, gridDim.x);
     const int r0 = b * (BS * W);
     const int r = r0 + threadIdx.x * W;
-    const bool inner = rows_inside(r0, BS * W, S.lo, S.hi, n);
+    const bool inner = S.inner.holds(r0, BS * W);
     constexpr bool SD = OP == OP_JACOBI && DIV == DIV_L1;
     VT fr[W], xr[W], dr[W], t[W], sd[W];
 #pragma unroll
@@ -240,8 +240,8 @@ __global__ __launch_bounds__(BS) void k_spmv_dots_sym(int n, SymRef<double> S,
         const double zr = (double)z[r], rr = rv[r];
         const double tor = K > 2 ? to[r] : 0.0;
         double tr[1], unused[1];
-        sym_rows<double, double, ZT, KO, 1, false>(n, r, rows_inside(r0, BS, S.lo, S.hi, n), S, z,
-                                                   tr, unused);
+        sym_rows<double, double, ZT, KO, 1, false>(n, r, S.inner.holds(r0, BS), S, z, tr,
+                                                   unused);
         t[r] = tr[0];
         sdot[0] = rr * zr;
         sdot[1] = tr[0] * zr;
@@ -261,8 +261,7 @@ SymRef<MT> sym_ref(const DevCsr &A)
     else
         S.u = Y.u32.get();
     S.ld = Y.ld;
-    S.lo = Y.off[0];
-    S.hi = Y.off[Y.k - 1];
+    S.inner = inner_rows(A.n, Y.off[0], Y.off[Y.k - 1]);
     for (int k = 0; k < PAT_MAX; k++) {
         S.off[k] = k < Y.k ? Y.off[k] : 0;
         S.up[k] = k < Y.k ? std::abs(k - Y.k / 2) : 0;

@@ -17,11 +17,16 @@ constexpr int group_row(unsigned block, unsigned thread, int G)
     return (int)(block * (unsigned)(ROW_BS / G) + thread / (unsigned)G);
 }
 
-/* Whether rows [r0, r0 + rows) lie in [0, n) with every neighbour at offsets lo
-   to hi (r0 + hi passes 2^31 from 2^30 rows on). */
-constexpr bool rows_inside(int r0, int rows, int lo, int hi, int n)
+/* The rows of [0, n) whose neighbours at offsets lo to hi lie in it too: from
+   `first` on and before `last`. A block of rows from r0 on is inside then when
+   r0 >= first and r0 <= last - rows; r0 + hi would pass 2^31 from 2^30 rows on. */
+struct InnerRows {
+    int first, last;
+    constexpr bool holds(int r0, int rows) const { return r0 >= first && r0 <= last - rows; }
+};
+constexpr InnerRows inner_rows(int n, int lo, int hi)
 {
-    return r0 + lo >= 0 && (long long)r0 + rows + (hi > 0 ? hi : 0) <= n;
+    return InnerRows{lo < 0 ? -lo : 0, n - (hi > 0 ? hi : 0)};
 }
 
 /* Workgroups for n rows of G lanes. A launch takes less than 2^32 lanes, which

@@ -62,7 +62,7 @@ def test_blocks_inside_the_operator(tmp_path):
                 for (long long r0 : {0ll, 256ll, n / 512 * 256, n / 256 * 256 - 256}) {
                     if (hi < lo || r0 < 0 || r0 >= n) continue;
                     const bool want = r0 + lo >= 0 && r0 + 256 + hi <= n && r0 + 256 <= n;
-                    if (rows_inside((int)r0, 256, (int)lo, (int)hi, (int)n) != want)
+                    if (inner_rows((int)n, (int)lo, (int)hi).holds((int)r0, 256) != want)
                         std::printf("n %lld lo %lld hi %lld r0 %lld\\n", n, lo, hi, r0);
                 }
     """)
