@@ -222,6 +222,9 @@ struct DevCsr {
     int pk = 0;
     int poff[PAT_MAX] = {};
     bool cols_analysed = false; /* narrow copy and pattern considered */
+    /* distinct column offsets (PAT_MAX + 1: more) and the smallest and largest,
+       known with row classes and the symmetric stencil */
+    int noff = 0, off_lo = 0, off_hi = 0;
     RowClasses cls;
     int band = -1;              /* largest |column - row|; -1: not determined */
     SymStencil sym;
@@ -255,6 +258,9 @@ void resolve_tiles(Ctx &c, const std::vector<DevCsr *> &mats);
    columns the row kernels do not read, get them only when asked for
    (bcmg_csr_set_columns): at 160^3 they are 61 MB. */
 void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats, bool asked = false);
+/* bytes a column of what make_narrow would keep for an operator whose offsets
+   are known: 0 the pattern, 2 the 16-bit columns, else 4 */
+int narrow_bytes(const DevCsr &A);
 /* find the band and the row classes (at most CLS_MAX forms) of every square
    operator in mats that has rows of at most CLS_ROW entries, their tiles
    resolved (one round trip for the lot) */

@@ -145,10 +145,11 @@ void d2h(bcmg_ctx ctx, void *dst, const void *src, size_t bytes)
     BCMG_HIP(hipStreamSynchronize(ctx->c.stream));
 }
 
-/* the narrow column copies of an operator that is read in another form */
+/* the narrow column copies of an operator that is read in another form, when
+   it will have them */
 void narrow_copies(bcmg_csr A)
 {
-    if (A->A.cls.n == 0 && A->A.sym.k == 0) return;
+    if (A->A.noff == 0 || narrow_bytes(A->A) == 4) return;
     CtxScope scope_(A->ctx);
     make_narrow(A->ctx->c, {&A->A}, true);
 }
@@ -406,10 +407,12 @@ int bcmg_csr_info(bcmg_csr A, int *n, int *nnz)
 int bcmg_csr_column_bytes(bcmg_csr A, int *bytes)
 {
     if (!A || !bytes) return BCMG_EINVAL;
-    API_BEGIN
-    narrow_copies(A);
-    *bytes = A->A.use_pattern() ? 0 : A->A.use_narrow() ? 2 : 4;
-    API_END
+    const DevCsr &M = A->A;
+    *bytes = M.noff > 0 && !M.cols_analysed && M.col_mode == 3 ? narrow_bytes(M)
+             : M.use_pattern()                                 ? 0
+             : M.use_narrow()                                  ? 2
+                                                               : 4;
+    return BCMG_OK;
 }
 
 int bcmg_csr_form(bcmg_csr A, int *form)
@@ -426,7 +429,7 @@ int bcmg_csr_set_columns(bcmg_csr A, int bytes)
 {
     if (!A) return BCMG_EINVAL;
     API_BEGIN
-    narrow_copies(A);
+    if (bytes == 0 || bytes == 2) narrow_copies(A);
     if (bytes == 4) {
         A->A.col_mode = 0;
     } else if (bytes == 2) {

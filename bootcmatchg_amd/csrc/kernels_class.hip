@@ -1067,6 +1067,15 @@ void take_classes(Ctx &c, DevCsr &A, ClassWork *w, const ClassHead &h)
         idx = li.data();
         val = lv.data();
     }
+    std::vector<int> off(idx + R.n, idx + ni);
+    for (int k = 0; k < R.row; k++)
+        for (int q = 0; q < R.n; q++)
+            if (k >= idx[q]) off[(size_t)k * R.n + q] = 0; /* no entry; a diagonal there is */
+    std::sort(off.begin(), off.end());
+    off.erase(std::unique(off.begin(), off.end()), off.end());
+    A.noff = std::min((int)off.size(), PAT_MAX + 1);
+    A.off_lo = off.front();
+    A.off_hi = off.back();
     MaskTable T;
     if (constant_stencil(R, idx, val, T)) {
         k_class_masks<<<(A.n + BS - 1) / BS, BS, 0, c.stream>>>(A.n, T, R.code.get());

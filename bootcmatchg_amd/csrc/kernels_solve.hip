@@ -1038,6 +1038,14 @@ bool offsets_found(const int *info, std::vector<int> &off)
     return info[0] == 0 && !off.empty() && off.size() <= PAT_MAX;
 }
 
+int narrow_bytes(const DevCsr &A)
+{
+    const size_t stream = (size_t)A.nnz * 12;
+    if (A.n != A.m || stream <= PAT_MIN_BYTES) return 4;
+    if (A.noff <= PAT_MAX) return 0;
+    return stream > NT_BYTES && A.off_lo >= -32768 && A.off_hi <= 32767 ? 2 : 4;
+}
+
 void make_narrow(Ctx &c, const std::vector<DevCsr *> &mats, bool asked)
 {
     std::vector<DevCsr *> cand;

@@ -340,7 +340,9 @@ void make_sym(Ctx &c, DevCsr &A, const std::vector<int> &off)
         Y.u.release();
         return;
     }
-    Y.k = k;
+    Y.k = A.noff = k;
+    A.off_lo = off.front();
+    A.off_hi = off.back();
     for (int q = 0; q < k; q++) Y.off[q] = off[q];
 }
 

@@ -102,8 +102,7 @@ int bcmg_csr_info(bcmg_csr A, int *n, int *nnz);
    copies use them when their 32-bit-column stream also exceeds 192 MB), else
    4. The row kernels read the narrowest copy that is kept unless
    bcmg_csr_form tells another form, which goes before them; an operator with
-   such a form gets its copies at the first call of this or of
-   bcmg_csr_set_columns.
+   such a form gets its copies when bcmg_csr_set_columns asks for one.
    Results are the same bits in every form. No counterpart in the reference
    (which always streams 32-bit columns). */
 int bcmg_csr_column_bytes(bcmg_csr A, int *bytes);

@@ -91,7 +91,9 @@ def test_a_stencil_keeps_no_column_copies(ctx):
     assert dA.form == bc.FORM_STENCIL
     assert held <= rounded(8 * nnz) + rounded(4 * nnz) + rounded(4 * (n + 1)) + (34 << 20)
     assert dA.column_bytes == 0
-    assert device_bytes_in_use() - before >= held + 2 * nnz
+    assert device_bytes_in_use() - before == held
+    dA.set_columns(2)
+    assert dA.column_bytes == 2 and device_bytes_in_use() - before >= held + 2 * nnz
     dA.free()
     c.close()
 
@@ -132,4 +134,45 @@ def test_offsets_of_any_number(ctx, count):
     dA.set_columns(4)
     bc.spmv(ctx, dA, x, y)
     assert np.array_equal(bits(got), bits(y.numpy()))
+    dA.free()
+
+
+def eight_of_nine(N):
+    """2D 9-point, every row without one corner, even and odd rows without
+    another one: rows of 8 entries at 9 offsets."""
+    T = sp.diags([np.ones(N - 1), np.ones(N), np.ones(N - 1)], [-1, 0, 1])
+    S = sp.csr_matrix(10.0 * sp.eye(N * N) - sp.kron(T, T))
+    S.sort_indices()
+    r = np.repeat(np.arange(N * N), np.diff(S.indptr))
+    drop = (S.indices - r) == np.where(r % 2 == 0, N + 1, -N - 1)
+    S.data[drop] = 0.0
+    S.eliminate_zeros()
+    return csr(S)
+
+
+@pytest.mark.parametrize("make,bytes_", [(lambda: ops.poisson3d(140), 0),
+                                         (lambda: ops.poisson3d(100), 4),
+                                         (lambda: eight_of_nine(1500), 2),
+                                         (lambda: ops.lognormal3d(120, 4.0, seed=1), 0)])
+def test_column_bytes_before_and_after_the_copies(ctx, make, bytes_):
+    """bcmg_csr_column_bytes says what the copies will be before they are made,
+    and what is not to come is refused."""
+    dA = bc.Csr(ctx, make())
+    assert dA.form != bc.FORM_COLUMNS and dA.column_bytes == bytes_
+    for form in (0, 2):
+        if form < bytes_:
+            with pytest.raises(bc.BcmgError) as e:
+                dA.set_columns(form)
+            assert e.value.code == bc.EUNSUP
+    if bytes_ < 4:
+        dA.set_columns(bytes_)
+        assert dA.form == bc.FORM_COLUMNS and dA.column_bytes == bytes_
+        x = bc.DeviceArray.from_numpy(ctx, ops.uniform_pm1(2, dA.n))
+        y = bc.DeviceArray(ctx, dA.n)
+        bc.spmv(ctx, dA, x, y)
+        got = y.numpy()
+        dA.set_columns(bc.COLUMNS_ANY)
+        assert dA.column_bytes == bytes_
+        bc.spmv(ctx, dA, x, y)
+        assert np.array_equal(bits(got), bits(y.numpy()))
     dA.free()
