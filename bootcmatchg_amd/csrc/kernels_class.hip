@@ -24,8 +24,11 @@
  * product 56.7 and 57.7 us with the one-byte mask and streamed values, 24.0
  * and 20.0 us from the table of forms, 13.5 and 12.1 us as a constant
  * stencil; the L1 sweep 63.3 -> 18.1 us (5.7 TB/s of its 102 MB; FP32
- * 30.9 -> 12.8 us). What bounds them now is the vectors' traffic through
- * L2 and the last-level cache.
+ * 30.9 -> 12.8 us). The FP64 sweep is bound by the vectors' traffic through L2
+ * and the last-level cache. The FP32 one is not (53 MB, 4.1 TB/s): half of the
+ * bytes, but as many instructions (5.1 M vector instructions a launch against
+ * 5.3, the same loads), which take 40 % of its cycles to issue, and its waves
+ * wait on them and on latency.
  */
 #include "kernels_common.h"
 
