@@ -764,6 +764,9 @@ void launch_kcycle_combine_il(hipStream_t s, int n, const double *ks, const VT *
 
 MultiWork &ensure_multi_into(Ctx &c, Boot &B, MultiWork &M, int kmax);
 MultiWork &multi_work(Ctx &c, Boot &B, MultiWork *&holder, int kmax);
+/* whether M holds what the composite's precision asks for (ensure_multi_into
+   makes it so) */
+bool multi_follows(const Boot &B, const MultiWork &M);
 /* device bytes a MultiWork of kmax slots takes on composite B */
 size_t multi_work_bytes(const Boot &B, int kmax);
 

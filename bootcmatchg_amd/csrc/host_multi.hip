@@ -71,6 +71,18 @@ inline int log2_cols(int k)
 
 } // namespace
 
+/* whether the cycle's result reaches FCG in FP32 */
+static bool hands_z32(const Boot &B)
+{
+    return B.prec != BCMG_PREC_FP64 && rows_sequential<double>(*B.A0);
+}
+
+bool multi_follows(const Boot &B, const MultiWork &M)
+{
+    return M.F.z32 == hands_z32(B) &&
+           (B.prec == BCMG_PREC_FP64 ? M.prec64 : M.prec == B.prec);
+}
+
 /* work space for kmax slots (kept and grown across calls) */
 MultiWork &ensure_multi_into(Ctx &c, Boot &B, MultiWork &M, int kmax)
 {
@@ -152,7 +164,7 @@ MultiWork &ensure_multi_into(Ctx &c, Boot &B, MultiWork &M, int kmax)
     } else {
         M.F.kflag = nullptr;
     }
-    M.F.z32 = B.prec != BCMG_PREC_FP64 && rows_sequential<double>(*B.A0);
+    M.F.z32 = hands_z32(B);
     M.F.nc = M.kmax;
     M.F.maxit = B.prm.itnlim;
     if (B.prec != BCMG_PREC_FP64 && M.prec != B.prec) {

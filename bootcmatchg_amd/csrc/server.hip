@@ -270,11 +270,27 @@ struct Server {
         return k;
     }
 
+    /* The work space of the composite's precision, which may have changed since
+       the lane's last launch: its buffers (allocated now, see open_lane) and
+       the type in which the cycle hands z to FCG. */
+    void follow_precision(Lane &L)
+    {
+        if (multi_follows(*L.B, *L.M)) return;
+        BCMG_HIP(hipStreamSynchronize(main.stream));
+        const size_t live0 = pool_live();
+        const OwnBlocks own;
+        ensure_multi_into(L.c, *L.B, *L.M, L.M->kmax);
+        const size_t grown = pool_live() - live0;
+        L.bytes += grown;
+        in_use += grown;
+    }
+
     /* wait, collect, retire (results recorded after the copies of x) */
     int finish(Lane &L)
     {
         SlotEngine &E = *L.E;
         if (E.launched) E.wait();
+        follow_precision(L);
         E.collect();
         bool retired = false;
         for (size_t j = 0; j < E.slots.size(); j++) {
@@ -313,16 +329,6 @@ struct Server {
        right-hand sides are done at admission and retired next step) */
     void admit(Lane &L, std::deque<Request> &q)
     {
-        if (L.B->prec != BCMG_PREC_FP64 && L.M->prec != L.B->prec) {
-            /* reduced-precision buffers are allocated now (see open_lane) */
-            BCMG_HIP(hipStreamSynchronize(main.stream));
-            const size_t live0 = pool_live();
-            const OwnBlocks own;
-            ensure_multi_into(L.c, *L.B, *L.M, L.M->kmax);
-            const size_t grown = pool_live() - live0;
-            L.bytes += grown;
-            in_use += grown;
-        }
         std::vector<int> js;
         std::vector<const double *> bs;
         for (size_t j = 0; j < L.E->slots.size() && !q.empty(); j++) {
