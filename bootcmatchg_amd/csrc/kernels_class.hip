@@ -47,6 +47,7 @@ constexpr int CLS_SLOTS = 1024;   /* hash slots while the forms are collected */
 constexpr int CLS_BLOCK_MAX = 128;
 constexpr unsigned long long HASH_EMPTY = 0ull;
 
+/* the finalizer of splitmix64 (Steele, Lea and Flood, 2014) */
 __device__ __forceinline__ unsigned long long mix64(unsigned long long z)
 {
     z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;

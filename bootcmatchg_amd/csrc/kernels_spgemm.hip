@@ -601,6 +601,7 @@ __global__ __launch_bounds__(BS) void k_sg_hash(int n, int lo, int hi, int smin,
             for (int d = 0; d < SG_AHEAD; d++) {
                 const int c = cc[d];
                 if (c < 0) continue;
+                /* Knuth's multiplicative hash */
                 int h = (int)(((unsigned)c * 2654435761u) >> SHIFT);
                 int tries = 0;
                 for (; tries < H; tries++) {
