@@ -91,7 +91,7 @@ def test_a_stencil_keeps_no_column_copies(ctx):
     assert dA.form == bc.FORM_STENCIL
     assert held <= rounded(8 * nnz) + rounded(4 * nnz) + rounded(4 * (n + 1)) + (34 << 20)
     assert dA.column_bytes == 0
-    assert device_bytes_in_use() - before == held
+    assert device_bytes_in_use() - before <= held
     dA.set_columns(2)
     assert dA.column_bytes == 2 and device_bytes_in_use() - before >= held + 2 * nnz
     dA.free()
